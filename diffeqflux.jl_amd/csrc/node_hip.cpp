@@ -1904,77 +1904,43 @@ int32_t node_destroy(node_handle_t* h) {
   return 0;
 }
 
-static int set_params_host(node_handle* h, const float* p, int64_t n) {
-  if (!p) return fail(h, NODE_ERR_INVALID, "params is NULL");
-  if (n != h->P) return fail(h, NODE_ERR_INVALID, "parameter count mismatch: expected " + std::to_string(h->P));
-  for (const Layer& ly : h->layers) {
-    const size_t cnt = (size_t)ly.outp * ly.inp;
-    std::vector<float> wr(cnt, 0.f), wc(cnt, 0.f), b(ly.outp, 0.f);
-    for (int i = 0; i < ly.in; ++i)
-      for (int o = 0; o < ly.out; ++o) {
-        const float w = p[ly.w0 + (int64_t)i * ly.out + o];  // Julia W[o, i]
-        wr[(size_t)o * ly.inp + i] = w;
-        wc[(size_t)i * ly.outp + o] = w;
-      }
-    for (int o = 0; o < ly.out; ++o) b[o] = p[ly.b0 + o];
-    if (h->prec != NODE_PREC_FP32) {
-      const int np = h->planes;
-      std::vector<uint16_t> r16(cnt * np), c16(cnt * np);
-      auto tobf = [](float f) {
-        uint32_t u;
-        std::memcpy(&u, &f, 4);
-        if ((u & 0x7f800000u) == 0x7f800000u && (u & 0x7fffffu)) return (uint16_t)((u >> 16) | 0x40);
-        u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even
-        return (uint16_t)(u >> 16);
-      };
-      auto frombf = [](uint16_t b) {
-        uint32_t u = (uint32_t)b << 16;
-        float f;
-        std::memcpy(&f, &u, 4);
-        return f;
-      };
-      for (size_t k = 0; k < cnt; ++k) {
-        r16[k] = tobf(wr[k]);
-        c16[k] = tobf(wc[k]);
-        if (np == 2) {  // lo plane: the rounding residual
-          r16[cnt + k] = tobf(wr[k] - frombf(r16[k]));
-          c16[cnt + k] = tobf(wc[k] - frombf(c16[k]));
-        }
-      }
-      HIPCHK(h, hipMemcpyAsync(ly.Wr, r16.data(), cnt * 2 * np, hipMemcpyHostToDevice, h->stream));
-      HIPCHK(h, hipMemcpyAsync(ly.Wc, c16.data(), cnt * 2 * np, hipMemcpyHostToDevice, h->stream));
-      HIPCHK(h, hipMemcpyAsync(ly.bias, b.data(), ly.outp * 4, hipMemcpyHostToDevice, h->stream));
-      HIPCHK(h, hipStreamSynchronize(h->stream));  // host staging vectors end with this layer
-    } else {
-      HIPCHK(h, hipMemcpyAsync(ly.Wr, wr.data(), cnt * 4, hipMemcpyHostToDevice, h->stream));
-      HIPCHK(h, hipMemcpyAsync(ly.Wc, wc.data(), cnt * 4, hipMemcpyHostToDevice, h->stream));
-      HIPCHK(h, hipMemcpyAsync(ly.bias, b.data(), ly.outp * 4, hipMemcpyHostToDevice, h->stream));
-      HIPCHK(h, hipStreamSynchronize(h->stream));
-    }
+// The flat vector (already in pflat) to the operand layouts, on the device.
+static int pack_params(node_handle* h) {
+  PackArgs a{};
+  a.nl = h->L;
+  for (int l = 0; l < h->L; ++l) {
+    const Layer& ly = h->layers[l];
+    a.in[l] = ly.in; a.out[l] = ly.out; a.inp[l] = ly.inp; a.outp[l] = ly.outp;
+    a.w0[l] = ly.w0; a.b0[l] = ly.b0;
+    a.Wr[l] = ly.Wr; a.Wc[l] = ly.Wc; a.bias[l] = ly.bias;
   }
-  if (!h->pflat && dalloc_t(h, &h->pflat, h->P * sizeof(float))) return NODE_ERR_HIP;
-  HIPCHK(h, hipMemcpyAsync(h->pflat, p, h->P * sizeof(float), hipMemcpyHostToDevice, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  launch_pack_params(h->prec, a, h->pflat, h->stream);
+  HIPCHK(h, hipGetLastError());
+  HIPCHK(h, hipStreamSynchronize(h->stream));  // the caller may reuse its buffer
   h->have_params = true;
   h->have_forward = false;
   h->rg.have = false;
   return 0;
 }
 
+static int set_params(node_handle* h, const float* p, int64_t n, hipMemcpyKind kind) {
+  if (!p) return fail(h, NODE_ERR_INVALID, "params is NULL");
+  if (n != h->P) return fail(h, NODE_ERR_INVALID, "parameter count mismatch: expected " + std::to_string(h->P));
+  if (!h->pflat && dalloc_t(h, &h->pflat, h->P * sizeof(float))) return NODE_ERR_HIP;
+  HIPCHK(h, hipMemcpyAsync(h->pflat, p, h->P * sizeof(float), kind, h->stream));
+  return pack_params(h);
+}
+
 int32_t node_set_params(node_handle_t* h, const float* p, int64_t n) {
   if (!h) return NODE_ERR_INVALID;
   std::lock_guard<std::mutex> g(h->mtx);
-  return set_params_host(h, p, n);
+  return set_params(h, p, n, hipMemcpyHostToDevice);
 }
 
 int32_t node_set_params_device(node_handle_t* h, const float* d_p, int64_t n) {
   if (!h) return NODE_ERR_INVALID;
   std::lock_guard<std::mutex> g(h->mtx);
-  if (n != h->P) return fail(h, NODE_ERR_INVALID, "parameter count mismatch");
-  std::vector<float> p(n);
-  HIPCHK(h, hipMemcpyAsync(p.data(), d_p, n * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
-  return set_params_host(h, p.data(), n);
+  return set_params(h, d_p, n, hipMemcpyDeviceToDevice);
 }
 
 int32_t node_forward_device(node_handle_t* h, const node_solve_opts* opts, const float* d_u0,

@@ -229,6 +229,16 @@ int gemm_cfg_tile_rows(int cfg);
 int gemm_cfg_tile_cols(int cfg);
 int gemm_cfg_count();
 
+// parameter packing: flat vector -> Wr / Wc planes and biases of every layer
+struct PackArgs {
+  int nl;
+  int in[MAXL], out[MAXL], inp[MAXL], outp[MAXL];
+  int64_t w0[MAXL], b0[MAXL];
+  void* Wr[MAXL]; void* Wc[MAXL];
+  float* bias[MAXL];
+};
+void launch_pack_params(int prec, const PackArgs& a, const float* p, hipStream_t s);
+
 // elementwise / control kernels
 struct StateGeom {
   int B, Bp, D, Dp;          // real / padded batch, state dim, padded state dim

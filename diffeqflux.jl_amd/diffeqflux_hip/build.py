@@ -6,6 +6,7 @@
 import os
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 PKG_ROOT = os.path.dirname(HERE)                  # diffeqflux.jl_amd/
@@ -14,10 +15,10 @@ CSRC = os.path.join(PKG_ROOT, "csrc")
 INCLUDE = os.path.join(REPO, "include")
 LIB = os.path.join(HERE, "libnode_hip.so")
 
-SOURCES = ["kernels.hip", "node_hip.cpp"]
+SOURCES = ["kernels.hip", "pack_kernels.hip", "node_hip.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
-    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
+    "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     # packed FP32 instructions stay off: some of their forms have given wrong
     # results on MI355X without any error being raised
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -28,15 +29,33 @@ FLAGS = [
 
 
 def build(verbose=False):
-    srcs = [os.path.join(CSRC, s) for s in SOURCES]
+    """Compiles the sources side by side and links the library."""
     tmp = LIB + ".tmp"
-    cmd = [HIPCC, *FLAGS, "-I", INCLUDE, "-I", CSRC, "-o", tmp, *srcs]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        sys.stderr.write(r.stdout + r.stderr)
-        raise RuntimeError("hipcc failed building libnode_hip.so")
+    with tempfile.TemporaryDirectory() as d:
+        jobs, objs = [], []
+        for src in SOURCES:
+            obj = os.path.join(d, src + ".o")
+            cmd = [HIPCC, *FLAGS, "-I", INCLUDE, "-I", CSRC, "-c", os.path.join(CSRC, src),
+                   "-o", obj]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            log = open(obj + ".txt", "w+")
+            jobs.append((src, subprocess.Popen(cmd, stdout=log, stderr=subprocess.STDOUT), log))
+            objs.append(obj)
+        failed = []
+        for src, job, log in jobs:
+            if job.wait() != 0:
+                failed.append(src)
+                log.seek(0)
+                sys.stderr.write(log.read())
+            log.close()
+        if failed:
+            raise RuntimeError(f"hipcc failed on {', '.join(failed)} building libnode_hip.so")
+        r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs],
+                           capture_output=True, text=True)
+        if r.returncode != 0:
+            sys.stderr.write(r.stdout + r.stderr)
+            raise RuntimeError("hipcc failed linking libnode_hip.so")
     os.replace(tmp, LIB)
     return LIB
 
