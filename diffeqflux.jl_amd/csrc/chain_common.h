@@ -1,0 +1,237 @@
+// The Dense chain over a block of rows, shared by the fused step kernels.
+//
+// A workgroup of four or eight waves (NW) owns a block of 16 * NT columns of MFMA tiles
+// (one column per trajectory; a flow's block holds its rows twice, primal and
+// tangent) and runs every layer with the activations in LDS.  Weights are the
+// A operand (16 output features per tile), read straight from L2 into
+// registers: they are packed in fragment order, one 16-byte vector per lane,
+// so a wave reads 1 KB contiguous per fragment and each fragment is read by
+// one wave of the workgroup only.  The activations are the B operand,
+// [row][feature] in LDS, a 16-byte vector per lane as well.  An accumulator
+// lane holds four consecutive features of one row, which is again one vector
+// of the next layer's operand: no transposition between layers.
+#pragma once
+#include "chain.h"
+#include "device_util.h"
+
+namespace nodehip {
+
+// Tsit5 tableau as compile-time constants of the step kernels (the same values
+// as the GEMM epilogues' tables)
+static __device__ const float chA[7][7] = {
+    {0, 0, 0, 0, 0, 0, 0},
+    {0.161, 0, 0, 0, 0, 0, 0},
+    {-0.008480655492356989, 0.335480655492357, 0, 0, 0, 0, 0},
+    {2.897153057105493, -6.359448489975075, 4.3622954328695815, 0, 0, 0, 0},
+    {5.325864828439257, -11.748883564062828, 7.4955393428898365, -0.09249506636175525, 0, 0, 0},
+    {5.86145544294642, -12.92096931784711, 8.159367898576159, -0.071584973281401,
+     -0.028269050394068383, 0, 0},
+    {0.09646076681806523, 0.01, 0.4798896504144996, 1.379008574103742, -3.290069515436081,
+     2.324710524099774, 0}};
+static __device__ const float chBT[7] = {-0.00178001105222577714, -0.0008164344596567469,
+                                         0.007880878010261995,    -0.1447110071732629,
+                                         0.5823571654525552,      -0.45808210592918697,
+                                         0.015151515151515152};
+
+// features per K tile, values per lane and K tile
+template <class PP> struct ChainK { static constexpr int KT = 32, V = 8; };
+template <> struct ChainK<PF32> { static constexpr int KT = 16, V = 4; };
+
+// One MFMA K tile of a 16 x 16 block.  FP32: four 16x16x4 steps, lane l
+// supplying k = 4 (l / 16) + j to step j for both operands.  Split BF16:
+// hi*hi + lo*hi + hi*lo, as the GEMM path orders them.
+template <class PP> struct ChainFrag {
+  u32x4 p[PP::SPLIT ? 2 : 1];
+};
+template <class PP>
+__device__ __forceinline__ void chain_mfma(f32x4v& c, const ChainFrag<PP>& a, const ChainFrag<PP>& b) {
+  if constexpr (sizeof(typename PP::T) == 4) {
+    const f32x4v fa = __builtin_bit_cast(f32x4v, a.p[0]), fb = __builtin_bit_cast(f32x4v, b.p[0]);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa.x, fb.x, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa.y, fb.y, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa.z, fb.z, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa.w, fb.w, c, 0, 0, 0);
+  } else {
+    auto m = [&](const u32x4& x, const u32x4& y) {
+      c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x),
+                                                  __builtin_bit_cast(bf16x8, y), c, 0, 0, 0);
+    };
+    m(a.p[0], b.p[0]);
+    if constexpr (PP::SPLIT) {
+      m(a.p[1], b.p[0]);
+      m(a.p[0], b.p[1]);
+    }
+  }
+}
+
+// The workgroup's LDS.  Buffers are handed on as element offsets into it, not
+// as pointers: through a pointer picked at run time the compiler loses the
+// address space and emits FLAT accesses, which wait for every load in flight.
+__device__ __forceinline__ unsigned char* chain_lds() {
+  extern __shared__ __attribute__((aligned(16))) unsigned char ch_lds[];
+  return ch_lds;
+}
+// A buffer of activations in LDS: [plane][row][pitch] elements at `off`
+template <class PP> struct ChainBuf {
+  int off, pitch, plane;
+  __device__ __forceinline__ typename PP::T* at(int row, int f) const {
+    return (typename PP::T*)chain_lds() + off + row * pitch + f;
+  }
+};
+
+// acc[m][n] += W tiles (first tile t0, MT of them, K tiles [k0, k1)) x columns.
+// The fragments of PF K tiles are in flight (ring in registers, loads
+// unconditional: the index is clamped instead).
+template <class PP, int NT, int MT, int PF>
+__device__ __forceinline__ void chain_mma(f32x4v (&acc)[MT][NT], const void* __restrict__ W, int t0,
+                                          int tlast, int kt, int k0, int k1, const ChainBuf<PP>& in,
+                                          int lane) {
+  constexpr int P = PP::SPLIT ? 2 : 1;
+  const u32x4* w[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int t = t0 + m < tlast ? t0 + m : tlast;
+    w[m] = (const u32x4*)W + (int64_t)t * kt * P * 64 + lane;
+  }
+  const typename PP::T* b = in.at(lane & 15, ChainK<PP>::V * (lane >> 4));
+  ChainFrag<PP> a[PF][MT];
+  auto load = [&](ChainFrag<PP>& f, int m, int k) {
+    k = k < k1 ? k : k1 - 1;
+#pragma unroll
+    for (int q = 0; q < P; ++q) f.p[q] = w[m][(k * P + q) * 64];
+  };
+  auto step = [&](ChainFrag<PP> (&f)[MT], int k, bool refill) {
+    ChainFrag<PP> x[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int q = 0; q < P; ++q)
+        x[n].p[q] = *(const u32x4*)(b + q * in.plane + n * 16 * in.pitch + k * ChainK<PP>::KT);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+      for (int n = 0; n < NT; ++n) chain_mfma<PP>(acc[m][n], f[m], x[n]);
+      if (refill) load(f[m], m, k + PF);
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < PF; ++j)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) load(a[j][m], m, k0 + j);
+  int k = k0;
+  for (; k + PF <= k1; k += PF) {
+#pragma unroll
+    for (int j = 0; j < PF; ++j) step(a[j], k + j, true);
+  }
+#pragma unroll
+  for (int j = 0; j < PF - 1; ++j)
+    if (k + j < k1) step(a[j], k + j, false);
+}
+
+// ring depth: enough K tiles in flight to cover an L2 read (~600 cycles)
+// against MT * NT * (128 FP32 / 48 split) MFMA cycles per tile (a fragment is
+// refilled as soon as its MFMAs are issued)
+template <class PP, int NT, int MT> constexpr int chain_pf() {
+  const int c = MT * NT * (sizeof(typename PP::T) == 4 ? 128 : PP::SPLIT ? 48 : 16);
+  return c >= 1024 ? 1 : c >= 384 ? 2 : c >= 128 ? 4 : 8;
+}
+
+template <class PP, int NT, int MT, class Epi>
+__device__ __forceinline__ void chain_chunk(const void* W, int t0, int tlast, int kt,
+                                            const ChainBuf<PP>& in, int lane, bool sync, Epi&& epi) {
+  f32x4v acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[m][n] = (f32x4v){0.f, 0.f, 0.f, 0.f};
+  chain_mma<PP, NT, MT, chain_pf<PP, NT, MT>()>(acc, W, t0, tlast, kt, 0, kt, in, lane);
+  if (sync) __syncthreads();  // in place: every wave has read the inputs
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+    if (t0 + m <= tlast) epi(t0 + m, acc[m]);
+}
+
+// One wide layer (mt output tiles over the waves): epi(tile, acc[NT]) for
+// every tile.  INPLACE: the outputs may overwrite the inputs (a wave holds all
+// its tiles' accumulators until the barrier; mt <= 4 NW); else chunks of at
+// most four tiles and the output goes to another buffer.  Ends with a barrier.
+template <class PP, int NT, int NW, bool INPLACE, class Epi>
+__device__ __forceinline__ void chain_layer(const void* W, int mt, int kt, const ChainBuf<PP>& in,
+                                            int wave, int lane, Epi&& epi) {
+  const int per = (mt + NW - 1) / NW;
+  int t = wave * per;
+  const int last = (t + per < mt ? t + per : mt) - 1;
+  if constexpr (INPLACE) {
+    // (a wave without tiles computes the last one again and drops it)
+    const int tl = last < mt - 1 ? last : mt - 1;
+    if (per > 2) chain_chunk<PP, NT, 4>(W, t, tl, kt, in, lane, true, epi);
+    else if (per > 1) chain_chunk<PP, NT, 2>(W, t, tl, kt, in, lane, true, epi);
+    else chain_chunk<PP, NT, 1>(W, t, tl, kt, in, lane, true, epi);
+  } else {
+    for (; t + 4 <= last + 1; t += 4) chain_chunk<PP, NT, 4>(W, t, last, kt, in, lane, false, epi);
+    if (t + 2 <= last + 1) { chain_chunk<PP, NT, 2>(W, t, last, kt, in, lane, false, epi); t += 2; }
+    if (t <= last) chain_chunk<PP, NT, 1>(W, t, last, kt, in, lane, false, epi);
+  }
+  __syncthreads();
+}
+
+// A narrow layer (state-sized output, mt <= 4 tiles): the K tiles are split
+// over the waves left over (at most four splits); partial products go to LDS
+// as FP32 [split][row][16 mt + 4], summed by the reader.  Ends with a barrier.
+template <int NW> __host__ __device__ __forceinline__ int chain_splits(int mt) {
+  const int s = NW / mt;
+  return s > 4 ? 4 : s;
+}
+template <class PP, int NT, int NW>
+__device__ __forceinline__ void chain_narrow(const void* W, int mt, int kt, const ChainBuf<PP>& in,
+                                             float* part, int wave, int lane) {
+  const int ks = chain_splits<NW>(mt), t = wave % mt, s = wave / mt;
+  if (s < ks) {
+    f32x4v acc[1][NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[0][n] = (f32x4v){0.f, 0.f, 0.f, 0.f};
+    const int k0 = kt * s / ks, k1 = kt * (s + 1) / ks;
+    if (k0 < k1) chain_mma<PP, NT, 1, 4>(acc, W, t, t, kt, k0, k1, in, lane);
+    const int pd = 16 * mt + 4;
+    float* o = part + s * (16 * NT) * pd + (lane & 15) * pd + 16 * t + 4 * (lane >> 4);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) *(f32x4v*)(o + n * 16 * pd) = acc[0][n];
+  }
+  __syncthreads();
+}
+template <int NW>
+__device__ __forceinline__ float chain_sum(const float* part, int mt, int cols, int row, int c) {
+  const int ks = chain_splits<NW>(mt), pd = 16 * mt + 4;
+  float v = part[row * pd + c];
+  for (int s = 1; s < ks; ++s) v += part[(s * cols + row) * pd + c];
+  return v;
+}
+
+// activation of four values, chosen once
+__device__ __forceinline__ f32x4v act_f4(int a, f32x4v z) {
+  switch (a) {
+    case 1: return (f32x4v){act_f(1, z.x), act_f(1, z.y), act_f(1, z.z), act_f(1, z.w)};
+    case 2: return (f32x4v){act_f(2, z.x), act_f(2, z.y), act_f(2, z.z), act_f(2, z.w)};
+    case 3: return (f32x4v){act_f(3, z.x), act_f(3, z.y), act_f(3, z.z), act_f(3, z.w)};
+    case 4: return (f32x4v){act_f(4, z.x), act_f(4, z.y), act_f(4, z.z), act_f(4, z.w)};
+    default: return z;
+  }
+}
+__device__ __forceinline__ f32x4v act_d4(int a, f32x4v z, f32x4v y) {
+  switch (a) {
+    case 1: return (f32x4v){act_d(1, z.x, y.x), act_d(1, z.y, y.y), act_d(1, z.z, y.z), act_d(1, z.w, y.w)};
+    case 2: return (f32x4v){act_d(2, z.x, y.x), act_d(2, z.y, y.y), act_d(2, z.z, y.z), act_d(2, z.w, y.w)};
+    case 3: return (f32x4v){act_d(3, z.x, y.x), act_d(3, z.y, y.y), act_d(3, z.z, y.z), act_d(3, z.w, y.w)};
+    case 4: return (f32x4v){act_d(4, z.x, y.x), act_d(4, z.y, y.y), act_d(4, z.z, y.z), act_d(4, z.w, y.w)};
+    default: return (f32x4v){1.f, 1.f, 1.f, 1.f};
+  }
+}
+
+// four features of one row into an LDS buffer
+template <class PP>
+__device__ __forceinline__ void chain_put4(const ChainBuf<PP>& o, int row, int f, f32x4v v) {
+  const float x[4] = {v.x, v.y, v.z, v.w};
+  put4<PP>(o.at(row, f), o.plane, x);
+}
+
+}  // namespace nodehip

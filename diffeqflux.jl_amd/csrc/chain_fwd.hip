@@ -1,0 +1,285 @@
+// Fused forward step of the Tsit5 solve: one launch per step attempt.
+//
+// Within an attempt a trajectory's stages depend on no other trajectory (the
+// shared step size couples them only through the error norm), so a workgroup
+// takes a block of rows through all six stages: stage input, the Dense chain
+// (chain_common.h), k_s, the embedded error's partial sum.  Bound by the MFMA
+// chain of the wide layers (FP32) or by the weights' way from L2 (split BF16);
+// it replaces eight kernels per right-hand side whose launches and drains cost
+// more than their work at these sizes.
+#include "chain_common.h"
+
+namespace nodehip {
+
+int chain_rows(int nt, bool cnf) { return cnf ? 8 * nt : 16 * nt; }
+
+// Pending saves of the last accepted step for the block's entries
+template <int THREADS>
+__device__ __forceinline__ void chain_saves(const ChainFwdArgs& a, int64_t e0, int n) {
+  const Ctl* ctl = a.ctl;
+  const int64_t lo = ctl->save_lo, hi = ctl->save_hi;
+  if (lo >= hi) return;
+  const float* ecur = a.tape + tape_slot(ctl, ctl->n) * a.ent;
+  const float* es = a.tape + tape_slot(ctl, ctl->save_step) * a.ent;
+  const double t = ctl->t, tprev = ctl->tprev, dts = ctl->dt_step;
+  const int64_t nreal = (int64_t)a.m.B * a.m.D;
+  for (int64_t si = lo; si < hi; ++si) {
+    const double ts = a.save_times[si];
+    float w[7];
+    const bool exact = ts == t;
+    if (!exact) interp_weights((ts - tprev) / dts, w);
+    float* o = a.out + si * nreal;
+    for (int i = threadIdx.x; i < n; i += THREADS) {
+      const int64_t idx = e0 + i;
+      if (idx >= nreal) break;
+      float v;
+      if (exact) v = ecur[idx];
+      else {
+        float sm = 0.f;
+#pragma unroll
+        for (int j = 0; j < 7; ++j) sm += w[j] * es[(1 + j) * a.sv + idx];
+        v = es[idx] + (float)dts * sm;
+      }
+      o[idx] = v;
+    }
+  }
+}
+
+template <class PP, int NT, int NW, bool CNF>
+__global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
+  using T = typename PP::T;
+  constexpr int CH_THREADS = 64 * NW;
+  constexpr int COLS = 16 * NT, R = CNF ? 8 * NT : COLS;
+  constexpr int NE = R * (CNF ? 32 : 64) / CH_THREADS;  // state entries per thread (D <= 64, flow 32)
+  constexpr int P = PP::SPLIT ? 2 : 1;
+  constexpr bool INPLACE = CNF && NT == 4;
+  const ChainModel& m = a.m;
+  const Ctl* ctl = a.ctl;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int D = m.D, L = m.L, mode = a.mode;
+  const int row0 = blockIdx.x * R;
+  const int64_t e0 = (int64_t)row0 * D;
+  const int ne = R * D;                       // entries of the block
+  if (mode == SM_STEP) {
+    chain_saves<CH_THREADS>(a, e0, ne);
+    if (ctl->done) return;
+  }
+  const int plane = COLS * m.pitch;
+  const int other = INPLACE ? 0 : P * plane;  // offset of the second buffer
+  const ChainBuf<PP> in0{0, m.pitch, plane};
+  float* part = (float*)(chain_lds() + (INPLACE ? 1 : 2) * P * plane * sizeof(T));
+
+  const int64_t n = mode == SM_STEP ? ctl->n : 0;
+  float* ent = a.tape + tape_slot(ctl, n) * a.ent;
+  float* nxt = a.tape + tape_slot(ctl, n + 1) * a.ent;
+  const float dt = (float)ctl->dt;
+  const float atol = (float)ctl->abstol, rtol = (float)ctl->reltol;
+
+  // this thread's state entries: row and column in the block
+  int row[NE], col[NE];
+  float u[NE], k[7][NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int i = tid + e * CH_THREADS;
+    row[e] = i / D;
+    col[e] = i - row[e] * D;
+    u[e] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 7; ++s) k[s][e] = 0.f;
+    if (i < ne) {
+      u[e] = ent[e0 + i];
+      if (mode == SM_STEP || mode == SM_INIT_F1) k[0][e] = ent[a.sv + e0 + i];
+    }
+  }
+  double sum = 0.0, flag = 0.0;
+  const int s0 = mode == SM_STEP ? 1 : 0, s1 = mode == SM_STEP ? 7 : 1;
+  float un[NE];
+  for (int s = s0; s < s1; ++s) {
+    // stage input
+    const double ts = mode == SM_STEP ? ctl->t + dC[s] * ctl->dt
+                      : mode == SM_INIT_F1 ? ctl->t + ctl->tdir * ctl->dt0 : ctl->t;
+    const int kin = m.ktf[0] * ChainK<PP>::KT;
+    for (int i = tid; i < COLS * (kin - m.dm); i += CH_THREADS) {
+      // columns past the model's own: zeros (the time column is written below)
+      const int r = i / (kin - m.dm), c = m.dm + i % (kin - m.dm);
+      const bool tc = CNF && m.tcat && c == m.dm && r < R;
+      put<PP>(in0.at(r, c), plane, tc ? (float)ts : 0.f);
+    }
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      if (tid + e * CH_THREADS >= ne) continue;
+      float v = u[e];
+      if (mode == SM_STEP) {
+        float sm = 0.f;
+#pragma unroll
+        for (int j = 5; j >= 0; --j) sm += chA[s][j] * k[j][e];
+        v = u[e] + dt * sm;
+        un[e] = v;
+      } else if (mode == SM_INIT_F1) {
+        v = u[e] + (float)(ctl->tdir * ctl->dt0) * k[0][e];
+      }
+      if (col[e] < m.dm) {
+        put<PP>(in0.at(row[e], col[e]), plane, map_f(m.map, v));
+        if constexpr (CNF) {
+          const int g = row0 + row[e];
+          put<PP>(in0.at(R + row[e], col[e]), plane,
+                  g < m.B ? a.probe[(int64_t)g * m.dm + col[e]] : 0.f);
+        }
+      }
+    }
+    if (mode == SM_STEP && s == 6) {
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+        if (tid + e * CH_THREADS < ne) nxt[e0 + tid + e * CH_THREADS] = un[e];
+    }
+    __syncthreads();
+    int cur = 0;
+    for (int l = 0; l < L - 1; ++l) {
+      const ChainBuf<PP> in{cur, m.pitch, plane}, o{other - cur, m.pitch, plane};
+      const float* bias = m.bias[l];
+      const int act = m.act[l];
+      auto epi = [&](int t, f32x4v (&acc)[NT]) {
+        const int f = 16 * t + 4 * (lane >> 4);
+        const f32x4v bv = *(const f32x4v*)(bias + f);
+#pragma unroll
+        for (int q = 0; q < (CNF ? NT / 2 : NT); ++q) {
+          const f32x4v z = acc[q] + bv, y = act_f4(act, z);
+          chain_put4<PP>(o, 16 * q + (lane & 15), f, y);
+          if constexpr (CNF)
+            chain_put4<PP>(o, R + 16 * q + (lane & 15), f, acc[q + NT / 2] * act_d4(act, z, y));
+        }
+      };
+      chain_layer<PP, NT, NW, INPLACE>(m.Wf[l], m.mtf[l], m.ktf[l], in, wave, lane, epi);
+      cur = other - cur;
+    }
+    const int ll = L - 1, mt = m.mtf[ll];
+    chain_narrow<PP, NT, NW>(m.Wf[ll], mt, m.ktf[ll], ChainBuf<PP>{cur, m.pitch, plane}, part, wave, lane);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      const int i = tid + e * CH_THREADS;
+      if (i >= ne) continue;
+      float kv;
+      if (!CNF || col[e] < m.dm) {
+        kv = act_f(m.act[ll], chain_sum<NW>(part, mt, COLS, row[e], col[e]) + m.bias[ll][col[e]]);
+      } else {  // log p: minus the probe's directional derivative of f
+        kv = 0.f;
+        const int g = row0 + row[e];
+        if (g < m.B)
+          for (int c = 0; c < m.dm; ++c)
+            kv -= a.probe[(int64_t)g * m.dm + c] * chain_sum<NW>(part, mt, COLS, R + row[e], c);
+      }
+      const int64_t idx = e0 + i;
+      const bool live = row0 + row[e] < m.B;
+      if (mode == SM_STEP) {
+        ent[(1 + s) * a.sv + idx] = kv;
+        if (s == 6) {
+          nxt[a.sv + idx] = kv;  // FSAL
+          float ut = chBT[6] * kv;
+#pragma unroll
+          for (int j = 0; j < 6; ++j) ut += chBT[j] * k[j][e];
+          ut *= dt;
+          const float sk = atol + fmaxf(fabsf(u[e]), fabsf(un[e])) * rtol;
+          if (live) {
+            const double q = (double)(ut / sk);
+            sum += q * q;
+            if (isnan(un[e])) flag = 1.0;
+          }
+        }
+#pragma unroll
+        for (int j = 1; j < 6; ++j) k[j][e] = j == s ? kv : k[j][e];
+      } else if (mode == SM_PLAIN) {
+        a.plain[idx] = kv;
+      } else {
+        const float sk = atol + fabsf(u[e]) * rtol;
+        const float d = mode == SM_INIT_F0 ? kv : kv - k[0][e];
+        if (mode == SM_INIT_F0) ent[a.sv + idx] = kv;
+        if (live) {
+          const double q = (double)(d / sk);
+          sum += q * q;
+          if (mode == SM_INIT_F1 && d != 0.f) flag = 1.0;
+        }
+      }
+    }
+  }
+  if (a.part) block_reduce_store(sum, flag, a.part, blockIdx.x);
+}
+
+static size_t chain_elt(int prec) { return prec == 0 ? 4 : prec == 1 ? 2 : 4; }  // bytes of all planes
+
+size_t chain_fwd_lds(int prec, const ChainModel& m, int nt) {
+  const bool inplace = nt == 4;
+  const int cols = 16 * nt, mt = m.mtf[m.L - 1];
+  const int ks = m.nw == 8 ? chain_splits<8>(mt) : chain_splits<4>(mt);
+  const size_t part = (size_t)ks * cols * (16 * mt + 4) * 4;
+  return (size_t)(inplace ? 1 : 2) * cols * m.pitch * chain_elt(prec) + part;
+}
+
+void launch_chain_fwd(int prec, int nt, bool cnf, const ChainFwdArgs& a, int grid, hipStream_t s) {
+  const size_t lds = chain_fwd_lds(prec, a.m, nt);
+  const int nw = a.m.nw;
+  auto go = [&](auto kern) {
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), lds, s, a);
+  };
+  if (prec == 0) {
+    if (cnf && nw == 8) go(k_chain_fwd<PF32, 2, 8, true>);
+    else if (cnf) go(k_chain_fwd<PF32, 2, 4, true>);
+    else if (nw == 8) go(k_chain_fwd<PF32, 1, 8, false>);
+    else go(k_chain_fwd<PF32, 1, 4, false>);
+  } else if (cnf) {
+    if (nt == 4) go(k_chain_fwd<PBF16X3, 4, 8, true>);
+    else if (nw == 8) go(k_chain_fwd<PBF16X3, 2, 8, true>);
+    else go(k_chain_fwd<PBF16X3, 2, 4, true>);
+  } else {
+    if (nt == 2) go(k_chain_fwd<PBF16X3, 2, 8, false>);
+    else if (nw == 8) go(k_chain_fwd<PBF16X3, 1, 8, false>);
+    else go(k_chain_fwd<PBF16X3, 1, 4, false>);
+  }
+}
+
+// Weights in fragment order.  One thread per lane of a fragment: V (4 FP32 or
+// 8 BF16) consecutive K values of one output feature, zero past the layer's
+// own size.  The forward fragments read the flat vector (W[o, i] at
+// i * out + o) along o, the backward ones V consecutive values of a row.
+template <class PP>
+__global__ void __launch_bounds__(256) k_pack_chain(ChainPack a, const float* __restrict__ p) {
+  using T = typename PP::T;
+  constexpr int V = ChainK<PP>::V, KT = ChainK<PP>::KT, P = PP::SPLIT ? 2 : 1;
+  const int l = blockIdx.y >> 1;
+  const bool bwd = blockIdx.y & 1;
+  T* W = (T*)(bwd ? a.Wb[l] : a.Wf[l]);
+  if (!W) return;
+  const int mt = bwd ? a.mtb[l] : a.mtf[l], kt = bwd ? a.ktb[l] : a.ktf[l];
+  const int in = a.in[l], out = a.out[l];
+  const float* w = p + a.w0[l];
+  const int64_t nfl = (int64_t)mt * kt * 64;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nfl;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    const int lane = (int)(i & 63);
+    const int64_t f = i >> 6;
+    const int t = (int)(f / kt), k = (int)(f % kt);
+    const int mrow = 16 * t + (lane & 15), k0 = k * KT + V * (lane >> 4);
+    T* d = W + (f * P * 64 + lane) * V;
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      const int kk = k0 + j;
+      const int o = bwd ? kk : mrow, ii = bwd ? mrow : kk;
+      const float v = o < out && ii < in ? w[(int64_t)ii * out + o] : 0.f;
+      put<PP>(d + j, 64 * V, v);
+    }
+  }
+}
+
+void launch_pack_chain(int prec, const ChainPack& a, const float* p, hipStream_t s) {
+  int64_t most = 1;
+  for (int l = 0; l < a.nl; ++l) {
+    const int64_t f = (int64_t)a.mtf[l] * a.ktf[l], b = (int64_t)a.mtb[l] * a.ktb[l];
+    most = f > most ? f : most;
+    most = b > most ? b : most;
+  }
+  const int grid = (int)((most + 3) / 4 < 1024 ? (most + 3) / 4 : 1024);
+  if (prec == 0) hipLaunchKernelGGL(k_pack_chain<PF32>, dim3(grid, 2 * a.nl), dim3(256), 0, s, a, p);
+  else hipLaunchKernelGGL(k_pack_chain<PBF16X3>, dim3(grid, 2 * a.nl), dim3(256), 0, s, a, p);
+}
+
+}  // namespace nodehip

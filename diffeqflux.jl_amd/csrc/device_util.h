@@ -29,6 +29,14 @@ static __device__ const double dRI[6][3] = {
     {-27.896526289197286, 65.09189467479366, -34.8706578614966},
     {1.5, -4.0, 2.5}};
 
+// dense-output weights at theta of a step: state = u + dt sum_i w[i] k_{i+1}
+__device__ __forceinline__ void interp_weights(double th, float* w) {
+  const double th2 = th * th;
+  w[0] = (float)(th * (dR1[0] + th * (dR1[1] + th * (dR1[2] + th * dR1[3]))));
+#pragma unroll
+  for (int i = 0; i < 6; ++i) w[i + 1] = (float)(th2 * (dRI[i][0] + th * (dRI[i][1] + th * dRI[i][2])));
+}
+
 // ---------------------------------------------------------------- helpers
 __device__ __forceinline__ bool gate_ok(const Ctl* c, int gate) {
   if (gate == GATE_ALWAYS) return true;

@@ -1693,12 +1693,6 @@ __device__ double block_sum_parts(const double* part, int n, double* flag_out) {
   return out;
 }
 
-__device__ __forceinline__ void interp_weights(double th, float* w) {
-  const double th2 = th * th;
-  w[0] = (float)(th * (dR1[0] + th * (dR1[1] + th * (dR1[2] + th * dR1[3]))));
-  for (int i = 0; i < 6; ++i) w[i + 1] = (float)(th2 * (dRI[i][0] + th * (dRI[i][1] + th * dRI[i][2])));
-}
-
 // SciMLBase sol(tau) on the forward record: exact stored state at a step
 // time, else the interpolant of the bracketing step with dt = t_i - t_{i-1}
 __device__ void set_interp(Ctl* c, int slot, double tau, const double* ft) {

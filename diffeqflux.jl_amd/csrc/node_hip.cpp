@@ -15,6 +15,7 @@
 #include <string>
 #include <vector>
 
+#include "chain.h"
 #include "node_internal.h"
 
 using namespace nodehip;
@@ -174,7 +175,8 @@ struct node_handle {
   // captured step-attempt graphs (re-captured when a captured pointer changes)
   bool use_graphs = true;
   hipGraphExec_t fwd_graph = nullptr, adj_graph = nullptr;
-  const void* fwd_graph_sig[3] = {nullptr, nullptr, nullptr};  // tape, save times, outputs
+  // tape, save times, outputs, fused steps
+  const void* fwd_graph_sig[4] = {nullptr, nullptr, nullptr, nullptr};
   // tape, save times, cotangents, saved states (BacksolveAdjoint checkpoints)
   const void* adj_graph_sig[4] = {nullptr, nullptr, nullptr, nullptr};
   int graph_attempts = 4;
@@ -212,6 +214,11 @@ struct node_handle {
     int* order = nullptr; int64_t order_cap = 0;
     double* part = nullptr; int64_t part_cap = 0;
   } ra;
+
+  // fused step kernels: model in fragment order, column tiles per row block
+  // (0: the forward runs on the GEMM path)
+  ChainModel chain{};
+  int chain_nt = 0;
 
   // profiling (node_prof_enable)
   uint64_t prof_mask = 0;
@@ -662,6 +669,98 @@ void vjp_eval(node_handle* h, int stage, int mode, int gate, int wflags, float c
   launch_bwd_last(h, stage, mode, gate, part, plain_out);
 }
 
+// ---------------------------------------------------------------- fused steps
+// Blocks of 16 rows (a flow's 16 columns of primal and tangent rows each) are
+// doubled when they would outnumber the CUs: the weights then pass L2 once
+// for twice the rows.
+int chain_tiles(const node_handle* h) {
+  const bool two = h->prec == NODE_PREC_BF16X3 && h->B > 16 * 256;
+  return h->cnf ? (two ? 4 : 2) : (two ? 2 : 1);
+}
+
+// Whether the forward runs as fused steps, and its model description (without
+// the weights' addresses).  Widths are bounded by LDS (the activations of a
+// row block) and by the in-place form of the four-tile block (32 tiles of
+// outputs).
+bool chain_plan(node_handle* h, ChainModel& m) {
+  m = ChainModel{};
+  if (h->prec == NODE_PREC_BF16 || h->cnf_reg || h->cnf_exact) return false;
+  if (h->D > (h->cnf ? 32 : 64)) return false;
+  const int KT = h->prec == NODE_PREC_FP32 ? 16 : 32;
+  m.L = h->L; m.map = h->desc.input_map; m.D = h->D; m.B = h->B;
+  m.dm = h->cnf ? h->cnf_dm : h->D;
+  m.tcat = h->desc.input_map == NODE_MAP_CNF_TIME ? 1 : 0;
+  int wide = 0;
+  for (int l = 0; l < h->L; ++l) {
+    const Layer& ly = h->layers[l];
+    m.in[l] = ly.in; m.out[l] = ly.out; m.act[l] = ly.act;
+    // hidden widths are padded to whole K tiles of the layer that reads them
+    m.ktf[l] = (ly.in + KT - 1) / KT;
+    m.ktb[l] = (ly.out + KT - 1) / KT;
+    m.mtf[l] = l < h->L - 1 ? m.ktb[l] * KT / 16 : (ly.out + 15) / 16;
+    m.mtb[l] = l > 0 ? m.ktf[l] * KT / 16 : (ly.in + 15) / 16;
+    wide = std::max(wide, std::max(m.ktf[l], m.ktb[l]) * KT);
+  }
+  if (wide > 1024 || (h->cnf && wide > 512)) return false;
+  // Past ~700k weights a block's way through them (2.2M: ~100 us per
+  // right-hand side, whatever the batch) costs what the GEMM path does at
+  // 4096 rows (split BF16) and twice that at 1000 (FP32: 116 against ~57).
+  int64_t weights = 0;
+  for (int l = 0; l < h->L; ++l) weights += (int64_t)h->layers[l].in * h->layers[l].out;
+  if (weights > 700000) return false;
+  m.pitch = wide + (h->prec == NODE_PREC_FP32 ? 4 : 8);
+  // two waves per SIMD where every wave of them has a tile of the wide layers
+  // (the four-tile in-place block needs them: four tiles per wave at 512)
+  m.nw = wide >= 128 || chain_tiles(h) > (h->cnf ? 2 : 1) ? 8 : 4;
+  return true;
+}
+
+int chain_alloc(node_handle* h) {
+  ChainModel m;
+  if (!chain_plan(h, m)) return 0;
+  int nt = chain_tiles(h);
+  if (chain_fwd_lds(h->prec, m, nt) > 160 * 1024) nt = h->cnf ? 2 : 1;
+  if (chain_fwd_lds(h->prec, m, nt) > 160 * 1024) return 0;
+  if ((h->B + chain_rows(nt, h->cnf) - 1) / chain_rows(nt, h->cnf) > MAX_PART) return 0;
+  const int V = h->prec == NODE_PREC_FP32 ? 4 : 8;
+  for (int l = 0; l < h->L; ++l) {
+    void *f = nullptr, *b = nullptr;
+    const size_t lane = (size_t)64 * V * h->esz * h->planes;
+    if (int rc = dalloc(h, &f, lane * m.mtf[l] * m.ktf[l])) return rc;
+    if (int rc = dalloc(h, &b, lane * m.mtb[l] * m.ktb[l])) return rc;
+    m.Wf[l] = f; m.Wb[l] = b;
+    m.bias[l] = h->layers[l].bias;
+  }
+  h->chain = m;
+  h->chain_nt = nt;
+  return 0;
+}
+
+// Whether this solve runs as fused steps.  Tape-budgeted solves stay on the
+// GEMM path: a checkpointed one starts its re-solves from the last, clipped
+// step of the interval before, so a difference in rounding moves the number
+// of tape entries that an interval needs, and with it what fits a budget.
+bool chain_on(const node_handle* h) { return h->chain_nt > 0 && h->tape_budget == 0; }
+
+int chain_grid(const node_handle* h) {
+  const int r = chain_rows(h->chain_nt, h->cnf);
+  return (h->B + r - 1) / r;
+}
+
+// One fused step attempt (SM_STEP), or one right-hand side of the initial-dt
+// heuristic, into the tape.
+void chain_forward(node_handle* h, int mode, double* part) {
+  ChainFwdArgs a{};
+  a.m = h->chain;
+  a.tape = h->tape;
+  a.sv = (int64_t)h->Bp * h->D;
+  a.ent = 8 * a.sv;
+  a.probe = h->probe;
+  a.save_times = h->save_times; a.out = h->out_dev;
+  a.part = part; a.ctl = h->ctl; a.mode = mode;
+  launch_chain_fwd(h->prec, h->chain_nt, h->cnf, a, chain_grid(h), h->stream);
+}
+
 int ensure_tape(node_handle* h, int64_t entries) {
   if (entries <= h->tape_cap) return 0;
   int64_t cap = std::max<int64_t>(entries, std::max<int64_t>(16, 2 * h->tape_cap));
@@ -982,20 +1081,30 @@ int fwd_run(node_handle* h, const node_solve_opts& o, const float* d_u0, int64_t
   const int nb = state_blocks(sg);
   const int64_t xpl = (int64_t)h->Bp * h->layers[0].inp;  // X0 plane stride
   launch_fwd_init(sg, d_u0, h->tape, h->X0, xpl, h->ctl, p0, nb, h->stream);
-  rhs_eval(h, 0, SM_INIT_F0, GATE_ALWAYS, px);
-  const int nx = rhs_last_tiles(h);
+  const bool fused = chain_on(h);
+  if (fused) chain_forward(h, SM_INIT_F0, px);
+  else rhs_eval(h, 0, SM_INIT_F0, GATE_ALWAYS, px);
+  const int nx = fused ? chain_grid(h) : rhs_last_tiles(h);
   const double nel = (double)h->B * h->D;
   if (!c.has_dt_) {
     launch_initdt_a(h->ctl, p0, nb, px, nx, nullptr, 0, nel, h->stream);
-    launch_fwd_initdt_prep(sg, h->tape, h->X0, xpl, h->ctl, h->stream);
-    rhs_eval(h, 0, SM_INIT_F1, GATE_ALWAYS, px);
+    if (fused) {
+      chain_forward(h, SM_INIT_F1, px);
+    } else {
+      launch_fwd_initdt_prep(sg, h->tape, h->X0, xpl, h->ctl, h->stream);
+      rhs_eval(h, 0, SM_INIT_F1, GATE_ALWAYS, px);
+    }
   }
   launch_initdt_b(h->ctl, px, nx, nullptr, 0, nel, h->save_times, 0, h->fwd_times, h->stream);
   HIPCHK(h, hipGetLastError());
 
   auto attempt = [&]() {
-    launch_fwd_step_begin(sg, h->tape, h->X0, xpl, h->save_times, h->out_dev, h->ctl, h->stream);
-    for (int s = 1; s < 7; ++s) rhs_eval(h, s, SM_STEP, GATE_ACTIVE, px);
+    if (fused) {
+      chain_forward(h, SM_STEP, px);
+    } else {
+      launch_fwd_step_begin(sg, h->tape, h->X0, xpl, h->save_times, h->out_dev, h->ctl, h->stream);
+      for (int s = 1; s < 7; ++s) rhs_eval(h, s, SM_STEP, GATE_ACTIVE, px);
+    }
     launch_fwd_controller(h->ctl, px, nx, h->save_times, h->fwd_times, nel, h->stream);
   };
   const bool graphs = h->use_graphs && h->prof_mask == 0;
@@ -1024,7 +1133,7 @@ int fwd_run(node_handle* h, const node_solve_opts& o, const float* d_u0, int64_t
     if (ring == 0)
       if (int rc = ensure_tape(h, h->hctl->n + chunk + 2)) return rc;
     if (!eager) {
-      const void* sig[3] = {h->tape, h->save_times, h->out_dev};
+      const void* sig[4] = {h->tape, h->save_times, h->out_dev, fused ? h : nullptr};
       if (h->fwd_graph && std::memcmp(sig, h->fwd_graph_sig, sizeof(sig)) != 0) {
         (void)hipGraphExecDestroy(h->fwd_graph);
         h->fwd_graph = nullptr;
@@ -1872,6 +1981,7 @@ int32_t node_create(const node_desc* desc, node_handle_t** out) {
     if (!rc) rc = dalloc(h, &e, hbt);
     h->H.push_back(a); h->HT.push_back(b); h->S.push_back(c); h->Dl.push_back(d); h->DlT.push_back(e);
   }
+  if (!rc) rc = chain_alloc(h);
   if (!rc) rc = dalloc_t(h, &h->ctl, sizeof(Ctl));
   if (!rc) rc = dalloc_t(h, &h->part, 4 * SEC * sizeof(double));
   if (!rc) rc = dalloc_t(h, &h->scratch, (size_t)h->Bp * h->D * sizeof(float));
@@ -1915,6 +2025,18 @@ static int pack_params(node_handle* h) {
     a.Wr[l] = ly.Wr; a.Wc[l] = ly.Wc; a.bias[l] = ly.bias;
   }
   launch_pack_params(h->prec, a, h->pflat, h->stream);
+  if (h->chain_nt > 0) {
+    ChainPack c{};
+    c.nl = h->L;
+    for (int l = 0; l < h->L; ++l) {
+      const ChainModel& m = h->chain;
+      c.in[l] = m.in[l]; c.out[l] = m.out[l];
+      c.mtf[l] = m.mtf[l]; c.ktf[l] = m.ktf[l]; c.mtb[l] = m.mtb[l]; c.ktb[l] = m.ktb[l];
+      c.w0[l] = h->layers[l].w0;
+      c.Wf[l] = (void*)m.Wf[l]; c.Wb[l] = (void*)m.Wb[l];
+    }
+    launch_pack_chain(h->prec, c, h->pflat, h->stream);
+  }
   HIPCHK(h, hipGetLastError());
   HIPCHK(h, hipStreamSynchronize(h->stream));  // the caller may reuse its buffer
   h->have_params = true;

@@ -15,7 +15,8 @@ CSRC = os.path.join(PKG_ROOT, "csrc")
 INCLUDE = os.path.join(REPO, "include")
 LIB = os.path.join(HERE, "libnode_hip.so")
 
-SOURCES = ["kernels.hip", "pack_kernels.hip", "node_hip.cpp"]
+SOURCES = ["kernels.hip", "pack_kernels.hip", "chain_fwd.hip",
+           "node_hip.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
