@@ -33,6 +33,58 @@ struct ChainFwdArgs {
   const Ctl* ctl;
   int mode;
 };
+// Operands of the weight gradients, kept per stage by the fused adjoint step:
+// for layer l its inputs h ([row][inp]) and output gradients d ([row][outp]),
+// T x planes (plane stride rows * width), rows = blocks * 16 nt (a flow's block
+// holds its primal rows first, then its tangent rows); widths padded to 64.
+// Slot of stage s: 1..5 -> s + 1; stages 0 and 6 share slots 0 and 1 (the last
+// stage of an accepted step is the next one's first: FSAL).
+struct ChainOps {
+  void* base;
+  int64_t slot;                // bytes per stage slot
+  int64_t h[MAXL], d[MAXL];    // byte offsets in a slot
+  int w[MAXL + 1];             // inp of layer l; w[L] = outp of the last
+  int64_t rows;
+};
+struct ChainAdjArgs {
+  ChainModel m;
+  ChainOps ops;
+  const float* tape; int64_t ent, sv;
+  float* lam; float* lam_new; float* kl;   // kl: slots 0 and 6 of 8 stage slots are used
+  const float* dLdout;
+  const float* probe;
+  float* slope; float* curve;  // act' (and act'' adot, flow) of the hidden layers, [l][rows][wmax]
+  int wmax;
+  // BacksolveAdjoint: u integrated with lambda (ubs != nullptr)
+  float* ubs; float* ubs_new; float* ku; const float* fsaved; int ckpt;
+  double* part;
+  const Ctl* ctl;
+  int mode;
+};
+struct ChainWgradArgs {
+  ChainModel m;
+  ChainOps ops;
+  int64_t rblk;                // rows of a block
+  int64_t rprim;               // of which primal (bias gradients sum these only)
+  int ntile;                   // 64 x 64 (FP32) or 128 x 128 (split) tiles of all layers
+  int tl[MAXL], tw[MAXL];      // first tile of a layer, its tiles along the outputs
+  int chunks; int64_t crows;   // row ranges and rows per range
+  float* part;                 // [chunk][2][ntile][65 x 64 or 129 x 128]
+  const Ctl* ctl;
+  int mode;
+};
+struct ChainMuArgs {
+  ChainWgradArgs w;
+  int64_t w0[MAXL], b0[MAXL], P;
+  int edge;                    // tile edge (64 / 128)
+  double* mu; float* g0;       // two mu buffers; gradient at the initial time
+  double* part;
+};
+size_t chain_adj_lds(int prec, const ChainModel& m, int nt);
+void launch_chain_adj(int prec, int nt, bool cnf, const ChainAdjArgs& a, int grid, hipStream_t s);
+void launch_chain_wgrad(int prec, const ChainWgradArgs& a, hipStream_t s);
+void launch_chain_mu(const ChainMuArgs& a, int nblk, hipStream_t s);
+
 // nt: 16-column MFMA tiles per block (rows per block: 16 nt, a flow 8 nt)
 int chain_rows(int nt, bool cnf);
 size_t chain_fwd_lds(int prec, const ChainModel& m, int nt);

@@ -1,0 +1,728 @@
+// Fused adjoint step: three launches per step attempt besides the controller.
+//
+// k_chain_adj takes a block of rows through all stages of the adjoint's Tsit5
+// step (step begin, u at the stage time, hidden recompute, data gradients,
+// k^lambda): lambda's rows are independent within an attempt, as the forward's
+// are.  It leaves each stage's layer inputs and output gradients behind, and
+// k_chain_wgrad forms from them the two sums over stages that the parameter
+// state needs (sum_s b_s G_s and sum_s bt_s G_s), one pass over the batch with
+// both sums in registers; k_chain_mu adds the row ranges' partial sums, forms
+// the speculative mu and its error norm.  Per-stage launches of one kernel per
+// GEMM, stage, fold and norm (12 per VJP) spent most of their time in launches,
+// drains and partial sums through memory.
+#include "chain_common.h"
+
+namespace nodehip {
+
+template <class PP, int NT, int NW, bool CNF>
+__global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
+  using T = typename PP::T;
+  constexpr int THREADS = 64 * NW;
+  constexpr int COLS = 16 * NT, R = CNF ? 8 * NT : COLS;
+  constexpr int NE = R * (CNF ? 32 : 64) / THREADS;
+  constexpr int P = PP::SPLIT ? 2 : 1;
+  constexpr bool INPLACE = CNF && NT == 4;
+  constexpr int NP = CNF ? NT / 2 : NT;        // column tiles of primal rows
+  const ChainModel& m = a.m;
+  const Ctl* ctl = a.ctl;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int D = m.D, L = m.L, mode = a.mode;
+  const int row0 = blockIdx.x * R;             // first trajectory
+  const int64_t orow0 = (int64_t)blockIdx.x * COLS;  // first operand row
+  const int64_t e0 = (int64_t)row0 * D;
+  const int ne = R * D;
+  const int64_t nreal = (int64_t)m.B * D;
+  const bool bs = !CNF && a.ubs != nullptr;
+  const float dt = (float)ctl->dt;
+  const float atol = (float)ctl->abstol, rtol = (float)ctl->reltol;
+  const int gsel = ctl->gsel;
+
+  int row[NE], col[NE];
+  float lam[NE], k[7][NE], ub[NE];
+  const int acc_ = mode == SM_STEP ? ctl->last_accept : 0;
+  const int jidx = mode == SM_STEP ? ctl->jump_idx : -1;
+  const bool re = mode == SM_STEP && ctl->fsal_reeval;
+  // step begin: lambda (and u) of the accepted step, the cotangent jump, the
+  // FSAL stage.  Idempotent: attempts enqueued past the end repeat it.
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    const int i = tid + e * THREADS;
+    row[e] = i / D;
+    col[e] = i - row[e] * D;
+    lam[e] = ub[e] = 0.f;
+#pragma unroll
+    for (int s = 0; s < 7; ++s) k[s][e] = 0.f;
+    if (i >= ne) continue;
+    const int64_t idx = e0 + i;
+    float l = acc_ ? a.lam_new[idx] : a.lam[idx];
+    if (acc_ && jidx >= 0 && idx < nreal) l += a.dLdout[(int64_t)jidx * nreal + idx];
+    lam[e] = l;
+    if (mode != SM_INIT_F0) k[0][e] = acc_ ? a.kl[6 * a.sv + idx] : a.kl[idx];
+    if (acc_) { a.lam[idx] = l; a.kl[idx] = k[0][e]; }
+    if (bs) {
+      float u = acc_ ? a.ubs_new[idx] : a.ubs[idx];
+      if (acc_ && jidx >= 0 && a.ckpt && idx < nreal) u = a.fsaved[(int64_t)jidx * nreal + idx];
+      ub[e] = u;
+      if (acc_) { a.ubs[idx] = u; a.ku[idx] = a.ku[6 * a.sv + idx]; }
+    }
+  }
+  if (mode == SM_STEP && ctl->done) return;
+
+  const int plane = COLS * m.pitch;
+  const int other = INPLACE ? 0 : P * plane;
+  const ChainBuf<PP> in0{0, m.pitch, plane};
+  float* part = (float*)(chain_lds() + (INPLACE ? 1 : 2) * P * plane * sizeof(T));
+  double sum = 0.0, flag = 0.0;
+  const int s0 = mode == SM_STEP && !re ? 1 : 0, s1 = mode == SM_STEP ? 7 : 1;
+  for (int s = s0; s < s1; ++s) {
+    const int slot = s == 0 ? (mode == SM_INIT_F1 ? 2 : gsel) : s == 6 ? (gsel ^ 1) : s + 1;
+    char* ob = (char*)a.ops.base + (int64_t)slot * a.ops.slot;
+    const int is = mode == SM_INIT_F1 ? 7 : s;   // interpolation slot
+    const double ts = mode == SM_INIT_F1 ? ctl->t + ctl->tdir * ctl->dt0 : ctl->t + dC[s] * ctl->dt;
+    // stage inputs: x = map(u(t_s)) now, lambda_s after the hidden recompute
+    const float* te = a.tape + (int64_t)ctl->st_step[is] * a.ent;
+    const bool ex = ctl->st_exact[is] != 0;
+    const float tdt = ctl->st_dt[is];
+    T* h0 = (T*)(ob + a.ops.h[0]);
+    const int64_t hpl = a.ops.rows * a.ops.w[0];
+    float ls[NE], us[NE];
+    {
+      const int kin = m.ktf[0] * ChainK<PP>::KT;
+      for (int i = tid; i < COLS * (kin - m.dm); i += THREADS) {
+        const int r = i / (kin - m.dm), c = m.dm + i % (kin - m.dm);
+        const bool tc = CNF && m.tcat && c == m.dm && r < R;
+        const float v = tc && row0 + r < m.B ? (float)ts : 0.f;
+        put<PP>(in0.at(r, c), plane, v);
+        if (tc) put<PP>(h0 + (orow0 + r) * a.ops.w[0] + c, hpl, v);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      ls[e] = us[e] = 0.f;
+      const int i = tid + e * THREADS;
+      if (i >= ne) continue;
+      const int64_t idx = e0 + i;
+      float u;
+      if (bs) {
+        // (u's stage values stay in memory: each is read by its own thread)
+        if (mode == SM_INIT_F1) u = ub[e] + (float)(ctl->tdir * ctl->dt0) * a.ku[idx];
+        else {
+          float sm = 0.f;
+          for (int j = s - 1; j >= 0; --j) sm += chA[s][j] * a.ku[j * a.sv + idx];
+          u = ub[e] + dt * sm;
+        }
+      } else {
+        u = te[idx];
+        if (!ex) {
+          float sm = 0.f;
+#pragma unroll
+          for (int j = 0; j < 7; ++j) sm += ctl->st_w[is][j] * te[(1 + j) * a.sv + idx];
+          u += tdt * sm;
+        }
+      }
+      us[e] = u;
+      if (mode == SM_INIT_F1) ls[e] = lam[e] + (float)(ctl->tdir * ctl->dt0) * k[0][e];
+      else {
+        float sm = 0.f;
+#pragma unroll
+        for (int j = 5; j >= 0; --j) sm += chA[s][j] * k[j][e];
+        ls[e] = lam[e] + dt * sm;
+      }
+      if (col[e] < m.dm) {
+        const float x = map_f(m.map, u);
+        put<PP>(in0.at(row[e], col[e]), plane, x);
+        put<PP>(h0 + (orow0 + row[e]) * a.ops.w[0] + col[e], hpl, x);
+        if constexpr (CNF) {
+          const int g = row0 + row[e];
+          const float p = g < m.B ? a.probe[(int64_t)g * m.dm + col[e]] : 0.f;
+          put<PP>(in0.at(R + row[e], col[e]), plane, p);
+          put<PP>(h0 + (orow0 + R + row[e]) * a.ops.w[0] + col[e], hpl, p);
+        }
+      }
+    }
+    if (mode == SM_STEP && s == 6) {
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const int i = tid + e * THREADS;
+        if (i >= ne) continue;
+        a.lam_new[e0 + i] = ls[e];
+        if (bs) a.ubs_new[e0 + i] = us[e];
+      }
+    }
+    __syncthreads();
+    // hidden recompute (a flow: with its tangent chain), act' and the
+    // second-order factor act'' adot kept for the way back.  The lane that
+    // writes an entry of them reads it again below: both sweeps deal a
+    // layer's tiles to the waves alike.
+    int cur = 0;
+    for (int l = 0; l < L - 1; ++l) {
+      const ChainBuf<PP> in{cur, m.pitch, plane}, o{other - cur, m.pitch, plane};
+      const float* bias = m.bias[l];
+      const int act = m.act[l], w = a.ops.w[l + 1];
+      T* hd = (T*)(ob + a.ops.h[l + 1]);
+      const int64_t pl = a.ops.rows * w;
+      float* sl = a.slope + ((int64_t)l * a.ops.rows + orow0) * a.wmax;
+      float* cv = a.curve + ((int64_t)l * a.ops.rows + orow0) * a.wmax;
+      auto epi = [&](int t, f32x4v (&acc)[NT]) {
+        const int f = 16 * t + 4 * (lane >> 4);
+        const f32x4v bv = *(const f32x4v*)(bias + f);
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          const int r = 16 * q + (lane & 15);
+          const f32x4v z = acc[q] + bv, y = act_f4(act, z), d = act_d4(act, z, y);
+          chain_put4<PP>(o, r, f, y);
+          const float yv[4] = {y.x, y.y, y.z, y.w};
+          put4<PP>(hd + (orow0 + r) * w + f, pl, yv);
+          *(f32x4v*)(sl + (int64_t)r * a.wmax + f) = d;
+          if constexpr (CNF) {
+            const f32x4v tv = acc[q + NP] * d;
+            chain_put4<PP>(o, R + r, f, tv);
+            const float tw[4] = {tv.x, tv.y, tv.z, tv.w};
+            put4<PP>(hd + (orow0 + R + r) * w + f, pl, tw);
+            // act'' adot in closed form (act' adot = t)
+            f32x4v c2 = {0.f, 0.f, 0.f, 0.f};
+            if (act == 1) c2 = -2.f * y * tv;
+            else if (act == 2) c2 = tv * (1.f - d);
+            else if (act == 4) c2 = tv * (1.f - 2.f * y);
+            *(f32x4v*)(cv + (int64_t)r * a.wmax + f) = c2;
+          }
+        }
+      };
+      chain_layer<PP, NT, NW, INPLACE>(m.Wf[l], m.mtf[l], m.ktf[l], in, wave, lane, epi);
+      cur = other - cur;
+    }
+    const int ll = L - 1;
+    float fu[NE];
+    if (bs) {  // f(u_s): u's own stage value
+      const int mt = m.mtf[ll];
+      chain_narrow<PP, NT, NW>(m.Wf[ll], mt, m.ktf[ll], ChainBuf<PP>{cur, m.pitch, plane}, part,
+                               wave, lane);
+#pragma unroll
+      for (int e = 0; e < NE; ++e)
+        fu[e] = tid + e * THREADS < ne
+                    ? chain_sum<NW, NT>(part, mt, row[e], col[e]) + m.bias[ll][col[e]] : 0.f;
+      __syncthreads();
+    }
+    // seeds at the output: lambda_s (a flow's tangent rows: -lambda_dlogp e)
+    cur = other - cur;
+    {
+      const ChainBuf<PP> o{cur, m.pitch, plane};
+      T* dd = (T*)(ob + a.ops.d[ll]);
+      const int w = a.ops.w[L];
+      const int64_t pl = a.ops.rows * w;
+      const int kin = m.ktb[ll] * ChainK<PP>::KT;
+      for (int i = tid; i < COLS * (kin - m.dm); i += THREADS) {
+        const int r = i / (kin - m.dm), c = m.dm + i % (kin - m.dm);
+        put<PP>(o.at(r, c), plane, 0.f);
+      }
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const int i = tid + e * THREADS;
+        if (i >= ne || col[e] >= m.dm) continue;
+        put<PP>(o.at(row[e], col[e]), plane, ls[e]);
+        put<PP>(dd + (orow0 + row[e]) * w + col[e], pl, ls[e]);
+        if constexpr (CNF) {  // (lambda_dlogp is constant over the solve)
+          const int g = row0 + row[e];
+          const float p = g < m.B ? -a.lam[(int64_t)g * D + m.dm] * a.probe[(int64_t)g * m.dm + col[e]] : 0.f;
+          put<PP>(o.at(R + row[e], col[e]), plane, p);
+          put<PP>(dd + (orow0 + R + row[e]) * w + col[e], pl, p);
+        }
+      }
+    }
+    __syncthreads();
+    for (int l = ll; l >= 1; --l) {
+      const ChainBuf<PP> in{cur, m.pitch, plane}, o{other - cur, m.pitch, plane};
+      const int w = a.ops.w[l];
+      T* dd = (T*)(ob + a.ops.d[l - 1]);
+      const int64_t pl = a.ops.rows * w;
+      const float* sl = a.slope + ((int64_t)(l - 1) * a.ops.rows + orow0) * a.wmax;
+      const float* cv = a.curve + ((int64_t)(l - 1) * a.ops.rows + orow0) * a.wmax;
+      auto epi = [&](int t, f32x4v (&acc)[NT]) {
+        const int f = 16 * t + 4 * (lane >> 4);
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          const int r = 16 * q + (lane & 15);
+          const f32x4v d = *(const f32x4v*)(sl + (int64_t)r * a.wmax + f);
+          f32x4v v = acc[q] * d;
+          if constexpr (CNF) {
+            const f32x4v c2 = *(const f32x4v*)(cv + (int64_t)r * a.wmax + f);
+            v += acc[q + NP] * c2;
+            const f32x4v tv = acc[q + NP] * d;
+            chain_put4<PP>(o, R + r, f, tv);
+            const float tw[4] = {tv.x, tv.y, tv.z, tv.w};
+            put4<PP>(dd + (orow0 + R + r) * w + f, pl, tw);
+          }
+          chain_put4<PP>(o, r, f, v);
+          const float vw[4] = {v.x, v.y, v.z, v.w};
+          put4<PP>(dd + (orow0 + r) * w + f, pl, vw);
+        }
+      };
+      chain_layer<PP, NT, NW, INPLACE>(m.Wb[l], m.mtb[l], m.ktb[l], in, wave, lane, epi);
+      cur = other - cur;
+    }
+    const int mt = m.mtb[0];
+    chain_narrow<PP, NT, NW>(m.Wb[0], mt, m.ktb[0], ChainBuf<PP>{cur, m.pitch, plane}, part, wave, lane);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      const int i = tid + e * THREADS;
+      if (i >= ne) continue;
+      float kv = 0.f;                            // (log p column: lambda constant)
+      if (!CNF || col[e] < m.dm) {
+        float g = chain_sum<NW, NT>(part, mt, row[e], col[e]);
+        if (m.map == 1) g *= 3.f * us[e] * us[e];
+        kv = -g;
+      }
+      const int64_t idx = e0 + i;
+      const bool live = idx < nreal;
+      auto add = [&](float d, float p, float q) {
+        const float sk = atol + fmaxf(fabsf(p), fabsf(q)) * rtol;
+        if (live) { const double v = (double)(d / sk); sum += v * v; }
+      };
+      if (mode == SM_STEP) {
+        if (s == 0) a.kl[idx] = kv;
+        if (bs) a.ku[s * a.sv + idx] = fu[e];
+        if (s == 6) {
+          a.kl[6 * a.sv + idx] = kv;
+          float ut = chBT[6] * kv;
+#pragma unroll
+          for (int j = 0; j < 6; ++j) ut += chBT[j] * k[j][e];
+          add(ut * dt, lam[e], ls[e]);
+          if (live && isnan(ls[e])) flag = 1.0;
+          if (bs) {
+            float uu = chBT[6] * fu[e];
+            for (int j = 0; j < 6; ++j) uu += chBT[j] * a.ku[j * a.sv + idx];
+            add(uu * dt, ub[e], us[e]);
+            if (live && isnan(us[e])) flag = 1.0;
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 6; ++j) k[j][e] = j == s ? kv : k[j][e];
+      } else if (mode == SM_INIT_F0) {
+        a.kl[idx] = kv;
+        add(kv, lam[e], 0.f);
+        if (bs) { a.ku[idx] = fu[e]; add(fu[e], ub[e], 0.f); }
+      } else {
+        add(kv - k[0][e], lam[e], 0.f);
+        if (live && kv != k[0][e]) flag = 1.0;
+        if (bs) {
+          const float f0 = a.ku[idx];
+          add(fu[e] - f0, ub[e], 0.f);
+          if (live && fu[e] != f0) flag = 1.0;
+        }
+      }
+    }
+    // (the next stage's inputs go to buffer 0; `part` is written again only
+    // after the barriers of its layers)
+    __syncthreads();
+  }
+  block_reduce_store(sum, flag, a.part, blockIdx.x);
+}
+
+size_t chain_adj_lds(int prec, const ChainModel& m, int nt) {
+  (void)prec;  // FP32, or two BF16 planes: four bytes per value
+  const size_t p0 = chain_part(m.nw, nt, m.mtf[m.L - 1]), p1 = chain_part(m.nw, nt, m.mtb[0]);
+  return (size_t)(nt == 4 ? 1 : 2) * 16 * nt * m.pitch * 4 + 4 * (p0 > p1 ? p0 : p1);
+}
+
+void launch_chain_adj(int prec, int nt, bool cnf, const ChainAdjArgs& a, int grid, hipStream_t s) {
+  const size_t lds = chain_adj_lds(prec, a.m, nt);
+  const int nw = a.m.nw;
+  auto go = [&](auto kern) {
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), lds, s, a);
+  };
+  if (prec == 0) {
+    if (cnf && nw == 8) go(k_chain_adj<PF32, 2, 8, true>);
+    else if (cnf) go(k_chain_adj<PF32, 2, 4, true>);
+    else if (nw == 8) go(k_chain_adj<PF32, 1, 8, false>);
+    else go(k_chain_adj<PF32, 1, 4, false>);
+  } else if (cnf) {
+    if (nt == 4) go(k_chain_adj<PBF16X3, 4, 8, true>);
+    else if (nw == 8) go(k_chain_adj<PBF16X3, 2, 8, true>);
+    else go(k_chain_adj<PBF16X3, 2, 4, true>);
+  } else {
+    if (nw == 8) go(k_chain_adj<PBF16X3, 1, 8, false>);
+    else go(k_chain_adj<PBF16X3, 1, 4, false>);
+  }
+}
+
+// ---------------------------------------------------------------- weight gradients
+// G_l[i][o] = sum over rows of h[row][i] d[row][o] per stage, K = rows, folded
+// into acc_b = sum_s b_s G_s and acc_e = sum_s bt_s G_s in registers.
+// Stage coefficients: the step's b and bt, or one stage alone (initial dt).
+__device__ __forceinline__ int wg_slot(int mode, int s, int gsel) {
+  if (mode == SM_INIT_F1) return 2;
+  return s == 0 ? gsel : s == 6 ? (gsel ^ 1) : s + 1;
+}
+
+// tile index -> layer, tile row (inputs) and column (outputs)
+__device__ __forceinline__ int wg_tile(const ChainWgradArgs& a, int tile, int& it, int& ot) {
+  int l = 0;
+  while (l + 1 < a.m.L && tile >= a.tl[l + 1]) ++l;
+  const int t = tile - a.tl[l];
+  it = t / a.tw[l];
+  ot = t % a.tw[l];
+  return l;
+}
+
+// FP32.  A wave owns a 64 x 64 tile over its share of a row range: both
+// operands come straight from memory, 16 bytes per lane (lane l: row l / 16 of
+// a group of four, features 4 (l % 16) ..), and component v of the vectors is
+// the operand of MFMA tile v, whose features are 4 (l % 16) + v.  32 B of
+// operands per lane feed 16 MFMAs (512 cycles), so neither LDS nor a second
+// read of the rows is needed; the four waves' sums meet in LDS at the end.
+constexpr int GT = 64;
+__global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
+  const Ctl* ctl = a.ctl;
+  if (a.mode == SM_STEP && ctl->done) return;
+  __shared__ float red[4][GT * GT / 2];
+  __shared__ float redb[4][2][GT];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  int it, ot;
+  const int l = wg_tile(a, blockIdx.x, it, ot);
+  const int64_t r0 = blockIdx.y * a.crows;
+  const int64_t r1 = r0 + a.crows < a.ops.rows ? r0 + a.crows : a.ops.rows;
+  const int wi = a.ops.w[l], wo = a.ops.w[l + 1];
+  const int gsel = ctl->gsel;
+  const int ns = a.mode == SM_STEP ? 7 : 1;
+  f32x4v g[4][4], ab[4][4], ae[4][4];
+  f32x4v gb, bb = {0.f, 0.f, 0.f, 0.f}, be = bb;
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+#pragma unroll
+    for (int y = 0; y < 4; ++y) ab[x][y] = ae[x][y] = bb;
+  const bool bias = it == 0;
+  const int64_t rr = r0 + 4 * wave + (lane >> 4);
+  for (int s = 0; s < ns; ++s) {
+    const char* ob = (const char*)a.ops.base + (int64_t)wg_slot(a.mode, s, gsel) * a.ops.slot;
+    const float* h = (const float*)(ob + a.ops.h[l]) + rr * wi + it * GT + 4 * (lane & 15);
+    const float* d = (const float*)(ob + a.ops.d[l]) + rr * wo + ot * GT + 4 * (lane & 15);
+    const f32x4v zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int y = 0; y < 4; ++y) g[x][y] = zero;
+    gb = zero;
+    const int n = (int)((r1 - r0) / 16);           // groups of 16 rows (4 per wave)
+    constexpr int PF = 2;
+    f32x4v hv[PF], dv[PF];
+    auto load = [&](int j, int k) {
+      k = k < n ? k : n - 1;
+      hv[j] = *(const f32x4v*)(h + (int64_t)k * 16 * wi);
+      dv[j] = *(const f32x4v*)(d + (int64_t)k * 16 * wo);
+    };
+    auto step = [&](int j, int k, bool refill) {
+      const f32x4v x = hv[j], y = dv[j];
+      if (refill) load(j, k + PF);
+      // bias: primal rows only
+      const int64_t row = rr + (int64_t)k * 16;
+      if (bias && (a.rprim == a.rblk || row % a.rblk < a.rprim)) gb += y;
+#pragma unroll
+      for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          g[p][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[p], y[q], g[p][q], 0, 0, 0);
+    };
+#pragma unroll
+    for (int j = 0; j < PF; ++j) load(j, j);
+    int k = 0;
+    for (; k + PF <= n; k += PF)
+#pragma unroll
+      for (int j = 0; j < PF; ++j) step(j, k + j, true);
+#pragma unroll
+    for (int j = 0; j < PF - 1; ++j)
+      if (k + j < n) step(j, k + j, false);
+    const float cb = a.mode == SM_STEP ? (s < 6 ? chA[6][s] : 0.f) : 1.f;
+    const float ce = a.mode == SM_STEP ? chBT[s] : 0.f;
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int y = 0; y < 4; ++y) {
+        ab[x][y] += cb * g[x][y];
+        ae[x][y] += ce * g[x][y];
+      }
+    bb += cb * gb;
+    be += ce * gb;
+  }
+  // sum over the waves, two halves of the tile at a time; acc element (p, q, v)
+  // of lane l is input 4 (4 (l / 16) + v) + p, output 4 (l % 16) + q
+  const int64_t tsz = GT * (GT + 1);
+  float* out = a.part + ((int64_t)blockIdx.y * 2 * a.ntile + blockIdx.x) * tsz;
+#pragma unroll
+  for (int which = 0; which < 2; ++which) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      __syncthreads();
+#pragma unroll
+      for (int pp = 0; pp < 2; ++pp) {
+        const int p = 2 * half + pp;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int ii = 4 * (lane >> 4) + v;    // input = 4 ii + p
+          f32x4v o;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) o[q] = which ? ae[p][q][v] : ab[p][q][v];
+          *(f32x4v*)&red[wave][(pp * 16 + ii) * GT + 4 * (lane & 15)] = o;
+        }
+      }
+      __syncthreads();
+      for (int e = threadIdx.x; e < GT * GT / 2; e += 256) {
+        const int rw = e / GT, c = e % GT;
+        const int i = 4 * (rw & 15) + 2 * half + (rw >> 4);
+        out[(int64_t)which * a.ntile * tsz + i * GT + c] =
+            (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
+      }
+    }
+  }
+  if (bias) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float x = bb[q], y = be[q];
+      x += __shfl_xor(x, 16); x += __shfl_xor(x, 32);
+      y += __shfl_xor(y, 16); y += __shfl_xor(y, 32);
+      if (lane < 16) { redb[wave][0][4 * lane + q] = x; redb[wave][1][4 * lane + q] = y; }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 * GT) {
+      const int which = threadIdx.x / GT, c = threadIdx.x % GT;
+      out[(int64_t)which * a.ntile * tsz + GT * GT + c] =
+          (redb[0][which][c] + redb[1][which][c]) + (redb[2][which][c] + redb[3][which][c]);
+    }
+  }
+}
+
+// Split BF16.  K = rows must be contiguous per lane, the operands are
+// row-major: a 128 x 128 tile stages 32 rows of both in LDS and reads them
+// through the transposing LDS load (a group of 16 lanes reads four rows of 16
+// features and gets each lane one feature of the four rows).  Row pitch 320 B:
+// the four rows of a read fall on different banks.  Four waves, each 64 x 64
+// (two 32 x 32 tiles each way, hi*hi + lo*hi + hi*lo) with both folded sums in
+// registers; the next 32 rows travel from memory to registers meanwhile.
+constexpr int GS = 128, GS_PITCH = 160, GS_K = 32;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
+__device__ __forceinline__ u32x4 wg_frag(const bf16* lds, int row, int col) {
+  const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(lds + row * GS_PITCH + col));
+  const s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4)(lds + (row + 4) * GS_PITCH + col));
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  const s16x8 v = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+  return __builtin_bit_cast(u32x4, v);
+}
+__global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
+  const Ctl* ctl = a.ctl;
+  if (a.mode == SM_STEP && ctl->done) return;
+  // [buffer][operand][plane][32 rows][pitch]
+  __shared__ __attribute__((aligned(16))) bf16 lt[2][2][2][GS_K * GS_PITCH];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  int it, ot;
+  const int l = wg_tile(a, blockIdx.x, it, ot);
+  const int64_t r0 = blockIdx.y * a.crows;
+  const int64_t r1 = r0 + a.crows < a.ops.rows ? r0 + a.crows : a.ops.rows;
+  const int wi = a.ops.w[l], wo = a.ops.w[l + 1];
+  const int gsel = ctl->gsel;
+  const int ns = a.mode == SM_STEP ? 7 : 1;
+  const int n = (int)((r1 - r0 + GS_K - 1) / GS_K);
+  const bool bias = it == 0;
+  // this thread's 16-byte pieces: 8 features (fc) of rows tr, tr + 16 of both
+  // operands and planes
+  const int fc = 8 * (tid & 15), tr = tid >> 4;
+  const bool hin = it * GS + fc < wi, din = ot * GS + fc < wo;
+  f32x16 g[2][2], ab[2][2], ae[2][2];
+  float gb[8], bb[8], be[8];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) ab[x][y][v] = ae[x][y][v] = 0.f;
+#pragma unroll
+  for (int v = 0; v < 8; ++v) bb[v] = be[v] = 0.f;
+  const int wr = 64 * (wave >> 1), wc = 64 * (wave & 1);
+  const int frow = 8 * (lane >> 5) + ((lane & 15) >> 2);          // first K row of this lane's reads
+  const int fcol = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  for (int s = 0; s < ns; ++s) {
+    const char* ob = (const char*)a.ops.base + (int64_t)wg_slot(a.mode, s, gsel) * a.ops.slot;
+    const bf16* h = (const bf16*)(ob + a.ops.h[l]) + it * GS + fc;
+    const bf16* d = (const bf16*)(ob + a.ops.d[l]) + ot * GS + fc;
+    const int64_t hp = a.ops.rows * wi, dp = a.ops.rows * wo;
+    u32x4 hv[2][2], dv[2][2];                                     // [row half][plane]
+    auto load = [&](int k) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int64_t r = r0 + (int64_t)k * GS_K + tr + 16 * q;
+        const bool in = r < r1;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          hv[q][p] = (u32x4){0, 0, 0, 0};
+          dv[q][p] = (u32x4){0, 0, 0, 0};
+          if (in && hin) hv[q][p] = *(const u32x4*)(h + p * hp + r * wi);
+          if (in && din) dv[q][p] = *(const u32x4*)(d + p * dp + r * wo);
+        }
+      }
+    };
+    auto store = [&](int b, int k) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          *(u32x4*)&lt[b][0][p][(tr + 16 * q) * GS_PITCH + fc] = hv[q][p];
+          *(u32x4*)&lt[b][1][p][(tr + 16 * q) * GS_PITCH + fc] = dv[q][p];
+        }
+        if (bias) {
+          const int64_t r = r0 + (int64_t)k * GS_K + tr + 16 * q;
+          if (a.rprim == a.rblk || r % a.rblk < a.rprim) {
+            const bf16x8 x = __builtin_bit_cast(bf16x8, dv[q][0]), y = __builtin_bit_cast(bf16x8, dv[q][1]);
+#pragma unroll
+            for (int v = 0; v < 8; ++v) gb[v] += (float)x[v] + (float)y[v];
+          }
+        }
+      }
+    };
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) g[x][y][v] = 0.f;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) gb[v] = 0.f;
+    load(0);
+    store(0, 0);
+    __syncthreads();
+    for (int k = 0; k < n; ++k) {
+      const int b = k & 1;
+      if (k + 1 < n) load(k + 1);
+#pragma unroll
+      for (int kk = 0; kk < GS_K; kk += 16) {
+        u32x4 x[2][2], y[2][2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            x[t][p] = wg_frag(lt[b][0][p], kk + frow, wr + 32 * t + fcol);
+            y[t][p] = wg_frag(lt[b][1][p], kk + frow, wc + 32 * t + fcol);
+          }
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            auto m = [&](const u32x4& p, const u32x4& q) {
+              g[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                  __builtin_bit_cast(bf16x8, p), __builtin_bit_cast(bf16x8, q), g[t][u], 0, 0, 0);
+            };
+            m(x[t][0], y[u][0]);
+            m(x[t][1], y[u][0]);
+            m(x[t][0], y[u][1]);
+          }
+      }
+      if (k + 1 < n) store(b ^ 1, k + 1);
+      __syncthreads();
+    }
+    const float cb = a.mode == SM_STEP ? (s < 6 ? chA[6][s] : 0.f) : 1.f;
+    const float ce = a.mode == SM_STEP ? chBT[s] : 0.f;
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        ab[x][y] += cb * g[x][y];
+        ae[x][y] += ce * g[x][y];
+      }
+#pragma unroll
+    for (int v = 0; v < 8; ++v) { bb[v] += cb * gb[v]; be[v] += ce * gb[v]; }
+  }
+  const int64_t tsz = GS * (GS + 1);
+  float* out = a.part + ((int64_t)blockIdx.y * 2 * a.ntile + blockIdx.x) * tsz;
+#pragma unroll
+  for (int which = 0; which < 2; ++which)
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int i = wr + 32 * t + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+          out[(int64_t)which * a.ntile * tsz + i * GS + wc + 32 * u + (lane & 31)] =
+              which ? ae[t][u][v] : ab[t][u][v];
+        }
+  if (bias) {
+    float* red = (float*)lt;                                      // [2][16][GS]
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      red[tr * GS + fc + v] = bb[v];
+      red[16 * GS + tr * GS + fc + v] = be[v];
+    }
+    __syncthreads();
+    const int which = tid / GS, c = tid % GS;
+    float x = 0.f;
+    for (int r = 0; r < 16; ++r) x += red[which * 16 * GS + r * GS + c];
+    out[(int64_t)which * a.ntile * tsz + GS * GS + c] = x;
+  }
+}
+
+// ---------------------------------------------------------------- parameter state
+// Adds the row ranges' partial sums in range order, forms the speculative mu in
+// the other buffer and its error norm (modes: step, initial-dt norms).  The
+// parameter equation is mu' = -lambda^T df/dp.
+__global__ void __launch_bounds__(256) k_chain_mu(ChainMuArgs a) {
+  const ChainWgradArgs& w = a.w;
+  const Ctl* c = w.ctl;
+  if (w.mode == SM_STEP && c->done) return;
+  const double atol = c->abstol, rtol = c->reltol, dt = c->dt;
+  const int ms = c->gsel_mu_;
+  const double* mu = ms ? a.mu + a.P : a.mu;
+  double* mo = ms ? a.mu : a.mu + a.P;
+  const int E = a.edge;
+  const int64_t tsz = (int64_t)E * (E + 1), half = (int64_t)w.ntile * tsz;
+  double sum = 0.0, flag = 0.0;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < a.P;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    int l = 0;
+    while (l + 1 < w.m.L && i >= a.w0[l + 1]) ++l;
+    const int out = w.m.out[l];
+    int64_t src;
+    if (i < a.b0[l]) {
+      const int q = (int)(i - a.w0[l]), in = q / out, o = q % out;
+      src = (int64_t)(w.tl[l] + in / E * w.tw[l] + o / E) * tsz + (in % E) * E + o % E;
+    } else {
+      const int o = (int)(i - a.b0[l]);
+      src = (int64_t)(w.tl[l] + o / E) * tsz + (int64_t)E * E + o % E;
+    }
+    float b = 0.f, e = 0.f;
+    if (w.mode == SM_STEP) {
+      for (int k = 0; k < w.chunks; ++k) {
+        b -= w.part[k * 2 * half + src];
+        e -= w.part[k * 2 * half + half + src];
+      }
+    } else {
+      for (int k = 0; k < w.chunks; ++k) b -= w.part[k * 2 * half + src];
+    }
+    const double m = mu[i];
+    double v;
+    if (w.mode == SM_STEP) {
+      const double mn = m + dt * (double)b;
+      mo[i] = mn;
+      v = dt * (double)e / (atol + fmax(fabs(m), fabs(mn)) * rtol);
+    } else if (w.mode == SM_INIT_F0) {
+      a.g0[i] = b;
+      v = (double)b / (atol + fabs(m) * rtol);
+    } else {
+      v = ((double)b - (double)a.g0[i]) / (atol + fabs(m) * rtol);
+      if (b != a.g0[i]) flag = 1.0;
+    }
+    sum += v * v;
+  }
+  block_reduce_store(sum, flag, a.part, blockIdx.x);
+}
+
+void launch_chain_wgrad(int prec, const ChainWgradArgs& a, hipStream_t s) {
+  if (prec == 0)
+    hipLaunchKernelGGL(k_chain_wgrad32, dim3(a.ntile, a.chunks), dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_chain_wgrad16, dim3(a.ntile, a.chunks), dim3(256), 0, s, a);
+}
+void launch_chain_mu(const ChainMuArgs& a, int nblk, hipStream_t s) {
+  hipLaunchKernelGGL(k_chain_mu, dim3(nblk), dim3(256), 0, s, a);
+}
+
+}  // namespace nodehip

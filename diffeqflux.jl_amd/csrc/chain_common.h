@@ -133,7 +133,7 @@ __device__ __forceinline__ void chain_mma(f32x4v (&acc)[MT][NT], const void* __r
 // refilled as soon as its MFMAs are issued)
 template <class PP, int NT, int MT> constexpr int chain_pf() {
   const int c = MT * NT * (sizeof(typename PP::T) == 4 ? 128 : PP::SPLIT ? 48 : 16);
-  return c >= 1024 ? 1 : c >= 384 ? 2 : c >= 128 ? 4 : 8;
+  return c >= 768 ? 1 : c >= 192 ? 2 : 4;
 }
 
 template <class PP, int NT, int MT, class Epi>
@@ -176,16 +176,17 @@ __device__ __forceinline__ void chain_layer(const void* W, int mt, int kt, const
 }
 
 // A narrow layer (state-sized output, mt <= 4 tiles): the K tiles are split
-// over the waves left over (at most four splits); partial products go to LDS
-// as FP32 [split][row][16 mt + 4], summed by the reader.  Ends with a barrier.
-template <int NW> __host__ __device__ __forceinline__ int chain_splits(int mt) {
-  const int s = NW / mt;
-  return s > 4 ? 4 : s;
+// over the waves left over (at most four splits, two where the block's
+// activations leave LDS for no more); partial products go to LDS as FP32
+// [split][row][16 mt + 4], summed by the reader.  Ends with a barrier.
+template <int NW, int NT> __host__ __device__ __forceinline__ int chain_splits(int mt) {
+  const int s = NW / mt, most = NT == 4 ? 2 : 4;
+  return s > most ? most : s;
 }
 template <class PP, int NT, int NW>
 __device__ __forceinline__ void chain_narrow(const void* W, int mt, int kt, const ChainBuf<PP>& in,
                                              float* part, int wave, int lane) {
-  const int ks = chain_splits<NW>(mt), t = wave % mt, s = wave / mt;
+  const int ks = chain_splits<NW, NT>(mt), t = wave % mt, s = wave / mt;
   if (s < ks) {
     f32x4v acc[1][NT];
 #pragma unroll
@@ -199,12 +200,18 @@ __device__ __forceinline__ void chain_narrow(const void* W, int mt, int kt, cons
   }
   __syncthreads();
 }
-template <int NW>
-__device__ __forceinline__ float chain_sum(const float* part, int mt, int cols, int row, int c) {
-  const int ks = chain_splits<NW>(mt), pd = 16 * mt + 4;
+template <int NW, int NT>
+__device__ __forceinline__ float chain_sum(const float* part, int mt, int row, int c) {
+  const int ks = chain_splits<NW, NT>(mt), pd = 16 * mt + 4;
   float v = part[row * pd + c];
-  for (int s = 1; s < ks; ++s) v += part[(s * cols + row) * pd + c];
+  for (int s = 1; s < ks; ++s) v += part[(s * 16 * NT + row) * pd + c];
   return v;
+}
+// floats of the partial products
+inline size_t chain_part(int nw, int nt, int mt) {
+  const int ks = nw == 8 ? (nt == 4 ? chain_splits<8, 4>(mt) : chain_splits<8, 1>(mt))
+                         : chain_splits<4, 1>(mt);
+  return (size_t)ks * 16 * nt * (16 * mt + 4);
 }
 
 // activation of four values, chosen once

@@ -160,13 +160,13 @@ __global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
       if (i >= ne) continue;
       float kv;
       if (!CNF || col[e] < m.dm) {
-        kv = act_f(m.act[ll], chain_sum<NW>(part, mt, COLS, row[e], col[e]) + m.bias[ll][col[e]]);
+        kv = act_f(m.act[ll], chain_sum<NW, NT>(part, mt, row[e], col[e]) + m.bias[ll][col[e]]);
       } else {  // log p: minus the probe's directional derivative of f
         kv = 0.f;
         const int g = row0 + row[e];
         if (g < m.B)
           for (int c = 0; c < m.dm; ++c)
-            kv -= a.probe[(int64_t)g * m.dm + c] * chain_sum<NW>(part, mt, COLS, R + row[e], c);
+            kv -= a.probe[(int64_t)g * m.dm + c] * chain_sum<NW, NT>(part, mt, R + row[e], c);
       }
       const int64_t idx = e0 + i;
       const bool live = row0 + row[e] < m.B;
@@ -208,10 +208,8 @@ static size_t chain_elt(int prec) { return prec == 0 ? 4 : prec == 1 ? 2 : 4; } 
 
 size_t chain_fwd_lds(int prec, const ChainModel& m, int nt) {
   const bool inplace = nt == 4;
-  const int cols = 16 * nt, mt = m.mtf[m.L - 1];
-  const int ks = m.nw == 8 ? chain_splits<8>(mt) : chain_splits<4>(mt);
-  const size_t part = (size_t)ks * cols * (16 * mt + 4) * 4;
-  return (size_t)(inplace ? 1 : 2) * cols * m.pitch * chain_elt(prec) + part;
+  return (size_t)(inplace ? 1 : 2) * 16 * nt * m.pitch * chain_elt(prec) +
+         4 * chain_part(m.nw, nt, m.mtf[m.L - 1]);
 }
 
 void launch_chain_fwd(int prec, int nt, bool cnf, const ChainFwdArgs& a, int grid, hipStream_t s) {

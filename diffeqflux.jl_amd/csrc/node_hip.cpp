@@ -178,7 +178,8 @@ struct node_handle {
   // tape, save times, outputs, fused steps
   const void* fwd_graph_sig[4] = {nullptr, nullptr, nullptr, nullptr};
   // tape, save times, cotangents, saved states (BacksolveAdjoint checkpoints)
-  const void* adj_graph_sig[4] = {nullptr, nullptr, nullptr, nullptr};
+  // (fifth: fused steps)
+  const void* adj_graph_sig[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   int graph_attempts = 4;
 
   // ragged batches: flat parameters and the last per-trajectory forward
@@ -219,6 +220,14 @@ struct node_handle {
   // (0: the forward runs on the GEMM path)
   ChainModel chain{};
   int chain_nt = 0;
+  // fused adjoint steps: column tiles per row block (0: GEMM path), operand
+  // store of the weight gradients, act' / act'' adot, partial sums
+  int chain_ant = 0;
+  ChainOps cops{};
+  ChainMuArgs cmu{};
+  float* cslope = nullptr;
+  float* ccurve = nullptr;
+  int cwmax = 0;
 
   // profiling (node_prof_enable)
   uint64_t prof_mask = 0;
@@ -715,6 +724,24 @@ bool chain_plan(node_handle* h, ChainModel& m) {
   return true;
 }
 
+// Layout of the operand store (without its address).
+constexpr int64_t CHAIN_OPS_MAX = int64_t(4) << 30;  // bytes a handle may keep for it
+ChainOps chain_ops(const node_handle* h, int nt) {
+  ChainOps o{};
+  const int r = chain_rows(nt, h->cnf);
+  o.rows = (int64_t)((h->B + r - 1) / r) * 16 * nt;
+  const int64_t elt = (int64_t)h->esz * h->planes;
+  for (int l = 0; l < h->L; ++l) o.w[l] = h->layers[l].inp;
+  o.w[h->L] = h->layers[h->L - 1].outp;
+  for (int l = 0; l < h->L; ++l) {
+    o.h[l] = o.slot;
+    o.slot += o.rows * o.w[l] * elt;
+    o.d[l] = o.slot;
+    o.slot += o.rows * o.w[l + 1] * elt;
+  }
+  return o;
+}
+
 int chain_alloc(node_handle* h) {
   ChainModel m;
   if (!chain_plan(h, m)) return 0;
@@ -733,7 +760,96 @@ int chain_alloc(node_handle* h) {
   }
   h->chain = m;
   h->chain_nt = nt;
+  // adjoint: linear last layer; a block's registers hold one column tile of
+  // rows with 64 state entries each (a flow's 32: two or four tiles)
+  const int ant = h->cnf ? nt : 1;
+  if (h->layers[h->L - 1].act == NODE_ACT_IDENTITY &&
+      chain_adj_lds(h->prec, m, ant) <= 160 * 1024 &&
+      (h->B + chain_rows(ant, h->cnf) - 1) / chain_rows(ant, h->cnf) <= MAX_PART &&
+      chain_ops(h, ant).slot * 7 <= CHAIN_OPS_MAX)
+    h->chain_ant = ant;
   return 0;
+}
+
+// Buffers of the fused adjoint, at its first use.
+int chain_adj_alloc(node_handle* h) {
+  if (h->cops.base) return 0;
+  ChainOps o = chain_ops(h, h->chain_ant);
+  const ChainModel& m = h->chain;
+  h->cwmax = 0;
+  for (int l = 0; l < h->L - 1; ++l) h->cwmax = std::max(h->cwmax, o.w[l + 1]);
+  const size_t sc = (size_t)std::max(h->L - 1, 1) * o.rows * std::max(h->cwmax, 4) * sizeof(float);
+  if (int rc = dalloc_t(h, &h->cslope, sc)) return rc;
+  if (h->cnf)
+    if (int rc = dalloc_t(h, &h->ccurve, sc)) return rc;
+  // weight-gradient tiles and row ranges: two workgroups (FP32) or one (split)
+  // per CU
+  ChainMuArgs& u = h->cmu;
+  ChainWgradArgs& w = u.w;
+  const int E = h->prec == NODE_PREC_FP32 ? 64 : 128, K = h->prec == NODE_PREC_FP32 ? 16 : 32;
+  w.m = m;
+  w.rblk = 16 * h->chain_ant;
+  w.rprim = chain_rows(h->chain_ant, h->cnf);
+  for (int l = 0; l < h->L; ++l) {
+    w.tl[l] = w.ntile;
+    w.tw[l] = (o.w[l + 1] + E - 1) / E;
+    w.ntile += w.tw[l] * ((o.w[l] + E - 1) / E);
+    u.w0[l] = h->layers[l].w0;
+    u.b0[l] = h->layers[l].b0;
+  }
+  const int64_t want = (h->prec == NODE_PREC_FP32 ? 512 : 256) / w.ntile;
+  w.chunks = (int)std::max<int64_t>(1, std::min<int64_t>(want, o.rows / 64));
+  w.crows = rup((o.rows + w.chunks - 1) / w.chunks, K);
+  w.chunks = (int)((o.rows + w.crows - 1) / w.crows);
+  if (int rc = dalloc_t(h, &w.part, (size_t)w.chunks * 2 * w.ntile * E * (E + 1) * sizeof(float))) return rc;
+  u.P = h->P;
+  u.edge = E;
+  void* base = nullptr;
+  if (int rc = dalloc(h, &base, (size_t)o.slot * 7)) return rc;
+  o.base = base;
+  w.ops = o;
+  h->cops = o;
+  return 0;
+}
+
+// Whether this adjoint runs as fused steps (see chain_on for tape budgets;
+// reduced weight-gradient precision is the GEMM path's).
+bool chain_adj_on(const node_handle* h) {
+  return h->chain_ant > 0 && h->tape_budget == 0 && h->wg_prec == h->prec;
+}
+
+int chain_adj_grid(const node_handle* h) {
+  const int r = chain_rows(h->chain_ant, h->cnf);
+  return (h->B + r - 1) / r;
+}
+int chain_mu_blocks(const node_handle* h) {
+  return (int)std::min<int64_t>((h->P + 255) / 256, 1024);
+}
+
+// One fused adjoint step attempt (SM_STEP) or one VJP of the initial-dt
+// heuristic: row pass, weight gradients, parameter state and its norm.
+void chain_adjoint(node_handle* h, const AdjBufs& ab, int mode, double* px, double* pm) {
+  ChainAdjArgs a{};
+  a.m = h->chain;
+  a.ops = h->cops;
+  a.tape = h->tape;
+  a.sv = (int64_t)h->Bp * h->D;
+  a.ent = 8 * a.sv;
+  a.lam = ab.lam; a.lam_new = ab.lam_new; a.kl = ab.kl;
+  a.dLdout = ab.dLdout;
+  a.probe = h->probe;
+  a.slope = h->cslope; a.curve = h->ccurve; a.wmax = h->cwmax;
+  a.ubs = ab.ubs; a.ubs_new = ab.ubs_new; a.ku = ab.ku; a.fsaved = ab.fsaved; a.ckpt = ab.ckpt;
+  a.part = px; a.ctl = h->ctl; a.mode = mode;
+  launch_chain_adj(h->prec, h->chain_ant, h->cnf, a, chain_adj_grid(h), h->stream);
+  ChainMuArgs u = h->cmu;
+  u.w.ctl = h->ctl;
+  u.w.mode = mode;
+  u.mu = h->mu;
+  u.g0 = h->gf0;
+  u.part = pm;
+  launch_chain_wgrad(h->prec, u.w, h->stream);
+  launch_chain_mu(u, chain_mu_blocks(h), h->stream);
 }
 
 // Whether this solve runs as fused steps.  Tape-budgeted solves stay on the
@@ -1162,7 +1278,9 @@ int forward_impl(node_handle* h, const node_solve_opts* o, const float* d_u0,
                  const double* saveat, int64_t n_saveat, node_stats* st) {
   if (!h->have_params) return fail(h, NODE_ERR_STATE, "parameters not set");
   if (!o) return fail(h, NODE_ERR_INVALID, "opts is NULL");
-  if (int rc = maybe_autotune(h)) return rc;
+  // (the GEMM plans are timed when a solve first needs them)
+  if (!chain_on(h) || !chain_adj_on(h))
+    if (int rc = maybe_autotune(h)) return rc;
   if (!(o->t1 != o->t0) || !std::isfinite(o->t0) || !std::isfinite(o->t1))
     return fail(h, NODE_ERR_INVALID, "tspan must be finite with t1 != t0");
   if (!o->adaptive && !(o->dt != 0.0)) return fail(h, NODE_ERR_INVALID, "fixed-step solve needs dt");
@@ -1369,7 +1487,12 @@ int backward_impl(node_handle* h, const float* d_dLdout, node_stats* st) {
     if (int rc = dalloc_t(h, &h->bs_ku, 8 * sv * 4)) return rc;
     if (int rc = dalloc_t(h, &h->bs_fu, sv * 4)) return rc;
   }
-  if (int rc = maybe_autotune(h)) return rc;
+  const bool fused = chain_adj_on(h);
+  if (fused) {
+    if (int rc = chain_adj_alloc(h)) return rc;
+  } else if (int rc = maybe_autotune(h)) {
+    return rc;
+  }
   const bool ck = h->fwd_ring;
   if (ck && h->sense != NODE_SENSE_INTERPOLATING)
     return fail(h, NODE_ERR_STATE, "the last forward kept checkpoints only "
@@ -1406,26 +1529,39 @@ int backward_impl(node_handle* h, const float* d_dLdout, node_stats* st) {
   double* px = h->part + SEC;
   double* pm = h->part + 2 * SEC;
   const int nb = state_blocks(sg);
-  const int nmb = mu_blocks(h->P);
-  const int nx = vjp_last_tiles(h);
+  const int nmb = fused ? chain_mu_blocks(h) : mu_blocks(h->P);
+  const int nx = fused ? chain_adj_grid(h) : vjp_last_tiles(h);
   // error norm over [lambda; mu], or [u; lambda; mu] when u is integrated too
   const double nel = (h->sense != NODE_SENSE_INTERPOLATING ? 2.0 : 1.0) * h->B * h->D + (double)h->P;
 
   launch_set_stage_interp(h->ctl, 0, o.t1, h->fwd_times, h->stream);
   launch_adj_init(sg, ab, h->ctl, p0, h->stream);
-  vjp_eval(h, 0, SM_INIT_F0, GATE_ALWAYS, WG_STORE_CUR, 0, 0, 0, 0, px, nullptr, nullptr);
-  launch_mu_norm(1, ab, h->ctl, pm, nmb, GATE_ALWAYS, h->stream);
+  if (fused) {
+    chain_adjoint(h, ab, SM_INIT_F0, px, pm);
+  } else {
+    vjp_eval(h, 0, SM_INIT_F0, GATE_ALWAYS, WG_STORE_CUR, 0, 0, 0, 0, px, nullptr, nullptr);
+    launch_mu_norm(1, ab, h->ctl, pm, nmb, GATE_ALWAYS, h->stream);
+  }
   if (!c.has_dt_) {
     launch_initdt_a(h->ctl, p0, nb, px, nx, pm, nmb, nel, h->stream);
     launch_set_stage_interp(h->ctl, 7, 0.0, h->fwd_times, h->stream);
-    launch_adj_initdt_prep(sg, ab, h->ctl, h->stream);
-    vjp_eval(h, 0, SM_INIT_F1, GATE_ALWAYS, WG_STORE_PTR, 0, 0, 0, 0, px, nullptr, h->accb);
-    launch_mu_norm(2, ab, h->ctl, pm, nmb, GATE_ALWAYS, h->stream);
+    if (fused) {
+      chain_adjoint(h, ab, SM_INIT_F1, px, pm);
+    } else {
+      launch_adj_initdt_prep(sg, ab, h->ctl, h->stream);
+      vjp_eval(h, 0, SM_INIT_F1, GATE_ALWAYS, WG_STORE_PTR, 0, 0, 0, 0, px, nullptr, h->accb);
+      launch_mu_norm(2, ab, h->ctl, pm, nmb, GATE_ALWAYS, h->stream);
+    }
   }
   launch_initdt_b(h->ctl, px, nx, pm, nmb, nel, h->save_times, 1, h->fwd_times, h->stream);
   HIPCHK(h, hipGetLastError());
 
   auto attempt = [&]() {
+    if (fused) {
+      chain_adjoint(h, ab, SM_STEP, px, pm);
+      launch_adj_controller(h->ctl, px, nx, pm, nmb, nel, h->save_times, h->fwd_times, h->stream);
+      return;
+    }
     launch_adj_step_begin(sg, ab, h->ctl, GATE_ALWAYS, h->stream);
     vjp_eval(h, 0, SM_STEP, GATE_FSAL, WG_STORE_CUR, 0, 0, 0, 0, px, nullptr, nullptr);
     for (int s = 1; s < 7; ++s) {
@@ -1472,7 +1608,7 @@ int backward_impl(node_handle* h, const float* d_dLdout, node_stats* st) {
     enqueued += chunk;
     if (graphs) {
       // the tape may have moved (a checkpoint re-solve grew it)
-      const void* asig[4] = {h->tape, h->save_times, d_dLdout, h->out_dev};
+      const void* asig[5] = {h->tape, h->save_times, d_dLdout, h->out_dev, fused ? h : nullptr};
       if (h->adj_graph && std::memcmp(asig, h->adj_graph_sig, sizeof(asig)) != 0) {
         (void)hipGraphExecDestroy(h->adj_graph);
         h->adj_graph = nullptr;
@@ -1492,7 +1628,11 @@ int backward_impl(node_handle* h, const float* d_dLdout, node_stats* st) {
     }
     HIPCHK(h, hipGetLastError());
   }
-  launch_adj_step_begin(sg, ab, h->ctl, GATE_ALWAYS, h->stream);
+  // lambda of the last step (and, on the GEMM path, mu: the fused step has
+  // written the accepted mu to the buffer that gsel_mu_ selects)
+  AdjBufs abf = ab;
+  if (fused) abf.P = 0;
+  launch_adj_step_begin(sg, abf, h->ctl, GATE_ALWAYS, h->stream);
   if (int rc = poll_ctl(h)) return rc;
   HIPCHK(h, hipGetLastError());
   const Ctl& r = *h->hctl;
@@ -2092,7 +2232,8 @@ int32_t node_forward(node_handle_t* h, const node_solve_opts* opts, const float*
   if (!u0) return fail(h, NODE_ERR_INVALID, "u0 is NULL");
   if (h->cnf) return fail(h, NODE_ERR_UNSUPPORTED, "CNF handle: use node_cnf_forward");
   if (n_saveat < 0 || (n_saveat > 0 && !saveat)) return fail(h, NODE_ERR_INVALID, "bad saveat");
-  if (int rc = maybe_autotune(h)) return rc;  // before u0 is staged in the scratch buffer
+  if (!chain_on(h) || !chain_adj_on(h))
+    if (int rc = maybe_autotune(h)) return rc;  // before u0 is staged in the scratch buffer
   float* du0 = h->scratch;  // u0 staged through the scratch state buffer
   HIPCHK(h, hipMemcpyAsync(du0, u0, (size_t)h->B * h->D * sizeof(float), hipMemcpyHostToDevice, h->stream));
   int rc = forward_impl(h, opts, du0, saveat, n_saveat, stats);
@@ -2116,7 +2257,8 @@ int32_t node_cnf_forward(node_handle_t* h, const node_solve_opts* opts, const fl
   if (!h->have_params) return fail(h, NODE_ERR_STATE, "parameters not set");
   h->cnf_fwd = false;
   if (int rc = ensure_adjoint(h)) return rc;  // Lm holds the probe for the data-gradient GEMMs
-  if (int rc = maybe_autotune(h)) return rc;
+  if (!chain_on(h) || !chain_adj_on(h))
+    if (int rc = maybe_autotune(h)) return rc;
   const int dm = h->cnf_dm, B = h->B;
   if (!h->probe && dalloc_t(h, &h->probe, (size_t)h->Bp * dm * sizeof(float))) return NODE_ERR_HIP;
   if (!h->fbuf && dalloc_t(h, &h->fbuf, (size_t)h->Bp * dm * sizeof(float))) return NODE_ERR_HIP;

@@ -15,7 +15,7 @@ CSRC = os.path.join(PKG_ROOT, "csrc")
 INCLUDE = os.path.join(REPO, "include")
 LIB = os.path.join(HERE, "libnode_hip.so")
 
-SOURCES = ["kernels.hip", "pack_kernels.hip", "chain_fwd.hip",
+SOURCES = ["kernels.hip", "pack_kernels.hip", "chain_fwd.hip", "chain_adj.hip",
            "node_hip.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
