@@ -15,6 +15,9 @@ struct ChainModel {
   const float* bias[MAXL];
   int pitch;                   // LDS row pitch (elements)
   int nw;                      // waves per workgroup (4 or 8)
+  // LDS byte offsets after the activation buffers: partial products of the
+  // narrow layers (0: over the activations), hidden biases (rows of wmax), probe
+  int lds_part, lds_bias, lds_probe, lds_bytes, wmax;
 };
 struct ChainPack {
   int nl;
@@ -53,8 +56,10 @@ struct ChainAdjArgs {
   float* lam; float* lam_new; float* kl;   // kl: slots 0 and 6 of 8 stage slots are used
   const float* dLdout;
   const float* probe;
-  float* slope; float* curve;  // act' (and act'' adot, flow) of the hidden layers, [l][rows][wmax]
-  int wmax;
+  // act' (and act'' adot, flow) of the hidden layers: per block and layer
+  // `stiles` feature tiles, each [primal column tile][lane][4]
+  float* slope; float* curve;
+  int stiles;
   // BacksolveAdjoint: u integrated with lambda (ubs != nullptr)
   float* ubs; float* ubs_new; float* ku; const float* fsaved; int ckpt;
   double* part;
@@ -80,14 +85,14 @@ struct ChainMuArgs {
   double* mu; float* g0;       // two mu buffers; gradient at the initial time
   double* part;
 };
-size_t chain_adj_lds(int prec, const ChainModel& m, int nt);
 void launch_chain_adj(int prec, int nt, bool cnf, const ChainAdjArgs& a, int grid, hipStream_t s);
 void launch_chain_wgrad(int prec, const ChainWgradArgs& a, hipStream_t s);
 void launch_chain_mu(const ChainMuArgs& a, int nblk, hipStream_t s);
 
 // nt: 16-column MFMA tiles per block (rows per block: 16 nt, a flow 8 nt)
 int chain_rows(int nt, bool cnf);
-size_t chain_fwd_lds(int prec, const ChainModel& m, int nt);
+// LDS layout of a model's step kernels (fills the lds_ fields)
+void chain_layout(ChainModel& m, int nt, bool cnf);
 void launch_chain_fwd(int prec, int nt, bool cnf, const ChainFwdArgs& a, int grid, hipStream_t s);
 
 }  // namespace nodehip

@@ -15,13 +15,15 @@
 namespace nodehip {
 
 template <class PP, int NT, int NW, bool CNF>
-__global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
+__global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdjArgs a) {
   using T = typename PP::T;
   constexpr int THREADS = 64 * NW;
   constexpr int COLS = 16 * NT, R = CNF ? 8 * NT : COLS;
   constexpr int NE = R * (CNF ? 32 : 64) / THREADS;
   constexpr int P = PP::SPLIT ? 2 : 1;
-  constexpr bool INPLACE = CNF && NT == 4;
+  constexpr bool INPLACE = CNF;
+  constexpr bool F32 = sizeof(T) == 4;
+  using Side = typename std::conditional<F32, ChainNoSide, ChainCopy<PP, THREADS>>::type;
   constexpr int NP = CNF ? NT / 2 : NT;        // column tiles of primal rows
   const ChainModel& m = a.m;
   const Ctl* ctl = a.ctl;
@@ -38,6 +40,7 @@ __global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
   const int gsel = ctl->gsel;
 
   int row[NE], col[NE];
+  float ld[NE];                                // a flow's lambda_dlogp of the row (constant)
   float lam[NE], k[7][NE], ub[NE];
   const int acc_ = mode == SM_STEP ? ctl->last_accept : 0;
   const int jidx = mode == SM_STEP ? ctl->jump_idx : -1;
@@ -49,7 +52,7 @@ __global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
     const int i = tid + e * THREADS;
     row[e] = i / D;
     col[e] = i - row[e] * D;
-    lam[e] = ub[e] = 0.f;
+    lam[e] = ub[e] = ld[e] = 0.f;
 #pragma unroll
     for (int s = 0; s < 7; ++s) k[s][e] = 0.f;
     if (i >= ne) continue;
@@ -57,6 +60,7 @@ __global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
     float l = acc_ ? a.lam_new[idx] : a.lam[idx];
     if (acc_ && jidx >= 0 && idx < nreal) l += a.dLdout[(int64_t)jidx * nreal + idx];
     lam[e] = l;
+    if (CNF && row0 + row[e] < m.B) ld[e] = a.lam[(int64_t)(row0 + row[e]) * D + m.dm];
     if (mode != SM_INIT_F0) k[0][e] = acc_ ? a.kl[6 * a.sv + idx] : a.kl[idx];
     if (acc_) { a.lam[idx] = l; a.kl[idx] = k[0][e]; }
     if (bs) {
@@ -71,29 +75,53 @@ __global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
   const int plane = COLS * m.pitch;
   const int other = INPLACE ? 0 : P * plane;
   const ChainBuf<PP> in0{0, m.pitch, plane};
-  float* part = (float*)(chain_lds() + (INPLACE ? 1 : 2) * P * plane * sizeof(T));
+  float* part = (float*)(chain_lds() + m.lds_part);
+  const float* lbias = (const float*)(chain_lds() + m.lds_bias);
+  const float* lprobe = (const float*)(chain_lds() + m.lds_probe);
+  __shared__ ChainShared sh;
+  chain_stage_init<THREADS, R, CNF, true>(m, ctl, sh, mode, a.probe, row0);
+  const float h0 = (float)(ctl->tdir * ctl->dt0);
+  const int64_t orows = a.ops.rows;
+  const int64_t sbase = (int64_t)blockIdx.x * (L - 1) * a.stiles;  // tiles of act' before the block
+  // FP32: where layer l's inputs / output gradients of the block go; split:
+  // the copy that takes them there from an LDS buffer
+  auto rows_at = [&](char* ob, int64_t off, int w) { return (T*)(ob + off) + orow0 * w; };
+  auto copy_of = [&](int buf, char* ob, int64_t off, int w, int used) {
+    if constexpr (F32) return Side{};
+    else return Side(ChainBuf<PP>{buf, m.pitch, plane}, ob + off, orows, orow0, w, used, COLS);
+  };
+  // u(t_s): the tape's entries are loaded a stage ahead
+  float tv[8][NE];
+  auto tape_load = [&](int is) {
+    const float* te = a.tape + (int64_t)sh.step[is] * a.ent + e0;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      const int i = tid + e * THREADS;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) tv[j][e] = te[j * a.sv + (i < ne ? i : 0)];
+    }
+  };
   double sum = 0.0, flag = 0.0;
   const int s0 = mode == SM_STEP && !re ? 1 : 0, s1 = mode == SM_STEP ? 7 : 1;
+  if (!bs) tape_load(mode == SM_INIT_F1 ? 7 : s0);
   for (int s = s0; s < s1; ++s) {
     const int slot = s == 0 ? (mode == SM_INIT_F1 ? 2 : gsel) : s == 6 ? (gsel ^ 1) : s + 1;
     char* ob = (char*)a.ops.base + (int64_t)slot * a.ops.slot;
     const int is = mode == SM_INIT_F1 ? 7 : s;   // interpolation slot
-    const double ts = mode == SM_INIT_F1 ? ctl->t + ctl->tdir * ctl->dt0 : ctl->t + dC[s] * ctl->dt;
+    const float ts = sh.A[s][7];
     // stage inputs: x = map(u(t_s)) now, lambda_s after the hidden recompute
-    const float* te = a.tape + (int64_t)ctl->st_step[is] * a.ent;
-    const bool ex = ctl->st_exact[is] != 0;
-    const float tdt = ctl->st_dt[is];
-    T* h0 = (T*)(ob + a.ops.h[0]);
-    const int64_t hpl = a.ops.rows * a.ops.w[0];
+    const bool ex = sh.exact[is] != 0;
+    const float tdt = sh.w[is][7];
     float ls[NE], us[NE];
+    T* const x0r = rows_at(ob, a.ops.h[0], a.ops.w[0]);
     {
       const int kin = m.ktf[0] * ChainK<PP>::KT;
       for (int i = tid; i < COLS * (kin - m.dm); i += THREADS) {
         const int r = i / (kin - m.dm), c = m.dm + i % (kin - m.dm);
         const bool tc = CNF && m.tcat && c == m.dm && r < R;
-        const float v = tc && row0 + r < m.B ? (float)ts : 0.f;
+        const float v = tc && row0 + r < m.B ? ts : 0.f;
         put<PP>(in0.at(r, c), plane, v);
-        if (tc) put<PP>(h0 + (orow0 + r) * a.ops.w[0] + c, hpl, v);
+        if constexpr (F32) if (tc) x0r[r * a.ops.w[0] + c] = v;
       }
     }
 #pragma unroll
@@ -105,38 +133,37 @@ __global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
       float u;
       if (bs) {
         // (u's stage values stay in memory: each is read by its own thread)
-        if (mode == SM_INIT_F1) u = ub[e] + (float)(ctl->tdir * ctl->dt0) * a.ku[idx];
+        if (mode == SM_INIT_F1) u = ub[e] + h0 * a.ku[idx];
         else {
           float sm = 0.f;
-          for (int j = s - 1; j >= 0; --j) sm += chA[s][j] * a.ku[j * a.sv + idx];
+          for (int j = s - 1; j >= 0; --j) sm += sh.A[s][j] * a.ku[j * a.sv + idx];
           u = ub[e] + dt * sm;
         }
       } else {
-        u = te[idx];
+        u = tv[0][e];
         if (!ex) {
           float sm = 0.f;
 #pragma unroll
-          for (int j = 0; j < 7; ++j) sm += ctl->st_w[is][j] * te[(1 + j) * a.sv + idx];
+          for (int j = 0; j < 7; ++j) sm += sh.w[is][j] * tv[1 + j][e];
           u += tdt * sm;
         }
       }
       us[e] = u;
-      if (mode == SM_INIT_F1) ls[e] = lam[e] + (float)(ctl->tdir * ctl->dt0) * k[0][e];
+      if (mode == SM_INIT_F1) ls[e] = lam[e] + h0 * k[0][e];
       else {
         float sm = 0.f;
 #pragma unroll
-        for (int j = 5; j >= 0; --j) sm += chA[s][j] * k[j][e];
+        for (int j = 5; j >= 0; --j) sm += sh.A[s][j] * k[j][e];
         ls[e] = lam[e] + dt * sm;
       }
       if (col[e] < m.dm) {
         const float x = map_f(m.map, u);
         put<PP>(in0.at(row[e], col[e]), plane, x);
-        put<PP>(h0 + (orow0 + row[e]) * a.ops.w[0] + col[e], hpl, x);
+        if constexpr (F32) x0r[row[e] * a.ops.w[0] + col[e]] = x;
         if constexpr (CNF) {
-          const int g = row0 + row[e];
-          const float p = g < m.B ? a.probe[(int64_t)g * m.dm + col[e]] : 0.f;
+          const float p = lprobe[row[e] * m.dm + col[e]];
           put<PP>(in0.at(R + row[e], col[e]), plane, p);
-          put<PP>(h0 + (orow0 + R + row[e]) * a.ops.w[0] + col[e], hpl, p);
+          if constexpr (F32) x0r[(R + row[e]) * a.ops.w[0] + col[e]] = p;
         }
       }
     }
@@ -149,7 +176,8 @@ __global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
         if (bs) a.ubs_new[e0 + i] = us[e];
       }
     }
-    __syncthreads();
+    if (!bs && s + 1 < s1) tape_load(s + 1);
+    chain_barrier();
     // hidden recompute (a flow: with its tangent chain), act' and the
     // second-order factor act'' adot kept for the way back.  The lane that
     // writes an entry of them reads it again below: both sweeps deal a
@@ -157,59 +185,65 @@ __global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
     int cur = 0;
     for (int l = 0; l < L - 1; ++l) {
       const ChainBuf<PP> in{cur, m.pitch, plane}, o{other - cur, m.pitch, plane};
-      const float* bias = m.bias[l];
-      const int act = m.act[l], w = a.ops.w[l + 1];
-      T* hd = (T*)(ob + a.ops.h[l + 1]);
-      const int64_t pl = a.ops.rows * w;
-      float* sl = a.slope + ((int64_t)l * a.ops.rows + orow0) * a.wmax;
-      float* cv = a.curve + ((int64_t)l * a.ops.rows + orow0) * a.wmax;
-      auto epi = [&](int t, f32x4v (&acc)[NT]) {
+      const float* bias = lbias + l * m.wmax;
+      const int act = m.act[l];
+      T* const hr = rows_at(ob, a.ops.h[l + 1], a.ops.w[l + 1]);
+      const int hw = a.ops.w[l + 1];
+      // act' (FP32 derives it from the stored output instead) and act'' adot in
+      // the lanes' own order: whole lines per access
+      f32x4v* sl = (f32x4v*)a.slope + (sbase + (int64_t)l * a.stiles) * NP * 64 + lane;
+      f32x4v* cv = (f32x4v*)a.curve + (sbase + (int64_t)l * a.stiles) * NP * 64 + lane;
+      auto epi = [&](int t, int, f32x4v (&acc)[NT]) {
         const int f = 16 * t + 4 * (lane >> 4);
         const f32x4v bv = *(const f32x4v*)(bias + f);
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
           const int r = 16 * q + (lane & 15);
-          const f32x4v z = acc[q] + bv, y = act_f4(act, z), d = act_d4(act, z, y);
+          const f32x4v z = acc[q] + bv, y = act_f4(act, z);
           chain_put4<PP>(o, r, f, y);
-          const float yv[4] = {y.x, y.y, y.z, y.w};
-          put4<PP>(hd + (orow0 + r) * w + f, pl, yv);
-          *(f32x4v*)(sl + (int64_t)r * a.wmax + f) = d;
+          if constexpr (F32) *(f32x4v*)(hr + r * hw + f) = y;
+          else sl[(t * NP + q) * 64] = act_d4(act, z, y);
           if constexpr (CNF) {
+            const f32x4v d = act_d4(act, z, y);
             const f32x4v tv = acc[q + NP] * d;
             chain_put4<PP>(o, R + r, f, tv);
-            const float tw[4] = {tv.x, tv.y, tv.z, tv.w};
-            put4<PP>(hd + (orow0 + R + r) * w + f, pl, tw);
+            if constexpr (F32) *(f32x4v*)(hr + (R + r) * hw + f) = tv;
             // act'' adot in closed form (act' adot = t)
             f32x4v c2 = {0.f, 0.f, 0.f, 0.f};
             if (act == 1) c2 = -2.f * y * tv;
             else if (act == 2) c2 = tv * (1.f - d);
             else if (act == 4) c2 = tv * (1.f - 2.f * y);
-            *(f32x4v*)(cv + (int64_t)r * a.wmax + f) = c2;
+            cv[(t * NP + q) * 64] = c2;
           }
         }
       };
-      chain_layer<PP, NT, NW, INPLACE>(m.Wf[l], m.mtf[l], m.ktf[l], in, wave, lane, epi);
+      // (split: the layer's input leaves for the weight gradients meanwhile)
+      Side copy = copy_of(cur, ob, a.ops.h[l], a.ops.w[l], m.ktf[l] * ChainK<PP>::KT);
+      chain_layer<PP, NT, NW, INPLACE>(m.Wf[l], m.mtf[l], m.ktf[l], in, wave, lane, copy,
+                                       [](int, int) {}, epi);
       cur = other - cur;
     }
     const int ll = L - 1;
+    // the last layer's input: copied under its own products (backsolve), or
+    // here
+    Side lastc = copy_of(cur, ob, a.ops.h[ll], a.ops.w[ll], m.ktf[ll] * ChainK<PP>::KT);
     float fu[NE];
     if (bs) {  // f(u_s): u's own stage value
       const int mt = m.mtf[ll];
-      chain_narrow<PP, NT, NW>(m.Wf[ll], mt, m.ktf[ll], ChainBuf<PP>{cur, m.pitch, plane}, part,
-                               wave, lane);
+      chain_narrow<PP, NT, NW, INPLACE>(m.Wf[ll], mt, m.ktf[ll], ChainBuf<PP>{cur, m.pitch, plane}, part,
+                                        wave, lane, lastc);
 #pragma unroll
       for (int e = 0; e < NE; ++e)
         fu[e] = tid + e * THREADS < ne
                     ? chain_sum<NW, NT>(part, mt, row[e], col[e]) + m.bias[ll][col[e]] : 0.f;
-      __syncthreads();
+      chain_barrier();
     }
+    lastc.finish();
+    if constexpr (INPLACE && !F32) chain_barrier();
     // seeds at the output: lambda_s (a flow's tangent rows: -lambda_dlogp e)
     cur = other - cur;
     {
       const ChainBuf<PP> o{cur, m.pitch, plane};
-      T* dd = (T*)(ob + a.ops.d[ll]);
-      const int w = a.ops.w[L];
-      const int64_t pl = a.ops.rows * w;
       const int kin = m.ktb[ll] * ChainK<PP>::KT;
       for (int i = tid; i < COLS * (kin - m.dm); i += THREADS) {
         const int r = i / (kin - m.dm), c = m.dm + i % (kin - m.dm);
@@ -219,49 +253,66 @@ __global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
       for (int e = 0; e < NE; ++e) {
         const int i = tid + e * THREADS;
         if (i >= ne || col[e] >= m.dm) continue;
+        T* const dr = rows_at(ob, a.ops.d[ll], a.ops.w[L]);
         put<PP>(o.at(row[e], col[e]), plane, ls[e]);
-        put<PP>(dd + (orow0 + row[e]) * w + col[e], pl, ls[e]);
-        if constexpr (CNF) {  // (lambda_dlogp is constant over the solve)
-          const int g = row0 + row[e];
-          const float p = g < m.B ? -a.lam[(int64_t)g * D + m.dm] * a.probe[(int64_t)g * m.dm + col[e]] : 0.f;
+        if constexpr (F32) dr[row[e] * a.ops.w[L] + col[e]] = ls[e];
+        if constexpr (CNF) {
+          const float p = -ld[e] * lprobe[row[e] * m.dm + col[e]];
           put<PP>(o.at(R + row[e], col[e]), plane, p);
-          put<PP>(dd + (orow0 + R + row[e]) * w + col[e], pl, p);
+          if constexpr (F32) dr[(R + row[e]) * a.ops.w[L] + col[e]] = p;
         }
       }
     }
-    __syncthreads();
+    chain_barrier();
     for (int l = ll; l >= 1; --l) {
       const ChainBuf<PP> in{cur, m.pitch, plane}, o{other - cur, m.pitch, plane};
-      const int w = a.ops.w[l];
-      T* dd = (T*)(ob + a.ops.d[l - 1]);
-      const int64_t pl = a.ops.rows * w;
-      const float* sl = a.slope + ((int64_t)(l - 1) * a.ops.rows + orow0) * a.wmax;
-      const float* cv = a.curve + ((int64_t)(l - 1) * a.ops.rows + orow0) * a.wmax;
-      auto epi = [&](int t, f32x4v (&acc)[NT]) {
+      T* const dr = rows_at(ob, a.ops.d[l - 1], a.ops.w[l]);
+      const int dw = a.ops.w[l], act = m.act[l - 1];
+      const T* const hr = rows_at(ob, a.ops.h[l], dw);
+      const f32x4v* sl = (const f32x4v*)a.slope + (sbase + (int64_t)(l - 1) * a.stiles) * NP * 64 + lane;
+      const f32x4v* cv = (const f32x4v*)a.curve + (sbase + (int64_t)(l - 1) * a.stiles) * NP * 64 + lane;
+      // FP32 blocks read act' ahead of the products, the split ones have no
+      // registers left for it
+      constexpr int ME = F32 ? (INPLACE && NW == 4 ? 8 : 4) : 1;
+      f32x4v sd[ME][NP], c2[CNF ? ME : 1][NP];
+      auto read = [&](int t, int mi) {
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+          if constexpr (F32)
+            sd[mi][q] = *(const f32x4v*)(hr + (16 * q + (lane & 15)) * dw + 16 * t + 4 * (lane >> 4));
+          else sd[mi][q] = sl[(t * NP + q) * 64];
+          if constexpr (CNF) c2[mi][q] = cv[(t * NP + q) * 64];
+        }
+      };
+      auto pro = [&](int t, int mi) { if constexpr (F32) read(t, mi); };
+      auto epi = [&](int t, int mi, f32x4v (&acc)[NT]) {
         const int f = 16 * t + 4 * (lane >> 4);
+        const int i = F32 ? mi : 0;
+        if constexpr (!F32) read(t, 0);
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
           const int r = 16 * q + (lane & 15);
-          const f32x4v d = *(const f32x4v*)(sl + (int64_t)r * a.wmax + f);
+          f32x4v d = sd[i][q];
+          if constexpr (F32) d = act_y4(act, d);
           f32x4v v = acc[q] * d;
           if constexpr (CNF) {
-            const f32x4v c2 = *(const f32x4v*)(cv + (int64_t)r * a.wmax + f);
-            v += acc[q + NP] * c2;
+            v += acc[q + NP] * c2[i][q];
             const f32x4v tv = acc[q + NP] * d;
             chain_put4<PP>(o, R + r, f, tv);
-            const float tw[4] = {tv.x, tv.y, tv.z, tv.w};
-            put4<PP>(dd + (orow0 + R + r) * w + f, pl, tw);
+            if constexpr (F32) *(f32x4v*)(dr + (R + r) * dw + f) = tv;
           }
           chain_put4<PP>(o, r, f, v);
-          const float vw[4] = {v.x, v.y, v.z, v.w};
-          put4<PP>(dd + (orow0 + r) * w + f, pl, vw);
+          if constexpr (F32) *(f32x4v*)(dr + r * dw + f) = v;
         }
       };
-      chain_layer<PP, NT, NW, INPLACE>(m.Wb[l], m.mtb[l], m.ktb[l], in, wave, lane, epi);
+      Side copy = copy_of(cur, ob, a.ops.d[l], a.ops.w[l + 1], m.ktb[l] * ChainK<PP>::KT);
+      chain_layer<PP, NT, NW, INPLACE>(m.Wb[l], m.mtb[l], m.ktb[l], in, wave, lane, copy, pro, epi);
       cur = other - cur;
     }
     const int mt = m.mtb[0];
-    chain_narrow<PP, NT, NW>(m.Wb[0], mt, m.ktb[0], ChainBuf<PP>{cur, m.pitch, plane}, part, wave, lane);
+    Side copy0 = copy_of(cur, ob, a.ops.d[0], a.ops.w[1], m.ktb[0] * ChainK<PP>::KT);
+    chain_narrow<PP, NT, NW, INPLACE>(m.Wb[0], mt, m.ktb[0], ChainBuf<PP>{cur, m.pitch, plane}, part,
+                                      wave, lane, copy0);
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
       const int i = tid + e * THREADS;
@@ -313,19 +364,13 @@ __global__ void __launch_bounds__(64 * NW) k_chain_adj(ChainAdjArgs a) {
     }
     // (the next stage's inputs go to buffer 0; `part` is written again only
     // after the barriers of its layers)
-    __syncthreads();
+    chain_barrier();
   }
   block_reduce_store(sum, flag, a.part, blockIdx.x);
 }
 
-size_t chain_adj_lds(int prec, const ChainModel& m, int nt) {
-  (void)prec;  // FP32, or two BF16 planes: four bytes per value
-  const size_t p0 = chain_part(m.nw, nt, m.mtf[m.L - 1]), p1 = chain_part(m.nw, nt, m.mtb[0]);
-  return (size_t)(nt == 4 ? 1 : 2) * 16 * nt * m.pitch * 4 + 4 * (p0 > p1 ? p0 : p1);
-}
-
 void launch_chain_adj(int prec, int nt, bool cnf, const ChainAdjArgs& a, int grid, hipStream_t s) {
-  const size_t lds = chain_adj_lds(prec, a.m, nt);
+  const size_t lds = a.m.lds_bytes;
   const int nw = a.m.nw;
   auto go = [&](auto kern) {
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

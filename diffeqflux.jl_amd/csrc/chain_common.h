@@ -71,6 +71,23 @@ __device__ __forceinline__ unsigned char* chain_lds() {
   extern __shared__ __attribute__((aligned(16))) unsigned char ch_lds[];
   return ch_lds;
 }
+// Barrier that orders LDS only (__syncthreads also waits for every global
+// access in flight).  Nothing that waves hand to each other here goes through
+// global memory: entries stored there are read by the lane that wrote them, or
+// by another launch.
+__device__ __forceinline__ void chain_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+// What every stage reads, in LDS: tableau rows, stage times and (adjoint) the
+// interpolation data of the stage times, and the hidden layers' biases.  As
+// scalar loads these cost a stage several dependent trips to memory.
+struct ChainShared {
+  float A[7][8];               // tableau rows; column 7: the stage time
+  float w[8][8];               // interpolation weights of a slot; column 7: its step
+  int step[8], exact[8];
+};
 // A buffer of activations in LDS: [plane][row][pitch] elements at `off`
 template <class PP> struct ChainBuf {
   int off, pitch, plane;
@@ -81,11 +98,12 @@ template <class PP> struct ChainBuf {
 
 // acc[m][n] += W tiles (first tile t0, MT of them, K tiles [k0, k1)) x columns.
 // The fragments of PF K tiles are in flight (ring in registers, loads
-// unconditional: the index is clamped instead).
-template <class PP, int NT, int MT, int PF>
+// unconditional: the index is clamped instead).  side.step(): a piece of other
+// work per K tile.
+template <class PP, int NT, int MT, int PF, class Side>
 __device__ __forceinline__ void chain_mma(f32x4v (&acc)[MT][NT], const void* __restrict__ W, int t0,
                                           int tlast, int kt, int k0, int k1, const ChainBuf<PP>& in,
-                                          int lane) {
+                                          int lane, Side& side) {
   constexpr int P = PP::SPLIT ? 2 : 1;
   const u32x4* w[MT];
 #pragma unroll
@@ -121,12 +139,68 @@ __device__ __forceinline__ void chain_mma(f32x4v (&acc)[MT][NT], const void* __r
   int k = k0;
   for (; k + PF <= k1; k += PF) {
 #pragma unroll
-    for (int j = 0; j < PF; ++j) step(a[j], k + j, true);
+    for (int j = 0; j < PF; ++j) {
+      step(a[j], k + j, true);
+      side.step();
+    }
   }
 #pragma unroll
   for (int j = 0; j < PF - 1; ++j)
     if (k + j < k1) step(a[j], k + j, false);
 }
+
+// FP32 blocks write their operand rows where they are produced (16 bytes per
+// lane; the copy's index arithmetic below cost the small blocks 5-25%).  Split
+// ones, at twice the values per row block and 8-byte pieces, copy:
+//
+// Copy of a block's activations (rows 0 .. rows of `buf`, all planes) from LDS
+// to an operand matrix of the weight gradients, 16 bytes per lane along the
+// rows.  Done a piece per K tile of the layer that reads the same buffer: as
+// stores of the producing epilogue all workgroups' writes met in the same
+// short phase (8-byte pieces of 16 rows each) while memory idled under the
+// products.
+struct ChainNoSide {
+  __device__ __forceinline__ void step() {}
+  __device__ __forceinline__ void finish() {}
+};
+template <class PP, int THREADS> struct ChainCopy {
+  static constexpr int E = 16 / sizeof(typename PP::T);  // elements per piece
+  ChainBuf<PP> buf;
+  typename PP::T* dst;         // the block's first row
+  int64_t plane;               // elements between the planes
+  int w, cpr, n, pos;          // row width, pieces per row, pieces, next piece
+  float rcpr;
+  u32x4 held;
+  typename PP::T* to;
+  __device__ __forceinline__ ChainCopy(ChainBuf<PP> b, void* base, int64_t rows, int64_t row0, int w_,
+                                       int used, int nrow)
+      : buf(b), dst((typename PP::T*)base + row0 * w_), plane(rows * w_), w(w_), cpr(used / E),
+        n((PP::SPLIT ? 2 : 1) * nrow * (used / E)), pos(threadIdx.x), rcpr(1.f / (used / E)),
+        held{0, 0, 0, 0}, to(nullptr) {
+    rows_ = nrow;
+  }
+  int rows_;
+  __device__ __forceinline__ void flush() {
+    if (to) *(u32x4*)to = held;
+    to = nullptr;
+  }
+  __device__ __forceinline__ void step() {
+    flush();
+    if (pos < n) {
+      int r = (int)(((float)pos + 0.5f) * rcpr);     // (exact: pos < 2^22)
+      const int c = (pos - r * cpr) * E;
+      int p = 0;
+      if (PP::SPLIT && r >= rows_) { p = 1; r -= rows_; }
+      held = *(const u32x4*)(buf.at(r, c) + p * buf.plane);
+      to = dst + p * plane + r * w + c;
+      pos += THREADS;
+    }
+  }
+  __device__ __forceinline__ void finish() {
+    while (pos < n) step();
+    flush();
+  }
+};
 
 // ring depth: enough K tiles in flight to cover an L2 read (~600 cycles)
 // against MT * NT * (128 FP32 / 48 split) MFMA cycles per tile (a fragment is
@@ -136,82 +210,129 @@ template <class PP, int NT, int MT> constexpr int chain_pf() {
   return c >= 768 ? 1 : c >= 192 ? 2 : 4;
 }
 
-template <class PP, int NT, int MT, class Epi>
+// One chunk of MT tiles.  pro(tile, m): loads that the epilogue needs, issued
+// before the products; epi(tile, m, acc[NT]).
+template <class PP, int NT, int MT, class Side, class Pro, class Epi>
 __device__ __forceinline__ void chain_chunk(const void* W, int t0, int tlast, int kt,
-                                            const ChainBuf<PP>& in, int lane, bool sync, Epi&& epi) {
+                                            const ChainBuf<PP>& in, int lane, bool sync, Side& side,
+                                            Pro&& pro, Epi&& epi) {
   f32x4v acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) pro(t0 + m < tlast ? t0 + m : tlast, m);
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int n = 0; n < NT; ++n) acc[m][n] = (f32x4v){0.f, 0.f, 0.f, 0.f};
-  chain_mma<PP, NT, MT, chain_pf<PP, NT, MT>()>(acc, W, t0, tlast, kt, 0, kt, in, lane);
-  if (sync) __syncthreads();  // in place: every wave has read the inputs
+  chain_mma<PP, NT, MT, chain_pf<PP, NT, MT>()>(acc, W, t0, tlast, kt, 0, kt, in, lane, side);
+  if (sync) {  // in place: every wave has read the inputs
+    side.finish();
+    chain_barrier();
+  }
 #pragma unroll
   for (int m = 0; m < MT; ++m)
-    if (t0 + m <= tlast) epi(t0 + m, acc[m]);
+    if (t0 + m <= tlast) epi(t0 + m, m, acc[m]);
 }
 
 // One wide layer (mt output tiles over the waves): epi(tile, acc[NT]) for
 // every tile.  INPLACE: the outputs may overwrite the inputs (a wave holds all
 // its tiles' accumulators until the barrier; mt <= 4 NW); else chunks of at
 // most four tiles and the output goes to another buffer.  Ends with a barrier.
-template <class PP, int NT, int NW, bool INPLACE, class Epi>
+template <class PP, int NT, int NW, bool INPLACE, class Side, class Pro, class Epi>
 __device__ __forceinline__ void chain_layer(const void* W, int mt, int kt, const ChainBuf<PP>& in,
-                                            int wave, int lane, Epi&& epi) {
+                                            int wave, int lane, Side& side, Pro&& pro,
+                                            Epi&& epi) {
   const int per = (mt + NW - 1) / NW;
   int t = wave * per;
   const int last = (t + per < mt ? t + per : mt) - 1;
   if constexpr (INPLACE) {
     // (a wave without tiles computes the last one again and drops it)
     const int tl = last < mt - 1 ? last : mt - 1;
-    if (per > 2) chain_chunk<PP, NT, 4>(W, t, tl, kt, in, lane, true, epi);
-    else if (per > 1) chain_chunk<PP, NT, 2>(W, t, tl, kt, in, lane, true, epi);
-    else chain_chunk<PP, NT, 1>(W, t, tl, kt, in, lane, true, epi);
+    // (mt <= 32; the eight-tile chunk would cost an eight-wave block spills)
+    if constexpr (NW == 4) {
+      if (per > 4) {
+        chain_chunk<PP, NT, 8>(W, t, tl, kt, in, lane, true, side, pro, epi);
+        chain_barrier();
+        return;
+      }
+    }
+    if (per > 2) chain_chunk<PP, NT, 4>(W, t, tl, kt, in, lane, true, side, pro, epi);
+    else if (per > 1) chain_chunk<PP, NT, 2>(W, t, tl, kt, in, lane, true, side, pro, epi);
+    else chain_chunk<PP, NT, 1>(W, t, tl, kt, in, lane, true, side, pro, epi);
   } else {
-    for (; t + 4 <= last + 1; t += 4) chain_chunk<PP, NT, 4>(W, t, last, kt, in, lane, false, epi);
-    if (t + 2 <= last + 1) { chain_chunk<PP, NT, 2>(W, t, last, kt, in, lane, false, epi); t += 2; }
-    if (t <= last) chain_chunk<PP, NT, 1>(W, t, last, kt, in, lane, false, epi);
+    for (; t + 4 <= last + 1; t += 4) chain_chunk<PP, NT, 4>(W, t, last, kt, in, lane, false, side, pro, epi);
+    if (t + 2 <= last + 1) { chain_chunk<PP, NT, 2>(W, t, last, kt, in, lane, false, side, pro, epi); t += 2; }
+    if (t <= last) chain_chunk<PP, NT, 1>(W, t, last, kt, in, lane, false, side, pro, epi);
+    side.finish();
   }
-  __syncthreads();
+  chain_barrier();
 }
 
 // A narrow layer (state-sized output, mt <= 4 tiles): the K tiles are split
-// over the waves left over (at most four splits, two where the block's
-// activations leave LDS for no more); partial products go to LDS as FP32
-// [split][row][16 mt + 4], summed by the reader.  Ends with a barrier.
-template <int NW, int NT> __host__ __device__ __forceinline__ int chain_splits(int mt) {
-  const int s = NW / mt, most = NT == 4 ? 2 : 4;
-  return s > most ? most : s;
+// over the waves left over (at most four splits); partial products go to LDS
+// as FP32 [split][row][16 mt + 4], summed by the reader.  Ends with a barrier.
+template <int NW> __host__ __device__ __forceinline__ int chain_splits(int mt) {
+  const int s = NW / mt;
+  return s > 4 ? 4 : s;
 }
-template <class PP, int NT, int NW>
+// ALIAS: the partial products overwrite the activations.
+template <class PP, int NT, int NW, bool ALIAS, class Side>
 __device__ __forceinline__ void chain_narrow(const void* W, int mt, int kt, const ChainBuf<PP>& in,
-                                             float* part, int wave, int lane) {
-  const int ks = chain_splits<NW, NT>(mt), t = wave % mt, s = wave / mt;
-  if (s < ks) {
-    f32x4v acc[1][NT];
+                                             float* part, int wave, int lane, Side& side) {
+  const int ks = chain_splits<NW>(mt), t = wave % mt, s = wave / mt;
+  f32x4v acc[1][NT];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) acc[0][n] = (f32x4v){0.f, 0.f, 0.f, 0.f};
-    const int k0 = kt * s / ks, k1 = kt * (s + 1) / ks;
-    if (k0 < k1) chain_mma<PP, NT, 1, 4>(acc, W, t, t, kt, k0, k1, in, lane);
+  for (int n = 0; n < NT; ++n) acc[0][n] = (f32x4v){0.f, 0.f, 0.f, 0.f};
+  const int k0 = kt * s / ks, k1 = kt * (s + 1) / ks;
+  if (s < ks && k0 < k1) chain_mma<PP, NT, 1, 4>(acc, W, t, t, kt, k0, k1, in, lane, side);
+  side.finish();
+  if constexpr (ALIAS) chain_barrier();
+  if (s < ks) {
     const int pd = 16 * mt + 4;
     float* o = part + s * (16 * NT) * pd + (lane & 15) * pd + 16 * t + 4 * (lane >> 4);
 #pragma unroll
     for (int n = 0; n < NT; ++n) *(f32x4v*)(o + n * 16 * pd) = acc[0][n];
   }
-  __syncthreads();
+  chain_barrier();
 }
 template <int NW, int NT>
 __device__ __forceinline__ float chain_sum(const float* part, int mt, int row, int c) {
-  const int ks = chain_splits<NW, NT>(mt), pd = 16 * mt + 4;
+  const int ks = chain_splits<NW>(mt), pd = 16 * mt + 4;
   float v = part[row * pd + c];
   for (int s = 1; s < ks; ++s) v += part[(s * 16 * NT + row) * pd + c];
   return v;
 }
-// floats of the partial products
-inline size_t chain_part(int nw, int nt, int mt) {
-  const int ks = nw == 8 ? (nt == 4 ? chain_splits<8, 4>(mt) : chain_splits<8, 1>(mt))
-                         : chain_splits<4, 1>(mt);
-  return (size_t)ks * 16 * nt * (16 * mt + 4);
+
+// Fills ChainShared, the biases and the probe (rows [row0, row0 + R) of
+// [B][dm], zero past B).  Ends with a barrier.
+template <int THREADS, int R, bool CNF, bool ADJ>
+__device__ __forceinline__ void chain_stage_init(const ChainModel& m, const Ctl* ctl, ChainShared& sh,
+                                                 int mode, const float* probe, int row0) {
+  const int tid = threadIdx.x;
+  if (tid < 56) {
+    const int s = tid >> 3, j = tid & 7;
+    float v;
+    if (j < 7) v = chA[s][j];
+    else v = (float)(mode == SM_INIT_F1 ? ctl->t + ctl->tdir * ctl->dt0
+                     : mode == SM_STEP ? ctl->t + dC[s] * ctl->dt : ctl->t);
+    sh.A[s][j] = v;
+  }
+  if constexpr (ADJ) {
+    const int i = tid - 64;
+    if (i >= 0 && i < 64) {
+      const int s = i >> 3, j = i & 7;
+      sh.w[s][j] = j < 7 ? ctl->st_w[s][j] : ctl->st_dt[s];
+      if (j == 0) { sh.step[s] = ctl->st_step[s]; sh.exact[s] = ctl->st_exact[s]; }
+    }
+  }
+  float* lb = (float*)(chain_lds() + m.lds_bias);
+  for (int l = 0; l < m.L - 1; ++l)
+    for (int i = tid; i < 16 * m.mtf[l]; i += THREADS) lb[l * m.wmax + i] = m.bias[l][i];
+  if constexpr (CNF) {
+    float* lp = (float*)(chain_lds() + m.lds_probe);
+    for (int i = tid; i < R * m.dm; i += THREADS)
+      lp[i] = row0 + i / m.dm < m.B ? probe[(int64_t)row0 * m.dm + i] : 0.f;
+  }
+  __syncthreads();
 }
 
 // activation of four values, chosen once
@@ -230,6 +351,17 @@ __device__ __forceinline__ f32x4v act_d4(int a, f32x4v z, f32x4v y) {
     case 2: return (f32x4v){act_d(2, z.x, y.x), act_d(2, z.y, y.y), act_d(2, z.z, y.z), act_d(2, z.w, y.w)};
     case 3: return (f32x4v){act_d(3, z.x, y.x), act_d(3, z.y, y.y), act_d(3, z.z, y.z), act_d(3, z.w, y.w)};
     case 4: return (f32x4v){act_d(4, z.x, y.x), act_d(4, z.y, y.y), act_d(4, z.z, y.z), act_d(4, z.w, y.w)};
+    default: return (f32x4v){1.f, 1.f, 1.f, 1.f};
+  }
+}
+
+// act' of four FP32 outputs
+__device__ __forceinline__ f32x4v act_y4(int a, f32x4v y) {
+  switch (a) {
+    case 1: return (f32x4v){act_d(1, 0.f, y.x), act_d(1, 0.f, y.y), act_d(1, 0.f, y.z), act_d(1, 0.f, y.w)};
+    case 2: return (f32x4v){act_d_y(2, y.x), act_d_y(2, y.y), act_d_y(2, y.z), act_d_y(2, y.w)};
+    case 3: return (f32x4v){act_d_y(3, y.x), act_d_y(3, y.y), act_d_y(3, y.z), act_d_y(3, y.w)};
+    case 4: return (f32x4v){act_d(4, 0.f, y.x), act_d(4, 0.f, y.y), act_d(4, 0.f, y.z), act_d(4, 0.f, y.w)};
     default: return (f32x4v){1.f, 1.f, 1.f, 1.f};
   }
 }

@@ -7,6 +7,8 @@
 // chain of the wide layers (FP32) or by the weights' way from L2 (split BF16);
 // it replaces eight kernels per right-hand side whose launches and drains cost
 // more than their work at these sizes.
+#include <algorithm>
+
 #include "chain_common.h"
 
 namespace nodehip {
@@ -46,13 +48,13 @@ __device__ __forceinline__ void chain_saves(const ChainFwdArgs& a, int64_t e0, i
 }
 
 template <class PP, int NT, int NW, bool CNF>
-__global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
+__global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwdArgs a) {
   using T = typename PP::T;
   constexpr int CH_THREADS = 64 * NW;
   constexpr int COLS = 16 * NT, R = CNF ? 8 * NT : COLS;
   constexpr int NE = R * (CNF ? 32 : 64) / CH_THREADS;  // state entries per thread (D <= 64, flow 32)
   constexpr int P = PP::SPLIT ? 2 : 1;
-  constexpr bool INPLACE = CNF && NT == 4;
+  constexpr bool INPLACE = CNF;
   const ChainModel& m = a.m;
   const Ctl* ctl = a.ctl;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -67,12 +69,16 @@ __global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
   const int plane = COLS * m.pitch;
   const int other = INPLACE ? 0 : P * plane;  // offset of the second buffer
   const ChainBuf<PP> in0{0, m.pitch, plane};
-  float* part = (float*)(chain_lds() + (INPLACE ? 1 : 2) * P * plane * sizeof(T));
+  float* part = (float*)(chain_lds() + m.lds_part);
+  const float* lbias = (const float*)(chain_lds() + m.lds_bias);
+  const float* lprobe = (const float*)(chain_lds() + m.lds_probe);
+  __shared__ ChainShared sh;
+  chain_stage_init<64 * NW, R, CNF, false>(m, ctl, sh, mode, a.probe, row0);
 
   const int64_t n = mode == SM_STEP ? ctl->n : 0;
   float* ent = a.tape + tape_slot(ctl, n) * a.ent;
   float* nxt = a.tape + tape_slot(ctl, n + 1) * a.ent;
-  const float dt = (float)ctl->dt;
+  const float dt = (float)ctl->dt, h0 = (float)(ctl->tdir * ctl->dt0);
   const float atol = (float)ctl->abstol, rtol = (float)ctl->reltol;
 
   // this thread's state entries: row and column in the block
@@ -92,18 +98,18 @@ __global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
     }
   }
   double sum = 0.0, flag = 0.0;
+  ChainNoSide none;
   const int s0 = mode == SM_STEP ? 1 : 0, s1 = mode == SM_STEP ? 7 : 1;
   float un[NE];
   for (int s = s0; s < s1; ++s) {
     // stage input
-    const double ts = mode == SM_STEP ? ctl->t + dC[s] * ctl->dt
-                      : mode == SM_INIT_F1 ? ctl->t + ctl->tdir * ctl->dt0 : ctl->t;
+    const float ts = sh.A[s][7];
     const int kin = m.ktf[0] * ChainK<PP>::KT;
     for (int i = tid; i < COLS * (kin - m.dm); i += CH_THREADS) {
       // columns past the model's own: zeros (the time column is written below)
       const int r = i / (kin - m.dm), c = m.dm + i % (kin - m.dm);
       const bool tc = CNF && m.tcat && c == m.dm && r < R;
-      put<PP>(in0.at(r, c), plane, tc ? (float)ts : 0.f);
+      put<PP>(in0.at(r, c), plane, tc ? ts : 0.f);
     }
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
@@ -112,19 +118,16 @@ __global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
       if (mode == SM_STEP) {
         float sm = 0.f;
 #pragma unroll
-        for (int j = 5; j >= 0; --j) sm += chA[s][j] * k[j][e];
+        for (int j = 5; j >= 0; --j) sm += sh.A[s][j] * k[j][e];
         v = u[e] + dt * sm;
         un[e] = v;
       } else if (mode == SM_INIT_F1) {
-        v = u[e] + (float)(ctl->tdir * ctl->dt0) * k[0][e];
+        v = u[e] + h0 * k[0][e];
       }
       if (col[e] < m.dm) {
         put<PP>(in0.at(row[e], col[e]), plane, map_f(m.map, v));
-        if constexpr (CNF) {
-          const int g = row0 + row[e];
-          put<PP>(in0.at(R + row[e], col[e]), plane,
-                  g < m.B ? a.probe[(int64_t)g * m.dm + col[e]] : 0.f);
-        }
+        if constexpr (CNF)
+          put<PP>(in0.at(R + row[e], col[e]), plane, lprobe[row[e] * m.dm + col[e]]);
       }
     }
     if (mode == SM_STEP && s == 6) {
@@ -132,13 +135,13 @@ __global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
       for (int e = 0; e < NE; ++e)
         if (tid + e * CH_THREADS < ne) nxt[e0 + tid + e * CH_THREADS] = un[e];
     }
-    __syncthreads();
+    chain_barrier();
     int cur = 0;
     for (int l = 0; l < L - 1; ++l) {
       const ChainBuf<PP> in{cur, m.pitch, plane}, o{other - cur, m.pitch, plane};
-      const float* bias = m.bias[l];
+      const float* bias = lbias + l * m.wmax;
       const int act = m.act[l];
-      auto epi = [&](int t, f32x4v (&acc)[NT]) {
+      auto epi = [&](int t, int, f32x4v (&acc)[NT]) {
         const int f = 16 * t + 4 * (lane >> 4);
         const f32x4v bv = *(const f32x4v*)(bias + f);
 #pragma unroll
@@ -149,11 +152,12 @@ __global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
             chain_put4<PP>(o, R + 16 * q + (lane & 15), f, acc[q + NT / 2] * act_d4(act, z, y));
         }
       };
-      chain_layer<PP, NT, NW, INPLACE>(m.Wf[l], m.mtf[l], m.ktf[l], in, wave, lane, epi);
+      chain_layer<PP, NT, NW, INPLACE>(m.Wf[l], m.mtf[l], m.ktf[l], in, wave, lane, none,
+                                       [](int, int) {}, epi);
       cur = other - cur;
     }
     const int ll = L - 1, mt = m.mtf[ll];
-    chain_narrow<PP, NT, NW>(m.Wf[ll], mt, m.ktf[ll], ChainBuf<PP>{cur, m.pitch, plane}, part, wave, lane);
+    chain_narrow<PP, NT, NW, INPLACE>(m.Wf[ll], mt, m.ktf[ll], ChainBuf<PP>{cur, m.pitch, plane}, part, wave, lane, none);
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
       const int i = tid + e * CH_THREADS;
@@ -163,10 +167,8 @@ __global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
         kv = act_f(m.act[ll], chain_sum<NW, NT>(part, mt, row[e], col[e]) + m.bias[ll][col[e]]);
       } else {  // log p: minus the probe's directional derivative of f
         kv = 0.f;
-        const int g = row0 + row[e];
-        if (g < m.B)
-          for (int c = 0; c < m.dm; ++c)
-            kv -= a.probe[(int64_t)g * m.dm + c] * chain_sum<NW, NT>(part, mt, R + row[e], c);
+        for (int c = 0; c < m.dm; ++c)
+          kv -= lprobe[row[e] * m.dm + c] * chain_sum<NW, NT>(part, mt, R + row[e], c);
       }
       const int64_t idx = e0 + i;
       const bool live = row0 + row[e] < m.B;
@@ -200,20 +202,30 @@ __global__ void __launch_bounds__(64 * NW) k_chain_fwd(ChainFwdArgs a) {
         }
       }
     }
+    chain_barrier();  // (in place: the partial products lie over the next stage's inputs)
   }
   if (a.part) block_reduce_store(sum, flag, a.part, blockIdx.x);
 }
 
-static size_t chain_elt(int prec) { return prec == 0 ? 4 : prec == 1 ? 2 : 4; }  // bytes of all planes
-
-size_t chain_fwd_lds(int prec, const ChainModel& m, int nt) {
-  const bool inplace = nt == 4;
-  return (size_t)(inplace ? 1 : 2) * 16 * nt * m.pitch * chain_elt(prec) +
-         4 * chain_part(m.nw, nt, m.mtf[m.L - 1]);
+void chain_layout(ChainModel& m, int nt, bool cnf) {
+  // four bytes per activation: FP32, or two BF16 planes
+  const int cols = 16 * nt, act = (cnf ? 1 : 2) * cols * m.pitch * 4;
+  const int mt[2] = {m.mtf[m.L - 1], m.mtb[0]};
+  int part = 0;
+  m.wmax = 4;
+  for (int x : mt) {
+    const int ks = m.nw == 8 ? chain_splits<8>(x) : chain_splits<4>(x);
+    part = std::max(part, ks * cols * (16 * x + 4) * 4);
+  }
+  for (int l = 0; l < m.L - 1; ++l) m.wmax = std::max(m.wmax, 16 * m.mtf[l]);
+  m.lds_part = cnf ? 0 : act;
+  m.lds_bias = cnf ? std::max(act, part) : act + part;
+  m.lds_probe = m.lds_bias + (m.L - 1) * m.wmax * 4;
+  m.lds_bytes = m.lds_probe + (cnf ? chain_rows(nt, true) * m.dm * 4 : 0);
 }
 
 void launch_chain_fwd(int prec, int nt, bool cnf, const ChainFwdArgs& a, int grid, hipStream_t s) {
-  const size_t lds = chain_fwd_lds(prec, a.m, nt);
+  const size_t lds = a.m.lds_bytes;
   const int nw = a.m.nw;
   auto go = [&](auto kern) {
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);

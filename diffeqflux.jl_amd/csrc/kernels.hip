@@ -218,31 +218,6 @@ __device__ __forceinline__ void epi_apply(const EpiHidden& e, f32x16 (&acc)[MR][
     tile_write<ST, false, BR, BC, NT>(lds, sv, g, lane, (ST*)e.S, e.ldo, 0, (ST*)nullptr, 0, 0);
 }
 
-// act' from the activation's output y (identity, softplus, relu):
-// softplus'(z) = sigmoid(z) = 1 - exp(-y) with y = softplus(z) > 0; below
-// y = 1/4 its Taylor series to y^6 (relative truncation < 5e-8, no
-// cancellation), above it the hardware exp2 (relative error < 1e-6)
-__device__ __forceinline__ float act_d_y(int a, float y) {
-  switch (a) {
-    case 2: {
-      if (y < 0.25f) {
-        float t = 1.f - y * (1.f / 6.f);
-        t = 1.f - y * (1.f / 5.f) * t;
-        t = 1.f - y * 0.25f * t;
-        t = 1.f - y * (1.f / 3.f) * t;
-        t = 1.f - y * 0.5f * t;
-        return y * t;
-      }
-      return 1.f - __builtin_amdgcn_exp2f(-y * LOG2E_F);
-    }
-    case 3: return y > 0.f ? 1.f : 0.f;
-    default: return 1.f;
-  }
-}
-
-// activations whose derivative the epilogues derive from the output
-__device__ __forceinline__ bool act_from_output_d(int a) { return a == 0 || a == 2 || a == 3; }
-
 // act' of this thread's accumulator
 // elements, loaded while the GEMM's last K tile is computed (padded columns
 // read the zero-filled padding)

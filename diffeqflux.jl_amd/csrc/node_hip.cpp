@@ -218,7 +218,7 @@ struct node_handle {
 
   // fused step kernels: model in fragment order, column tiles per row block
   // (0: the forward runs on the GEMM path)
-  ChainModel chain{};
+  ChainModel chain{}, chain_adj{};
   int chain_nt = 0;
   // fused adjoint steps: column tiles per row block (0: GEMM path), operand
   // store of the weight gradients, act' / act'' adot, partial sums
@@ -227,7 +227,7 @@ struct node_handle {
   ChainMuArgs cmu{};
   float* cslope = nullptr;
   float* ccurve = nullptr;
-  int cwmax = 0;
+  int cstiles = 0;
 
   // profiling (node_prof_enable)
   uint64_t prof_mask = 0;
@@ -679,18 +679,18 @@ void vjp_eval(node_handle* h, int stage, int mode, int gate, int wflags, float c
 }
 
 // ---------------------------------------------------------------- fused steps
-// Blocks of 16 rows (a flow's 16 columns of primal and tangent rows each) are
-// doubled when they would outnumber the CUs: the weights then pass L2 once
-// for twice the rows.
+// Column tiles of a row block.  One (16 rows), or two for a split-BF16 forward
+// whose blocks would outnumber the CUs: the weights then pass L2 once for twice
+// the rows.  A flow's two (four) tiles are 16 (32) primal and as many tangent
+// rows.
 int chain_tiles(const node_handle* h) {
-  const bool two = h->prec == NODE_PREC_BF16X3 && h->B > 16 * 256;
-  return h->cnf ? (two ? 4 : 2) : (two ? 2 : 1);
+  const bool many = h->prec == NODE_PREC_BF16X3 && h->B > 16 * 256;
+  return (h->cnf ? 2 : 1) * (many ? 2 : 1);
 }
 
 // Whether the forward runs as fused steps, and its model description (without
 // the weights' addresses).  Widths are bounded by LDS (the activations of a
-// row block) and by the in-place form of the four-tile block (32 tiles of
-// outputs).
+// row block) and by a flow's in-place layers (32 tiles of outputs).
 bool chain_plan(node_handle* h, ChainModel& m) {
   m = ChainModel{};
   if (h->prec == NODE_PREC_BF16 || h->cnf_reg || h->cnf_exact) return false;
@@ -718,13 +718,14 @@ bool chain_plan(node_handle* h, ChainModel& m) {
   for (int l = 0; l < h->L; ++l) weights += (int64_t)h->layers[l].in * h->layers[l].out;
   if (weights > 700000) return false;
   m.pitch = wide + (h->prec == NODE_PREC_FP32 ? 4 : 8);
-  // two waves per SIMD where every wave of them has a tile of the wide layers
-  // (the four-tile in-place block needs them: four tiles per wave at 512)
+  // eight waves (two per SIMD) where the wide layers have a tile for each; the
+  // larger blocks are built for eight
   m.nw = wide >= 128 || chain_tiles(h) > (h->cnf ? 2 : 1) ? 8 : 4;
   return true;
 }
 
 // Layout of the operand store (without its address).
+constexpr int CHAIN_LDS_MAX = 159 * 1024;  // (static LDS of the kernels aside)
 constexpr int64_t CHAIN_OPS_MAX = int64_t(4) << 30;  // bytes a handle may keep for it
 ChainOps chain_ops(const node_handle* h, int nt) {
   ChainOps o{};
@@ -746,8 +747,9 @@ int chain_alloc(node_handle* h) {
   ChainModel m;
   if (!chain_plan(h, m)) return 0;
   int nt = chain_tiles(h);
-  if (chain_fwd_lds(h->prec, m, nt) > 160 * 1024) nt = h->cnf ? 2 : 1;
-  if (chain_fwd_lds(h->prec, m, nt) > 160 * 1024) return 0;
+  chain_layout(m, nt, h->cnf);
+  if (m.lds_bytes > CHAIN_LDS_MAX) chain_layout(m, nt = h->cnf ? 2 : 1, h->cnf);
+  if (m.lds_bytes > CHAIN_LDS_MAX) return 0;
   if ((h->B + chain_rows(nt, h->cnf) - 1) / chain_rows(nt, h->cnf) > MAX_PART) return 0;
   const int V = h->prec == NODE_PREC_FP32 ? 4 : 8;
   for (int l = 0; l < h->L; ++l) {
@@ -760,14 +762,16 @@ int chain_alloc(node_handle* h) {
   }
   h->chain = m;
   h->chain_nt = nt;
-  // adjoint: linear last layer; a block's registers hold one column tile of
-  // rows with 64 state entries each (a flow's 32: two or four tiles)
+  // adjoint: linear last layer; one column tile of rows, a flow as its forward
   const int ant = h->cnf ? nt : 1;
-  if (h->layers[h->L - 1].act == NODE_ACT_IDENTITY &&
-      chain_adj_lds(h->prec, m, ant) <= 160 * 1024 &&
+  ChainModel am = m;
+  chain_layout(am, ant, h->cnf);
+  if (h->layers[h->L - 1].act == NODE_ACT_IDENTITY && am.lds_bytes <= CHAIN_LDS_MAX &&
       (h->B + chain_rows(ant, h->cnf) - 1) / chain_rows(ant, h->cnf) <= MAX_PART &&
-      chain_ops(h, ant).slot * 7 <= CHAIN_OPS_MAX)
+      chain_ops(h, ant).slot * 7 <= CHAIN_OPS_MAX) {
     h->chain_ant = ant;
+    h->chain_adj = am;
+  }
   return 0;
 }
 
@@ -775,10 +779,10 @@ int chain_alloc(node_handle* h) {
 int chain_adj_alloc(node_handle* h) {
   if (h->cops.base) return 0;
   ChainOps o = chain_ops(h, h->chain_ant);
-  const ChainModel& m = h->chain;
-  h->cwmax = 0;
-  for (int l = 0; l < h->L - 1; ++l) h->cwmax = std::max(h->cwmax, o.w[l + 1]);
-  const size_t sc = (size_t)std::max(h->L - 1, 1) * o.rows * std::max(h->cwmax, 4) * sizeof(float);
+  const ChainModel& m = h->chain_adj;
+  h->cstiles = 1;
+  for (int l = 0; l < h->L - 1; ++l) h->cstiles = std::max(h->cstiles, m.mtf[l]);
+  const size_t sc = (size_t)std::max(h->L - 1, 1) * o.rows * 16 * h->cstiles * sizeof(float);
   if (int rc = dalloc_t(h, &h->cslope, sc)) return rc;
   if (h->cnf)
     if (int rc = dalloc_t(h, &h->ccurve, sc)) return rc;
@@ -830,7 +834,7 @@ int chain_mu_blocks(const node_handle* h) {
 // heuristic: row pass, weight gradients, parameter state and its norm.
 void chain_adjoint(node_handle* h, const AdjBufs& ab, int mode, double* px, double* pm) {
   ChainAdjArgs a{};
-  a.m = h->chain;
+  a.m = h->chain_adj;
   a.ops = h->cops;
   a.tape = h->tape;
   a.sv = (int64_t)h->Bp * h->D;
@@ -838,7 +842,7 @@ void chain_adjoint(node_handle* h, const AdjBufs& ab, int mode, double* px, doub
   a.lam = ab.lam; a.lam_new = ab.lam_new; a.kl = ab.kl;
   a.dLdout = ab.dLdout;
   a.probe = h->probe;
-  a.slope = h->cslope; a.curve = h->ccurve; a.wmax = h->cwmax;
+  a.slope = h->cslope; a.curve = h->ccurve; a.stiles = h->cstiles;
   a.ubs = ab.ubs; a.ubs_new = ab.ubs_new; a.ku = ab.ku; a.fsaved = ab.fsaved; a.ckpt = ab.ckpt;
   a.part = px; a.ctl = h->ctl; a.mode = mode;
   launch_chain_adj(h->prec, h->chain_ant, h->cnf, a, chain_adj_grid(h), h->stream);
