@@ -1648,24 +1648,22 @@ void launch_fwd_step_begin(const StateGeom& sg, const float* tape, void* X0, int
 }
 
 // ---------------------------------------------------------------- controllers
+// Sum (and largest flag) of n partial pairs over a 256-thread block, in a fixed
+// order; the result in every thread.
 __device__ double block_sum_parts(const double* part, int n, double* flag_out) {
-  __shared__ double rs[256], rf[256];
+  __shared__ double rs[4], rf[4];
   double s = 0.0, f = 0.0;
   for (int i = threadIdx.x; i < n; i += blockDim.x) { s += part[2 * i]; f = fmax(f, part[2 * i + 1]); }
-  rs[threadIdx.x] = s;
-  rf[threadIdx.x] = f;
-  __syncthreads();
-  for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      rs[threadIdx.x] += rs[threadIdx.x + w];
-      rf[threadIdx.x] = fmax(rf[threadIdx.x], rf[threadIdx.x + w]);
-    }
-    __syncthreads();
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    s += __shfl_xor(s, off);
+    f = fmax(f, __shfl_xor(f, off));
   }
-  const double out = rs[0], fo = rf[0];
+  __syncthreads();  // (an earlier call's result has been read)
+  if ((threadIdx.x & 63) == 0) { rs[threadIdx.x >> 6] = s; rf[threadIdx.x >> 6] = f; }
   __syncthreads();
-  if (flag_out) *flag_out = fo;
-  return out;
+  if (flag_out) *flag_out = fmax(fmax(rf[0], rf[1]), fmax(rf[2], rf[3]));
+  return (rs[0] + rs[1]) + (rs[2] + rs[3]);
 }
 
 // SciMLBase sol(tau) on the forward record: exact stored state at a step
@@ -2021,16 +2019,11 @@ void launch_mu_norm(int mode, const AdjBufs& ab, const Ctl* ctl, double* part, i
   hipLaunchKernelGGL(k_mu_norm, dim3(nblk), dim3(EW_THREADS), 0, s, mode, ab, ctl, part, gate);
 }
 
-__global__ void k_adj_controller(Ctl* c, const double* pl, int nl, const double* pm, int nm,
-                                 double nel, const double* cbt, const double* ft) {
-  if (c->done) return;
-  double flag = 0.0;
-  const double sl = block_sum_parts(pl, nl, &flag);
-  const double sm = block_sum_parts(pm, nm, nullptr);
-  if (threadIdx.x != 0) return;
+// accept / reject, tstop and jump bookkeeping of one adjoint attempt (one
+// thread); false: the solve ended or pauses
+__device__ bool adj_control(Ctl* c, double eest, double flag, const double* cbt) {
   c->nf += c->fsal_reeval ? 7 : 6;
-  const double eest = c->adaptive ? sqrt((sl + sm) / nel) : 0.0;
-  if (c->adaptive && isnan(eest)) { c->retcode = 3; c->done = 1; c->commit_mu = 0; c->last_accept = 0; c->jump_idx = -1; return; }
+  if (c->adaptive && isnan(eest)) { c->retcode = 3; c->done = 1; c->commit_mu = 0; c->last_accept = 0; c->jump_idx = -1; return false; }
   const bool acc = pi_control(c, eest);
   c->accepted = acc;
   c->fsal_reeval = 0;
@@ -2053,8 +2046,8 @@ __global__ void k_adj_controller(Ctl* c, const double* pl, int nl, const double*
       c->save_next -= 1;
       c->fsal_reeval = 1;
     }
-    if (flag != 0.0) { c->retcode = 6; c->done = 1; return; }
-    if (c->t == c->t_end) { c->retcode = 1; c->done = 1; return; }
+    if (flag != 0.0) { c->retcode = 6; c->done = 1; return false; }
+    if (c->t == c->t_end) { c->retcode = 1; c->done = 1; return false; }
     c->dt = c->dtpropose;
   } else {
     c->nreject += 1;
@@ -2069,9 +2062,38 @@ __global__ void k_adj_controller(Ctl* c, const double* pl, int nl, const double*
     // and resumes (k_adj_resume sets the stage interpolation data)
     c->paused = 1;
     c->done = 1;
-    return;
+    return false;
   }
-  for (int s = 0; s < 7; ++s) set_interp(c, s, c->t + dC[s] * c->dt, ft);
+  return true;
+}
+
+// One block.  Latency only: the control itself is one thread's, the forward
+// steps that the next attempt's seven stage times fall in are looked up by
+// seven threads at once, in times copied to LDS beside the partial sums (one
+// thread's seven binary searches in global memory took half of the kernel:
+// 12 -> 8 us).
+constexpr int AC_TIMES = 512;
+__global__ void k_adj_controller(Ctl* c, const double* pl, int nl, const double* pm, int nm,
+                                 double nel, const double* cbt, const double* ft) {
+  __shared__ double times[AC_TIMES];
+  __shared__ Ctl lc;           // the block control, worked on in LDS
+  __shared__ int go;
+  static_assert(sizeof(Ctl) % 8 == 0, "copied by 8-byte words");
+  double* lw = (double*)&lc;
+  for (int i = threadIdx.x; i < (int)(sizeof(Ctl) / 8); i += blockDim.x) lw[i] = ((const double*)c)[i];
+  __syncthreads();
+  if (lc.done) return;
+  const int64_t nt = lc.n_fwd + 1;
+  for (int64_t i = threadIdx.x; i < nt && i < AC_TIMES; i += blockDim.x) times[i] = ft[i];
+  double flag = 0.0;
+  const double sl = block_sum_parts(pl, nl, &flag);
+  const double sm = block_sum_parts(pm, nm, nullptr);
+  if (threadIdx.x == 0) go = adj_control(&lc, lc.adaptive ? sqrt((sl + sm) / nel) : 0.0, flag, cbt);
+  __syncthreads();
+  if (go && threadIdx.x < 7)
+    set_interp(&lc, threadIdx.x, lc.t + dC[threadIdx.x] * lc.dt, nt <= AC_TIMES ? times : ft);
+  __syncthreads();
+  for (int i = threadIdx.x; i < (int)(sizeof(Ctl) / 8); i += blockDim.x) ((double*)c)[i] = lw[i];
 }
 
 // Resume a paused adjoint on the forward interval just re-solved (n_fwd
