@@ -15,6 +15,7 @@ struct ChainModel {
   const float* bias[MAXL];
   int pitch;                   // LDS row pitch (elements)
   int nw;                      // waves per workgroup (4 or 8)
+  int kt;                      // features per K tile
   // LDS byte offsets after the activation buffers: partial products of the
   // narrow layers (0: over the activations), hidden biases (rows of wmax), probe
   int lds_part, lds_bias, lds_probe, lds_bytes, wmax;

@@ -41,7 +41,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
 
   int row[NE], col[NE];
   float ld[NE];                                // a flow's lambda_dlogp of the row (constant)
-  float lam[NE], k[7][NE], ub[NE];
+  float lam[NE], k[7][NE], kl[NE], ub[NE];     // kl: the last stage's k
   const int acc_ = mode == SM_STEP ? ctl->last_accept : 0;
   const int jidx = mode == SM_STEP ? ctl->jump_idx : -1;
   const bool re = mode == SM_STEP && ctl->fsal_reeval;
@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
     const int i = tid + e * THREADS;
     row[e] = i / D;
     col[e] = i - row[e] * D;
-    lam[e] = ub[e] = ld[e] = 0.f;
+    lam[e] = ub[e] = ld[e] = kl[e] = 0.f;
 #pragma unroll
     for (int s = 0; s < 7; ++s) k[s][e] = 0.f;
     if (i >= ne) continue;
@@ -62,6 +62,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
     lam[e] = l;
     if (CNF && row0 + row[e] < m.B) ld[e] = a.lam[(int64_t)(row0 + row[e]) * D + m.dm];
     if (mode != SM_INIT_F0) k[0][e] = acc_ ? a.kl[6 * a.sv + idx] : a.kl[idx];
+    kl[e] = k[0][e];
     if (acc_) { a.lam[idx] = l; a.kl[idx] = k[0][e]; }
     if (bs) {
       float u = acc_ ? a.ubs_new[idx] : a.ubs[idx];
@@ -79,7 +80,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
   const float* lbias = (const float*)(chain_lds() + m.lds_bias);
   const float* lprobe = (const float*)(chain_lds() + m.lds_probe);
   __shared__ ChainShared sh;
-  chain_stage_init<THREADS, R, CNF, true>(m, ctl, sh, mode, a.probe, row0);
+  chain_stage_init<PP, THREADS, R, CNF, true>(m, ctl, sh, mode, a.probe, row0);
   const float h0 = (float)(ctl->tdir * ctl->dt0);
   const int64_t orows = a.ops.rows;
   const int64_t sbase = (int64_t)blockIdx.x * (L - 1) * a.stiles;  // tiles of act' before the block
@@ -96,9 +97,10 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
     const float* te = a.tape + (int64_t)sh.step[is] * a.ent + e0;
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
-      const int i = tid + e * THREADS;
+      if (e * THREADS >= ne) continue;   // (uniform: small states use the first entry only)
+      const int i = tid + e * THREADS < ne ? tid + e * THREADS : 0;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) tv[j][e] = te[j * a.sv + (i < ne ? i : 0)];
+      for (int j = 0; j < 8; ++j) tv[j][e] = (te + j * a.sv)[i];
     }
   };
   double sum = 0.0, flag = 0.0;
@@ -109,6 +111,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
     char* ob = (char*)a.ops.base + (int64_t)slot * a.ops.slot;
     const int is = mode == SM_INIT_F1 ? 7 : s;   // interpolation slot
     const float ts = sh.A[s][7];
+    const ChainRK rk(sh, s, dt);
     // stage inputs: x = map(u(t_s)) now, lambda_s after the hidden recompute
     const bool ex = sh.exact[is] != 0;
     const float tdt = sh.w[is][7];
@@ -116,54 +119,55 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
     T* const x0r = rows_at(ob, a.ops.h[0], a.ops.w[0]);
     {
       const int kin = m.ktf[0] * ChainK<PP>::KT;
-      for (int i = tid; i < COLS * (kin - m.dm); i += THREADS) {
-        const int r = i / (kin - m.dm), c = m.dm + i % (kin - m.dm);
+      for (int c = m.dm + tid / COLS; c < kin; c += THREADS / COLS) {
+        const int r = tid % COLS;
         const bool tc = CNF && m.tcat && c == m.dm && r < R;
         const float v = tc && row0 + r < m.B ? ts : 0.f;
-        put<PP>(in0.at(r, c), plane, v);
-        if constexpr (F32) if (tc) x0r[r * a.ops.w[0] + c] = v;
+        const int cp = chain_pos<PP>(c);
+        put<PP>(in0.at(r, cp), plane, v);
+        if constexpr (F32) if (tc) x0r[r * a.ops.w[0] + cp] = v;
       }
     }
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
       ls[e] = us[e] = 0.f;
+      if (e * THREADS >= ne) continue;
       const int i = tid + e * THREADS;
       if (i >= ne) continue;
       const int64_t idx = e0 + i;
       float u;
       if (bs) {
         // (u's stage values stay in memory: each is read by its own thread)
-        if (mode == SM_INIT_F1) u = ub[e] + h0 * a.ku[idx];
+        if (mode == SM_INIT_F1) u = fmaf(h0, a.ku[idx], ub[e]);
+        else if (s == 0) u = ub[e];
         else {
-          float sm = 0.f;
-          for (int j = s - 1; j >= 0; --j) sm += sh.A[s][j] * a.ku[j * a.sv + idx];
-          u = ub[e] + dt * sm;
+          float ku[7][1];  // (entries past the stage before are read, not used)
+#pragma unroll
+          for (int j = 0; j < 5; ++j) ku[j][0] = a.ku[j * a.sv + idx];
+          u = rk(ub[e], ku, a.ku[(s - 1) * a.sv + idx], 0);
         }
       } else {
         u = tv[0][e];
         if (!ex) {
           float sm = 0.f;
 #pragma unroll
-          for (int j = 0; j < 7; ++j) sm += sh.w[is][j] * tv[1 + j][e];
-          u += tdt * sm;
+          for (int j = 0; j < 7; ++j) sm = fmaf(sh.w[is][j], tv[1 + j][e], sm);
+          u = fmaf(tdt, sm, u);
         }
       }
       us[e] = u;
-      if (mode == SM_INIT_F1) ls[e] = lam[e] + h0 * k[0][e];
-      else {
-        float sm = 0.f;
-#pragma unroll
-        for (int j = 5; j >= 0; --j) sm += sh.A[s][j] * k[j][e];
-        ls[e] = lam[e] + dt * sm;
-      }
+      if (mode == SM_INIT_F1) ls[e] = fmaf(h0, k[0][e], lam[e]);
+      else if (s == 0) ls[e] = lam[e];
+      else ls[e] = rk(lam[e], k, kl[e], e);
       if (col[e] < m.dm) {
         const float x = map_f(m.map, u);
-        put<PP>(in0.at(row[e], col[e]), plane, x);
-        if constexpr (F32) x0r[row[e] * a.ops.w[0] + col[e]] = x;
+        const int cp = chain_pos<PP>(col[e]);
+        put<PP>(in0.at(row[e], cp), plane, x);
+        if constexpr (F32) x0r[row[e] * a.ops.w[0] + cp] = x;
         if constexpr (CNF) {
           const float p = lprobe[row[e] * m.dm + col[e]];
-          put<PP>(in0.at(R + row[e], col[e]), plane, p);
-          if constexpr (F32) x0r[(R + row[e]) * a.ops.w[0] + col[e]] = p;
+          put<PP>(in0.at(R + row[e], cp), plane, p);
+          if constexpr (F32) x0r[(R + row[e]) * a.ops.w[0] + cp] = p;
         }
       }
     }
@@ -235,7 +239,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
 #pragma unroll
       for (int e = 0; e < NE; ++e)
         fu[e] = tid + e * THREADS < ne
-                    ? chain_sum<NW, NT>(part, mt, row[e], col[e]) + m.bias[ll][col[e]] : 0.f;
+                    ? chain_sum<PP, NW, NT>(part, mt, m.ktf[ll], row[e], col[e]) + m.bias[ll][col[e]] : 0.f;
       chain_barrier();
     }
     lastc.finish();
@@ -245,21 +249,20 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
     {
       const ChainBuf<PP> o{cur, m.pitch, plane};
       const int kin = m.ktb[ll] * ChainK<PP>::KT;
-      for (int i = tid; i < COLS * (kin - m.dm); i += THREADS) {
-        const int r = i / (kin - m.dm), c = m.dm + i % (kin - m.dm);
-        put<PP>(o.at(r, c), plane, 0.f);
-      }
+      for (int c = m.dm + tid / COLS; c < kin; c += THREADS / COLS)
+        put<PP>(o.at(tid % COLS, chain_pos<PP>(c)), plane, 0.f);
 #pragma unroll
       for (int e = 0; e < NE; ++e) {
         const int i = tid + e * THREADS;
         if (i >= ne || col[e] >= m.dm) continue;
         T* const dr = rows_at(ob, a.ops.d[ll], a.ops.w[L]);
-        put<PP>(o.at(row[e], col[e]), plane, ls[e]);
-        if constexpr (F32) dr[row[e] * a.ops.w[L] + col[e]] = ls[e];
+        const int cp = chain_pos<PP>(col[e]);
+        put<PP>(o.at(row[e], cp), plane, ls[e]);
+        if constexpr (F32) dr[row[e] * a.ops.w[L] + cp] = ls[e];
         if constexpr (CNF) {
           const float p = -ld[e] * lprobe[row[e] * m.dm + col[e]];
-          put<PP>(o.at(R + row[e], col[e]), plane, p);
-          if constexpr (F32) dr[(R + row[e]) * a.ops.w[L] + col[e]] = p;
+          put<PP>(o.at(R + row[e], cp), plane, p);
+          if constexpr (F32) dr[(R + row[e]) * a.ops.w[L] + cp] = p;
         }
       }
     }
@@ -315,11 +318,12 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
                                       wave, lane, copy0);
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
+      if (e * THREADS >= ne) continue;
       const int i = tid + e * THREADS;
       if (i >= ne) continue;
       float kv = 0.f;                            // (log p column: lambda constant)
       if (!CNF || col[e] < m.dm) {
-        float g = chain_sum<NW, NT>(part, mt, row[e], col[e]);
+        float g = chain_sum<PP, NW, NT>(part, mt, m.ktb[0], row[e], col[e]);
         if (m.map == 1) g *= 3.f * us[e] * us[e];
         kv = -g;
       }
@@ -334,20 +338,19 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
         if (bs) a.ku[s * a.sv + idx] = fu[e];
         if (s == 6) {
           a.kl[6 * a.sv + idx] = kv;
-          float ut = chBT[6] * kv;
-#pragma unroll
-          for (int j = 0; j < 6; ++j) ut += chBT[j] * k[j][e];
+          const float ut = chain_err(k, e, kv);
           add(ut * dt, lam[e], ls[e]);
           if (live && isnan(ls[e])) flag = 1.0;
           if (bs) {
-            float uu = chBT[6] * fu[e];
-            for (int j = 0; j < 6; ++j) uu += chBT[j] * a.ku[j * a.sv + idx];
+            float uu = fmaf(chBT[6], fu[e], chBT[0] * a.ku[idx]);
+            for (int j = 1; j < 6; ++j) uu = fmaf(chBT[j], a.ku[j * a.sv + idx], uu);
             add(uu * dt, ub[e], us[e]);
             if (live && isnan(us[e])) flag = 1.0;
           }
         }
 #pragma unroll
         for (int j = 0; j < 6; ++j) k[j][e] = j == s ? kv : k[j][e];
+        kl[e] = kv;
       } else if (mode == SM_INIT_F0) {
         a.kl[idx] = kv;
         add(kv, lam[e], 0.f);
@@ -726,21 +729,33 @@ __global__ void __launch_bounds__(256) k_chain_mu(ChainMuArgs a) {
     while (l + 1 < w.m.L && i >= a.w0[l + 1]) ++l;
     const int out = w.m.out[l];
     int64_t src;
+    const bool f32 = E == 64;                      // (FP32 operand rows: chain_feat order)
     if (i < a.b0[l]) {
-      const int q = (int)(i - a.w0[l]), in = q / out, o = q % out;
+      const int q = (int)(i - a.w0[l]), qi = q / out, qo = q % out;
+      const int in = f32 ? chain_posn(qi) : qi, o = f32 ? chain_posn(qo) : qo;
       src = (int64_t)(w.tl[l] + in / E * w.tw[l] + o / E) * tsz + (in % E) * E + o % E;
     } else {
-      const int o = (int)(i - a.b0[l]);
+      const int qo = (int)(i - a.b0[l]), o = f32 ? chain_posn(qo) : qo;
       src = (int64_t)(w.tl[l] + o / E) * tsz + (int64_t)E * E + o % E;
     }
+    // (four ranges' loads in flight: a chain of 20 otherwise)
     float b = 0.f, e = 0.f;
-    if (w.mode == SM_STEP) {
-      for (int k = 0; k < w.chunks; ++k) {
-        b -= w.part[k * 2 * half + src];
-        e -= w.part[k * 2 * half + half + src];
+    const bool st = w.mode == SM_STEP;
+    const float* p = w.part + src;
+    int k = 0;
+    for (; k + 4 <= w.chunks; k += 4, p += 8 * half) {
+      float x[4], y[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        x[j] = p[2 * j * half];
+        y[j] = st ? p[(2 * j + 1) * half] : 0.f;
       }
-    } else {
-      for (int k = 0; k < w.chunks; ++k) b -= w.part[k * 2 * half + src];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) { b -= x[j]; e -= y[j]; }
+    }
+    for (; k < w.chunks; ++k, p += 2 * half) {
+      b -= p[0];
+      if (st) e -= p[half];
     }
     const double m = mu[i];
     double v;

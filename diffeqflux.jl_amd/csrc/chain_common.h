@@ -33,6 +33,23 @@ static __device__ const float chBT[7] = {-0.00178001105222577714, -0.00081643445
                                          0.5823571654525552,      -0.45808210592918697,
                                          0.015151515151515152};
 
+// Feature order of FP32 blocks.  An FP32 MFMA adds its K products one after the
+// other, so the order in which a dot product meets them is part of its
+// rounding; the adaptive solves' first error estimates sit on that rounding
+// (two terms of 1e-7 that cancel), and another order means other step sizes.
+// Features are therefore stored (LDS, operand rows, fragments) in an order
+// within each 16 that makes the four 16x16x4 steps take them as the GEMM path's
+// eight 32x32x2 steps do: 0 4 1 5 2 6 3 7, 8 12 9 13 10 14 11 15.
+__host__ __device__ __forceinline__ int chain_feat(int p) {  // position -> feature
+  return (p & ~15) + ((p & 2) << 2) + ((p >> 3) & 1) + ((p & 1) << 1) + (((p >> 2) & 1) << 2);
+}
+__host__ __device__ __forceinline__ int chain_posn(int f) {  // feature -> position
+  return (f & ~15) + ((f & 1) << 3) + (((f >> 2) & 1) << 2) + (((f >> 3) & 1) << 1) + ((f >> 1) & 1);
+}
+template <class PP> __device__ __forceinline__ int chain_pos(int f) {
+  return sizeof(typename PP::T) == 4 ? chain_posn(f) : f;
+}
+
 // features per K tile, values per lane and K tile
 template <class PP> struct ChainK { static constexpr int KT = 32, V = 8; };
 template <> struct ChainK<PF32> { static constexpr int KT = 16, V = 4; };
@@ -83,7 +100,7 @@ __device__ __forceinline__ void chain_barrier() {
 // What every stage reads, in LDS: tableau rows, stage times and (adjoint) the
 // interpolation data of the stage times, and the hidden layers' biases.  As
 // scalar loads these cost a stage several dependent trips to memory.
-struct ChainShared {
+struct alignas(16) ChainShared {
   float A[7][8];               // tableau rows; column 7: the stage time
   float w[8][8];               // interpolation weights of a slot; column 7: its step
   int step[8], exact[8];
@@ -202,11 +219,13 @@ template <class PP, int THREADS> struct ChainCopy {
   }
 };
 
-// ring depth: enough K tiles in flight to cover an L2 read (~600 cycles)
-// against MT * NT * (128 FP32 / 48 split) MFMA cycles per tile (a fragment is
-// refilled as soon as its MFMAs are issued)
+// ring depth: enough K tiles in flight to cover an L2 read under load (~1000
+// cycles) with two waves per SIMD at MT * NT * (128 FP32 / 48 split) MFMA
+// cycles per tile, as far as the registers go
 template <class PP, int NT, int MT> constexpr int chain_pf() {
-  const int c = MT * NT * (sizeof(typename PP::T) == 4 ? 128 : PP::SPLIT ? 48 : 16);
+  constexpr bool f32 = sizeof(typename PP::T) == 4;
+  const int c = MT * NT * (f32 ? 128 : PP::SPLIT ? 48 : 16);
+  if (f32) return c >= 512 ? 2 : 4;
   return c >= 768 ? 1 : c >= 192 ? 2 : 4;
 }
 
@@ -268,43 +287,96 @@ __device__ __forceinline__ void chain_layer(const void* W, int mt, int kt, const
 }
 
 // A narrow layer (state-sized output, mt <= 4 tiles): the K tiles are split
-// over the waves left over (at most four splits); partial products go to LDS
-// as FP32 [split][row][16 mt + 4], summed by the reader.  Ends with a barrier.
-template <int NW> __host__ __device__ __forceinline__ int chain_splits(int mt) {
+// over the waves; partial products go to LDS as FP32 [split][row][16 mt + 4],
+// summed by the reader.  Up to 64 inputs in two splits of 32 features (FP32:
+// the GEMM path's plan at these widths, see chain_feat), else four (the waves
+// left over).  ALIAS: the partial products overwrite the activations.  Ends
+// with a barrier.
+template <int NW> __host__ __device__ __forceinline__ int chain_splits(int mt, int kt, int KT) {
+  if (kt * KT <= 64) return 2;
   const int s = NW / mt;
   return s > 4 ? 4 : s;
 }
-// ALIAS: the partial products overwrite the activations.
 template <class PP, int NT, int NW, bool ALIAS, class Side>
 __device__ __forceinline__ void chain_narrow(const void* W, int mt, int kt, const ChainBuf<PP>& in,
                                              float* part, int wave, int lane, Side& side) {
-  const int ks = chain_splits<NW>(mt), t = wave % mt, s = wave / mt;
-  f32x4v acc[1][NT];
+  constexpr int KT = ChainK<PP>::KT;
+  const int ks = chain_splits<NW>(mt, kt, KT);
+  f32x4v acc[2][1][NT];
 #pragma unroll
-  for (int n = 0; n < NT; ++n) acc[0][n] = (f32x4v){0.f, 0.f, 0.f, 0.f};
-  const int k0 = kt * s / ks, k1 = kt * (s + 1) / ks;
-  if (s < ks && k0 < k1) chain_mma<PP, NT, 1, 4>(acc, W, t, t, kt, k0, k1, in, lane, side);
+  for (int u = 0; u < 2; ++u)
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[u][0][n] = (f32x4v){0.f, 0.f, 0.f, 0.f};
+  // (at most two units of work per wave: mt ks <= 2 NW)
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int w = wave + u * NW;
+    if (w >= mt * ks) break;
+    const int t = w % mt, s = w / mt;
+    int k0 = kt * s / ks, k1 = kt * (s + 1) / ks;
+    if (kt * KT <= 64) { k0 = s ? 32 / KT : 0; k1 = s ? kt : kt < 32 / KT ? kt : 32 / KT; }
+    if (k0 < k1) chain_mma<PP, NT, 1, 4>(acc[u], W, t, t, kt, k0, k1, in, lane, side);
+  }
   side.finish();
   if constexpr (ALIAS) chain_barrier();
-  if (s < ks) {
-    const int pd = 16 * mt + 4;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int w = wave + u * NW;
+    if (w >= mt * ks) break;
+    const int t = w % mt, s = w / mt, pd = 16 * mt + 4;
     float* o = part + s * (16 * NT) * pd + (lane & 15) * pd + 16 * t + 4 * (lane >> 4);
 #pragma unroll
-    for (int n = 0; n < NT; ++n) *(f32x4v*)(o + n * 16 * pd) = acc[0][n];
+    for (int n = 0; n < NT; ++n) *(f32x4v*)(o + n * 16 * pd) = acc[u][0][n];
   }
   chain_barrier();
 }
-template <int NW, int NT>
-__device__ __forceinline__ float chain_sum(const float* part, int mt, int row, int c) {
-  const int ks = chain_splits<NW>(mt), pd = 16 * mt + 4;
+template <class PP, int NW, int NT>
+__device__ __forceinline__ float chain_sum(const float* part, int mt, int kt, int row, int c) {
+  const int ks = chain_splits<NW>(mt, kt, ChainK<PP>::KT), pd = 16 * mt + 4;
   float v = part[row * pd + c];
   for (int s = 1; s < ks; ++s) v += part[(s * 16 * NT + row) * pd + c];
   return v;
 }
 
+// Runge-Kutta stage values u + dt sum_j A[s][j] k_j: the latest stage first,
+// the others in order, the first stage's product with dt * A (the GEMM path's
+// stage kernels' order; fused multiply-adds in words, since the compiler moves
+// sums across branches and then splits them).  The row is read once and the
+// terms are selected, not branched on: a dozen branches per entry were a tenth
+// of a small block's stage.  kl: the stage before s.
+struct ChainRK {
+  float w[5], wl, h;
+  int s;
+  __device__ __forceinline__ ChainRK(const ChainShared& sh, int s_, float dt) : s(s_) {
+    const f32x4v a = *(const f32x4v*)sh.A[s_];
+    w[0] = a.x; w[1] = a.y; w[2] = a.z; w[3] = a.w; w[4] = sh.A[s_][4];
+    wl = sh.A[s_][s_ > 0 ? s_ - 1 : 0];
+    h = s_ == 1 ? dt * wl : dt;
+  }
+  template <int NE>
+  __device__ __forceinline__ float operator()(float u, const float (&k)[7][NE], float kl, int e) const {
+    float sm = wl * kl;
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+      const float t = fmaf(w[j], k[j][e], sm);
+      sm = j < s - 1 ? t : sm;
+    }
+    sm = s == 1 ? kl : sm;
+    return fmaf(h, sm, u);
+  }
+};
+
+// error estimate / dt, the same way (k7: the last stage, not in `k` yet)
+template <int NE> __device__ __forceinline__ float chain_err(const float (&k)[7][NE], int e, float k7) {
+  float v = fmaf(chBT[6], k7, chBT[0] * k[0][e]);
+#pragma unroll
+  for (int j = 1; j < 6; ++j) v = fmaf(chBT[j], k[j][e], v);
+  return v;
+}
+
 // Fills ChainShared, the biases and the probe (rows [row0, row0 + R) of
 // [B][dm], zero past B).  Ends with a barrier.
-template <int THREADS, int R, bool CNF, bool ADJ>
+template <class PP, int THREADS, int R, bool CNF, bool ADJ>
 __device__ __forceinline__ void chain_stage_init(const ChainModel& m, const Ctl* ctl, ChainShared& sh,
                                                  int mode, const float* probe, int row0) {
   const int tid = threadIdx.x;
@@ -326,7 +398,7 @@ __device__ __forceinline__ void chain_stage_init(const ChainModel& m, const Ctl*
   }
   float* lb = (float*)(chain_lds() + m.lds_bias);
   for (int l = 0; l < m.L - 1; ++l)
-    for (int i = tid; i < 16 * m.mtf[l]; i += THREADS) lb[l * m.wmax + i] = m.bias[l][i];
+    for (int i = tid; i < 16 * m.mtf[l]; i += THREADS) lb[l * m.wmax + chain_pos<PP>(i)] = m.bias[l][i];
   if constexpr (CNF) {
     float* lp = (float*)(chain_lds() + m.lds_probe);
     for (int i = tid; i < R * m.dm; i += THREADS)

@@ -73,17 +73,18 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
   const float* lbias = (const float*)(chain_lds() + m.lds_bias);
   const float* lprobe = (const float*)(chain_lds() + m.lds_probe);
   __shared__ ChainShared sh;
-  chain_stage_init<64 * NW, R, CNF, false>(m, ctl, sh, mode, a.probe, row0);
+  chain_stage_init<PP, 64 * NW, R, CNF, false>(m, ctl, sh, mode, a.probe, row0);
 
   const int64_t n = mode == SM_STEP ? ctl->n : 0;
-  float* ent = a.tape + tape_slot(ctl, n) * a.ent;
-  float* nxt = a.tape + tape_slot(ctl, n + 1) * a.ent;
+  // (the block's entries: uniform bases, 32-bit offsets)
+  float* ent = a.tape + tape_slot(ctl, n) * a.ent + e0;
+  float* nxt = a.tape + tape_slot(ctl, n + 1) * a.ent + e0;
   const float dt = (float)ctl->dt, h0 = (float)(ctl->tdir * ctl->dt0);
   const float atol = (float)ctl->abstol, rtol = (float)ctl->reltol;
 
   // this thread's state entries: row and column in the block
   int row[NE], col[NE];
-  float u[NE], k[7][NE];
+  float u[NE], k[7][NE], kl[NE];               // kl: the last stage's k
 #pragma unroll
   for (int e = 0; e < NE; ++e) {
     const int i = tid + e * CH_THREADS;
@@ -93,9 +94,10 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
 #pragma unroll
     for (int s = 0; s < 7; ++s) k[s][e] = 0.f;
     if (i < ne) {
-      u[e] = ent[e0 + i];
-      if (mode == SM_STEP || mode == SM_INIT_F1) k[0][e] = ent[a.sv + e0 + i];
+      u[e] = ent[i];
+      if (mode == SM_STEP || mode == SM_INIT_F1) k[0][e] = (ent + a.sv)[i];
     }
+    kl[e] = k[0][e];
   }
   double sum = 0.0, flag = 0.0;
   ChainNoSide none;
@@ -104,36 +106,35 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
   for (int s = s0; s < s1; ++s) {
     // stage input
     const float ts = sh.A[s][7];
+    const ChainRK rk(sh, s, dt);
     const int kin = m.ktf[0] * ChainK<PP>::KT;
-    for (int i = tid; i < COLS * (kin - m.dm); i += CH_THREADS) {
-      // columns past the model's own: zeros (the time column is written below)
-      const int r = i / (kin - m.dm), c = m.dm + i % (kin - m.dm);
-      const bool tc = CNF && m.tcat && c == m.dm && r < R;
-      put<PP>(in0.at(r, c), plane, tc ? ts : 0.f);
+    // columns past the state's: the time column, zeros
+    for (int c = m.dm + tid / COLS; c < kin; c += CH_THREADS / COLS) {
+      const int r = tid % COLS;
+      put<PP>(in0.at(r, chain_pos<PP>(c)), plane, CNF && m.tcat && c == m.dm && r < R ? ts : 0.f);
     }
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
+      if (e * CH_THREADS >= ne) continue;   // (uniform: small states use the first entry only)
       if (tid + e * CH_THREADS >= ne) continue;
       float v = u[e];
       if (mode == SM_STEP) {
-        float sm = 0.f;
-#pragma unroll
-        for (int j = 5; j >= 0; --j) sm += sh.A[s][j] * k[j][e];
-        v = u[e] + dt * sm;
+        v = rk(u[e], k, kl[e], e);
         un[e] = v;
       } else if (mode == SM_INIT_F1) {
-        v = u[e] + h0 * k[0][e];
+        v = fmaf(h0, k[0][e], u[e]);
       }
       if (col[e] < m.dm) {
-        put<PP>(in0.at(row[e], col[e]), plane, map_f(m.map, v));
+        const int cp = chain_pos<PP>(col[e]);
+        put<PP>(in0.at(row[e], cp), plane, map_f(m.map, v));
         if constexpr (CNF)
-          put<PP>(in0.at(R + row[e], col[e]), plane, lprobe[row[e] * m.dm + col[e]]);
+          put<PP>(in0.at(R + row[e], cp), plane, lprobe[row[e] * m.dm + col[e]]);
       }
     }
     if (mode == SM_STEP && s == 6) {
 #pragma unroll
       for (int e = 0; e < NE; ++e)
-        if (tid + e * CH_THREADS < ne) nxt[e0 + tid + e * CH_THREADS] = un[e];
+        if (tid + e * CH_THREADS < ne) nxt[tid + e * CH_THREADS] = un[e];
     }
     chain_barrier();
     int cur = 0;
@@ -160,26 +161,23 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
     chain_narrow<PP, NT, NW, INPLACE>(m.Wf[ll], mt, m.ktf[ll], ChainBuf<PP>{cur, m.pitch, plane}, part, wave, lane, none);
 #pragma unroll
     for (int e = 0; e < NE; ++e) {
+      if (e * CH_THREADS >= ne) continue;
       const int i = tid + e * CH_THREADS;
       if (i >= ne) continue;
       float kv;
       if (!CNF || col[e] < m.dm) {
-        kv = act_f(m.act[ll], chain_sum<NW, NT>(part, mt, row[e], col[e]) + m.bias[ll][col[e]]);
+        kv = act_f(m.act[ll], chain_sum<PP, NW, NT>(part, mt, m.ktf[ll], row[e], col[e]) + m.bias[ll][col[e]]);
       } else {  // log p: minus the probe's directional derivative of f
         kv = 0.f;
         for (int c = 0; c < m.dm; ++c)
-          kv -= lprobe[row[e] * m.dm + c] * chain_sum<NW, NT>(part, mt, R + row[e], c);
+          kv -= lprobe[row[e] * m.dm + c] * chain_sum<PP, NW, NT>(part, mt, m.ktf[ll], R + row[e], c);
       }
-      const int64_t idx = e0 + i;
       const bool live = row0 + row[e] < m.B;
       if (mode == SM_STEP) {
-        ent[(1 + s) * a.sv + idx] = kv;
+        (ent + (1 + s) * a.sv)[i] = kv;
         if (s == 6) {
-          nxt[a.sv + idx] = kv;  // FSAL
-          float ut = chBT[6] * kv;
-#pragma unroll
-          for (int j = 0; j < 6; ++j) ut += chBT[j] * k[j][e];
-          ut *= dt;
+          (nxt + a.sv)[i] = kv;  // FSAL
+          const float ut = dt * chain_err(k, e, kv);
           const float sk = atol + fmaxf(fabsf(u[e]), fabsf(un[e])) * rtol;
           if (live) {
             const double q = (double)(ut / sk);
@@ -189,12 +187,13 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
         }
 #pragma unroll
         for (int j = 1; j < 6; ++j) k[j][e] = j == s ? kv : k[j][e];
+        kl[e] = kv;
       } else if (mode == SM_PLAIN) {
-        a.plain[idx] = kv;
+        (a.plain + e0)[i] = kv;
       } else {
         const float sk = atol + fabsf(u[e]) * rtol;
         const float d = mode == SM_INIT_F0 ? kv : kv - k[0][e];
-        if (mode == SM_INIT_F0) ent[a.sv + idx] = kv;
+        if (mode == SM_INIT_F0) (ent + a.sv)[i] = kv;
         if (live) {
           const double q = (double)(d / sk);
           sum += q * q;
@@ -210,11 +209,11 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
 void chain_layout(ChainModel& m, int nt, bool cnf) {
   // four bytes per activation: FP32, or two BF16 planes
   const int cols = 16 * nt, act = (cnf ? 1 : 2) * cols * m.pitch * 4;
-  const int mt[2] = {m.mtf[m.L - 1], m.mtb[0]};
   int part = 0;
   m.wmax = 4;
-  for (int x : mt) {
-    const int ks = m.nw == 8 ? chain_splits<8>(x) : chain_splits<4>(x);
+  for (int i = 0; i < 2; ++i) {
+    const int x = i ? m.mtb[0] : m.mtf[m.L - 1], k = i ? m.ktb[0] : m.ktf[m.L - 1];
+    const int ks = m.nw == 8 ? chain_splits<8>(x, k, m.kt) : chain_splits<4>(x, k, m.kt);
     part = std::max(part, ks * cols * (16 * x + 4) * 4);
   }
   for (int l = 0; l < m.L - 1; ++l) m.wmax = std::max(m.wmax, 16 * m.mtf[l]);
@@ -261,6 +260,8 @@ __global__ void __launch_bounds__(256) k_pack_chain(ChainPack a, const float* __
   if (!W) return;
   const int mt = bwd ? a.mtb[l] : a.mtf[l], kt = bwd ? a.ktb[l] : a.ktf[l];
   const int in = a.in[l], out = a.out[l];
+  const bool hid = bwd ? l > 0 : l < a.nl - 1;   // hidden features on the M side
+  constexpr bool F32 = sizeof(T) == 4;           // (stored in chain_feat order)
   const float* w = p + a.w0[l];
   const int64_t nfl = (int64_t)mt * kt * 64;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nfl;
@@ -268,11 +269,12 @@ __global__ void __launch_bounds__(256) k_pack_chain(ChainPack a, const float* __
     const int lane = (int)(i & 63);
     const int64_t f = i >> 6;
     const int t = (int)(f / kt), k = (int)(f % kt);
-    const int mrow = 16 * t + (lane & 15), k0 = k * KT + V * (lane >> 4);
+    const int mr = 16 * t + (lane & 15), k0 = k * KT + V * (lane >> 4);
+    const int mrow = F32 && hid ? chain_feat(mr) : mr;
     T* d = W + (f * P * 64 + lane) * V;
 #pragma unroll
     for (int j = 0; j < V; ++j) {
-      const int kk = k0 + j;
+      const int kk = F32 ? chain_feat(k0 + j) : k0 + j;
       const int o = bwd ? kk : mrow, ii = bwd ? mrow : kk;
       const float v = o < out && ii < in ? w[(int64_t)ii * out + o] : 0.f;
       put<PP>(d + j, 64 * V, v);

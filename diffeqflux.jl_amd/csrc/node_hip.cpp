@@ -696,7 +696,7 @@ bool chain_plan(node_handle* h, ChainModel& m) {
   if (h->prec == NODE_PREC_BF16 || h->cnf_reg || h->cnf_exact) return false;
   if (h->D > (h->cnf ? 32 : 64)) return false;
   const int KT = h->prec == NODE_PREC_FP32 ? 16 : 32;
-  m.L = h->L; m.map = h->desc.input_map; m.D = h->D; m.B = h->B;
+  m.L = h->L; m.map = h->desc.input_map; m.D = h->D; m.B = h->B; m.kt = KT;
   m.dm = h->cnf ? h->cnf_dm : h->D;
   m.tcat = h->desc.input_map == NODE_MAP_CNF_TIME ? 1 : 0;
   int wide = 0;
