@@ -413,6 +413,17 @@ __device__ __forceinline__ int wg_tile(const ChainWgradArgs& a, int tile, int& i
   return l;
 }
 
+// Block -> (tile, row range).  Blocks go to the eight XCDs in turn; each XCD
+// gets a contiguous piece of the (range, tile) sequence, so that a range's rows
+// are read into one L2 and serve all its tiles there (spread over the XCDs every
+// L2 read every row).  False: no work.
+__device__ __forceinline__ bool wg_block(const ChainWgradArgs& a, int& tile, int& chunk) {
+  const int m = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  chunk = m / a.ntile;
+  tile = m - chunk * a.ntile;
+  return chunk < a.chunks;
+}
+
 // FP32.  A wave owns a 64 x 64 tile over its share of a row range: both
 // operands come straight from memory, 16 bytes per lane (lane l: row l / 16 of
 // a group of four, features 4 (l % 16) ..), and component v of the vectors is
@@ -426,9 +437,10 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
   __shared__ float red[4][GT * GT / 2];
   __shared__ float redb[4][2][GT];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  int it, ot;
-  const int l = wg_tile(a, blockIdx.x, it, ot);
-  const int64_t r0 = blockIdx.y * a.crows;
+  int it, ot, tile, chunk;
+  if (!wg_block(a, tile, chunk)) return;
+  const int l = wg_tile(a, tile, it, ot);
+  const int64_t r0 = chunk * a.crows;
   const int64_t r1 = r0 + a.crows < a.ops.rows ? r0 + a.crows : a.ops.rows;
   const int wi = a.ops.w[l], wo = a.ops.w[l + 1];
   const int gsel = ctl->gsel;
@@ -495,7 +507,7 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
   // sum over the waves, two halves of the tile at a time; acc element (p, q, v)
   // of lane l is input 4 (4 (l / 16) + v) + p, output 4 (l % 16) + q
   const int64_t tsz = GT * (GT + 1);
-  float* out = a.part + ((int64_t)blockIdx.y * 2 * a.ntile + blockIdx.x) * tsz;
+  float* out = a.part + ((int64_t)chunk * 2 * a.ntile + tile) * tsz;
 #pragma unroll
   for (int which = 0; which < 2; ++which) {
 #pragma unroll
@@ -545,7 +557,15 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
 // features and gets each lane one feature of the four rows).  Row pitch 320 B:
 // the four rows of a read fall on different banks.  Four waves, each 64 x 64
 // (two 32 x 32 tiles each way, hi*hi + lo*hi + hi*lo) with both folded sums in
-// registers; the next 32 rows travel from memory to registers meanwhile.
+// registers, one wave per SIMD: nothing but the wave's own instructions hides a
+// load, so three groups of 32 rows travel from memory at a time (a ring of
+// registers; with one group, a read under load took four times the products it
+// travelled under: 24% of the matrix rate) and LDS holds three: one written, one
+// whose second half is read while its first half multiplies and the other way
+// round with the next one (reading all of a group and then multiplying took as
+// long again as the products).  Loads are unconditional: rows
+// are padded to whole groups with zeros, columns past a layer's width repeat
+// the last ones and end in tile entries nobody reads.
 constexpr int GS = 128, GS_PITCH = 160, GS_K = 32;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4;
@@ -560,21 +580,24 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
   const Ctl* ctl = a.ctl;
   if (a.mode == SM_STEP && ctl->done) return;
   // [buffer][operand][plane][32 rows][pitch]
-  __shared__ __attribute__((aligned(16))) bf16 lt[2][2][2][GS_K * GS_PITCH];
+  __shared__ __attribute__((aligned(16))) bf16 lt[3 * 2 * 2 * GS_K * GS_PITCH];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  int it, ot;
-  const int l = wg_tile(a, blockIdx.x, it, ot);
-  const int64_t r0 = blockIdx.y * a.crows;
+  int it, ot, tile, chunk;
+  if (!wg_block(a, tile, chunk)) return;
+  const int l = wg_tile(a, tile, it, ot);
+  const int64_t r0 = chunk * a.crows;
   const int64_t r1 = r0 + a.crows < a.ops.rows ? r0 + a.crows : a.ops.rows;
   const int wi = a.ops.w[l], wo = a.ops.w[l + 1];
   const int gsel = ctl->gsel;
   const int ns = a.mode == SM_STEP ? 7 : 1;
-  const int n = (int)((r1 - r0 + GS_K - 1) / GS_K);
+  const int n = (int)((r1 - r0) / GS_K);
+  const int rblk = (int)a.rblk, rprim = (int)a.rprim;
   const bool bias = it == 0;
   // this thread's 16-byte pieces: 8 features (fc) of rows tr, tr + 16 of both
   // operands and planes
   const int fc = 8 * (tid & 15), tr = tid >> 4;
-  const bool hin = it * GS + fc < wi, din = ot * GS + fc < wo;
+  const int hc = it * GS + fc < wi ? it * GS + fc : wi - 8, dc = ot * GS + fc < wo ? ot * GS + fc : wo - 8;
+  const unsigned hoff = 2 * (tr * wi + hc), doff = 2 * (tr * wo + dc);
   f32x16 g[2][2], ab[2][2], ae[2][2];
   float gb[8], bb[8], be[8];
 #pragma unroll
@@ -588,43 +611,73 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
   const int wr = 64 * (wave >> 1), wc = 64 * (wave & 1);
   const int frow = 8 * (lane >> 5) + ((lane & 15) >> 2);          // first K row of this lane's reads
   const int fcol = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+  const int64_t hp = a.ops.rows * wi, dp = a.ops.rows * wo;
+  constexpr int OPER = 2 * GS_K * GS_PITCH, BUF = 2 * OPER;       // LDS elements of an operand, a group
   for (int s = 0; s < ns; ++s) {
     const char* ob = (const char*)a.ops.base + (int64_t)wg_slot(a.mode, s, gsel) * a.ops.slot;
-    const bf16* h = (const bf16*)(ob + a.ops.h[l]) + it * GS + fc;
-    const bf16* d = (const bf16*)(ob + a.ops.d[l]) + ot * GS + fc;
-    const int64_t hp = a.ops.rows * wi, dp = a.ops.rows * wo;
-    u32x4 hv[2][2], dv[2][2];                                     // [row half][plane]
-    auto load = [&](int k) {
+    const bf16* h = (const bf16*)(ob + a.ops.h[l]) + r0 * wi;       // (uniform; lane offsets apart)
+    const bf16* d = (const bf16*)(ob + a.ops.d[l]) + r0 * wo;
+    u32x4 hv[3][2][2], dv[3][2][2];                               // [ring][row half][plane]
+    auto load = [&](int j, int k) {
+      k = k < n ? k : n - 1;
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int64_t r = r0 + (int64_t)k * GS_K + tr + 16 * q;
-        const bool in = r < r1;
+      for (int q = 0; q < 2; ++q)
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-          hv[q][p] = (u32x4){0, 0, 0, 0};
-          dv[q][p] = (u32x4){0, 0, 0, 0};
-          if (in && hin) hv[q][p] = *(const u32x4*)(h + p * hp + r * wi);
-          if (in && din) dv[q][p] = *(const u32x4*)(d + p * dp + r * wo);
+          hv[j][q][p] = *(const u32x4*)((const char*)(h + p * hp + (int64_t)(k * GS_K + 16 * q) * wi) + hoff);
+          dv[j][q][p] = *(const u32x4*)((const char*)(d + p * dp + (int64_t)(k * GS_K + 16 * q) * wo) + doff);
+        }
+    };
+    auto store = [&](int j, int k) {
+      bf16* o = lt + j * BUF + tr * GS_PITCH + fc;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          *(u32x4*)(o + (p * GS_K + 16 * q) * GS_PITCH) = hv[j][q][p];
+          *(u32x4*)(o + OPER + (p * GS_K + 16 * q) * GS_PITCH) = dv[j][q][p];
+        }
+        // (a block's rows: a power of two, the primal ones first)
+        if (bias && k < n && (((int)r0 + k * GS_K + tr + 16 * q) & (rblk - 1)) < rprim) {
+          const bf16x8 x = __builtin_bit_cast(bf16x8, dv[j][q][0]), y = __builtin_bit_cast(bf16x8, dv[j][q][1]);
+#pragma unroll
+          for (int v = 0; v < 8; ++v) gb[v] += (float)x[v] + (float)y[v];
         }
       }
     };
-    auto store = [&](int b, int k) {
+    struct Frags { u32x4 x[2][2], y[2][2]; };                     // [tile][plane] of 16 K rows
+    auto read = [&](Frags& f, int j, int kk) {
+      const bf16* in = lt + j * BUF;
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
+      for (int p = 0; p < 2; ++p)
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          *(u32x4*)&lt[b][0][p][(tr + 16 * q) * GS_PITCH + fc] = hv[q][p];
-          *(u32x4*)&lt[b][1][p][(tr + 16 * q) * GS_PITCH + fc] = dv[q][p];
+        for (int t = 0; t < 2; ++t) {
+          f.x[t][p] = wg_frag(in + p * GS_K * GS_PITCH, 16 * kk + frow, wr + 32 * t + fcol);
+          f.y[t][p] = wg_frag(in + OPER + p * GS_K * GS_PITCH, 16 * kk + frow, wc + 32 * t + fcol);
         }
-        if (bias) {
-          const int64_t r = r0 + (int64_t)k * GS_K + tr + 16 * q;
-          if (a.rprim == a.rblk || r % a.rblk < a.rprim) {
-            const bf16x8 x = __builtin_bit_cast(bf16x8, dv[q][0]), y = __builtin_bit_cast(bf16x8, dv[q][1]);
+    };
+    auto mul = [&](const Frags& f) {
 #pragma unroll
-            for (int v = 0; v < 8; ++v) gb[v] += (float)x[v] + (float)y[v];
-          }
-        }
-      }
+      for (int pq = 0; pq < 3; ++pq)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+            g[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                __builtin_bit_cast(bf16x8, f.x[t][pq == 1]), __builtin_bit_cast(bf16x8, f.y[u][pq == 2]),
+                g[t][u], 0, 0, 0);
+    };
+    Frags fa, fb;
+    // group k (k % 3 = j; its first half is in fa): group k + 2 to LDS, group
+    // k + 5 from memory, each half's products over the other's reads
+    auto step = [&](int j, int k) {
+      store((j + 2) % 3, k + 2);                                  // (past the last: not used)
+      load((j + 2) % 3, k + 5);
+      read(fb, j, 1);
+      mul(fa);
+      read(fa, (j + 1) % 3, 0);
+      mul(fb);
+      chain_barrier();
     };
 #pragma unroll
     for (int x = 0; x < 2; ++x)
@@ -634,38 +687,21 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
         for (int v = 0; v < 16; ++v) g[x][y][v] = 0.f;
 #pragma unroll
     for (int v = 0; v < 8; ++v) gb[v] = 0.f;
-    load(0);
-    store(0, 0);
-    __syncthreads();
-    for (int k = 0; k < n; ++k) {
-      const int b = k & 1;
-      if (k + 1 < n) load(k + 1);
 #pragma unroll
-      for (int kk = 0; kk < GS_K; kk += 16) {
-        u32x4 x[2][2], y[2][2];
+    for (int j = 0; j < 3; ++j) load(j, j);
 #pragma unroll
-        for (int p = 0; p < 2; ++p)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            x[t][p] = wg_frag(lt[b][0][p], kk + frow, wr + 32 * t + fcol);
-            y[t][p] = wg_frag(lt[b][1][p], kk + frow, wc + 32 * t + fcol);
-          }
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int u = 0; u < 2; ++u) {
-            auto m = [&](const u32x4& p, const u32x4& q) {
-              g[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                  __builtin_bit_cast(bf16x8, p), __builtin_bit_cast(bf16x8, q), g[t][u], 0, 0, 0);
-            };
-            m(x[t][0], y[u][0]);
-            m(x[t][1], y[u][0]);
-            m(x[t][0], y[u][1]);
-          }
-      }
-      if (k + 1 < n) store(b ^ 1, k + 1);
-      __syncthreads();
+    for (int j = 0; j < 2; ++j) {
+      store(j, j);
+      load(j, j + 3);
     }
+    chain_barrier();
+    read(fa, 0, 0);
+    int k = 0;
+    for (; k + 3 <= n; k += 3)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) step(j, k + j);
+    if (k < n) step(0, k);
+    if (k + 1 < n) step(1, k + 1);
     const float cb = a.mode == SM_STEP ? (s < 6 ? chA[6][s] : 0.f) : 1.f;
     const float ce = a.mode == SM_STEP ? chBT[s] : 0.f;
 #pragma unroll
@@ -679,7 +715,7 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
     for (int v = 0; v < 8; ++v) { bb[v] += cb * gb[v]; be[v] += ce * gb[v]; }
   }
   const int64_t tsz = GS * (GS + 1);
-  float* out = a.part + ((int64_t)blockIdx.y * 2 * a.ntile + blockIdx.x) * tsz;
+  float* out = a.part + ((int64_t)chunk * 2 * a.ntile + tile) * tsz;
 #pragma unroll
   for (int which = 0; which < 2; ++which)
 #pragma unroll
@@ -694,7 +730,6 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
         }
   if (bias) {
     float* red = (float*)lt;                                      // [2][16][GS]
-    __syncthreads();
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
       red[tr * GS + fc + v] = bb[v];
@@ -776,10 +811,9 @@ __global__ void __launch_bounds__(256) k_chain_mu(ChainMuArgs a) {
 }
 
 void launch_chain_wgrad(int prec, const ChainWgradArgs& a, hipStream_t s) {
-  if (prec == 0)
-    hipLaunchKernelGGL(k_chain_wgrad32, dim3(a.ntile, a.chunks), dim3(256), 0, s, a);
-  else
-    hipLaunchKernelGGL(k_chain_wgrad16, dim3(a.ntile, a.chunks), dim3(256), 0, s, a);
+  const dim3 grid(8 * ((a.ntile * a.chunks + 7) / 8));
+  if (prec == 0) hipLaunchKernelGGL(k_chain_wgrad32, grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL(k_chain_wgrad16, grid, dim3(256), 0, s, a);
 }
 void launch_chain_mu(const ChainMuArgs& a, int nblk, hipStream_t s) {
   hipLaunchKernelGGL(k_chain_mu, dim3(nblk), dim3(256), 0, s, a);

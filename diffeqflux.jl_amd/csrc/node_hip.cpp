@@ -730,7 +730,9 @@ constexpr int64_t CHAIN_OPS_MAX = int64_t(4) << 30;  // bytes a handle may keep 
 ChainOps chain_ops(const node_handle* h, int nt) {
   ChainOps o{};
   const int r = chain_rows(nt, h->cnf);
-  o.rows = (int64_t)((h->B + r - 1) / r) * 16 * nt;
+  // (split: whole groups of the weight gradients' 32 rows; those past the blocks
+  // stay zero)
+  o.rows = rup((int64_t)((h->B + r - 1) / r) * 16 * nt, h->prec == NODE_PREC_FP32 ? 16 : 32);
   const int64_t elt = (int64_t)h->esz * h->planes;
   for (int l = 0; l < h->L; ++l) o.w[l] = h->layers[l].inp;
   o.w[h->L] = h->layers[h->L - 1].outp;
