@@ -1865,28 +1865,31 @@ int ragged_backward_impl(node_handle* h, const float* dLdout, float* dLdu0, doub
   if (ragged_model(h, m, why)) return fail(h, NODE_ERR_UNSUPPORTED, why);
   const int64_t n = r.n, ns = r.ns, P = h->P, Pn = m.Pn;
   const int D = h->D, Dp = (D + 15) / 16 * 16;
-  // A workgroup per CU (the weights fill its LDS) of up to 4 waves, one per
-  // SIMD.  A wave's time is its VJP rounds (as many as its longest slot
-  // needs) plus one parameter pass per step of every slot, each pass bound
-  // by the wave's own memory latency: so the trajectories are spread over as
-  // many waves as the SIMDs hold (spw slots of 16 active per wave), and all
-  // of them start at once when they fit.
-  const int64_t max_waves = 4 * (int64_t)h->n_cu;
-  const int spw = (int)std::min<int64_t>(RG_SLOTS, std::max<int64_t>(1, (n + max_waves - 1) / max_waves));
-  const int64_t waves_all = (n + spw - 1) / spw;
-  const int waves = (int)std::min<int64_t>(4, std::max<int64_t>(1, (waves_all + h->n_cu - 1) / h->n_cu));
-  const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(h->n_cu, (waves_all + waves - 1) / waves));
-  const int64_t slots = (int64_t)grid * waves * RG_SLOTS;      // stage blocks, row buffers
-  const int64_t nslots = (int64_t)grid * waves * spw;          // active slots
-  // act' of the VJPs in LDS beside the weights when every wave's area fits
+  // Workgroups of up to 4 waves, one per SIMD, as many on a CU as the width
+  // class's registers and the LDS (weights, and act' of the VJPs beside them
+  // where every wave's area fits) allow.  A wave's time is its VJP rounds (as
+  // many as its longest slot needs) plus one parameter pass per step of every
+  // slot, each pass bound by the wave's own memory latency: so the
+  // trajectories are spread over as many waves as the SIMDs hold (spw slots of
+  // 16 active per wave), and all of them start at once when they fit.
   int act_tiles = 0;
   for (int l = 0; l < m.L; ++l) {
     m.act_off[l] = act_tiles;
     act_tiles += m.to[l];
   }
-  m.act_stride = act_tiles * 256;
-  if (((int64_t)m.lds_floats + (int64_t)waves * m.act_stride) * (int64_t)sizeof(float) > 160 * 1024)
-    m.act_stride = 0;
+  auto lds_of = [&](int w, bool act) {
+    return ((int64_t)m.lds_floats + (act ? (int64_t)w * act_tiles * 256 : 0)) * (int64_t)sizeof(float);
+  };
+  constexpr int64_t LDS = 160 * 1024;
+  const int occ = (int)std::max<int64_t>(
+      1, std::min<int64_t>(ragged_waves(m.rw), LDS / lds_of(4, lds_of(4, true) <= LDS)));
+  const int64_t max_waves = 4 * (int64_t)h->n_cu * occ;
+  const int spw = (int)std::min<int64_t>(RG_SLOTS, std::max<int64_t>(1, (n + max_waves - 1) / max_waves));
+  const int64_t waves_all = (n + spw - 1) / spw;
+  const int waves = (int)std::min<int64_t>(4, std::max<int64_t>(1, (waves_all + h->n_cu - 1) / h->n_cu));
+  const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)h->n_cu * occ, (waves_all + waves - 1) / waves));
+  const int64_t nslots = (int64_t)grid * waves * spw;          // slots: stage blocks, row buffers
+  m.act_stride = lds_of(waves, true) <= LDS ? act_tiles * 256 : 0;
   // start order (a schedule only: each trajectory's arithmetic is the same
   // in any slot).  A wave runs until its last slot's trajectory is done and
   // does one parameter pass per step of every slot, so the waves' sums of
@@ -1918,8 +1921,8 @@ int ragged_backward_impl(node_handle* h, const float* dLdout, float* dLdu0, doub
       grow(h, &b.dLdout, std::max<int64_t>(ns * D, 1), b.dLdout_cap, std::max<int64_t>(ns * D, 64)) ||
       grow(h, &b.dLdu0, n * D, b.dLdu0_cap, n * D) ||
       grow(h, &b.rows, n * Pn, b.rows_cap, n * Pn) ||
-      grow(h, &b.tmp, slots * Pn, b.tmp_cap, slots * Pn) ||
-      grow(h, &b.sbuf, (slots + 1) * 8 * m.sv, b.sbuf_cap, (slots + 1) * 8 * m.sv) ||
+      grow(h, &b.tmp, nslots * Pn, b.tmp_cap, nslots * Pn) ||
+      grow(h, &b.sbuf, (nslots + 1) * 8 * m.sv, b.sbuf_cap, (nslots + 1) * 8 * m.sv) ||
       grow(h, &b.dp, P, b.dp_cap, P) ||
       grow(h, &b.part, RG_SUM_CHUNKS * P, b.part_cap, RG_SUM_CHUNKS * P))
     return NODE_ERR_HIP;
@@ -1938,7 +1941,7 @@ int ragged_backward_impl(node_handle* h, const float* dLdout, float* dLdu0, doub
   a.last_rec = r.last; a.rec_t = r.rec_t; a.rec_prev = r.rec_prev; a.rec_data = r.rec_data;
   a.dLdu0 = b.dLdu0; a.dLdp_traj = b.rows; a.mu_tmp = b.tmp; a.sbuf = b.sbuf;
   a.queue = r.ctr; a.retcode = r.ret; a.traj_stats = r.tstats;
-  a.order = b.order; a.norder = norder; a.nslots = nslots; a.spw = spw; a.nslots_all = slots;
+  a.order = b.order; a.norder = norder; a.nslots = nslots; a.spw = spw;
   a.vjp_bf16 = h->rg_vjp_prec == NODE_PREC_BF16;
   const node_solve_opts* o = &r.opts;
   a.t0 = o->t0;

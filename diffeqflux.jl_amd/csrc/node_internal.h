@@ -385,9 +385,8 @@ struct RaggedAdjArgs {
   const float* rec_data;
   float* dLdu0;                       // [n][D]
   float* dLdp_traj;                   // [n][Pn] per-trajectory parameter gradients (zeroed)
-  float* mu_tmp;                      // [slots][Pn]
-  float* sbuf;                        // [slots + 1][8][sv] stage blocks (the last: sink of idle columns)
-  int64_t nslots_all;                 // slots of the launch (16 per wave)
+  float* mu_tmp;                      // [nslots][Pn]
+  float* sbuf;                        // [nslots + 1][8][sv] stage blocks (the last: sink of idle columns)
   int* queue;
   // start order: the trajectory at each queue position (-1: none).  A wave
   // runs trajectories in its first spw slots only (spw <= 16: more waves, each
@@ -405,6 +404,8 @@ struct RaggedAdjArgs {
   int adaptive;
   unsigned long long* stats;
 };
+// waves per SIMD the kernels of a width class (m.rw) are compiled for
+int ragged_waves(int rw);
 void launch_ragged_adj(const RaggedAdjArgs& a, int grid, int waves, hipStream_t s);
 // part: [RG_SUM_CHUNKS][P] FP64 scratch (the per-range sums)
 void launch_ragged_sum(const float* rows, int64_t n, int64_t P, int64_t stride, double* part,

@@ -34,6 +34,13 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <class T> using gp = __attribute__((address_space(1))) T*;
 template <class T> __device__ __forceinline__ gp<T> glb(T* p) { return (gp<T>)p; }
 
+// The kernels are compiled per width class HT (the longest tile dimension of
+// any layer, 1, 2, 4 or 8 tiles), with as many waves per SIMD as the class's
+// registers allow: a class-1 VJP is a dozen dependent LDS reads and MFMAs, a
+// parameter pass a few dependent memory reads, and the other waves run under
+// them.  (2-16-2 model, 10240 trajectories: see k_ragged_adj.)
+__host__ __device__ constexpr int rg_waves(int ht) { return ht <= 4 ? 2 : 1; }
+
 struct SlotCtl {
   double t, dt, tprev, dtpropose, qold, q11, eest, tdir, dtmax_abs, dtmin, t_end, dt_fixed;
   int64_t iter, maxiters;
@@ -55,55 +62,6 @@ __device__ __forceinline__ rg_s4 rg_bf4(const f32x4& v) {
 }
 __device__ __forceinline__ f32x4 rg_mfma_bf(rg_s4 a, rg_s4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-}
-
-// z[ot] = W x for output tiles ot < nto (no bias); x: nti input tiles
-template <int NTI, int NTO>
-__device__ __forceinline__ void rg_fwd_gemm(const float* W, int pitch, const f32x4 (&x)[NTI],
-                                            int nti, int nto, f32x4 (&z)[NTO], int lane) {
-  const int r = lane & 15, g = lane >> 4;
-#pragma unroll
-  for (int ot = 0; ot < NTO; ++ot) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (ot < nto) {
-      const float* wrow = W + (16 * ot + r) * pitch + 4 * g;
-#pragma unroll
-      for (int it = 0; it < NTI; ++it) {
-        if (it < nti) {
-          const f32x4 a = *(const f32x4*)(wrow + 16 * it);
-          acc = rg_mfma(a.x, x[it].x, acc);
-          acc = rg_mfma(a.y, x[it].y, acc);
-          acc = rg_mfma(a.z, x[it].z, acc);
-          acc = rg_mfma(a.w, x[it].w, acc);
-        }
-      }
-    }
-    z[ot] = acc;
-  }
-}
-
-// out[it] = W^T d for input tiles it < nti; d: nto output-feature tiles
-template <int NTI, int NTO>
-__device__ __forceinline__ void rg_bwd_gemm(const float* W, int pitch, const f32x4 (&d)[NTO],
-                                            int nti, int nto, f32x4 (&out)[NTI], int lane) {
-  const int r = lane & 15, g = lane >> 4;
-#pragma unroll
-  for (int it = 0; it < NTI; ++it) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (it < nti) {
-#pragma unroll
-      for (int ot = 0; ot < NTO; ++ot) {
-        if (ot < nto) {
-          const float* wc = W + (16 * ot + 4 * g) * pitch + 16 * it + r;
-          acc = rg_mfma(wc[0], d[ot].x, acc);
-          acc = rg_mfma(wc[pitch], d[ot].y, acc);
-          acc = rg_mfma(wc[2 * pitch], d[ot].z, acc);
-          acc = rg_mfma(wc[3 * pitch], d[ot].w, acc);
-        }
-      }
-    }
-    out[it] = acc;
-  }
 }
 
 // one Dense layer, tile by tile: y[ot] = act(W x + b) for ot < nto
@@ -137,18 +95,18 @@ __device__ __forceinline__ void rg_layer(const float* W, int pitch, const float*
 // map applied) -> f (DT tiles).  One rolled loop body over the layers (the
 // output is copied into place after each layer) keeps the code small enough
 // for the instruction cache.
-template <int DT>
+template <int DT, int HT>
 __device__ __forceinline__ void rg_mlp(const RaggedModel& m, const float* lds,
                                        const f32x4 (&x)[DT], f32x4 (&f)[DT], int lane) {
-  f32x4 hin[RG_HT], hout[RG_HT];
+  f32x4 hin[HT], hout[HT];
 #pragma unroll
-  for (int t = 0; t < RG_HT; ++t) hin[t] = t < DT ? x[t < DT ? t : 0] : f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < HT; ++t) hin[t] = t < DT ? x[t < DT ? t : 0] : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
   for (int l = 0; l < m.L; ++l) {
-    rg_layer<RG_HT, RG_HT>(lds + m.lw[l], m.pitch[l], lds + m.lb[l], m.act[l], hin, m.ti[l],
+    rg_layer<HT, HT>(lds + m.lw[l], m.pitch[l], lds + m.lb[l], m.act[l], hin, m.ti[l],
                            m.to[l], hout, lane);
 #pragma unroll
-    for (int t = 0; t < RG_HT; ++t) hin[t] = hout[t];
+    for (int t = 0; t < HT; ++t) hin[t] = hout[t];
   }
 #pragma unroll
   for (int t = 0; t < DT; ++t) f[t] = hin[t];
@@ -224,7 +182,7 @@ __device__ __forceinline__ int rg_record(const RaggedFwdArgs& a, double t, int p
   return idx;
 }
 
-template <int DT>
+template <int DT, int HT>
 __global__ void __launch_bounds__(256) k_ragged_fwd(RaggedFwdArgs a) {
   extern __shared__ __attribute__((aligned(16))) float rg_lds[];
   const RaggedModel& m = a.m;
@@ -306,7 +264,7 @@ __global__ void __launch_bounds__(256) k_ragged_fwd(RaggedFwdArgs a) {
       for (int q = 0; q < 4; ++q) x[t][q] = rg_map(m.map, v[q]);
     }
     f32x4 fo[DT];
-    rg_mlp<DT>(m, rg_lds, x, fo, lane);
+    rg_mlp<DT, HT>(m, rg_lds, x, fo, lane);
     if (traj < 0) continue;
     ++nf;
     bool fin = false;
@@ -476,17 +434,30 @@ __global__ void __launch_bounds__(256) k_ragged_fwd(RaggedFwdArgs a) {
   }
 }
 
+// (state tiles, width class): m.rw is at least the state's tiles
+#define RG_DISPATCH(GO)                    \
+  do {                                     \
+    if (a.Dp <= 16) {                      \
+      if (a.m.rw == 1) GO(1, 1);           \
+      else if (a.m.rw == 2) GO(1, 2);      \
+      else if (a.m.rw == 4) GO(1, 4);      \
+      else GO(1, RG_HT);                   \
+    } else {                               \
+      if (a.m.rw == 2) GO(2, 2);           \
+      else if (a.m.rw == 4) GO(2, 4);      \
+      else GO(2, RG_HT);                   \
+    }                                      \
+  } while (0)
+
 void launch_ragged_fwd(const RaggedFwdArgs& a, int grid, hipStream_t s) {
   const size_t lds = (size_t)a.m.lds_floats * sizeof(float);
-  if (a.Dp <= 16) {
-    (void)hipFuncSetAttribute((const void*)k_ragged_fwd<1>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(k_ragged_fwd<1>, dim3(grid), dim3(256), lds, s, a);
-  } else {
-    (void)hipFuncSetAttribute((const void*)k_ragged_fwd<2>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(k_ragged_fwd<2>, dim3(grid), dim3(256), lds, s, a);
-  }
+  auto go = [&](auto kern) {
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, s, a);
+  };
+#define RG_GO(DT, HT) go(k_ragged_fwd<DT, HT>)
+  RG_DISPATCH(RG_GO);
+#undef RG_GO
 }
 
 // ---------------------------------------------------------------- adjoint
@@ -519,18 +490,18 @@ __device__ __forceinline__ void rg_act4(int act, const f32x4& z, f32x4& y, f32x4
 // or in the block's delta area when m.act_stride is 0) and returns
 // g = W_0^T delta_0 (the input-map derivative is applied by the caller).
 // BF: the products on BF16 operands (rounded to nearest), FP32 accumulation.
-template <bool BF>
+template <bool BF, int HT>
 __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, float* act_lds,
-                                       const f32x4 (&x0)[RG_HT], const f32x4 (&lam)[RG_HT],
-                                       gp<float> blk, f32x4 (&gout)[RG_HT], int lane) {
+                                       const f32x4 (&x0)[HT], const f32x4 (&lam)[HT],
+                                       gp<float> blk, f32x4 (&gout)[HT], int lane) {
   const int r = lane & 15, g4 = 4 * (lane >> 4);
   const int L = m.L;
   // one rolled loop body per sweep (the layer's input is copied into place
   // after each layer): the unrolled-over-layers form did not fit the
   // instruction cache
-  f32x4 hin[RG_HT], hout[RG_HT];
+  f32x4 hin[HT], hout[HT];
 #pragma unroll
-  for (int t = 0; t < RG_HT; ++t) {
+  for (int t = 0; t < HT; ++t) {
     hin[t] = x0[t];
     if (t < m.ti[0]) *(gp<f32x4>)(blk + m.sh[0] + 16 * t + g4) = x0[t];
   }
@@ -539,24 +510,24 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
     const float* W = lds + m.lw[l];
     const float* bias = lds + m.lb[l];
     const int pitch = m.pitch[l], nti = m.ti[l], nto = m.to[l], act = m.act[l];
-    rg_s4 hb[RG_HT];
+    rg_s4 hb[HT];
     if (BF) {
 #pragma unroll
-      for (int t = 0; t < RG_HT; ++t) hb[t] = rg_bf4(hin[t]);
+      for (int t = 0; t < HT; ++t) hb[t] = rg_bf4(hin[t]);
     }
     // a hidden tanh layer of 8 x 8 tiles with act' parked in LDS (the usual
     // shape): one straight-line block, so the compiler can run a tile's
     // activation and stores under the next tile's reads and MFMAs
-    if (nti == RG_HT && nto == RG_HT && act == 1 && m.act_stride && l < L - 1) {
+    if (HT == RG_HT && nti == HT && nto == HT && act == 1 && m.act_stride && l < L - 1) {
 #pragma unroll
-      for (int ot = 0; ot < RG_HT; ++ot) {
+      for (int ot = 0; ot < HT; ++ot) {
         f32x4 acc = *(const f32x4*)(bias + 16 * ot + g4);
         const float* wrow = W + (16 * ot + r) * pitch + g4;
-        f32x4 a[RG_HT];
+        f32x4 a[HT];
 #pragma unroll
-        for (int it = 0; it < RG_HT; ++it) a[it] = *(const f32x4*)(wrow + 16 * it);
+        for (int it = 0; it < HT; ++it) a[it] = *(const f32x4*)(wrow + 16 * it);
 #pragma unroll
-        for (int it = 0; it < RG_HT; ++it) {
+        for (int it = 0; it < HT; ++it) {
           if (BF) {
             acc = rg_mfma_bf(rg_bf4(a[it]), hb[it], acc);
           } else {
@@ -576,10 +547,10 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
         *(gp<f32x4>)(blk + m.sh[l + 1] + 16 * ot + g4) = y;
         hout[ot] = y;
       }
-    } else if (nti == 1 && nto == RG_HT && act == 1 && m.act_stride && l < L - 1) {
+    } else if (HT == RG_HT && nti == 1 && nto == HT && act == 1 && m.act_stride && l < L - 1) {
       // the same for a first layer of 1 x 8 tiles (inputs <= 16)
 #pragma unroll
-      for (int ot = 0; ot < RG_HT; ++ot) {
+      for (int ot = 0; ot < HT; ++ot) {
         f32x4 acc = *(const f32x4*)(bias + 16 * ot + g4);
         const f32x4 a = *(const f32x4*)(W + (16 * ot + r) * pitch + g4);
         if (BF) {
@@ -602,20 +573,20 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
       }
     } else {
 #pragma unroll
-    for (int ot = 0; ot < RG_HT; ++ot) {
+    for (int ot = 0; ot < HT; ++ot) {
       hout[ot] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (ot < nto) {
+      if (HT == 1 || ot < nto) {
         f32x4 acc = *(const f32x4*)(bias + 16 * ot + g4);
         const float* wrow = W + (16 * ot + r) * pitch + g4;
         // the tile's weight vectors read in one batch at constant offsets:
         // one LDS wait per tile, not per k-tile (k-tiles past nti read the
         // next rows or the zero pad after the weights, and go unused)
-        f32x4 a[RG_HT];
+        f32x4 a[HT];
 #pragma unroll
-        for (int it = 0; it < RG_HT; ++it) a[it] = *(const f32x4*)(wrow + 16 * it);
+        for (int it = 0; it < HT; ++it) a[it] = *(const f32x4*)(wrow + 16 * it);
 #pragma unroll
-        for (int it = 0; it < RG_HT; ++it) {
-          if (it < nti) {
+        for (int it = 0; it < HT; ++it) {
+          if (HT == 1 || it < nti) {
             if (BF) {
               acc = rg_mfma_bf(rg_bf4(a[it]), hb[it], acc);
             } else {
@@ -636,38 +607,38 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
     }
     }
 #pragma unroll
-    for (int t = 0; t < RG_HT; ++t) hin[t] = hout[t];
+    for (int t = 0; t < HT; ++t) hin[t] = hout[t];
   }
   // backward sweep: gi = gradient entering layer l
-  f32x4 gi[RG_HT], go[RG_HT];
+  f32x4 gi[HT], go[HT];
 #pragma unroll
-  for (int t = 0; t < RG_HT; ++t) gi[t] = lam[t];
+  for (int t = 0; t < HT; ++t) gi[t] = lam[t];
 #pragma unroll 1
   for (int l = L - 1; l >= 0; --l) {
     const int nti = m.ti[l], nto = m.to[l], pitch = m.pitch[l];
     const float* W = lds + m.lw[l];
-    if (nti == RG_HT && nto == RG_HT && m.act_stride) {
+    if (HT == RG_HT && nti == HT && nto == HT && m.act_stride) {
       // 8 x 8 tiles, act' in LDS: the same straight-line form as the forward
 #pragma unroll
-      for (int ot = 0; ot < RG_HT; ++ot) {
+      for (int ot = 0; ot < HT; ++ot) {
         const f32x4 ad = *(const f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane);
         const f32x4 d = gi[ot] * ad;
         *(gp<f32x4>)(blk + m.sd[l] + 16 * ot + g4) = d;
         gi[ot] = d;
       }
 #pragma unroll
-      for (int it = 0; it < RG_HT; ++it) go[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int it = 0; it < HT; ++it) go[it] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ot = 0; ot < RG_HT; ++ot) {
+      for (int ot = 0; ot < HT; ++ot) {
         const float* wc = W + (16 * ot + g4) * pitch + r;
-        float w[RG_HT][4];
+        float w[HT][4];
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-          for (int it = 0; it < RG_HT; ++it) w[it][v] = wc[v * pitch + 16 * it];
+          for (int it = 0; it < HT; ++it) w[it][v] = wc[v * pitch + 16 * it];
         const rg_s4 gb = rg_bf4(gi[ot]);
 #pragma unroll
-        for (int it = 0; it < RG_HT; ++it) {
+        for (int it = 0; it < HT; ++it) {
           if (BF) {
             go[it] = rg_mfma_bf(rg_bf4(f32x4{w[it][0], w[it][1], w[it][2], w[it][3]}), gb, go[it]);
           } else {
@@ -679,32 +650,32 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
         }
       }
 #pragma unroll
-      for (int t = 0; t < RG_HT; ++t) gi[t] = go[t];
+      for (int t = 0; t < HT; ++t) gi[t] = go[t];
       continue;
     }
-    if (m.act_stride && ((nti == RG_HT && nto == 1) || (nti == 1 && nto == RG_HT))) {
+    if (HT == RG_HT && m.act_stride && ((nti == HT && nto == 1) || (nti == 1 && nto == HT))) {
       // the last layer's 8 x 1 and the first layer's 1 x 8 tiles, likewise:
       // NTO output tiles by NTI input tiles, one of them 1
       const bool last = nto == 1;
 #pragma unroll
-      for (int ot = 0; ot < RG_HT; ++ot) {
+      for (int ot = 0; ot < HT; ++ot) {
         if (ot > 0 && last) break;
         const f32x4 d = gi[ot] * *(const f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane);
         *(gp<f32x4>)(blk + m.sd[l] + 16 * ot + g4) = d;
         gi[ot] = d;
       }
 #pragma unroll
-      for (int it = 0; it < RG_HT; ++it) go[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int it = 0; it < HT; ++it) go[it] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (last) {
         const float* wc = W + g4 * pitch + r;
-        float w[RG_HT][4];
+        float w[HT][4];
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-          for (int it = 0; it < RG_HT; ++it) w[it][v] = wc[v * pitch + 16 * it];
+          for (int it = 0; it < HT; ++it) w[it][v] = wc[v * pitch + 16 * it];
         const rg_s4 gb = rg_bf4(gi[0]);
 #pragma unroll
-        for (int it = 0; it < RG_HT; ++it) {
+        for (int it = 0; it < HT; ++it) {
           if (BF) {
             go[it] = rg_mfma_bf(rg_bf4(f32x4{w[it][0], w[it][1], w[it][2], w[it][3]}), gb, go[it]);
           } else {
@@ -715,13 +686,13 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
           }
         }
       } else {
-        float w[RG_HT][4];
+        float w[HT][4];
 #pragma unroll
-        for (int ot = 0; ot < RG_HT; ++ot)
+        for (int ot = 0; ot < HT; ++ot)
 #pragma unroll
           for (int v = 0; v < 4; ++v) w[ot][v] = W[(16 * ot + g4 + v) * pitch + r];
 #pragma unroll
-        for (int ot = 0; ot < RG_HT; ++ot) {
+        for (int ot = 0; ot < HT; ++ot) {
           if (BF) {
             go[0] = rg_mfma_bf(rg_bf4(f32x4{w[ot][0], w[ot][1], w[ot][2], w[ot][3]}), rg_bf4(gi[ot]), go[0]);
           } else {
@@ -733,12 +704,12 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
         }
       }
 #pragma unroll
-      for (int t = 0; t < RG_HT; ++t) gi[t] = go[t];
+      for (int t = 0; t < HT; ++t) gi[t] = go[t];
       continue;
     }
 #pragma unroll
-    for (int ot = 0; ot < RG_HT; ++ot) {
-      if (ot < nto) {
+    for (int ot = 0; ot < HT; ++ot) {
+      if (HT == 1 || ot < nto) {
         gp<float> pd = blk + m.sd[l] + 16 * ot + g4;
         const f32x4 ad = m.act_stride ? *(const f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane)
                                       : *(gp<const f32x4>)pd;
@@ -751,20 +722,20 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
     // W^T row bases of an output tile serve all input tiles at constant
     // offsets (k-tiles past nti read the next rows or the zero pad, unused)
 #pragma unroll
-    for (int it = 0; it < RG_HT; ++it) go[it] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int it = 0; it < HT; ++it) go[it] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ot = 0; ot < RG_HT; ++ot) {
-      if (ot < nto) {
+    for (int ot = 0; ot < HT; ++ot) {
+      if (HT == 1 || ot < nto) {
         const float* wc = W + (16 * ot + g4) * pitch + r;
-        float w[RG_HT][4];
+        float w[HT][4];
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-          for (int it = 0; it < RG_HT; ++it) w[it][v] = wc[v * pitch + 16 * it];
+          for (int it = 0; it < HT; ++it) w[it][v] = wc[v * pitch + 16 * it];
         const rg_s4 gb = rg_bf4(gi[ot]);
 #pragma unroll
-        for (int it = 0; it < RG_HT; ++it) {
-          if (it < nti) {
+        for (int it = 0; it < HT; ++it) {
+          if (HT == 1 || it < nti) {
             if (BF) {
               go[it] = rg_mfma_bf(rg_bf4(f32x4{w[it][0], w[it][1], w[it][2], w[it][3]}), gb, go[it]);
             } else {
@@ -778,26 +749,25 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
       }
     }
 #pragma unroll
-    for (int t = 0; t < RG_HT; ++t) gi[t] = go[t];
+    for (int t = 0; t < HT; ++t) gi[t] = go[t];
   }
 #pragma unroll
-  for (int t = 0; t < RG_HT; ++t) gout[t] = gi[t];
+  for (int t = 0; t < HT; ++t) gout[t] = gi[t];
 }
 
-// One entry of the parameter part from its pre-scaled stage sums (MODE as in
-// rg_mu_pass): kb = -dt sum_j b_j g~_j (MODE 0) or the g_0 sum (MODE 1), ke
+// One entry of the parameter part from its pre-scaled stage sums (mode as in
+// rg_mu_pass): kb = -dt sum_j b_j g~_j (mode 0) or the g_0 sum (mode 1), ke
 // the error sum.  The error's denominator is kept at least FLT_MIN, so padded
 // entries (all zero) add 0 also for atol = 0; v_rcp_f32 (1 ulp) stands in for
 // the divide, whose IEEE expansion cost a dozen instructions per entry.
-template <int MODE>
-__device__ __forceinline__ float rg_mu_err(float kb, float ke, float atf, float rtf, float m0,
+__device__ __forceinline__ float rg_mu_err(int mode, float kb, float ke, float atf, float rtf, float m0,
                                            float& mn, float& fl) {
   float num, mx;
-  if (MODE == 0) {
+  if (mode == 0) {
     mn = m0 + kb;
     mx = fmaxf(fabsf(m0), fabsf(mn));
     num = ke;
-  } else if (MODE == 1) {
+  } else if (mode == 1) {
     mx = fabsf(m0);
     num = kb;
   } else {
@@ -905,11 +875,12 @@ __device__ __attribute__((noinline)) double rg_mu_pass(uint64_t kargs, gp<const 
   // a load under a lane-dependent branch makes the wave wait for everything
   // in flight where the branch joins.
   const int Lm1 = mm.L - 1;
-  float bm[RG_MAXL][2], bkb[RG_MAXL][2], bke[RG_MAXL][2];
+  constexpr int CB = RW > 4 ? 2 : 1;   // 64-wide rounds of a layer's outputs
+  float bm[RG_MAXL][CB], bkb[RG_MAXL][CB], bke[RG_MAXL][CB];
 #pragma unroll
   for (int l = 0; l < RG_MAXL; ++l)
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < CB; ++c) {
       const int lc = l < mm.L ? l : Lm1, out = mm.out[lc];
       const int o = 64 * c + lane, oc = o < out ? o : out - 1;
       const float keep = (l < mm.L && o < out) ? 1.f : 0.f;
@@ -937,11 +908,11 @@ __device__ __attribute__((noinline)) double rg_mu_pass(uint64_t kargs, gp<const 
 #pragma unroll
   for (int l = 0; l < RG_MAXL; ++l)
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < CB; ++c) {
       const int o = 64 * c + lane;
       if (l < mm.L && o < mm.out[l]) {
         float mn = 0.f;
-        const float ev = rg_mu_err<MODE>(bkb[l][c], bke[l][c], atf, rtf, bm[l][c], mn, fl);
+        const float ev = rg_mu_err(MODE, bkb[l][c], bke[l][c], atf, rtf, bm[l][c], mn, fl);
         if (MODE == 0) mu_new[mm.nb0[l] + o] = mn;
         acc += ev * ev;
       }
@@ -1000,7 +971,7 @@ __device__ __attribute__((noinline)) double rg_mu_pass(uint64_t kargs, gp<const 
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           float mv = 0.f;
-          const float ev = rg_mu_err<MODE>(kb[v], ke[v], atf, rtf, buf[k][v], mv, fl);
+          const float ev = rg_mu_err(MODE, kb[v], ke[v], atf, rtf, buf[k][v], mv, fl);
           mn[v] = mv;
           acc = fmaf(ev, ev, acc);
         }
@@ -1021,23 +992,160 @@ __device__ __attribute__((noinline)) double rg_mu_pass(uint64_t kargs, gp<const 
   return sum;
 }
 
-// The pass for the model's row width (1, 2, 4 or 8 tiles) and mode.
-__device__ __forceinline__ double rg_mu_call(uint64_t kargs, int rw, int mode, gp<const float> sbs,
-                                             int p0, double dt, double atol, double rtol,
-                                             gp<const float> mu, gp<float> mun, double* fl, int lane) {
-#define RG_MU_RW(R)                                                                          \
-  if (rw == R) {                                                                            \
-    if (mode == 0) return rg_mu_pass<0, R>(kargs, sbs, p0, dt, atol, rtol, mu, mun, nullptr, lane); \
-    if (mode == 1) return rg_mu_pass<1, R>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, nullptr, lane); \
-    return rg_mu_pass<2, R>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, fl, lane);                \
+// The same for the classes of one and two tiles: inlined, the mode a run-time
+// value (kb and ke are both formed; the coefficients of the one a mode does not
+// use are 0).  The biases of 64 / (16 RW) layers go to one round of lanes, and
+// their squares are summed in the lanes and order rg_mu_pass sums them in.
+template <int RW>
+__device__ __forceinline__ double rg_mu_small(const RaggedModel& mm, int mode, gp<const float> sbs,
+                                              int p0, double dt, double atol, double rtol,
+                                              gp<const float> __restrict__ mu,
+                                              gp<float> __restrict__ mu_new, double* flag, int lane) {
+  constexpr int LW = 16 * RW, LR = 64 / LW, NR = RG_MAXL / LR;  // lanes per layer, layers per round, rounds
+  const int r = lane & 15, g = lane >> 4;
+  const float dtf = (float)dt, atf = (float)atol, rtf = (float)rtol;
+  const float sb = mode == 0 ? -dtf : -1.f, se = mode == 0 ? dtf : -1.f;
+  // stage j's block and its weights in the two sums
+  auto block = [&](int j) {
+    return mode == 0 ? (j == 0 ? p0 : j == 6 ? 7 - p0 : j < 7 ? j : 0) : (j == 0 || mode == 1) ? p0 : 7 - p0;
+  };
+  auto wb = [&](int j) { return mode == 0 ? (j < 6 ? cA[6][j] : 0.f) : mode == 1 && j == 0 ? 1.f : 0.f; };
+  auto we = [&](int j) {
+    return mode == 0 ? (j < 7 ? cBT[j] : 0.f) : mode == 2 ? (j == 0 ? -1.f : j == 1 ? 1.f : 0.f) : 0.f;
+  };
+  int boff[2];
+  float cb[2], ce[2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int j = 4 * q + g;
+    boff[q] = block(j) * mm.sv;
+    cb[q] = wb(j) * sb;
+    ce[q] = we(j) * se;
   }
-  RG_MU_RW(1)
-  RG_MU_RW(2)
-  RG_MU_RW(4)
-#undef RG_MU_RW
-  if (mode == 0) return rg_mu_pass<0, RG_HT>(kargs, sbs, p0, dt, atol, rtol, mu, mun, nullptr, lane);
-  if (mode == 1) return rg_mu_pass<1, RG_HT>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, nullptr, lane);
-  return rg_mu_pass<2, RG_HT>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, fl, lane);
+  const gp<const f32x4> wsrc = (gp<const f32x4>)mu + lane;
+  const gp<f32x4> wdst = (gp<f32x4>)mu_new + lane;
+  const int tlast = mm.ntile - 1;
+  f32x4 buf[RW];
+#pragma unroll
+  for (int k = 0; k < RW; ++k) buf[k] = wsrc[(k < tlast ? k : tlast) * 64];
+  float acc = 0.f, fl = 0.f;
+
+  // ---- biases
+  float bm[NR], bkb[NR], bke[NR];
+  bool bok[NR];
+  int bat[NR];
+#pragma unroll
+  for (int n = 0; n < NR; ++n) {
+    const int l = n * LR + lane / LW, o = lane % LW;
+    int out = 1, sd = mm.sd[0], nb = (int)mm.nb0[0];
+    bool ok = false;
+#pragma unroll
+    for (int i = 0; i < RG_MAXL; ++i)
+      if (i == l && i < mm.L) { out = mm.out[i]; sd = mm.sd[i]; nb = (int)mm.nb0[i]; ok = o < mm.out[i]; }
+    const int oc = o < out ? o : out - 1;
+    bok[n] = ok;
+    bat[n] = nb + oc;
+    bm[n] = mu[nb + oc];
+    float kb = 0.f, ke = 0.f;
+    float d[7];
+#pragma unroll
+    for (int j = 0; j < 7; ++j) d[j] = sbs[block(j) * mm.sv + sd + oc];
+    if (mode == 0) {
+#pragma unroll
+      for (int j = 0; j < 7; ++j) {
+        kb += (j < 6 ? cA[6][j] : 0.f) * d[j];
+        ke += cBT[j] * d[j];
+      }
+      kb *= sb;
+      ke *= se;
+    } else if (mode == 1) {
+      kb = sb * d[0];
+    } else {
+      ke = se * (d[1] - d[0]);
+    }
+    bkb[n] = ok ? kb : 0.f;
+    bke[n] = ok ? ke : 0.f;
+  }
+#pragma unroll
+  for (int n = 0; n < NR; ++n) {
+    float mn = 0.f;
+    const float e = rg_mu_err(mode, bkb[n], bke[n], atf, rtf, bm[n], mn, fl);
+    if (mode == 0 && bok[n]) mu_new[bat[n]] = mn;
+    const float ev = bok[n] ? e : 0.f;
+#pragma unroll
+    for (int i = 0; i < LR; ++i) {
+      const float x = __shfl(ev, LW * i + lane % LW);
+      if (lane < LW) acc = fmaf(x, x, acc);
+    }
+  }
+
+  // ---- weight tiles (as in rg_mu_pass)
+#pragma unroll 1
+  for (int l = 0; l < mm.L; ++l) {
+    const int in = mm.in[l], out = mm.out[l];
+    const bool ro = mm.rowout[l];
+    float tB[RW][2], tE[RW][2], cB[RW][2], cE[RW][2];
+#pragma unroll
+    for (int t = 0; t < RW; ++t) {
+      const int i = 16 * t + r;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const float hv = sbs[boff[q] + mm.sh[l] + (i < in ? i : in - 1)];
+        const float dv = sbs[boff[q] + mm.sd[l] + (i < out ? i : out - 1)];
+        const float h = (i < in ? 1.f : 0.f) * hv;
+        const float dm = (i < out ? 1.f : 0.f) * dv;
+        const float bq = cb[q] * dm, eq = ce[q] * dm;
+        tB[t][q] = ro ? h : bq;
+        tE[t][q] = ro ? h : eq;
+        cB[t][q] = ro ? bq : h;
+        cE[t][q] = ro ? eq : h;
+      }
+    }
+    const int T0 = (int)(mm.nw0[l] >> 8), nr = mm.nrow[l];
+#pragma unroll
+    for (int a = 0; a < RW; ++a) {
+      if (a >= nr) break;
+#pragma unroll
+      for (int k = 0; k < RW; ++k) {
+        const int T = T0 + a * RW + k;
+        f32x4 kb = {0.f, 0.f, 0.f, 0.f}, ke = kb, mn = kb;
+        kb = rg_mfma(tB[a][0], cB[k][0], kb);
+        kb = rg_mfma(tB[a][1], cB[k][1], kb);
+        ke = rg_mfma(tE[a][0], cE[k][0], ke);
+        ke = rg_mfma(tE[a][1], cE[k][1], ke);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          float mv = 0.f;
+          const float ev = rg_mu_err(mode, kb[v], ke[v], atf, rtf, buf[k][v], mv, fl);
+          mn[v] = mv;
+          acc = fmaf(ev, ev, acc);
+        }
+        if (mode == 0) wdst[T * 64] = mn;
+        const int Tn = T + RW;
+        buf[k] = wsrc[(Tn < tlast ? Tn : tlast) * 64];
+      }
+    }
+  }
+  double sum = (double)acc, flg = (double)fl;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    sum += __shfl_xor(sum, off);
+    flg = fmax(flg, __shfl_xor(flg, off));
+  }
+  *flag = flg;
+  return sum;
+}
+
+// The pass of a width class (m.rw = RW).
+template <int RW>
+__device__ __forceinline__ double rg_mu_call(const RaggedModel& m, uint64_t kargs, int mode,
+                                             gp<const float> sbs, int p0, double dt, double atol,
+                                             double rtol, gp<const float> mu, gp<float> mun,
+                                             double* fl, int lane) {
+  if constexpr (RW <= 2) return rg_mu_small<RW>(m, mode, sbs, p0, dt, atol, rtol, mu, mun, fl, lane);
+  if (mode == 0) return rg_mu_pass<0, RW>(kargs, sbs, p0, dt, atol, rtol, mu, mun, nullptr, lane);
+  if (mode == 1) return rg_mu_pass<1, RW>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, nullptr, lane);
+  return rg_mu_pass<2, RW>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, fl, lane);
 }
 
 // A finished trajectory's row from the tile-row order to the flat
@@ -1098,20 +1206,20 @@ __device__ __forceinline__ void rg_tape_u(const RaggedAdjArgs& a, int cj, double
   }
 }
 
-template <int DT, bool BF>
-__global__ void __launch_bounds__(256) k_ragged_adj(RaggedAdjArgs a) {
+template <int DT, bool BF, int HT>
+__global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs a) {
   static_assert(offsetof(RaggedAdjArgs, m) == 0, "the model leads the argument struct");
   extern __shared__ __attribute__((aligned(16))) float rg_lds[];
   const RaggedModel& m = a.m;
   const uint64_t kargs = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
   rg_load_weights(m, rg_lds);
   const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
-  const int64_t wslot0 = ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * RG_SLOTS;
+  const int64_t wslot0 = ((int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * a.spw;
   // stage blocks of the slot's VJPs; the columns past spw never hold a
   // trajectory, and their VJP writes (garbage that stays in its own MFMA
   // column) go to one sink block shared by all of them, which stays in L2
   const gp<float> sb = r < a.spw ? glb(a.sbuf) + (wslot0 + r) * 8 * m.sv
-                                 : glb(a.sbuf) + a.nslots_all * 8 * m.sv;
+                                 : glb(a.sbuf) + a.nslots * 8 * m.sv;
   const int D = a.D;
   const int64_t P = m.P;
   const double nel = (double)D + (double)P;
@@ -1135,7 +1243,7 @@ __global__ void __launch_bounds__(256) k_ragged_adj(RaggedAdjArgs a) {
       need_start = false;
       // the slot's own position first (slots >= spw stay idle), then
       // positions from the queue
-      int64_t pos = r < a.spw ? wslot0 / RG_SLOTS * a.spw + r : a.norder;
+      int64_t pos = r < a.spw ? wslot0 + r : a.norder;
       if (!first_start) {
         int q = 0;
         if (g == 0) q = atomicAdd(a.queue, 1);
@@ -1209,9 +1317,9 @@ __global__ void __launch_bounds__(256) k_ragged_adj(RaggedAdjArgs a) {
       }
       rg_tape_u<DT>(a, cj, tcj, tnx, tau, uc, lane);
     }
-    f32x4 x0[RG_HT], lg[RG_HT], gv[RG_HT];
+    f32x4 x0[HT], lg[HT], gv[HT];
 #pragma unroll
-    for (int t = 0; t < RG_HT; ++t) {
+    for (int t = 0; t < HT; ++t) {
       x0[t] = lg[t] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (t < DT && traj >= 0) {
 #pragma unroll
@@ -1219,7 +1327,7 @@ __global__ void __launch_bounds__(256) k_ragged_adj(RaggedAdjArgs a) {
         lg[t] = ls[t];
       }
     }
-    rg_vjp<BF>(m, rg_lds, rg_lds + m.lds_floats + (threadIdx.x >> 6) * m.act_stride, x0, lg,
+    rg_vjp<BF, HT>(m, rg_lds, rg_lds + m.lds_floats + (threadIdx.x >> 6) * m.act_stride, x0, lg,
            sb + blkid * m.sv, gv, lane);
     // k = -(lambda^T df/du): input-map derivative 3u^2 for x.^3
     f32x4 kn[DT];
@@ -1293,12 +1401,12 @@ __global__ void __launch_bounds__(256) k_ragged_adj(RaggedAdjArgs a) {
     // ---- parameter part, slot by slot with the whole wave
     __threadfence_block();
     double smu = 0.0, flmu = 0.0;
-    for (int s = 0; s < RG_SLOTS; ++s) {
-      const int ms = __shfl(mode, s);
+    for (int s = 0; s < a.spw; ++s) {
+      const int ms = __builtin_amdgcn_readlane(mode, s);
       if (ms < 0) continue;
-      const int trs = __shfl(traj, s);
-      const int p0s = __shfl(p0, s);
-      const int mfs = __shfl(muflip, s);
+      const int trs = __builtin_amdgcn_readlane(traj, s);
+      const int p0s = __builtin_amdgcn_readlane(p0, s);
+      const int mfs = __builtin_amdgcn_readlane(muflip, s);
       const double dts = __shfl(c.dt, s);
       const gp<const float> sbs = glb(a.sbuf) + (wslot0 + s) * 8 * m.sv;
       const gp<float> row = glb(a.dLdp_traj) + (int64_t)trs * m.Pn;
@@ -1306,7 +1414,7 @@ __global__ void __launch_bounds__(256) k_ragged_adj(RaggedAdjArgs a) {
       const gp<const float> mu = mfs ? tmp : row;
       const gp<float> mun = mfs ? row : tmp;
       double fl = 0.0, sm;
-      sm = rg_mu_call(kargs, m.rw, ms, sbs, p0s, dts, a.abstol, a.reltol, mu, mun, &fl, lane);
+      sm = rg_mu_call<HT>(m, kargs, ms, sbs, p0s, dts, a.abstol, a.reltol, mu, mun, &fl, lane);
       if (r == s) { smu = sm; flmu = fl; }
     }
     // ---- consume, part 2: control
@@ -1420,12 +1528,12 @@ __global__ void __launch_bounds__(256) k_ragged_adj(RaggedAdjArgs a) {
     // flat parameter order (whole wave, converged): the tile-major row is
     // first copied to the slot's row when it is not there already
     if (__any(fin)) {
-      for (int s = 0; s < RG_SLOTS; ++s) {
-        if (!__shfl((int)fin, s)) continue;
-        const int trs = __shfl(traj, s);
+      for (int s = 0; s < a.spw; ++s) {
+        if (!__builtin_amdgcn_readlane((int)fin, s)) continue;
+        const int trs = __builtin_amdgcn_readlane(traj, s);
         const gp<float> tmp = glb(a.mu_tmp) + (wslot0 + s) * m.Pn;
         const gp<float> row = glb(a.dLdp_traj) + (int64_t)trs * m.Pn;
-        if (!__shfl(muflip, s)) {
+        if (!__builtin_amdgcn_readlane(muflip, s)) {
           for (int64_t i = 4 * lane; i < m.Pn; i += 256) *(gp<f32x4>)(tmp + i) = *(gp<const f32x4>)(row + i);
           __threadfence_block();
         }
@@ -1435,20 +1543,22 @@ __global__ void __launch_bounds__(256) k_ragged_adj(RaggedAdjArgs a) {
   }
 }
 
-// `waves` (1..4) waves of RG_SLOTS slots per workgroup
+int ragged_waves(int rw) { return rg_waves(rw); }
+
+// `waves` (1..4) waves of up to RG_SLOTS slots per workgroup
 void launch_ragged_adj(const RaggedAdjArgs& a, int grid, int waves, hipStream_t s) {
   const size_t lds = ((size_t)a.m.lds_floats + (size_t)waves * a.m.act_stride) * sizeof(float);
   auto go = [&](auto kern) {
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * waves), lds, s, a);
   };
-  if (a.Dp <= 16) {
-    if (a.vjp_bf16) go(k_ragged_adj<1, true>);
-    else go(k_ragged_adj<1, false>);
-  } else {
-    if (a.vjp_bf16) go(k_ragged_adj<2, true>);
-    else go(k_ragged_adj<2, false>);
-  }
+#define RG_GO(DT, HT)                                  \
+  do {                                                 \
+    if (a.vjp_bf16) go(k_ragged_adj<DT, true, HT>);    \
+    else go(k_ragged_adj<DT, false, HT>);              \
+  } while (0)
+  RG_DISPATCH(RG_GO);
+#undef RG_GO
 }
 
 // dL/dp = sum over trajectories of their FP32 rows (first P of every `stride`
