@@ -551,6 +551,94 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
   }
 }
 
+// FP32, ranges of 16 rows (small batches).  With one group of rows per range
+// the kernel above is a chain: a memory latency per stage and a sum over waves
+// in four LDS rounds (12.7 us for one trajectory's 2 tiles, 21 us for 333 rows).
+// Here all stages' operands are requested at once, and a wave takes all 16 rows
+// of a quarter of the tile (inputs 4 i + wave), so nothing is summed across
+// waves.
+__global__ void __launch_bounds__(256, 2) k_chain_wgrad32s(ChainWgradArgs a) {
+  const Ctl* ctl = a.ctl;
+  if (a.mode == SM_STEP && ctl->done) return;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  int it, ot, tile, chunk;
+  if (!wg_block(a, tile, chunk)) return;
+  const int l = wg_tile(a, tile, it, ot);
+  const int wi = a.ops.w[l], wo = a.ops.w[l + 1];
+  const int gsel = ctl->gsel;
+  const bool bias = it == 0 && wave == 0;
+  const int64_t rr = chunk * 16 + (lane >> 4);
+  const int64_t ho = rr * wi + it * GT + 4 * (lane & 15) + wave, dof = rr * wo + ot * GT + 4 * (lane & 15);
+  const f32x4v zero = {0.f, 0.f, 0.f, 0.f};
+  f32x4v ab[4], ae[4], bb = zero, be = zero;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) ab[q] = ae[q] = zero;
+  float hv[7][4];
+  f32x4v dv[7][4];
+  auto load = [&](int s) {
+    const char* ob = (const char*)a.ops.base + (int64_t)wg_slot(a.mode, s, gsel) * a.ops.slot;
+    const float* h = (const float*)(ob + a.ops.h[l]) + ho;
+    const float* d = (const float*)(ob + a.ops.d[l]) + dof;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      hv[s][j] = h[4 * j * wi];
+      dv[s][j] = *(const f32x4v*)(d + 4 * j * wo);
+    }
+  };
+  auto fold = [&](int s, float cb, float ce) {
+    f32x4v gb = zero;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (bias && (a.rprim == a.rblk || (rr + 4 * j) % a.rblk < a.rprim)) gb += dv[s][j];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      f32x4v g = zero;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) g = __builtin_amdgcn_mfma_f32_16x16x4f32(hv[s][j], dv[s][j][q], g, 0, 0, 0);
+      ab[q] += cb * g;
+      ae[q] += ce * g;
+    }
+    bb += cb * gb;
+    be += ce * gb;
+  };
+  load(0);
+  if (a.mode == SM_STEP) {
+#pragma unroll
+    for (int s = 1; s < 7; ++s) load(s);
+#pragma unroll
+    for (int s = 0; s < 7; ++s) fold(s, s < 6 ? chA[6][s] : 0.f, chBT[s]);
+  } else {
+    fold(0, 1.f, 0.f);
+  }
+  // acc element (q, v) of lane l: input 4 (4 (l / 16) + v) + wave, output 4 (l % 16) + q
+  const int64_t tsz = GT * (GT + 1);
+  float* out = a.part + ((int64_t)chunk * 2 * a.ntile + tile) * tsz;
+#pragma unroll
+  for (int which = 0; which < 2; ++which)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      f32x4v o;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o[q] = which ? ae[q][v] : ab[q][v];
+      *(f32x4v*)(out + (int64_t)which * a.ntile * tsz + (4 * (4 * (lane >> 4) + v) + wave) * GT +
+                 4 * (lane & 15)) = o;
+    }
+  if (bias) {
+    f32x4v x, y;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      x[q] = bb[q] + __shfl_xor(bb[q], 16);
+      x[q] += __shfl_xor(x[q], 32);
+      y[q] = be[q] + __shfl_xor(be[q], 16);
+      y[q] += __shfl_xor(y[q], 32);
+    }
+    if (lane < 16) {
+      *(f32x4v*)(out + GT * GT + 4 * lane) = x;
+      *(f32x4v*)(out + (int64_t)a.ntile * tsz + GT * GT + 4 * lane) = y;
+    }
+  }
+}
+
 // Split BF16.  K = rows must be contiguous per lane, the operands are
 // row-major: a 128 x 128 tile stages 32 rows of both in LDS and reads them
 // through the transposing LDS load (a group of 16 lanes reads four rows of 16
@@ -773,20 +861,20 @@ __global__ void __launch_bounds__(256) k_chain_mu(ChainMuArgs a) {
       const int qo = (int)(i - a.b0[l]), o = f32 ? chain_posn(qo) : qo;
       src = (int64_t)(w.tl[l] + o / E) * tsz + (int64_t)E * E + o % E;
     }
-    // (four ranges' loads in flight: a chain of 20 otherwise)
+    // (eight ranges' loads in flight: a chain of 20 otherwise)
     float b = 0.f, e = 0.f;
     const bool st = w.mode == SM_STEP;
     const float* p = w.part + src;
     int k = 0;
-    for (; k + 4 <= w.chunks; k += 4, p += 8 * half) {
-      float x[4], y[4];
+    for (; k + 8 <= w.chunks; k += 8, p += 16 * half) {
+      float x[8], y[8];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < 8; ++j) {
         x[j] = p[2 * j * half];
         y[j] = st ? p[(2 * j + 1) * half] : 0.f;
       }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) { b -= x[j]; e -= y[j]; }
+      for (int j = 0; j < 8; ++j) { b -= x[j]; e -= y[j]; }
     }
     for (; k < w.chunks; ++k, p += 2 * half) {
       b -= p[0];
@@ -812,7 +900,8 @@ __global__ void __launch_bounds__(256) k_chain_mu(ChainMuArgs a) {
 
 void launch_chain_wgrad(int prec, const ChainWgradArgs& a, hipStream_t s) {
   const dim3 grid(8 * ((a.ntile * a.chunks + 7) / 8));
-  if (prec == 0) hipLaunchKernelGGL(k_chain_wgrad32, grid, dim3(256), 0, s, a);
+  if (prec == 0 && a.crows == 16) hipLaunchKernelGGL(k_chain_wgrad32s, grid, dim3(256), 0, s, a);
+  else if (prec == 0) hipLaunchKernelGGL(k_chain_wgrad32, grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL(k_chain_wgrad16, grid, dim3(256), 0, s, a);
 }
 void launch_chain_mu(const ChainMuArgs& a, int nblk, hipStream_t s) {

@@ -804,7 +804,10 @@ int chain_adj_alloc(node_handle* h) {
     u.b0[l] = h->layers[l].b0;
   }
   const int64_t want = (h->prec == NODE_PREC_FP32 ? 512 : 256) / w.ntile;
-  w.chunks = (int)std::max<int64_t>(1, std::min<int64_t>(want, o.rows / 64));
+  // (FP32 batches of up to 32 groups of 16 rows: a range each, the kernel made
+  // for it; k_chain_mu adds the ranges one after the other, so no more)
+  const bool few = h->prec == NODE_PREC_FP32 && o.rows / 16 <= std::min<int64_t>(want, 32);
+  w.chunks = (int)std::max<int64_t>(1, std::min<int64_t>(want, o.rows / (few ? 16 : 64)));
   w.crows = rup((o.rows + w.chunks - 1) / w.chunks, K);
   w.chunks = (int)((o.rows + w.crows - 1) / w.crows);
   if (int rc = dalloc_t(h, &w.part, (size_t)w.chunks * 2 * w.ntile * E * (E + 1) * sizeof(float))) return rc;
