@@ -444,6 +444,7 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
   const int64_t r1 = r0 + a.crows < a.ops.rows ? r0 + a.crows : a.ops.rows;
   const int wi = a.ops.w[l], wo = a.ops.w[l + 1];
   const int gsel = ctl->gsel;
+  const int rblk = (int)a.rblk, rprim = (int)a.rprim;
   const int ns = a.mode == SM_STEP ? 7 : 1;
   f32x4v g[4][4], ab[4][4], ae[4][4];
   f32x4v gb, bb = {0.f, 0.f, 0.f, 0.f}, be = bb;
@@ -475,8 +476,8 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
       const f32x4v x = hv[j], y = dv[j];
       if (refill) load(j, k + PF);
       // bias: primal rows only
-      const int64_t row = rr + (int64_t)k * 16;
-      if (bias && (a.rprim == a.rblk || row % a.rblk < a.rprim)) gb += y;
+      // (a block's rows: a power of two)
+      if (bias && (((int)rr + k * 16) & (rblk - 1)) < rprim) gb += y;
 #pragma unroll
       for (int p = 0; p < 4; ++p)
 #pragma unroll
@@ -573,6 +574,10 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32s(ChainWgradArgs a) {
   f32x4v ab[4], ae[4], bb = zero, be = zero;
 #pragma unroll
   for (int q = 0; q < 4; ++q) ab[q] = ae[q] = zero;
+  // bias: primal rows only (a block's rows: a power of two, the primal first)
+  bool keep[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) keep[j] = (((int)rr + 4 * j) & ((int)a.rblk - 1)) < (int)a.rprim;
   float hv[7][4];
   f32x4v dv[7][4];
   auto load = [&](int s) {
@@ -589,7 +594,7 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32s(ChainWgradArgs a) {
     f32x4v gb = zero;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (bias && (a.rprim == a.rblk || (rr + 4 * j) % a.rblk < a.rprim)) gb += dv[s][j];
+      gb += keep[j] ? dv[s][j] : zero;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       f32x4v g = zero;
