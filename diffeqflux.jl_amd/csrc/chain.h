@@ -15,6 +15,7 @@ struct ChainModel {
   const float* bias[MAXL];
   int pitch;                   // LDS row pitch (elements)
   int nw;                      // waves per workgroup (4 or 8)
+  int cw, tf;                  // rows and features of an MFMA tile (16 x 16, or 4 x 64)
   int kt;                      // features per K tile
   // LDS byte offsets after the activation buffers: partial products of the
   // narrow layers (0: over the activations), hidden biases (rows of wmax), probe
@@ -25,6 +26,7 @@ struct ChainPack {
   int in[MAXL], out[MAXL], mtf[MAXL], ktf[MAXL], mtb[MAXL], ktb[MAXL];
   int64_t w0[MAXL];
   void* Wf[MAXL]; void* Wb[MAXL];
+  int tf;
 };
 void launch_pack_chain(int prec, const ChainPack& a, const float* p, hipStream_t s);
 struct ChainFwdArgs {
@@ -39,7 +41,7 @@ struct ChainFwdArgs {
 };
 // Operands of the weight gradients, kept per stage by the fused adjoint step:
 // for layer l its inputs h ([row][inp]) and output gradients d ([row][outp]),
-// T x planes (plane stride rows * width), rows = blocks * 16 nt (a flow's block
+// T x planes (plane stride rows * width), rows = blocks * cw nt (a flow's block
 // holds its primal rows first, then its tangent rows); widths padded to 64.
 // Slot of stage s: 1..5 -> s + 1; stages 0 and 6 share slots 0 and 1 (the last
 // stage of an accepted step is the next one's first: FSAL).
@@ -90,8 +92,8 @@ void launch_chain_adj(int prec, int nt, bool cnf, const ChainAdjArgs& a, int gri
 void launch_chain_wgrad(int prec, const ChainWgradArgs& a, hipStream_t s);
 void launch_chain_mu(const ChainMuArgs& a, int nblk, hipStream_t s);
 
-// nt: 16-column MFMA tiles per block (rows per block: 16 nt, a flow 8 nt)
-int chain_rows(int nt, bool cnf);
+// nt: column tiles (of cw) per block (rows per block: cw nt, a flow half)
+int chain_rows(const ChainModel& m, int nt, bool cnf);
 // LDS layout of a model's step kernels (fills the lds_ fields)
 void chain_layout(ChainModel& m, int nt, bool cnf);
 void launch_chain_fwd(int prec, int nt, bool cnf, const ChainFwdArgs& a, int grid, hipStream_t s);

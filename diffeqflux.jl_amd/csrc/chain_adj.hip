@@ -18,7 +18,8 @@ template <class PP, int NT, int NW, bool CNF>
 __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdjArgs a) {
   using T = typename PP::T;
   constexpr int THREADS = 64 * NW;
-  constexpr int COLS = 16 * NT, R = CNF ? 8 * NT : COLS;
+  constexpr int CW = ChainK<PP>::CW, TF = ChainK<PP>::TF;
+  constexpr int COLS = CW * NT, R = CNF ? COLS / 2 : COLS;
   constexpr int NE = R * (CNF ? 32 : 64) / THREADS;
   constexpr int P = PP::SPLIT ? 2 : 1;
   constexpr bool INPLACE = CNF;
@@ -198,11 +199,11 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
       f32x4v* sl = (f32x4v*)a.slope + (sbase + (int64_t)l * a.stiles) * NP * 64 + lane;
       f32x4v* cv = (f32x4v*)a.curve + (sbase + (int64_t)l * a.stiles) * NP * 64 + lane;
       auto epi = [&](int t, int, f32x4v (&acc)[NT]) {
-        const int f = 16 * t + 4 * (lane >> 4);
+        const int f = TF * t + 4 * (lane / CW);
         const f32x4v bv = *(const f32x4v*)(bias + f);
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
-          const int r = 16 * q + (lane & 15);
+          const int r = CW * q + (lane & (CW - 1));
           const f32x4v z = acc[q] + bv, y = act_f4(act, z);
           chain_put4<PP>(o, r, f, y);
           if constexpr (F32) *(f32x4v*)(hr + r * hw + f) = y;
@@ -282,19 +283,19 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
           if constexpr (F32)
-            sd[mi][q] = *(const f32x4v*)(hr + (16 * q + (lane & 15)) * dw + 16 * t + 4 * (lane >> 4));
+            sd[mi][q] = *(const f32x4v*)(hr + (CW * q + (lane & (CW - 1))) * dw + TF * t + 4 * (lane / CW));
           else sd[mi][q] = sl[(t * NP + q) * 64];
           if constexpr (CNF) c2[mi][q] = cv[(t * NP + q) * 64];
         }
       };
       auto pro = [&](int t, int mi) { if constexpr (F32) read(t, mi); };
       auto epi = [&](int t, int mi, f32x4v (&acc)[NT]) {
-        const int f = 16 * t + 4 * (lane >> 4);
+        const int f = TF * t + 4 * (lane / CW);
         const int i = F32 ? mi : 0;
         if constexpr (!F32) read(t, 0);
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
-          const int r = 16 * q + (lane & 15);
+          const int r = CW * q + (lane & (CW - 1));
           f32x4v d = sd[i][q];
           if constexpr (F32) d = act_y4(act, d);
           f32x4v v = acc[q] * d;
@@ -379,7 +380,10 @@ void launch_chain_adj(int prec, int nt, bool cnf, const ChainAdjArgs& a, int gri
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), lds, s, a);
   };
-  if (prec == 0) {
+  if (prec == 0 && a.m.cw == 4) {
+    if (nw == 8) go(k_chain_adj<PF32S, 2, 8, false>);
+    else go(k_chain_adj<PF32S, 2, 4, false>);
+  } else if (prec == 0) {
     if (cnf && nw == 8) go(k_chain_adj<PF32, 2, 8, true>);
     else if (cnf) go(k_chain_adj<PF32, 2, 4, true>);
     else if (nw == 8) go(k_chain_adj<PF32, 1, 8, false>);

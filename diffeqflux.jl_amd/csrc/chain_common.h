@@ -50,9 +50,18 @@ template <class PP> __device__ __forceinline__ int chain_pos(int f) {
   return sizeof(typename PP::T) == 4 ? chain_posn(f) : f;
 }
 
-// features per K tile, values per lane and K tile
-template <class PP> struct ChainK { static constexpr int KT = 32, V = 8; };
-template <> struct ChainK<PF32> { static constexpr int KT = 16, V = 4; };
+// FP32 in blocks of few rows: tiles of 64 features x 4 rows (v_mfma_4x4x1, one
+// K step of 16 four by four blocks) instead of 16 x 16.  The rate is the same,
+// so a block of 8 rows spends half the matrix time of one of 16, and a batch
+// that fills only some of the CUs with blocks of 16 spreads over twice as many.
+struct PF32S : PF32 {};
+
+// features per K tile, values per lane and K tile; rows (columns of the MFMA)
+// and features of a tile.  An accumulator lane holds the features
+// 4 (l / CW) .. + 3 of row l % CW in both shapes.
+template <class PP> struct ChainK { static constexpr int KT = 32, V = 8, CW = 16, TF = 16; };
+template <> struct ChainK<PF32> { static constexpr int KT = 16, V = 4, CW = 16, TF = 16; };
+template <> struct ChainK<PF32S> { static constexpr int KT = 16, V = 4, CW = 4, TF = 64; };
 
 // One MFMA K tile of a 16 x 16 block.  FP32: four 16x16x4 steps, lane l
 // supplying k = 4 (l / 16) + j to step j for both operands.  Split BF16:
@@ -117,10 +126,65 @@ template <class PP> struct ChainBuf {
 // The fragments of PF K tiles are in flight (ring in registers, loads
 // unconditional: the index is clamped instead).  side.step(): a piece of other
 // work per K tile.
+// The same on 64 x 4 tiles: a lane holds one feature's 16 K values (four
+// vectors) and reads its row's, in the order that the 16 x 16 steps take them.
+template <int NT, int MT, int PF>
+__device__ __forceinline__ void chain_mma4(f32x4v (&acc)[MT][NT], const void* __restrict__ W, int t0,
+                                           int tlast, int kt, int k0, int k1, const ChainBuf<PF32S>& in,
+                                           int lane) {
+  const f32x4v* w[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int t = t0 + m < tlast ? t0 + m : tlast;
+    w[m] = (const f32x4v*)W + (int64_t)t * kt * 256 + lane;
+  }
+  const float* b = in.at(lane & 3, 0);
+  f32x4v a[PF][MT][4];
+  auto load = [&](f32x4v (&f)[4], int m, int k) {
+    k = k < k1 ? k : k1 - 1;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) f[v] = w[m][(k * 4 + v) * 64];
+  };
+  auto step = [&](f32x4v (&f)[MT][4], int k, bool refill) {
+    f32x4v x[NT][4];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) x[n][v] = *(const f32x4v*)(b + n * 4 * in.pitch + k * 16 + 4 * v);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int n = 0; n < NT; ++n)
+            acc[m][n] = __builtin_amdgcn_mfma_f32_4x4x1f32(f[m][v][j], x[n][v][j], acc[m][n], 0, 0, 0);
+    if (refill)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) load(f[m], m, k + PF);
+  };
+#pragma unroll
+  for (int j = 0; j < PF; ++j)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) load(a[j][m], m, k0 + j);
+  int k = k0;
+  for (; k + PF <= k1; k += PF)
+#pragma unroll
+    for (int j = 0; j < PF; ++j) step(a[j], k + j, true);
+#pragma unroll
+  for (int j = 0; j < PF - 1; ++j)
+    if (k + j < k1) step(a[j], k + j, false);
+}
+
 template <class PP, int NT, int MT, int PF, class Side>
 __device__ __forceinline__ void chain_mma(f32x4v (&acc)[MT][NT], const void* __restrict__ W, int t0,
                                           int tlast, int kt, int k0, int k1, const ChainBuf<PP>& in,
                                           int lane, Side& side) {
+  if constexpr (ChainK<PP>::CW == 4) {
+    chain_mma4<NT, MT, (MT <= 2 ? 4 / MT : 2)>(acc, W, t0, tlast, kt, k0, k1, in, lane);
+    return;
+  } else {
   constexpr int P = PP::SPLIT ? 2 : 1;
   const u32x4* w[MT];
 #pragma unroll
@@ -164,6 +228,7 @@ __device__ __forceinline__ void chain_mma(f32x4v (&acc)[MT][NT], const void* __r
 #pragma unroll
   for (int j = 0; j < PF - 1; ++j)
     if (k + j < k1) step(a[j], k + j, false);
+  }
 }
 
 // FP32 blocks write their operand rows where they are produced (16 bytes per
@@ -323,18 +388,19 @@ __device__ __forceinline__ void chain_narrow(const void* W, int mt, int kt, cons
   for (int u = 0; u < 2; ++u) {
     const int w = wave + u * NW;
     if (w >= mt * ks) break;
-    const int t = w % mt, s = w / mt, pd = 16 * mt + 4;
-    float* o = part + s * (16 * NT) * pd + (lane & 15) * pd + 16 * t + 4 * (lane >> 4);
+    constexpr int CW = ChainK<PP>::CW, TF = ChainK<PP>::TF;
+    const int t = w % mt, s = w / mt, pd = TF * mt + 4;
+    float* o = part + s * (CW * NT) * pd + (lane & (CW - 1)) * pd + TF * t + 4 * (lane / CW);
 #pragma unroll
-    for (int n = 0; n < NT; ++n) *(f32x4v*)(o + n * 16 * pd) = acc[u][0][n];
+    for (int n = 0; n < NT; ++n) *(f32x4v*)(o + n * CW * pd) = acc[u][0][n];
   }
   chain_barrier();
 }
 template <class PP, int NW, int NT>
 __device__ __forceinline__ float chain_sum(const float* part, int mt, int kt, int row, int c) {
-  const int ks = chain_splits<NW>(mt, kt, ChainK<PP>::KT), pd = 16 * mt + 4;
+  const int ks = chain_splits<NW>(mt, kt, ChainK<PP>::KT), pd = ChainK<PP>::TF * mt + 4;
   float v = part[row * pd + c];
-  for (int s = 1; s < ks; ++s) v += part[(s * 16 * NT + row) * pd + c];
+  for (int s = 1; s < ks; ++s) v += part[(s * ChainK<PP>::CW * NT + row) * pd + c];
   return v;
 }
 
@@ -398,7 +464,7 @@ __device__ __forceinline__ void chain_stage_init(const ChainModel& m, const Ctl*
   }
   float* lb = (float*)(chain_lds() + m.lds_bias);
   for (int l = 0; l < m.L - 1; ++l)
-    for (int i = tid; i < 16 * m.mtf[l]; i += THREADS) lb[l * m.wmax + chain_pos<PP>(i)] = m.bias[l][i];
+    for (int i = tid; i < ChainK<PP>::TF * m.mtf[l]; i += THREADS) lb[l * m.wmax + chain_pos<PP>(i)] = m.bias[l][i];
   if constexpr (CNF) {
     float* lp = (float*)(chain_lds() + m.lds_probe);
     for (int i = tid; i < R * m.dm; i += THREADS)

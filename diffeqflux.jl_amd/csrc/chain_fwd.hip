@@ -13,7 +13,7 @@
 
 namespace nodehip {
 
-int chain_rows(int nt, bool cnf) { return cnf ? 8 * nt : 16 * nt; }
+int chain_rows(const ChainModel& m, int nt, bool cnf) { return m.cw * nt / (cnf ? 2 : 1); }
 
 // Pending saves of the last accepted step for the block's entries
 template <int THREADS>
@@ -51,7 +51,8 @@ template <class PP, int NT, int NW, bool CNF>
 __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwdArgs a) {
   using T = typename PP::T;
   constexpr int CH_THREADS = 64 * NW;
-  constexpr int COLS = 16 * NT, R = CNF ? 8 * NT : COLS;
+  constexpr int CW = ChainK<PP>::CW, TF = ChainK<PP>::TF;
+  constexpr int COLS = CW * NT, R = CNF ? COLS / 2 : COLS;
   constexpr int NE = R * (CNF ? 32 : 64) / CH_THREADS;  // state entries per thread (D <= 64, flow 32)
   constexpr int P = PP::SPLIT ? 2 : 1;
   constexpr bool INPLACE = CNF;
@@ -143,14 +144,14 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
       const float* bias = lbias + l * m.wmax;
       const int act = m.act[l];
       auto epi = [&](int t, int, f32x4v (&acc)[NT]) {
-        const int f = 16 * t + 4 * (lane >> 4);
+        const int f = TF * t + 4 * (lane / CW), r = lane & (CW - 1);
         const f32x4v bv = *(const f32x4v*)(bias + f);
 #pragma unroll
         for (int q = 0; q < (CNF ? NT / 2 : NT); ++q) {
           const f32x4v z = acc[q] + bv, y = act_f4(act, z);
-          chain_put4<PP>(o, 16 * q + (lane & 15), f, y);
+          chain_put4<PP>(o, CW * q + r, f, y);
           if constexpr (CNF)
-            chain_put4<PP>(o, R + 16 * q + (lane & 15), f, acc[q + NT / 2] * act_d4(act, z, y));
+            chain_put4<PP>(o, R + CW * q + r, f, acc[q + NT / 2] * act_d4(act, z, y));
         }
       };
       chain_layer<PP, NT, NW, INPLACE>(m.Wf[l], m.mtf[l], m.ktf[l], in, wave, lane, none,
@@ -208,19 +209,19 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
 
 void chain_layout(ChainModel& m, int nt, bool cnf) {
   // four bytes per activation: FP32, or two BF16 planes
-  const int cols = 16 * nt, act = (cnf ? 1 : 2) * cols * m.pitch * 4;
+  const int cols = m.cw * nt, act = (cnf ? 1 : 2) * cols * m.pitch * 4;
   int part = 0;
   m.wmax = 4;
   for (int i = 0; i < 2; ++i) {
     const int x = i ? m.mtb[0] : m.mtf[m.L - 1], k = i ? m.ktb[0] : m.ktf[m.L - 1];
     const int ks = m.nw == 8 ? chain_splits<8>(x, k, m.kt) : chain_splits<4>(x, k, m.kt);
-    part = std::max(part, ks * cols * (16 * x + 4) * 4);
+    part = std::max(part, ks * cols * (m.tf * x + 4) * 4);
   }
-  for (int l = 0; l < m.L - 1; ++l) m.wmax = std::max(m.wmax, 16 * m.mtf[l]);
+  for (int l = 0; l < m.L - 1; ++l) m.wmax = std::max(m.wmax, m.tf * m.mtf[l]);
   m.lds_part = cnf ? 0 : act;
   m.lds_bias = cnf ? std::max(act, part) : act + part;
   m.lds_probe = m.lds_bias + (m.L - 1) * m.wmax * 4;
-  m.lds_bytes = m.lds_probe + (cnf ? chain_rows(nt, true) * m.dm * 4 : 0);
+  m.lds_bytes = m.lds_probe + (cnf ? chain_rows(m, nt, true) * m.dm * 4 : 0);
 }
 
 void launch_chain_fwd(int prec, int nt, bool cnf, const ChainFwdArgs& a, int grid, hipStream_t s) {
@@ -230,7 +231,10 @@ void launch_chain_fwd(int prec, int nt, bool cnf, const ChainFwdArgs& a, int gri
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), lds, s, a);
   };
-  if (prec == 0) {
+  if (prec == 0 && a.m.cw == 4) {
+    if (nw == 8) go(k_chain_fwd<PF32S, 2, 8, false>);
+    else go(k_chain_fwd<PF32S, 2, 4, false>);
+  } else if (prec == 0) {
     if (cnf && nw == 8) go(k_chain_fwd<PF32, 2, 8, true>);
     else if (cnf) go(k_chain_fwd<PF32, 2, 4, true>);
     else if (nw == 8) go(k_chain_fwd<PF32, 1, 8, false>);
@@ -254,6 +258,7 @@ template <class PP>
 __global__ void __launch_bounds__(256) k_pack_chain(ChainPack a, const float* __restrict__ p) {
   using T = typename PP::T;
   constexpr int V = ChainK<PP>::V, KT = ChainK<PP>::KT, P = PP::SPLIT ? 2 : 1;
+  constexpr int TF = ChainK<PP>::TF, NV = TF / 16;   // vectors of a K tile per lane (64 x 4 tiles: four)
   const int l = blockIdx.y >> 1;
   const bool bwd = blockIdx.y & 1;
   T* W = (T*)(bwd ? a.Wb[l] : a.Wf[l]);
@@ -263,13 +268,13 @@ __global__ void __launch_bounds__(256) k_pack_chain(ChainPack a, const float* __
   const bool hid = bwd ? l > 0 : l < a.nl - 1;   // hidden features on the M side
   constexpr bool F32 = sizeof(T) == 4;           // (stored in chain_feat order)
   const float* w = p + a.w0[l];
-  const int64_t nfl = (int64_t)mt * kt * 64;
+  const int64_t nfl = (int64_t)mt * kt * NV * 64;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < nfl;
        i += (int64_t)gridDim.x * blockDim.x) {
     const int lane = (int)(i & 63);
-    const int64_t f = i >> 6;
-    const int t = (int)(f / kt), k = (int)(f % kt);
-    const int mr = 16 * t + (lane & 15), k0 = k * KT + V * (lane >> 4);
+    const int64_t f = i >> 6;                        // (fragment, vector)
+    const int t = (int)(f / NV / kt), k = (int)(f / NV % kt);
+    const int mr = TF * t + (lane & (TF - 1)), k0 = k * KT + V * (TF == 64 ? (int)(f & 3) : lane >> 4);
     const int mrow = F32 && hid ? chain_feat(mr) : mr;
     T* d = W + (f * P * 64 + lane) * V;
 #pragma unroll
@@ -290,7 +295,9 @@ void launch_pack_chain(int prec, const ChainPack& a, const float* p, hipStream_t
     most = b > most ? b : most;
   }
   const int grid = (int)((most + 3) / 4 < 1024 ? (most + 3) / 4 : 1024);
-  if (prec == 0) hipLaunchKernelGGL(k_pack_chain<PF32>, dim3(grid, 2 * a.nl), dim3(256), 0, s, a, p);
+  if (prec == 0 && a.tf == 64)
+    hipLaunchKernelGGL(k_pack_chain<PF32S>, dim3(grid, 2 * a.nl), dim3(256), 0, s, a, p);
+  else if (prec == 0) hipLaunchKernelGGL(k_pack_chain<PF32>, dim3(grid, 2 * a.nl), dim3(256), 0, s, a, p);
   else hipLaunchKernelGGL(k_pack_chain<PBF16X3>, dim3(grid, 2 * a.nl), dim3(256), 0, s, a, p);
 }
 

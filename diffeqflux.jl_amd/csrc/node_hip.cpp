@@ -683,7 +683,8 @@ void vjp_eval(node_handle* h, int stage, int mode, int gate, int wflags, float c
 // whose blocks would outnumber the CUs: the weights then pass L2 once for twice
 // the rows.  A flow's two (four) tiles are 16 (32) primal and as many tangent
 // rows.
-int chain_tiles(const node_handle* h) {
+int chain_tiles(const node_handle* h, const ChainModel& m) {
+  if (m.cw == 4) return 2;
   const bool many = h->prec == NODE_PREC_BF16X3 && h->B > 16 * 256;
   return (h->cnf ? 2 : 1) * (many ? 2 : 1);
 }
@@ -699,16 +700,30 @@ bool chain_plan(node_handle* h, ChainModel& m) {
   m.L = h->L; m.map = h->desc.input_map; m.D = h->D; m.B = h->B; m.kt = KT;
   m.dm = h->cnf ? h->cnf_dm : h->D;
   m.tcat = h->desc.input_map == NODE_MAP_CNF_TIME ? 1 : 0;
-  int wide = 0;
+  int wide = 0, mid = 0;
+  for (int l = 0; l < h->L; ++l) mid = std::max(mid, std::min(h->layers[l].in, h->layers[l].out));
+  // 64 x 4 tiles, blocks of 8 rows: less matrix time per block (a chain of one
+  // MFMA per K step, ~17 cycles each, against two waves' shares of 32), worth it
+  // where a layer is wide both ways and the blocks fit the chip at once.  Fixed
+  // steps, forward / adjoint us at 300 rows, 16-row against 8-row blocks:
+  // 64-128-128-64 955 / 1921 and 1024 / 2067, 64-160-160-64 1257 / 2657 and
+  // 1132 / 2360, 64-256-256-64 1590 / 3366 and 1334 / 2919, 64-512-512-64
+  // 3678 / 7928 and 2422 / 5837; 8-1024-8 1028 / 2595 and 1106 / 2434.
+  const bool small = h->prec == NODE_PREC_FP32 && !h->cnf && mid > 128 && h->B <= 8 * 256;
+  m.cw = small ? 4 : 16;
+  m.tf = small ? 64 : 16;
+  wide = 0;
   for (int l = 0; l < h->L; ++l) {
     const Layer& ly = h->layers[l];
     m.in[l] = ly.in; m.out[l] = ly.out; m.act[l] = ly.act;
     // hidden widths are padded to whole K tiles of the layer that reads them
     m.ktf[l] = (ly.in + KT - 1) / KT;
     m.ktb[l] = (ly.out + KT - 1) / KT;
-    m.mtf[l] = l < h->L - 1 ? m.ktb[l] * KT / 16 : (ly.out + 15) / 16;
-    m.mtb[l] = l > 0 ? m.ktf[l] * KT / 16 : (ly.in + 15) / 16;
+    auto tiles = [&](int f) { return (f + m.tf - 1) / m.tf; };
+    m.mtf[l] = tiles(l < h->L - 1 ? m.ktb[l] * KT : ly.out);
+    m.mtb[l] = tiles(l > 0 ? m.ktf[l] * KT : ly.in);
     wide = std::max(wide, std::max(m.ktf[l], m.ktb[l]) * KT);
+    if (l < h->L - 1) wide = std::max(wide, m.mtf[l] * m.tf);
   }
   if (wide > 1024 || (h->cnf && wide > 512)) return false;
   // Past ~700k weights a block's way through them (2.2M: ~100 us per
@@ -720,19 +735,19 @@ bool chain_plan(node_handle* h, ChainModel& m) {
   m.pitch = wide + (h->prec == NODE_PREC_FP32 ? 4 : 8);
   // eight waves (two per SIMD) where the wide layers have a tile for each; the
   // larger blocks are built for eight
-  m.nw = wide >= 128 || chain_tiles(h) > (h->cnf ? 2 : 1) ? 8 : 4;
+  m.nw = small ? (wide > 256 ? 8 : 4) : wide >= 128 || chain_tiles(h, m) > (h->cnf ? 2 : 1) ? 8 : 4;
   return true;
 }
 
 // Layout of the operand store (without its address).
 constexpr int CHAIN_LDS_MAX = 159 * 1024;  // (static LDS of the kernels aside)
 constexpr int64_t CHAIN_OPS_MAX = int64_t(4) << 30;  // bytes a handle may keep for it
-ChainOps chain_ops(const node_handle* h, int nt) {
+ChainOps chain_ops(const node_handle* h, const ChainModel& m, int nt) {
   ChainOps o{};
-  const int r = chain_rows(nt, h->cnf);
+  const int r = chain_rows(m, nt, h->cnf);
   // (split: whole groups of the weight gradients' 32 rows; those past the blocks
   // stay zero)
-  o.rows = rup((int64_t)((h->B + r - 1) / r) * 16 * nt, h->prec == NODE_PREC_FP32 ? 16 : 32);
+  o.rows = rup((int64_t)((h->B + r - 1) / r) * m.cw * nt, h->prec == NODE_PREC_FP32 ? 16 : 32);
   const int64_t elt = (int64_t)h->esz * h->planes;
   for (int l = 0; l < h->L; ++l) o.w[l] = h->layers[l].inp;
   o.w[h->L] = h->layers[h->L - 1].outp;
@@ -748,15 +763,15 @@ ChainOps chain_ops(const node_handle* h, int nt) {
 int chain_alloc(node_handle* h) {
   ChainModel m;
   if (!chain_plan(h, m)) return 0;
-  int nt = chain_tiles(h);
+  int nt = chain_tiles(h, m);
   chain_layout(m, nt, h->cnf);
-  if (m.lds_bytes > CHAIN_LDS_MAX) chain_layout(m, nt = h->cnf ? 2 : 1, h->cnf);
+  if (m.lds_bytes > CHAIN_LDS_MAX) chain_layout(m, nt = h->cnf || m.cw == 4 ? 2 : 1, h->cnf);
   if (m.lds_bytes > CHAIN_LDS_MAX) return 0;
-  if ((h->B + chain_rows(nt, h->cnf) - 1) / chain_rows(nt, h->cnf) > MAX_PART) return 0;
+  if ((h->B + chain_rows(m, nt, h->cnf) - 1) / chain_rows(m, nt, h->cnf) > MAX_PART) return 0;
   const int V = h->prec == NODE_PREC_FP32 ? 4 : 8;
   for (int l = 0; l < h->L; ++l) {
     void *f = nullptr, *b = nullptr;
-    const size_t lane = (size_t)64 * V * h->esz * h->planes;
+    const size_t lane = (size_t)64 * V * h->esz * h->planes * (m.tf / 16);
     if (int rc = dalloc(h, &f, lane * m.mtf[l] * m.ktf[l])) return rc;
     if (int rc = dalloc(h, &b, lane * m.mtb[l] * m.ktb[l])) return rc;
     m.Wf[l] = f; m.Wb[l] = b;
@@ -765,12 +780,12 @@ int chain_alloc(node_handle* h) {
   h->chain = m;
   h->chain_nt = nt;
   // adjoint: linear last layer; one column tile of rows, a flow as its forward
-  const int ant = h->cnf ? nt : 1;
+  const int ant = h->cnf || m.cw == 4 ? nt : 1;
   ChainModel am = m;
   chain_layout(am, ant, h->cnf);
   if (h->layers[h->L - 1].act == NODE_ACT_IDENTITY && am.lds_bytes <= CHAIN_LDS_MAX &&
-      (h->B + chain_rows(ant, h->cnf) - 1) / chain_rows(ant, h->cnf) <= MAX_PART &&
-      chain_ops(h, ant).slot * 7 <= CHAIN_OPS_MAX) {
+      (h->B + chain_rows(m, ant, h->cnf) - 1) / chain_rows(m, ant, h->cnf) <= MAX_PART &&
+      chain_ops(h, m, ant).slot * 7 <= CHAIN_OPS_MAX) {
     h->chain_ant = ant;
     h->chain_adj = am;
   }
@@ -780,8 +795,8 @@ int chain_alloc(node_handle* h) {
 // Buffers of the fused adjoint, at its first use.
 int chain_adj_alloc(node_handle* h) {
   if (h->cops.base) return 0;
-  ChainOps o = chain_ops(h, h->chain_ant);
   const ChainModel& m = h->chain_adj;
+  ChainOps o = chain_ops(h, m, h->chain_ant);
   h->cstiles = 1;
   for (int l = 0; l < h->L - 1; ++l) h->cstiles = std::max(h->cstiles, m.mtf[l]);
   const size_t sc = (size_t)std::max(h->L - 1, 1) * o.rows * 16 * h->cstiles * sizeof(float);
@@ -794,8 +809,8 @@ int chain_adj_alloc(node_handle* h) {
   ChainWgradArgs& w = u.w;
   const int E = h->prec == NODE_PREC_FP32 ? 64 : 128, K = h->prec == NODE_PREC_FP32 ? 16 : 32;
   w.m = m;
-  w.rblk = 16 * h->chain_ant;
-  w.rprim = chain_rows(h->chain_ant, h->cnf);
+  w.rblk = m.cw * h->chain_ant;
+  w.rprim = chain_rows(m, h->chain_ant, h->cnf);
   for (int l = 0; l < h->L; ++l) {
     w.tl[l] = w.ntile;
     w.tw[l] = (o.w[l + 1] + E - 1) / E;
@@ -828,7 +843,7 @@ bool chain_adj_on(const node_handle* h) {
 }
 
 int chain_adj_grid(const node_handle* h) {
-  const int r = chain_rows(h->chain_ant, h->cnf);
+  const int r = chain_rows(h->chain_adj, h->chain_ant, h->cnf);
   return (h->B + r - 1) / r;
 }
 int chain_mu_blocks(const node_handle* h) {
@@ -868,7 +883,7 @@ void chain_adjoint(node_handle* h, const AdjBufs& ab, int mode, double* px, doub
 bool chain_on(const node_handle* h) { return h->chain_nt > 0 && h->tape_budget == 0; }
 
 int chain_grid(const node_handle* h) {
-  const int r = chain_rows(h->chain_nt, h->cnf);
+  const int r = chain_rows(h->chain, h->chain_nt, h->cnf);
   return (h->B + r - 1) / r;
 }
 
@@ -2180,6 +2195,7 @@ static int pack_params(node_handle* h) {
   if (h->chain_nt > 0) {
     ChainPack c{};
     c.nl = h->L;
+    c.tf = h->chain.tf;
     for (int l = 0; l < h->L; ++l) {
       const ChainModel& m = h->chain;
       c.in[l] = m.in[l]; c.out[l] = m.out[l];

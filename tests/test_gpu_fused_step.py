@@ -39,7 +39,8 @@ def model(widths, acts, seed=0, imap=0):
 @pytest.mark.parametrize("hidden,D,B", [
     ([], 5, 3), ([1], 1, 1), ([16], 2, 16), ([17], 2, 17), ([50], 2, 1), ([33, 70], 33, 65),
     ([128, 32], 16, 33), ([100, 300, 40], 64, 20), ([512], 64, 16), ([256, 256], 32, 130),
-    ([24], 3, 4097), ([70], 5, 512), ([70], 5, 513)])
+    ([24], 3, 4097), ([70], 5, 512), ([70], 5, 513),
+    ([130, 200], 7, 9), ([129, 513], 64, 21), ([140, 130], 3, 2048), ([140, 130], 3, 2049)])
 def test_neural_ode(hidden, D, B, prec):
     from diffeqflux_hip import Handle
     widths = [D] + hidden + [D]
