@@ -33,6 +33,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // scalar access in flight.  The hot loops go through these instead.
 template <class T> using gp = __attribute__((address_space(1))) T*;
 template <class T> __device__ __forceinline__ gp<T> glb(T* p) { return (gp<T>)p; }
+// The slots' stage blocks are in LDS where they fit, else in global memory.
+template <class T> using lp = __attribute__((address_space(3))) T*;
+__device__ __forceinline__ gp<f32x4> rg_v4(gp<float> p) { return (gp<f32x4>)p; }
+__device__ __forceinline__ lp<f32x4> rg_v4(lp<float> p) { return (lp<f32x4>)p; }
 
 // The kernels are compiled per width class HT (the longest tile dimension of
 // any layer, 1, 2, 4 or 8 tiles), with as many waves per SIMD as the class's
@@ -490,10 +494,10 @@ __device__ __forceinline__ void rg_act4(int act, const f32x4& z, f32x4& y, f32x4
 // or in the block's delta area when m.act_stride is 0) and returns
 // g = W_0^T delta_0 (the input-map derivative is applied by the caller).
 // BF: the products on BF16 operands (rounded to nearest), FP32 accumulation.
-template <bool BF, int HT>
+template <bool BF, int HT, class BP>
 __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, float* act_lds,
                                        const f32x4 (&x0)[HT], const f32x4 (&lam)[HT],
-                                       gp<float> blk, f32x4 (&gout)[HT], int lane) {
+                                       BP blk, f32x4 (&gout)[HT], int lane) {
   const int r = lane & 15, g4 = 4 * (lane >> 4);
   const int L = m.L;
   // one rolled loop body per sweep (the layer's input is copied into place
@@ -503,7 +507,7 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
 #pragma unroll
   for (int t = 0; t < HT; ++t) {
     hin[t] = x0[t];
-    if (t < m.ti[0]) *(gp<f32x4>)(blk + m.sh[0] + 16 * t + g4) = x0[t];
+    if (t < m.ti[0]) *rg_v4(blk + m.sh[0] + 16 * t + g4) = x0[t];
   }
 #pragma unroll 1
   for (int l = 0; l < L; ++l) {
@@ -544,7 +548,7 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
           sd[v] = act_d(1, acc[v], y[v]);
         }
         *(f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane) = sd;
-        *(gp<f32x4>)(blk + m.sh[l + 1] + 16 * ot + g4) = y;
+        *rg_v4(blk + m.sh[l + 1] + 16 * ot + g4) = y;
         hout[ot] = y;
       }
     } else if (HT == RG_HT && nti == 1 && nto == HT && act == 1 && m.act_stride && l < L - 1) {
@@ -568,7 +572,7 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
           sd[v] = act_d(1, acc[v], y[v]);
         }
         *(f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane) = sd;
-        *(gp<f32x4>)(blk + m.sh[l + 1] + 16 * ot + g4) = y;
+        *rg_v4(blk + m.sh[l + 1] + 16 * ot + g4) = y;
         hout[ot] = y;
       }
     } else {
@@ -600,8 +604,8 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
         f32x4 y, sd;
         rg_act4(act, acc, y, sd);
         if (m.act_stride) *(f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane) = sd;
-        else *(gp<f32x4>)(blk + m.sd[l] + 16 * ot + g4) = sd;
-        if (l < L - 1) *(gp<f32x4>)(blk + m.sh[l + 1] + 16 * ot + g4) = y;
+        else *rg_v4(blk + m.sd[l] + 16 * ot + g4) = sd;
+        if (l < L - 1) *rg_v4(blk + m.sh[l + 1] + 16 * ot + g4) = y;
         hout[ot] = y;
       }
     }
@@ -623,7 +627,7 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
       for (int ot = 0; ot < HT; ++ot) {
         const f32x4 ad = *(const f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane);
         const f32x4 d = gi[ot] * ad;
-        *(gp<f32x4>)(blk + m.sd[l] + 16 * ot + g4) = d;
+        *rg_v4(blk + m.sd[l] + 16 * ot + g4) = d;
         gi[ot] = d;
       }
 #pragma unroll
@@ -661,7 +665,7 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
       for (int ot = 0; ot < HT; ++ot) {
         if (ot > 0 && last) break;
         const f32x4 d = gi[ot] * *(const f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane);
-        *(gp<f32x4>)(blk + m.sd[l] + 16 * ot + g4) = d;
+        *rg_v4(blk + m.sd[l] + 16 * ot + g4) = d;
         gi[ot] = d;
       }
 #pragma unroll
@@ -710,11 +714,11 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
 #pragma unroll
     for (int ot = 0; ot < HT; ++ot) {
       if (HT == 1 || ot < nto) {
-        gp<float> pd = blk + m.sd[l] + 16 * ot + g4;
+        BP pd = blk + m.sd[l] + 16 * ot + g4;
         const f32x4 ad = m.act_stride ? *(const f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane)
-                                      : *(gp<const f32x4>)pd;
+                                      : *rg_v4(pd);
         const f32x4 d = gi[ot] * ad;
-        *(gp<f32x4>)pd = d;
+        *rg_v4(pd) = d;
         gi[ot] = d;
       }
     }
@@ -996,8 +1000,8 @@ __device__ __attribute__((noinline)) double rg_mu_pass(uint64_t kargs, gp<const 
 // value (kb and ke are both formed; the coefficients of the one a mode does not
 // use are 0).  The biases of 64 / (16 RW) layers go to one round of lanes, and
 // their squares are summed in the lanes and order rg_mu_pass sums them in.
-template <int RW>
-__device__ __forceinline__ double rg_mu_small(const RaggedModel& mm, int mode, gp<const float> sbs,
+template <int RW, class SP>
+__device__ __forceinline__ double rg_mu_small(const RaggedModel& mm, int mode, SP sbs,
                                               int p0, double dt, double atol, double rtol,
                                               gp<const float> __restrict__ mu,
                                               gp<float> __restrict__ mu_new, double* flag, int lane) {
@@ -1126,26 +1130,26 @@ __device__ __forceinline__ double rg_mu_small(const RaggedModel& mm, int mode, g
       }
     }
   }
-  double sum = (double)acc, flg = (double)fl;
+  double sum = (double)acc;
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    sum += __shfl_xor(sum, off);
-    flg = fmax(flg, __shfl_xor(flg, off));
-  }
-  *flag = flg;
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+  *flag = __any(fl != 0.f) ? 1.0 : 0.0;
   return sum;
 }
 
 // The pass of a width class (m.rw = RW).
-template <int RW>
+template <int RW, class SP>
 __device__ __forceinline__ double rg_mu_call(const RaggedModel& m, uint64_t kargs, int mode,
-                                             gp<const float> sbs, int p0, double dt, double atol,
+                                             SP sbs, int p0, double dt, double atol,
                                              double rtol, gp<const float> mu, gp<float> mun,
                                              double* fl, int lane) {
-  if constexpr (RW <= 2) return rg_mu_small<RW>(m, mode, sbs, p0, dt, atol, rtol, mu, mun, fl, lane);
+  if constexpr (RW <= 2) {
+    return rg_mu_small<RW>(m, mode, sbs, p0, dt, atol, rtol, mu, mun, fl, lane);
+  } else {
   if (mode == 0) return rg_mu_pass<0, RW>(kargs, sbs, p0, dt, atol, rtol, mu, mun, nullptr, lane);
   if (mode == 1) return rg_mu_pass<1, RW>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, nullptr, lane);
   return rg_mu_pass<2, RW>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, fl, lane);
+  }
 }
 
 // A finished trajectory's row from the tile-row order to the flat
@@ -1172,21 +1176,56 @@ __device__ void rg_row_to_flat(const RaggedModel& m, gp<const float> __restrict_
   }
 }
 
+// Where a slot stands on its trajectory's tape: record j (start time t, the
+// next one's tn) and the record before it (p, its start time tp and its own
+// predecessor pp), which a stage time usually falls in if not in j itself.  The
+// links are read when the cursor moves, not one after the other at every stage.
+struct TapeCursor {
+  int j, p, pp;
+  double t, tn, tp;
+  __device__ __forceinline__ void before(const RaggedAdjArgs& a) {
+    const int q = p >= 0 ? p : j;
+    tp = glb(a.rec_t)[q];
+    pp = glb(a.rec_prev)[q];
+  }
+  __device__ __forceinline__ void start(const RaggedAdjArgs& a, int last) {
+    j = last;
+    t = glb(a.rec_t)[j];
+    p = glb(a.rec_prev)[j];
+    tn = INFINITY;
+    before(a);
+  }
+  __device__ __forceinline__ void back_to(const RaggedAdjArgs& a, double tau) {
+    while (t > tau && p >= 0) {
+      tn = t;
+      j = p;
+      t = tp;
+      p = pp;
+      before(a);
+    }
+  }
+};
+
 // u(tau) of the slot's trajectory from its forward tape: the stored state when
 // tau is a step time, else the step's free interpolant (dt = t_{j+1} - t_j);
-// (cj, tcj, tnx): a record at or before tau's step and the time after it
+// the cursor is at or after tau's step
 template <int DT>
-__device__ __forceinline__ void rg_tape_u(const RaggedAdjArgs& a, int cj, double tcj, double tnx,
-                                          double tau, f32x4 (&uu)[DT], int lane) {
+__device__ __forceinline__ void rg_tape_u(const RaggedAdjArgs& a, const TapeCursor& c, double tau,
+                                          f32x4 (&uu)[DT], int lane) {
   const int g4 = 4 * (lane >> 4);
-  int j = cj;
-  double tj = tcj, tn = tnx;
-  const gp<const int> rprev = glb(a.rec_prev);
-  const gp<const double> rt = glb(a.rec_t);
-  while (tj > tau && rprev[j] >= 0) {
+  int j = c.j, p = c.p, pp = c.pp;
+  double tj = c.t, tn = c.tn, tp = c.tp;
+  bool first = true;
+  while (tj > tau && p >= 0) {
+    if (!first) {   // (the first step back is the cursor's own)
+      tp = glb(a.rec_t)[p];
+      pp = glb(a.rec_prev)[p];
+    }
+    first = false;
     tn = tj;
-    j = rprev[j];
-    tj = rt[j];
+    j = p;
+    tj = tp;
+    p = pp;
   }
   const gp<const float> rd = glb(a.rec_data) + (int64_t)j * 8 * a.Dp;
   if (tj == tau || !(tn > tj)) {
@@ -1206,7 +1245,7 @@ __device__ __forceinline__ void rg_tape_u(const RaggedAdjArgs& a, int cj, double
   }
 }
 
-template <int DT, bool BF, int HT>
+template <int DT, bool BF, int HT, bool SL>
 __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs a) {
   static_assert(offsetof(RaggedAdjArgs, m) == 0, "the model leads the argument struct");
   extern __shared__ __attribute__((aligned(16))) float rg_lds[];
@@ -1218,14 +1257,25 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
   // stage blocks of the slot's VJPs; the columns past spw never hold a
   // trajectory, and their VJP writes (garbage that stays in its own MFMA
   // column) go to one sink block shared by all of them, which stays in L2
-  const gp<float> sb = r < a.spw ? glb(a.sbuf) + (wslot0 + r) * 8 * m.sv
-                                 : glb(a.sbuf) + a.nslots * 8 * m.sv;
+  using SP = typename std::conditional<SL, lp<float>, gp<float>>::type;
+  const int bsv = 8 * m.sv;
+  SP sb0, sb;
+  if constexpr (SL) {
+    const int nw = blockDim.x >> 6, w = threadIdx.x >> 6;
+    lp<float> all = (lp<float>)rg_lds + m.lds_floats + nw * m.act_stride;
+    sb0 = all + w * a.spw * bsv;
+    sb = r < a.spw ? sb0 + r * bsv : all + nw * a.spw * bsv;
+  } else {
+    sb0 = glb(a.sbuf) + wslot0 * bsv;
+    sb = r < a.spw ? sb0 + r * bsv : glb(a.sbuf) + a.nslots * bsv;
+  }
   const int D = a.D;
   const int64_t P = m.P;
   const double nel = (double)D + (double)P;
   const float atol = (float)a.abstol, rtol = (float)a.reltol;
 
-  int traj = -1, phase = 0, stage = 0, p0 = 0, pad = 0, fsal_re = 0, muflip = 0, cj = 0;
+  int traj = -1, phase = 0, stage = 0, p0 = 0, pad = 0, fsal_re = 0, muflip = 0;
+  TapeCursor cur{};
   bool need_start = true, first_start = true;
   SlotCtl c{};
   f32x4 lam[DT], lnew[DT], kl[7][DT], uc[DT];
@@ -1236,7 +1286,7 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
     for (int j = 0; j < 7; ++j) kl[j][t] = lam[t];
   }
   int64_t s_lo = 0, snext = -1, nf = 0, nacc = 0, nrej = 0;
-  double tcj = 0.0, tnx = 0.0, dt0 = 0.0, d0 = 0.0, d1 = 0.0, s1l = 0.0;
+  double dt0 = 0.0, d0 = 0.0, d1 = 0.0, s1l = 0.0;
 
   for (;;) {
     if (need_start) {
@@ -1282,9 +1332,7 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
           }
         s0 = rg_slot_sum(s0);
         d0 = sqrt(s0 / nel);
-        cj = a.last_rec[traj];
-        tcj = a.rec_t[cj];
-        tnx = INFINITY;
+        cur.start(a, a.last_rec[traj]);
         p0 = 0;
         muflip = 0;
         fsal_re = 0;
@@ -1315,7 +1363,7 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
           for (int t = 0; t < DT; ++t) ls[t] = lam[t] + h * rg_stage_sum(kl, stage, t);
         }
       }
-      rg_tape_u<DT>(a, cj, tcj, tnx, tau, uc, lane);
+      rg_tape_u<DT>(a, cur, tau, uc, lane);
     }
     f32x4 x0[HT], lg[HT], gv[HT];
 #pragma unroll
@@ -1399,7 +1447,9 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
       fll = rg_slot_sum(fll);
     }
     // ---- parameter part, slot by slot with the whole wave
-    __threadfence_block();
+    // (a wave's LDS accesses are in order: only the compiler has to keep them so)
+    if constexpr (SL) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    else __threadfence_block();
     double smu = 0.0, flmu = 0.0;
     for (int s = 0; s < a.spw; ++s) {
       const int ms = __builtin_amdgcn_readlane(mode, s);
@@ -1408,7 +1458,7 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
       const int p0s = __builtin_amdgcn_readlane(p0, s);
       const int mfs = __builtin_amdgcn_readlane(muflip, s);
       const double dts = __shfl(c.dt, s);
-      const gp<const float> sbs = glb(a.sbuf) + (wslot0 + s) * 8 * m.sv;
+      const SP sbs = sb0 + s * bsv;
       const gp<float> row = glb(a.dLdp_traj) + (int64_t)trs * m.Pn;
       const gp<float> tmp = glb(a.mu_tmp) + (wslot0 + s) * m.Pn;
       const gp<const float> mu = mfs ? tmp : row;
@@ -1487,11 +1537,7 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
           fsal_re = 1;
         }
         // tape cursor back to the record holding the new time
-        while (tcj > c.t && a.rec_prev[cj] >= 0) {
-          tnx = tcj;
-          cj = a.rec_prev[cj];
-          tcj = a.rec_t[cj];
-        }
+        cur.back_to(a, c.t);
         if (!c.adaptive) c.dtpropose = c.dt;
         c.last_accept = 1;
         if (fll != 0.0) { c.retcode = 6; c.done = 1; }
@@ -1528,6 +1574,7 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
     // flat parameter order (whole wave, converged): the tile-major row is
     // first copied to the slot's row when it is not there already
     if (__any(fin)) {
+      if constexpr (SL) __threadfence_block();   // (the parameter pass's rows, read by other lanes)
       for (int s = 0; s < a.spw; ++s) {
         if (!__builtin_amdgcn_readlane((int)fin, s)) continue;
         const int trs = __builtin_amdgcn_readlane(traj, s);
@@ -1547,15 +1594,22 @@ int ragged_waves(int rw) { return rg_waves(rw); }
 
 // `waves` (1..4) waves of up to RG_SLOTS slots per workgroup
 void launch_ragged_adj(const RaggedAdjArgs& a, int grid, int waves, hipStream_t s) {
-  const size_t lds = ((size_t)a.m.lds_floats + (size_t)waves * a.m.act_stride) * sizeof(float);
+  const size_t lds = ((size_t)a.m.lds_floats + (size_t)waves * a.m.act_stride +
+                      (a.stage_lds ? (size_t)(waves * a.spw + 1) * 8 * a.m.sv : 0)) * sizeof(float);
   auto go = [&](auto kern) {
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * waves), lds, s, a);
   };
-#define RG_GO(DT, HT)                                  \
-  do {                                                 \
-    if (a.vjp_bf16) go(k_ragged_adj<DT, true, HT>);    \
-    else go(k_ragged_adj<DT, false, HT>);              \
+#define RG_GO(DT, HT)                                                          \
+  do {                                                                         \
+    constexpr bool SL = HT <= 2;                                               \
+    if (SL && a.stage_lds) {                                                   \
+      if (a.vjp_bf16) go(k_ragged_adj<DT, true, HT, SL>);                      \
+      else go(k_ragged_adj<DT, false, HT, SL>);                                \
+    } else {                                                                   \
+      if (a.vjp_bf16) go(k_ragged_adj<DT, true, HT, false>);                   \
+      else go(k_ragged_adj<DT, false, HT, false>);                             \
+    }                                                                          \
   } while (0)
   RG_DISPATCH(RG_GO);
 #undef RG_GO

@@ -17,7 +17,7 @@ from oracle.mlp import MLP
 
 pytestmark = pytest.mark.gpu
 
-CLASSES = [
+CLASSES = [  # (repeated 700 times; the last so often that its stage data leaves LDS)
     ([3, 13, 3], ["tanh", "identity"]),
     ([2, 16, 16, 9, 2], ["tanh", "softplus", "sigmoid", "identity"]),
     ([9, 17, 31, 9], ["softplus", "tanh", "identity"]),
@@ -26,6 +26,7 @@ CLASSES = [
     ([30, 50, 30], ["tanh", "identity"]),
     ([5, 65, 5], ["tanh", "identity"]),
     ([18, 100, 18], ["softplus", "identity"]),
+    ([2, 16, 16, 8, 2], ["tanh", "softplus", "sigmoid", "identity"]),
 ]
 
 
@@ -33,7 +34,7 @@ CLASSES = [
 @pytest.mark.parametrize("widths,acts", CLASSES, ids=["-".join(map(str, w)) for w, _ in CLASSES])
 def test_every_width_class(widths, acts, vjp):
     from diffeqflux_hip import Handle
-    tol, distinct, copies = 1e-6, 4, 700
+    tol, distinct, copies = 1e-6, 4, 4000 if widths == CLASSES[-1][0] else 700
     m = MLP(widths, acts)
     rng = np.random.default_rng(sum(widths))
     p32 = m.glorot_init(rng).astype(np.float32)
