@@ -2070,8 +2070,8 @@ __device__ bool adj_control(Ctl* c, double eest, double flag, const double* cbt)
 // One block.  Latency only: the control itself is one thread's, the forward
 // steps that the next attempt's seven stage times fall in are looked up by
 // seven threads at once, in times copied to LDS beside the partial sums (one
-// thread's seven binary searches in global memory took half of the kernel:
-// 12 -> 8 us).
+// thread's seven binary searches in global memory, and control fields fetched
+// one after the other, took most of the kernel: 12 -> 5.5 us).
 constexpr int AC_TIMES = 512;
 __global__ void k_adj_controller(Ctl* c, const double* pl, int nl, const double* pm, int nm,
                                  double nel, const double* cbt, const double* ft) {
