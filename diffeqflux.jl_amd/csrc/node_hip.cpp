@@ -792,6 +792,16 @@ int chain_alloc(node_handle* h) {
   return 0;
 }
 
+void chain_adj_free(node_handle* h) {
+  dfree(h, h->cslope);
+  dfree(h, h->ccurve);
+  dfree(h, h->cmu.w.part);
+  dfree(h, h->cops.base);
+  h->cslope = h->ccurve = nullptr;
+  h->cmu = ChainMuArgs{};
+  h->cops = ChainOps{};
+}
+
 // Buffers of the fused adjoint, at its first use.
 int chain_adj_alloc(node_handle* h) {
   if (h->cops.base) return 0;
@@ -800,7 +810,8 @@ int chain_adj_alloc(node_handle* h) {
   h->cstiles = 1;
   for (int l = 0; l < h->L - 1; ++l) h->cstiles = std::max(h->cstiles, m.mtf[l]);
   const size_t sc = (size_t)std::max(h->L - 1, 1) * o.rows * 16 * h->cstiles * sizeof(float);
-  if (int rc = dalloc_t(h, &h->cslope, sc)) return rc;
+  if (h->prec != NODE_PREC_FP32)               // (FP32 derives act' from the outputs)
+    if (int rc = dalloc_t(h, &h->cslope, sc)) return rc;
   if (h->cnf)
     if (int rc = dalloc_t(h, &h->ccurve, sc)) return rc;
   // weight-gradient tiles and row ranges: two workgroups (FP32) or one (split)
@@ -1511,12 +1522,16 @@ int backward_impl(node_handle* h, const float* d_dLdout, node_stats* st) {
     if (int rc = dalloc_t(h, &h->bs_ku, 8 * sv * 4)) return rc;
     if (int rc = dalloc_t(h, &h->bs_fu, sv * 4)) return rc;
   }
-  const bool fused = chain_adj_on(h);
-  if (fused) {
-    if (int rc = chain_adj_alloc(h)) return rc;
-  } else if (int rc = maybe_autotune(h)) {
-    return rc;
+  // (no memory for the fused step's operand slots: the GEMM path needs none)
+  if (chain_adj_on(h) && chain_adj_alloc(h)) {
+    chain_adj_free(h);
+    h->chain_ant = 0;
+    h->err.clear();
+    (void)hipGetLastError();
   }
+  const bool fused = chain_adj_on(h);
+  if (!fused)
+    if (int rc = maybe_autotune(h)) return rc;
   const bool ck = h->fwd_ring;
   if (ck && h->sense != NODE_SENSE_INTERPOLATING)
     return fail(h, NODE_ERR_STATE, "the last forward kept checkpoints only "
