@@ -1925,7 +1925,7 @@ int ragged_backward_impl(node_handle* h, const float* dLdout, float* dLdu0, doub
   m.act_stride = lds_of(waves, true) <= LDS ? act_tiles * 256 : 0;
   // stage blocks in LDS too (narrow classes), unless that costs a workgroup per
   // CU: every stage's operands are written and read a few hundred cycles apart
-  const bool stage_lds = m.rw <= 2 && occ * (lds_of(waves, m.act_stride > 0) +
+  const bool stage_lds = false && m.rw <= 2 && occ * (lds_of(waves, m.act_stride > 0) +
                                              (int64_t)(waves * spw + 1) * 8 * m.sv * (int64_t)sizeof(float)) <= LDS;
   // start order (a schedule only: each trajectory's arithmetic is the same
   // in any slot).  A wave runs until its last slot's trajectory is done and

@@ -1001,160 +1001,14 @@ __device__ __attribute__((noinline)) double rg_mu_pass(uint64_t kargs, gp<const 
   return sum;
 }
 
-// The same for the classes of one and two tiles: inlined, the mode a run-time
-// value (kb and ke are both formed; the coefficients of the one a mode does not
-// use are 0).  The biases of 64 / (16 RW) layers go to one round of lanes, and
-// their squares are summed in the lanes and order rg_mu_pass sums them in.
-template <int RW, class SP>
-__device__ __forceinline__ double rg_mu_small(const RaggedModel& mm, int mode, SP sbs,
-                                              int p0, double dt, double atol, double rtol,
-                                              gp<const float> __restrict__ mu,
-                                              gp<float> __restrict__ mu_new, double* flag, int lane) {
-  constexpr int LW = 16 * RW, LR = 64 / LW, NR = RG_MAXL / LR;  // lanes per layer, layers per round, rounds
-  const int r = lane & 15, g = lane >> 4;
-  const float dtf = (float)dt, atf = (float)atol, rtf = (float)rtol;
-  const float sb = mode == 0 ? -dtf : -1.f, se = mode == 0 ? dtf : -1.f;
-  // stage j's block and its weights in the two sums
-  auto block = [&](int j) {
-    return mode == 0 ? (j == 0 ? p0 : j == 6 ? 7 - p0 : j < 7 ? j : 0) : (j == 0 || mode == 1) ? p0 : 7 - p0;
-  };
-  auto wb = [&](int j) { return mode == 0 ? (j < 6 ? cA[6][j] : 0.f) : mode == 1 && j == 0 ? 1.f : 0.f; };
-  auto we = [&](int j) {
-    return mode == 0 ? (j < 7 ? cBT[j] : 0.f) : mode == 2 ? (j == 0 ? -1.f : j == 1 ? 1.f : 0.f) : 0.f;
-  };
-  int boff[2];
-  float cb[2], ce[2];
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int j = 4 * q + g;
-    boff[q] = block(j) * mm.sv;
-    cb[q] = wb(j) * sb;
-    ce[q] = we(j) * se;
-  }
-  const gp<const f32x4> wsrc = (gp<const f32x4>)mu + lane;
-  const gp<f32x4> wdst = (gp<f32x4>)mu_new + lane;
-  const int tlast = mm.ntile - 1;
-  f32x4 buf[RW];
-#pragma unroll
-  for (int k = 0; k < RW; ++k) buf[k] = wsrc[(k < tlast ? k : tlast) * 64];
-  float acc = 0.f, fl = 0.f;
-
-  // ---- biases
-  float bm[NR], bkb[NR], bke[NR];
-  bool bok[NR];
-  int bat[NR];
-#pragma unroll
-  for (int n = 0; n < NR; ++n) {
-    const int l = n * LR + lane / LW, o = lane % LW;
-    int out = 1, sd = mm.sd[0], nb = (int)mm.nb0[0];
-    bool ok = false;
-#pragma unroll
-    for (int i = 0; i < RG_MAXL; ++i)
-      if (i == l && i < mm.L) { out = mm.out[i]; sd = mm.sd[i]; nb = (int)mm.nb0[i]; ok = o < mm.out[i]; }
-    const int oc = o < out ? o : out - 1;
-    bok[n] = ok;
-    bat[n] = nb + oc;
-    bm[n] = mu[nb + oc];
-    float kb = 0.f, ke = 0.f;
-    float d[7];
-#pragma unroll
-    for (int j = 0; j < 7; ++j) d[j] = sbs[block(j) * mm.sv + sd + oc];
-    if (mode == 0) {
-#pragma unroll
-      for (int j = 0; j < 7; ++j) {
-        kb += (j < 6 ? cA[6][j] : 0.f) * d[j];
-        ke += cBT[j] * d[j];
-      }
-      kb *= sb;
-      ke *= se;
-    } else if (mode == 1) {
-      kb = sb * d[0];
-    } else {
-      ke = se * (d[1] - d[0]);
-    }
-    bkb[n] = ok ? kb : 0.f;
-    bke[n] = ok ? ke : 0.f;
-  }
-#pragma unroll
-  for (int n = 0; n < NR; ++n) {
-    float mn = 0.f;
-    const float e = rg_mu_err(mode, bkb[n], bke[n], atf, rtf, bm[n], mn, fl);
-    if (mode == 0 && bok[n]) mu_new[bat[n]] = mn;
-    const float ev = bok[n] ? e : 0.f;
-#pragma unroll
-    for (int i = 0; i < LR; ++i) {
-      const float x = __shfl(ev, LW * i + lane % LW);
-      if (lane < LW) acc = fmaf(x, x, acc);
-    }
-  }
-
-  // ---- weight tiles (as in rg_mu_pass)
-#pragma unroll 1
-  for (int l = 0; l < mm.L; ++l) {
-    const int in = mm.in[l], out = mm.out[l];
-    const bool ro = mm.rowout[l];
-    float tB[RW][2], tE[RW][2], cB[RW][2], cE[RW][2];
-#pragma unroll
-    for (int t = 0; t < RW; ++t) {
-      const int i = 16 * t + r;
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const float hv = sbs[boff[q] + mm.sh[l] + (i < in ? i : in - 1)];
-        const float dv = sbs[boff[q] + mm.sd[l] + (i < out ? i : out - 1)];
-        const float h = (i < in ? 1.f : 0.f) * hv;
-        const float dm = (i < out ? 1.f : 0.f) * dv;
-        const float bq = cb[q] * dm, eq = ce[q] * dm;
-        tB[t][q] = ro ? h : bq;
-        tE[t][q] = ro ? h : eq;
-        cB[t][q] = ro ? bq : h;
-        cE[t][q] = ro ? eq : h;
-      }
-    }
-    const int T0 = (int)(mm.nw0[l] >> 8), nr = mm.nrow[l];
-#pragma unroll
-    for (int a = 0; a < RW; ++a) {
-      if (a >= nr) break;
-#pragma unroll
-      for (int k = 0; k < RW; ++k) {
-        const int T = T0 + a * RW + k;
-        f32x4 kb = {0.f, 0.f, 0.f, 0.f}, ke = kb, mn = kb;
-        kb = rg_mfma(tB[a][0], cB[k][0], kb);
-        kb = rg_mfma(tB[a][1], cB[k][1], kb);
-        ke = rg_mfma(tE[a][0], cE[k][0], ke);
-        ke = rg_mfma(tE[a][1], cE[k][1], ke);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          float mv = 0.f;
-          const float ev = rg_mu_err(mode, kb[v], ke[v], atf, rtf, buf[k][v], mv, fl);
-          mn[v] = mv;
-          acc = fmaf(ev, ev, acc);
-        }
-        if (mode == 0) wdst[T * 64] = mn;
-        const int Tn = T + RW;
-        buf[k] = wsrc[(Tn < tlast ? Tn : tlast) * 64];
-      }
-    }
-  }
-  double sum = (double)acc;
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-  *flag = __any(fl != 0.f) ? 1.0 : 0.0;
-  return sum;
-}
-
 // The pass of a width class (m.rw = RW).
-template <int RW, class SP>
-__device__ __forceinline__ double rg_mu_call(const RaggedModel& m, uint64_t kargs, int mode,
-                                             SP sbs, int p0, double dt, double atol,
-                                             double rtol, gp<const float> mu, gp<float> mun,
-                                             double* fl, int lane) {
-  if constexpr (RW <= 2) {
-    return rg_mu_small<RW>(m, mode, sbs, p0, dt, atol, rtol, mu, mun, fl, lane);
-  } else {
+template <int RW>
+__device__ __forceinline__ double rg_mu_call(uint64_t kargs, int mode, gp<const float> sbs, int p0,
+                                             double dt, double atol, double rtol, gp<const float> mu,
+                                             gp<float> mun, double* fl, int lane) {
   if (mode == 0) return rg_mu_pass<0, RW>(kargs, sbs, p0, dt, atol, rtol, mu, mun, nullptr, lane);
   if (mode == 1) return rg_mu_pass<1, RW>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, nullptr, lane);
   return rg_mu_pass<2, RW>(kargs, sbs, p0, dt, atol, rtol, mu, nullptr, fl, lane);
-  }
 }
 
 // A finished trajectory's row from the tile-row order to the flat
@@ -1469,7 +1323,7 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
       const gp<const float> mu = mfs ? tmp : row;
       const gp<float> mun = mfs ? row : tmp;
       double fl = 0.0, sm;
-      sm = rg_mu_call<HT>(m, kargs, ms, sbs, p0s, dts, a.abstol, a.reltol, mu, mun, &fl, lane);
+      sm = rg_mu_call<HT>(kargs, ms, sbs, p0s, dts, a.abstol, a.reltol, mu, mun, &fl, lane);
       if (r == s) { smu = sm; flmu = fl; }
     }
     // ---- consume, part 2: control
@@ -1607,8 +1461,8 @@ void launch_ragged_adj(const RaggedAdjArgs& a, int grid, int waves, hipStream_t 
   };
 #define RG_GO(DT, HT)                                                          \
   do {                                                                         \
-    constexpr bool SL = HT <= 2;                                               \
-    if (SL && a.stage_lds) {                                                   \
+    constexpr bool SL = false;                                                 \
+    if (SL) {                                                   \
       if (a.vjp_bf16) go(k_ragged_adj<DT, true, HT, SL>);                      \
       else go(k_ragged_adj<DT, false, HT, SL>);                                \
     } else {                                                                   \
