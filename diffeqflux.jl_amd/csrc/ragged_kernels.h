@@ -42,12 +42,9 @@ __device__ __forceinline__ lp<f32x4> rg_v4(lp<float> p) { return (lp<f32x4>)p; }
 // any layer, 1, 2, 4 or 8 tiles), with as many waves per SIMD as the class's
 // registers allow: a class-1 VJP is a dozen dependent LDS reads and MFMAs, a
 // parameter pass a few dependent memory reads, and the other wave runs under
-// them.  Three waves (168 registers) spill 360-750 B per lane.  One kernel for
-// all widths, one wave per SIMD, against this (forward + adjoint): 2-16-2 over
-// 15,360 segments 6.7 -> 5.6 ms, 3-16-16-3 x 10,000 7.1 -> 4.95, 8-32-32-8 x
-// 2,000 9.9 -> 7.9, 12-60-12 x 5,000 12.9 -> 11.3, 5-40-5 x 20 7.1 -> 5.4;
-// 16-128-128-16 x 10,000 (class 8, one wave as before: its weights fill the
-// LDS) 83.5 -> 82.2.
+// them.  Three waves (168 registers) spill 360-750 B per lane.  16-128-128-16 x
+// 10,000 (class 8, one wave as before: its weights fill the LDS) 83.5 -> 82.2
+// ms forward + adjoint, 12-60-12 x 5,000 12.9 -> 11.3.
 __host__ __device__ constexpr int rg_waves(int ht) { return ht <= 4 ? 2 : 1; }
 
 struct SlotCtl {
