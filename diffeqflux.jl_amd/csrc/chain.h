@@ -63,6 +63,10 @@ struct ChainAdjArgs {
   // `stiles` feature tiles, each [primal column tile][lane][4]
   float* slope; float* curve;
   int stiles;
+  // split BF16: sums of the hidden layers' output gradients over a block's
+  // primal rows, [slot][block][hidden layer][bw] (the bias gradients come from
+  // the FP32 values; the operand rows keep ~16 bits of them)
+  float* bsum; int bw;
   // BacksolveAdjoint: u integrated with lambda (ubs != nullptr)
   float* ubs; float* ubs_new; float* ku; const float* fsaved; int ckpt;
   double* part;
@@ -77,6 +81,7 @@ struct ChainWgradArgs {
   int ntile;                   // 64 x 64 (FP32) or 128 x 128 (split) tiles of all layers
   int tl[MAXL], tw[MAXL];      // first tile of a layer, its tiles along the outputs
   int chunks; int64_t crows;   // row ranges and rows per range
+  const float* bsum; int bw, nblk;  // (split) bias sums per block, as in ChainAdjArgs
   float* part;                 // [chunk][2][ntile][65 x 64 or 129 x 128]
   const Ctl* ctl;
   int mode;

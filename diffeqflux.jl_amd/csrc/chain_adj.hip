@@ -26,6 +26,19 @@
 
 namespace nodehip {
 
+// Sum over the 16 lanes of a row of the wave (in every one of them)
+__device__ __forceinline__ float row16_sum(float x) {
+  auto ror = [](float v, auto n) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + n(),
+                                                                 0xf, 0xf, true));
+  };
+  x += ror(x, std::integral_constant<int, 8>{});
+  x += ror(x, std::integral_constant<int, 4>{});
+  x += ror(x, std::integral_constant<int, 2>{});
+  x += ror(x, std::integral_constant<int, 1>{});
+  return x;
+}
+
 template <class PP, int NT, int NW, bool CNF>
 __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdjArgs a) {
   using T = typename PP::T;
@@ -284,6 +297,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
       const ChainBuf<PP> in{cur, m.pitch, plane}, o{other - cur, m.pitch, plane};
       T* const dr = rows_at(ob, a.ops.d[l - 1], a.ops.w[l]);
       const int dw = a.ops.w[l], act = m.act[l - 1];
+      float* const bsr = a.bsum + (((int64_t)slot * gridDim.x + blockIdx.x) * (L - 1) + l - 1) * a.bw;
       const T* const hr = rows_at(ob, a.ops.h[l], dw);
       const f32x4v* sl = (const f32x4v*)a.slope + (sbase + (int64_t)(l - 1) * a.stiles) * NP * 64 + lane;
       const f32x4v* cv = (const f32x4v*)a.curve + (sbase + (int64_t)(l - 1) * a.stiles) * NP * 64 + lane;
@@ -305,6 +319,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
         const int f = TF * t + 4 * (lane / CW);
         const int i = F32 ? mi : 0;
         if constexpr (!F32) read(t, 0);
+        f32x4v bs4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
           const int r = CW * q + (lane & (CW - 1));
@@ -319,6 +334,12 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
           }
           chain_put4<PP>(o, r, f, v);
           if constexpr (F32) *(f32x4v*)(dr + r * dw + f) = v;
+          else bs4 += v;
+        }
+        if constexpr (!F32) {  // (the 16 lanes of a row of the wave hold a row of the block each)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) bs4[j] = row16_sum(bs4[j]);
+          if ((lane & 15) == 0) *(f32x4v*)(bsr + f) = bs4;
         }
       };
       Side copy = copy_of(cur, ob, a.ops.d[l], a.ops.w[l + 1], m.ktb[l] * ChainK<PP>::KT);
@@ -707,7 +728,7 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
   const int ns = a.mode == SM_STEP ? 7 : 1;
   const int n = (int)((r1 - r0) / GS_K);
   const int rblk = (int)a.rblk, rprim = (int)a.rprim;
-  const bool bias = it == 0;
+  const bool bias = it == 0, lastb = bias && l == a.m.L - 1;
   // this thread's 16-byte pieces: 8 features (fc) of rows tr, tr + 16 of both
   // operands and planes
   const int fc = 8 * (tid & 15), tr = tid >> 4;
@@ -723,6 +744,32 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
       for (int v = 0; v < 16; ++v) ab[x][y][v] = ae[x][y][v] = 0.f;
 #pragma unroll
   for (int v = 0; v < 8; ++v) bb[v] = be[v] = 0.f;
+  // hidden biases: the blocks' sums (blocks that begin in this row range; 16
+  // threads share a feature), all stages' loads in flight at once
+  if (bias && !lastb) {
+    const int hl = a.m.L - 1;
+    const int64_t ss = (int64_t)a.nblk * hl * a.bw;
+    for (int64_t b = (r0 + rblk - 1) / rblk + tr; b * rblk < r1 && b < a.nblk; b += 16) {
+      const float* q = a.bsum + (b * hl + l) * a.bw + ot * GS + fc;
+      f32x4v x[7][2];
+#pragma unroll
+      for (int s = 0; s < 7; ++s)
+        if (s < ns)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) x[s][j] = *(const f32x4v*)(q + wg_slot(a.mode, s, gsel) * ss + 4 * j);
+#pragma unroll
+      for (int s = 0; s < 7; ++s)
+        if (s < ns) {
+          const float cb = a.mode == SM_STEP ? (s < 6 ? chA[6][s] : 0.f) : 1.f;
+          const float ce = a.mode == SM_STEP ? chBT[s] : 0.f;
+#pragma unroll
+          for (int v = 0; v < 8; ++v) {
+            bb[v] += cb * x[s][v >> 2][v & 3];
+            be[v] += ce * x[s][v >> 2][v & 3];
+          }
+        }
+    }
+  }
   const int wr = 64 * (wave >> 1), wc = 64 * (wave & 1);
   const int frow = 8 * (lane >> 5) + ((lane & 15) >> 2);          // first K row of this lane's reads
   const int fcol = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
@@ -752,8 +799,9 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
           *(u32x4*)(o + (p * GS_K + 16 * q) * GS_PITCH) = hv[j][q][p];
           *(u32x4*)(o + OPER + (p * GS_K + 16 * q) * GS_PITCH) = dv[j][q][p];
         }
-        // (a block's rows: a power of two, the primal ones first)
-        if (bias && k < n && (((int)r0 + k * GS_K + tr + 16 * q) & (rblk - 1)) < rprim) {
+        // last layer's bias: lambda, as the products read it (a block's rows: a
+        // power of two, the primal ones first)
+        if (lastb && k < n && (((int)r0 + k * GS_K + tr + 16 * q) & (rblk - 1)) < rprim) {
           const bf16x8 x = __builtin_bit_cast(bf16x8, dv[j][q][0]), y = __builtin_bit_cast(bf16x8, dv[j][q][1]);
 #pragma unroll
           for (int v = 0; v < 8; ++v) gb[v] += (float)x[v] + (float)y[v];

@@ -227,6 +227,7 @@ struct node_handle {
   ChainMuArgs cmu{};
   float* cslope = nullptr;
   float* ccurve = nullptr;
+  float* cbsum = nullptr;      // bias sums per block (split BF16)
   int cstiles = 0;
 
   // profiling (node_prof_enable)
@@ -795,9 +796,10 @@ int chain_alloc(node_handle* h) {
 void chain_adj_free(node_handle* h) {
   dfree(h, h->cslope);
   dfree(h, h->ccurve);
+  dfree(h, h->cbsum);
   dfree(h, h->cmu.w.part);
   dfree(h, h->cops.base);
-  h->cslope = h->ccurve = nullptr;
+  h->cslope = h->ccurve = h->cbsum = nullptr;
   h->cmu = ChainMuArgs{};
   h->cops = ChainOps{};
 }
@@ -828,6 +830,12 @@ int chain_adj_alloc(node_handle* h) {
     w.ntile += w.tw[l] * ((o.w[l] + E - 1) / E);
     u.w0[l] = h->layers[l].w0;
     u.b0[l] = h->layers[l].b0;
+  }
+  if (h->prec != NODE_PREC_FP32) {
+    for (int l = 1; l < h->L; ++l) w.bw = std::max(w.bw, (int)rup(o.w[l], E));
+    w.nblk = (h->B + (int)w.rprim - 1) / (int)w.rprim;
+    if (int rc = dalloc_t(h, &h->cbsum, (size_t)7 * w.nblk * std::max(h->L - 1, 1) * std::max(w.bw, 1) * sizeof(float))) return rc;
+    w.bsum = h->cbsum;
   }
   const int64_t want = (h->prec == NODE_PREC_FP32 ? 512 : 256) / w.ntile;
   // (FP32 batches of up to 32 groups of 16 rows: a range each, the kernel made
@@ -874,6 +882,7 @@ void chain_adjoint(node_handle* h, const AdjBufs& ab, int mode, double* px, doub
   a.dLdout = ab.dLdout;
   a.probe = h->probe;
   a.slope = h->cslope; a.curve = h->ccurve; a.stiles = h->cstiles;
+  a.bsum = h->cbsum; a.bw = h->cmu.w.bw;
   a.ubs = ab.ubs; a.ubs_new = ab.ubs_new; a.ku = ab.ku; a.fsaved = ab.fsaved; a.ckpt = ab.ckpt;
   a.part = px; a.ctl = h->ctl; a.mode = mode;
   launch_chain_adj(h->prec, h->chain_ant, h->cnf, a, chain_adj_grid(h), h->stream);
