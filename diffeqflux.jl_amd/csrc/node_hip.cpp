@@ -761,22 +761,32 @@ ChainOps chain_ops(const node_handle* h, const ChainModel& m, int nt) {
   return o;
 }
 
-int chain_alloc(node_handle* h) {
+// The fused steps' weight copies, when the model fits them.  Without memory for
+// them the handle runs on the GEMM path, which needs none.
+void chain_alloc(node_handle* h) {
   ChainModel m;
-  if (!chain_plan(h, m)) return 0;
+  if (!chain_plan(h, m)) return;
   int nt = chain_tiles(h, m);
   chain_layout(m, nt, h->cnf);
   if (m.lds_bytes > CHAIN_LDS_MAX) chain_layout(m, nt = h->cnf || m.cw == 4 ? 2 : 1, h->cnf);
-  if (m.lds_bytes > CHAIN_LDS_MAX) return 0;
-  if ((h->B + chain_rows(m, nt, h->cnf) - 1) / chain_rows(m, nt, h->cnf) > MAX_PART) return 0;
+  if (m.lds_bytes > CHAIN_LDS_MAX) return;
+  if ((h->B + chain_rows(m, nt, h->cnf) - 1) / chain_rows(m, nt, h->cnf) > MAX_PART) return;
   const int V = h->prec == NODE_PREC_FP32 ? 4 : 8;
   for (int l = 0; l < h->L; ++l) {
     void *f = nullptr, *b = nullptr;
     const size_t lane = (size_t)64 * V * h->esz * h->planes * (m.tf / 16);
-    if (int rc = dalloc(h, &f, lane * m.mtf[l] * m.ktf[l])) return rc;
-    if (int rc = dalloc(h, &b, lane * m.mtb[l] * m.ktb[l])) return rc;
+    const bool none = dalloc(h, &f, lane * m.mtf[l] * m.ktf[l]) || dalloc(h, &b, lane * m.mtb[l] * m.ktb[l]);
     m.Wf[l] = f; m.Wb[l] = b;
     m.bias[l] = h->layers[l].bias;
+    if (none) {
+      for (int i = 0; i <= l; ++i) {
+        dfree(h, (void*)m.Wf[i]);
+        dfree(h, (void*)m.Wb[i]);
+      }
+      h->err.clear();
+      (void)hipGetLastError();
+      return;
+    }
   }
   h->chain = m;
   h->chain_nt = nt;
@@ -790,7 +800,6 @@ int chain_alloc(node_handle* h) {
     h->chain_ant = ant;
     h->chain_adj = am;
   }
-  return 0;
 }
 
 void chain_adj_free(node_handle* h) {
@@ -2177,7 +2186,7 @@ int32_t node_create(const node_desc* desc, node_handle_t** out) {
     if (!rc) rc = dalloc(h, &e, hbt);
     h->H.push_back(a); h->HT.push_back(b); h->S.push_back(c); h->Dl.push_back(d); h->DlT.push_back(e);
   }
-  if (!rc) rc = chain_alloc(h);
+  if (!rc) chain_alloc(h);
   if (!rc) rc = dalloc_t(h, &h->ctl, sizeof(Ctl));
   if (!rc) rc = dalloc_t(h, &h->part, 4 * SEC * sizeof(double));
   if (!rc) rc = dalloc_t(h, &h->scratch, (size_t)h->Bp * h->D * sizeof(float));
