@@ -97,6 +97,12 @@ void launch_chain_adj(int prec, int nt, bool cnf, const ChainAdjArgs& a, int gri
 void launch_chain_wgrad(int prec, const ChainWgradArgs& a, hipStream_t s);
 void launch_chain_mu(const ChainMuArgs& a, int nblk, hipStream_t s);
 
+// Dynamic LDS of a step kernel at most (its static LDS comes on top).  Also what
+// the launches set as the kernels' limit, whatever they need themselves: the
+// limit belongs to the process, and handles of other sizes set it from other
+// threads.
+constexpr int CHAIN_LDS_MAX = 159 * 1024;
+
 // nt: column tiles (of cw) per block (rows per block: cw nt, a flow half)
 int chain_rows(const ChainModel& m, int nt, bool cnf);
 // LDS layout of a model's step kernels (fills the lds_ fields)

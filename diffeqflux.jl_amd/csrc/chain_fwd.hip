@@ -234,7 +234,7 @@ void launch_chain_fwd(int prec, int nt, bool cnf, const ChainFwdArgs& a, int gri
   const size_t lds = a.m.lds_bytes;
   const int nw = a.m.nw;
   auto go = [&](auto kern) {
-    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, CHAIN_LDS_MAX);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * nw), lds, s, a);
   };
   if (prec == 0 && a.m.cw == 4) {

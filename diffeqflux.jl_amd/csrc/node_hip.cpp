@@ -741,7 +741,6 @@ bool chain_plan(node_handle* h, ChainModel& m) {
 }
 
 // Layout of the operand store (without its address).
-constexpr int CHAIN_LDS_MAX = 159 * 1024;  // (static LDS of the kernels aside)
 constexpr int64_t CHAIN_OPS_MAX = int64_t(4) << 30;  // bytes a handle may keep for it
 ChainOps chain_ops(const node_handle* h, const ChainModel& m, int nt) {
   ChainOps o{};

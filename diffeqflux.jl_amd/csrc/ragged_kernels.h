@@ -440,6 +440,11 @@ __global__ void __launch_bounds__(256) k_ragged_fwd(RaggedFwdArgs a) {
   }
 }
 
+// dynamic LDS of a launch at most: all of a CU's.  Set as the kernels' limit by
+// every launch, whatever it needs itself: the limit belongs to the process, and
+// handles of other sizes set it from other threads.
+constexpr int RG_LDS_MAX = 160 * 1024;
+
 // (state tiles, width class): m.rw is at least the state's tiles
 #define RG_DISPATCH(GO)                    \
   do {                                     \
@@ -458,7 +463,7 @@ __global__ void __launch_bounds__(256) k_ragged_fwd(RaggedFwdArgs a) {
 void launch_ragged_fwd(const RaggedFwdArgs& a, int grid, hipStream_t s) {
   const size_t lds = (size_t)a.m.lds_floats * sizeof(float);
   auto go = [&](auto kern) {
-    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, RG_LDS_MAX);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), lds, s, a);
   };
 #define RG_GO(DT, HT) go(k_ragged_fwd<DT, HT>)
@@ -1453,7 +1458,7 @@ void launch_ragged_adj(const RaggedAdjArgs& a, int grid, int waves, hipStream_t 
   const size_t lds = ((size_t)a.m.lds_floats + (size_t)waves * a.m.act_stride +
                       (a.stage_lds ? (size_t)(waves * a.spw + 1) * 8 * a.m.sv : 0)) * sizeof(float);
   auto go = [&](auto kern) {
-    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, RG_LDS_MAX);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * waves), lds, s, a);
   };
 #define RG_GO(DT, HT)                                                          \

@@ -112,3 +112,38 @@ for k in range(n):
 print("made", made)
 """)
     assert out.split()[-1] == str(2 * (len(widths) - 1))
+
+
+def test_lds_limits_do_not_depend_on_the_handle(run):
+    """The dynamic-LDS limit of a kernel is the process's, not a launch's: handles
+    of other sizes, driven by other threads, set the same one."""
+    out = run("""
+import numpy as np
+o = _lib.SolveOpts()
+o.t0, o.t1, o.abstol, o.reltol, o.adaptive, o.maxiters = 0.0, 1.0, 1e-6, 1e-6, 1, 4
+keep = []
+for kind in ("fwd", "ragged"):
+    for hidden in (50, 20, 33):
+        rc, h = create([2, hidden, 2], 3)
+        assert rc == 0
+        p = np.zeros(5 * hidden + 2, np.float32)
+        assert lib.node_set_params(h, p.ctypes.data, p.size) == 0
+        u = np.zeros((3, 2), np.float32)
+        if kind == "fwd":  # (the step counter never moves here)
+            st = _lib.Stats()
+            assert lib.node_forward(h, ctypes.byref(o), u.ctypes.data, None, 0, None, 0,
+                                    ctypes.byref(st)) == -3
+        else:
+            t1, off, ts = np.ones(3), np.arange(4), np.ones(3)
+            res = [np.zeros(s, d) for s, d in (((3, 2), np.float32), (3, np.int32), ((3, 4), np.int32))]
+            rs = _lib.RaggedStats()
+            rc = lib.node_ragged_forward(h, ctypes.byref(o), 3, t1.ctypes.data, u.ctypes.data,
+                                         off.ctypes.data, ts.ctypes.data, *[x.ctypes.data for x in res],
+                                         ctypes.byref(rs))
+            print(kind, rc, lib.node_last_error(h))
+print("sets", counter("stub_attrs").value, "changes", counter("stub_attr_changes").value)
+""")
+    print(out)
+    words = out.split()
+    assert int(words[words.index("sets") + 1]) > 0
+    assert words[-1] == "0"
