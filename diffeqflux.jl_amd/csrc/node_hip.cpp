@@ -1940,10 +1940,6 @@ int ragged_backward_impl(node_handle* h, const float* dLdout, float* dLdu0, doub
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((int64_t)h->n_cu * occ, (waves_all + waves - 1) / waves));
   const int64_t nslots = (int64_t)grid * waves * spw;          // slots: stage blocks, row buffers
   m.act_stride = lds_of(waves, true) <= LDS ? act_tiles * 256 : 0;
-  // stage blocks in LDS too (narrow classes), unless that costs a workgroup per
-  // CU: every stage's operands are written and read a few hundred cycles apart
-  const bool stage_lds = false && m.rw <= 2 && occ * (lds_of(waves, m.act_stride > 0) +
-                                             (int64_t)(waves * spw + 1) * 8 * m.sv * (int64_t)sizeof(float)) <= LDS;
   // start order (a schedule only: each trajectory's arithmetic is the same
   // in any slot).  A wave runs until its last slot's trajectory is done and
   // does one parameter pass per step of every slot, so the waves' sums of
@@ -1976,7 +1972,7 @@ int ragged_backward_impl(node_handle* h, const float* dLdout, float* dLdu0, doub
       grow(h, &b.dLdu0, n * D, b.dLdu0_cap, n * D) ||
       grow(h, &b.rows, n * Pn, b.rows_cap, n * Pn) ||
       grow(h, &b.tmp, nslots * Pn, b.tmp_cap, nslots * Pn) ||
-      (!stage_lds && grow(h, &b.sbuf, (nslots + 1) * 8 * m.sv, b.sbuf_cap, (nslots + 1) * 8 * m.sv)) ||
+      grow(h, &b.sbuf, (nslots + 1) * 8 * m.sv, b.sbuf_cap, (nslots + 1) * 8 * m.sv) ||
       grow(h, &b.dp, P, b.dp_cap, P) ||
       grow(h, &b.part, RG_SUM_CHUNKS * P, b.part_cap, RG_SUM_CHUNKS * P))
     return NODE_ERR_HIP;
@@ -1996,7 +1992,6 @@ int ragged_backward_impl(node_handle* h, const float* dLdout, float* dLdu0, doub
   a.dLdu0 = b.dLdu0; a.dLdp_traj = b.rows; a.mu_tmp = b.tmp; a.sbuf = b.sbuf;
   a.queue = r.ctr; a.retcode = r.ret; a.traj_stats = r.tstats;
   a.order = b.order; a.norder = norder; a.nslots = nslots; a.spw = spw;
-  a.stage_lds = stage_lds;
   a.vjp_bf16 = h->rg_vjp_prec == NODE_PREC_BF16;
   const node_solve_opts* o = &r.opts;
   a.t0 = o->t0;

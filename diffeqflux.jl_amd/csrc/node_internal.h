@@ -396,7 +396,6 @@ struct RaggedAdjArgs {
   const int* order;                   // [norder]
   int64_t norder, nslots;
   int spw;
-  int stage_lds;                      // stage blocks in LDS after act' ((waves * spw + 1) per workgroup), not in sbuf
   int vjp_bf16;                       // VJP products on BF16 operands (NODE_OPT_RAGGED_VJP_PRECISION)
   int* retcode;                       // [n]
   int* traj_stats;                    // [n][4]

@@ -33,10 +33,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // scalar access in flight.  The hot loops go through these instead.
 template <class T> using gp = __attribute__((address_space(1))) T*;
 template <class T> __device__ __forceinline__ gp<T> glb(T* p) { return (gp<T>)p; }
-// The slots' stage blocks are in LDS where they fit, else in global memory.
-template <class T> using lp = __attribute__((address_space(3))) T*;
 __device__ __forceinline__ gp<f32x4> rg_v4(gp<float> p) { return (gp<f32x4>)p; }
-__device__ __forceinline__ lp<f32x4> rg_v4(lp<float> p) { return (lp<f32x4>)p; }
 
 // The kernels are compiled per width class HT (the longest tile dimension of
 // any layer, 1, 2, 4 or 8 tiles), with as many waves per SIMD as the class's
@@ -501,10 +498,10 @@ __device__ __forceinline__ void rg_act4(int act, const f32x4& z, f32x4& y, f32x4
 // or in the block's delta area when m.act_stride is 0) and returns
 // g = W_0^T delta_0 (the input-map derivative is applied by the caller).
 // BF: the products on BF16 operands (rounded to nearest), FP32 accumulation.
-template <bool BF, int HT, class BP>
+template <bool BF, int HT>
 __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, float* act_lds,
                                        const f32x4 (&x0)[HT], const f32x4 (&lam)[HT],
-                                       BP blk, f32x4 (&gout)[HT], int lane) {
+                                       gp<float> blk, f32x4 (&gout)[HT], int lane) {
   const int r = lane & 15, g4 = 4 * (lane >> 4);
   const int L = m.L;
   // one rolled loop body per sweep (the layer's input is copied into place
@@ -721,7 +718,7 @@ __device__ __forceinline__ void rg_vjp(const RaggedModel& m, const float* lds, f
 #pragma unroll
     for (int ot = 0; ot < HT; ++ot) {
       if (HT == 1 || ot < nto) {
-        BP pd = blk + m.sd[l] + 16 * ot + g4;
+        const gp<float> pd = blk + m.sd[l] + 16 * ot + g4;
         const f32x4 ad = m.act_stride ? *(const f32x4*)(act_lds + (m.act_off[l] + ot) * 256 + 4 * lane)
                                       : *rg_v4(pd);
         const f32x4 d = gi[ot] * ad;
@@ -1106,7 +1103,7 @@ __device__ __forceinline__ void rg_tape_u(const RaggedAdjArgs& a, const TapeCurs
   }
 }
 
-template <int DT, bool BF, int HT, bool SL>
+template <int DT, bool BF, int HT>
 __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs a) {
   static_assert(offsetof(RaggedAdjArgs, m) == 0, "the model leads the argument struct");
   extern __shared__ __attribute__((aligned(16))) float rg_lds[];
@@ -1118,18 +1115,9 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
   // stage blocks of the slot's VJPs; the columns past spw never hold a
   // trajectory, and their VJP writes (garbage that stays in its own MFMA
   // column) go to one sink block shared by all of them, which stays in L2
-  using SP = typename std::conditional<SL, lp<float>, gp<float>>::type;
   const int bsv = 8 * m.sv;
-  SP sb0, sb;
-  if constexpr (SL) {
-    const int nw = blockDim.x >> 6, w = threadIdx.x >> 6;
-    lp<float> all = (lp<float>)rg_lds + m.lds_floats + nw * m.act_stride;
-    sb0 = all + w * a.spw * bsv;
-    sb = r < a.spw ? sb0 + r * bsv : all + nw * a.spw * bsv;
-  } else {
-    sb0 = glb(a.sbuf) + wslot0 * bsv;
-    sb = r < a.spw ? sb0 + r * bsv : glb(a.sbuf) + a.nslots * bsv;
-  }
+  const gp<float> sb0 = glb(a.sbuf) + wslot0 * bsv;
+  const gp<float> sb = r < a.spw ? sb0 + r * bsv : glb(a.sbuf) + a.nslots * bsv;
   const int D = a.D;
   const int64_t P = m.P;
   const double nel = (double)D + (double)P;
@@ -1308,9 +1296,7 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
       fll = rg_slot_sum(fll);
     }
     // ---- parameter part, slot by slot with the whole wave
-    // (a wave's LDS accesses are in order: only the compiler has to keep them so)
-    if constexpr (SL) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    else __threadfence_block();
+    __threadfence_block();
     double smu = 0.0, flmu = 0.0;
     for (int s = 0; s < a.spw; ++s) {
       const int ms = __builtin_amdgcn_readlane(mode, s);
@@ -1319,7 +1305,7 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
       const int p0s = __builtin_amdgcn_readlane(p0, s);
       const int mfs = __builtin_amdgcn_readlane(muflip, s);
       const double dts = __shfl(c.dt, s);
-      const SP sbs = sb0 + s * bsv;
+      const gp<const float> sbs = sb0 + s * bsv;
       const gp<float> row = glb(a.dLdp_traj) + (int64_t)trs * m.Pn;
       const gp<float> tmp = glb(a.mu_tmp) + (wslot0 + s) * m.Pn;
       const gp<const float> mu = mfs ? tmp : row;
@@ -1435,7 +1421,6 @@ __global__ void __launch_bounds__(256, rg_waves(HT)) k_ragged_adj(RaggedAdjArgs 
     // flat parameter order (whole wave, converged): the tile-major row is
     // first copied to the slot's row when it is not there already
     if (__any(fin)) {
-      if constexpr (SL) __threadfence_block();   // (the parameter pass's rows, read by other lanes)
       for (int s = 0; s < a.spw; ++s) {
         if (!__builtin_amdgcn_readlane((int)fin, s)) continue;
         const int trs = __builtin_amdgcn_readlane(traj, s);
@@ -1455,22 +1440,15 @@ int ragged_waves(int rw) { return rg_waves(rw); }
 
 // `waves` (1..4) waves of up to RG_SLOTS slots per workgroup
 void launch_ragged_adj(const RaggedAdjArgs& a, int grid, int waves, hipStream_t s) {
-  const size_t lds = ((size_t)a.m.lds_floats + (size_t)waves * a.m.act_stride +
-                      (a.stage_lds ? (size_t)(waves * a.spw + 1) * 8 * a.m.sv : 0)) * sizeof(float);
+  const size_t lds = ((size_t)a.m.lds_floats + (size_t)waves * a.m.act_stride) * sizeof(float);
   auto go = [&](auto kern) {
     (void)hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, RG_LDS_MAX);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * waves), lds, s, a);
   };
 #define RG_GO(DT, HT)                                                          \
   do {                                                                         \
-    constexpr bool SL = false;                                                 \
-    if (SL) {                                                   \
-      if (a.vjp_bf16) go(k_ragged_adj<DT, true, HT, SL>);                      \
-      else go(k_ragged_adj<DT, false, HT, SL>);                                \
-    } else {                                                                   \
-      if (a.vjp_bf16) go(k_ragged_adj<DT, true, HT, false>);                   \
-      else go(k_ragged_adj<DT, false, HT, false>);                             \
-    }                                                                          \
+    if (a.vjp_bf16) go(k_ragged_adj<DT, true, HT>);                            \
+    else go(k_ragged_adj<DT, false, HT>);                                      \
   } while (0)
   RG_DISPATCH(RG_GO);
 #undef RG_GO
