@@ -295,7 +295,10 @@ GemmPlan plan(int rows, int cols, int min_cfg = 0) {
 }
 
 enum ProfRole { PR_FWD_HIDDEN = 0, PR_FWD_STAGE = 1, PR_ADJ_HIDDEN = 2, PR_BWD_DATA = 3,
-                PR_WGRAD = 4, PR_BWD_LAST = 5 };
+                PR_WGRAD = 4, PR_BWD_LAST = 5,
+                // fused steps: "layer" 0; adjoint 0 row pass, 1 weight gradients,
+                // 2 parameter state
+                PR_FUSED_FWD = 6, PR_FUSED_ADJ = 7 };
 
 hipEvent_t prof_event(node_handle* h) {
   if (!h->ev_pool.empty()) {
@@ -893,14 +896,21 @@ void chain_adjoint(node_handle* h, const AdjBufs& ab, int mode, double* px, doub
   a.bsum = h->cbsum; a.bw = h->cmu.w.bw;
   a.ubs = ab.ubs; a.ubs_new = ab.ubs_new; a.ku = ab.ku; a.fsaved = ab.fsaved; a.ckpt = ab.ckpt;
   a.part = px; a.ctl = h->ctl; a.mode = mode;
-  launch_chain_adj(h->prec, h->chain_ant, h->cnf, a, chain_adj_grid(h), h->stream);
+  {
+    ProfScope ps(h, PR_FUSED_ADJ, 0);
+    launch_chain_adj(h->prec, h->chain_ant, h->cnf, a, chain_adj_grid(h), h->stream);
+  }
   ChainMuArgs u = h->cmu;
   u.w.ctl = h->ctl;
   u.w.mode = mode;
   u.mu = h->mu;
   u.g0 = h->gf0;
   u.part = pm;
-  launch_chain_wgrad(h->prec, u.w, h->stream);
+  {
+    ProfScope ps(h, PR_FUSED_ADJ, 1);
+    launch_chain_wgrad(h->prec, u.w, h->stream);
+  }
+  ProfScope ps(h, PR_FUSED_ADJ, 2);
   launch_chain_mu(u, chain_mu_blocks(h), h->stream);
 }
 
@@ -926,6 +936,7 @@ void chain_forward(node_handle* h, int mode, double* part) {
   a.probe = h->probe;
   a.save_times = h->save_times; a.out = h->out_dev;
   a.part = part; a.ctl = h->ctl; a.mode = mode;
+  ProfScope ps(h, PR_FUSED_FWD, 0);
   launch_chain_fwd(h->prec, h->chain_nt, h->cnf, a, chain_grid(h), h->stream);
 }
 

@@ -302,7 +302,8 @@ class Handle:
             self._sense = int(value)
 
     def plans(self):
-        """{(role name, layer): (tile rows, tile cols, ksplit)} currently in use."""
+        """{(role name, layer): (tile rows, tile cols, ksplit)} of the GEMM path (a
+        handle whose solves run as fused steps uses it for ``rhs`` and ``vjp``)."""
         out = {}
         L = len(self.widths) - 1
         for role, name in self.ROLES.items():
@@ -324,10 +325,13 @@ class Handle:
     # ------------------------------------------------------------ profiling
     ROLES = {0: "fwd_hidden", 1: "fwd_stage", 2: "adj_hidden", 3: "bwd_data",
              4: "wgrad", 5: "bwd_last"}
+    # fused steps (no plans): role 6 layer 0, role 7 layers 0..2
+    FUSED_ROLES = {(6, 0): "fused_fwd", (7, 0): "fused_adj", (7, 1): "fused_wgrad",
+                   (7, 2): "fused_mu"}
 
     def prof_enable(self, keys=None):
-        """Record HIP-event timings around GEMM launches.  ``keys``: iterable
-        of (role, layer) or None for all; ``[]`` disables."""
+        """Record HIP-event timings around GEMM and fused step launches.
+        ``keys``: iterable of (role, layer) or None for all; ``[]`` disables."""
         if keys is None:
             mask = (1 << 64) - 1
         else:

@@ -321,17 +321,25 @@ enum { NODE_OPT_GRAPHS = 1, NODE_OPT_GRAPH_ATTEMPTS = 2, NODE_OPT_AUTOTUNE = 3,
        NODE_OPT_TAPE_BUDGET = 7, NODE_OPT_RAGGED_VJP_PRECISION = 8 };
 enum { NODE_SENSE_INTERPOLATING = 0, NODE_SENSE_BACKSOLVE = 1, NODE_SENSE_BACKSOLVE_NOCKPT = 2 };
 int32_t node_set_option(node_handle_t* h, int32_t key, int64_t value);
-/* Tile plan chosen for a GEMM role (roles as for node_prof_enable below) and
- * layer: tile rows x cols and split-K factor. */
+/* Tile plan chosen for a GEMM role (roles 0 to 5 of node_prof_enable below) and
+ * layer: tile rows x cols and split-K factor.  Solves that run as fused steps
+ * (see node_prof_enable) use none; the plans of such a handle are the ones its
+ * GEMM path (node_rhs, node_vjp, a tape budget) has or would start from. */
 int32_t node_get_plan(node_handle_t* h, int32_t role, int32_t layer, int32_t* tile_rows,
                       int32_t* tile_cols, int32_t* ksplit);
 
 /* Profiling hook (no counterpart in the reference; for measurement tools).
- * Records a HIP-event pair on the handle's stream around every GEMM launch
- * whose key (role * 8 + layer) has its bit set in key_mask; 0 disables.
+ * Records a HIP-event pair on the handle's stream around every GEMM or fused
+ * step launch whose key (role * 8 + layer) has its bit set in key_mask; 0
+ * disables.
  * Roles: 0 forward hidden layer, 1 forward last layer (stage epilogue),
  * 2 adjoint forward recompute, 3 adjoint data gradient, 4 weight gradient,
- * 5 adjoint layer-1 data gradient (stage epilogue). */
+ * 5 adjoint layer-1 data gradient (stage epilogue).  Models that fit a
+ * workgroup (state <= 64, a flow 32, widths <= 1024, a flow 512, <= 700k
+ * weights; FP32 or BF16X3; no exact trace, regularisers, tape budget or reduced
+ * weight-gradient precision) solve in fused steps instead: 6 (layer 0) a
+ * forward step attempt, 7 an adjoint one (layer 0 row pass, 1 weight gradients,
+ * 2 parameter state). */
 int32_t node_prof_enable(node_handle_t* h, uint64_t key_mask);
 /* Per-launch durations (ms) and keys recorded since enabling; clears them. */
 int32_t node_prof_collect(node_handle_t* h, int32_t* keys, float* ms, int64_t cap,
