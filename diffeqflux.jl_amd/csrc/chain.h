@@ -34,7 +34,6 @@ struct ChainFwdArgs {
   float* tape; int64_t ent, sv;
   const float* probe;          // flow: [B][dm]
   const double* save_times; float* out;
-  float* plain;                // SM_PLAIN: input state in tape[0..], output here
   double* part;
   const Ctl* ctl;
   int mode;

@@ -303,7 +303,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
       const f32x4v* cv = (const f32x4v*)a.curve + (sbase + (int64_t)(l - 1) * a.stiles) * NP * 64 + lane;
       // FP32 blocks read act' ahead of the products, the split ones have no
       // registers left for it
-      constexpr int ME = F32 ? (INPLACE && NW == 4 ? 8 : 4) : 1;
+      constexpr int ME = F32 ? (INPLACE ? chain_inplace<NW>() : 4) : 1;
       f32x4v sd[ME][NP], c2[CNF ? ME : 1][NP];
       auto read = [&](int t, int mi) {
 #pragma unroll

@@ -122,12 +122,9 @@ template <class PP> struct ChainBuf {
   }
 };
 
-// acc[m][n] += W tiles (first tile t0, MT of them, K tiles [k0, k1)) x columns.
-// The fragments of PF K tiles are in flight (ring in registers, loads
-// unconditional: the index is clamped instead).  side.step(): a piece of other
-// work per K tile.
-// The same on 64 x 4 tiles: a lane holds one feature's 16 K values (four
-// vectors) and reads its row's, in the order that the 16 x 16 steps take them.
+// chain_mma (below) on 64 x 4 tiles: a lane holds one feature's 16 K values
+// (four vectors) and reads its row's, in the order that the 16 x 16 steps take
+// them.
 template <int NT, int MT, int PF>
 __device__ __forceinline__ void chain_mma4(f32x4v (&acc)[MT][NT], const void* __restrict__ W, int t0,
                                            int tlast, int kt, int k0, int k1, const ChainBuf<PF32S>& in,
@@ -177,6 +174,10 @@ __device__ __forceinline__ void chain_mma4(f32x4v (&acc)[MT][NT], const void* __
     if (k + j < k1) step(a[j], k + j, false);
 }
 
+// acc[m][n] += W tiles (first tile t0, MT of them, K tiles [k0, k1)) x columns.
+// The fragments of PF K tiles are in flight (ring in registers, loads
+// unconditional: the index is clamped instead).  side.step(): a piece of other
+// work per K tile.
 template <class PP, int NT, int MT, int PF, class Side>
 __device__ __forceinline__ void chain_mma(f32x4v (&acc)[MT][NT], const void* __restrict__ W, int t0,
                                           int tlast, int kt, int k0, int k1, const ChainBuf<PP>& in,
@@ -317,10 +318,15 @@ __device__ __forceinline__ void chain_chunk(const void* W, int t0, int tlast, in
     if (t0 + m <= tlast) epi(t0 + m, m, acc[m]);
 }
 
+// Tiles of a wave in place: four-wave blocks have layers narrower than 128 (under
+// 8 tiles), eight-wave ones up to 512 (32 tiles), by chain_plan's limits
+template <int NW> constexpr int chain_inplace() { return NW == 4 ? 2 : 4; }
+
 // One wide layer (mt output tiles over the waves): epi(tile, acc[NT]) for
 // every tile.  INPLACE: the outputs may overwrite the inputs (a wave holds all
-// its tiles' accumulators until the barrier; mt <= 4 NW); else chunks of at
-// most four tiles and the output goes to another buffer.  Ends with a barrier.
+// its tiles' accumulators until the barrier: chain_inplace<NW> of them at most);
+// else chunks of at most four tiles and the output goes to another buffer.  Ends
+// with a barrier.
 template <class PP, int NT, int NW, bool INPLACE, class Side, class Pro, class Epi>
 __device__ __forceinline__ void chain_layer(const void* W, int mt, int kt, const ChainBuf<PP>& in,
                                             int wave, int lane, Side& side, Pro&& pro,
@@ -331,15 +337,7 @@ __device__ __forceinline__ void chain_layer(const void* W, int mt, int kt, const
   if constexpr (INPLACE) {
     // (a wave without tiles computes the last one again and drops it)
     const int tl = last < mt - 1 ? last : mt - 1;
-    // (mt <= 32; the eight-tile chunk would cost an eight-wave block spills)
-    if constexpr (NW == 4) {
-      if (per > 4) {
-        chain_chunk<PP, NT, 8>(W, t, tl, kt, in, lane, true, side, pro, epi);
-        chain_barrier();
-        return;
-      }
-    }
-    if (per > 2) chain_chunk<PP, NT, 4>(W, t, tl, kt, in, lane, true, side, pro, epi);
+    if (chain_inplace<NW>() > 2 && per > 2) chain_chunk<PP, NT, chain_inplace<NW>()>(W, t, tl, kt, in, lane, true, side, pro, epi);
     else if (per > 1) chain_chunk<PP, NT, 2>(W, t, tl, kt, in, lane, true, side, pro, epi);
     else chain_chunk<PP, NT, 1>(W, t, tl, kt, in, lane, true, side, pro, epi);
   } else {

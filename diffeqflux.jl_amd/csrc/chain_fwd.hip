@@ -195,22 +195,25 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
 #pragma unroll
         for (int j = 1; j < 6; ++j) k[j][e] = j == s ? kv : k[j][e];
         kl[e] = kv;
-      } else if (mode == SM_PLAIN) {
-        (a.plain + e0)[i] = kv;
-      } else {
+      } else if (mode == SM_INIT_F0) {
+        (ent + a.sv)[i] = kv;
         const float sk = atol + fabsf(u[e]) * rtol;
-        const float d = mode == SM_INIT_F0 ? kv : kv - k[0][e];
-        if (mode == SM_INIT_F0) (ent + a.sv)[i] = kv;
+        if (live) {
+          const double q = (double)(kv / sk);
+          sum += q * q;
+        }
+      } else {
+        const float sk = atol + fabsf(u[e]) * rtol, d = kv - k[0][e];
         if (live) {
           const double q = (double)(d / sk);
           sum += q * q;
-          if (mode == SM_INIT_F1 && d != 0.f) flag = 1.0;
+          if (d != 0.f) flag = 1.0;
         }
       }
     }
     chain_barrier();  // (in place: the partial products lie over the next stage's inputs)
   }
-  if (a.part) block_reduce_store(sum, flag, a.part, blockIdx.x);
+  block_reduce_store(sum, flag, a.part, blockIdx.x);
 }
 
 void chain_layout(ChainModel& m, int nt, bool cnf) {
