@@ -11,13 +11,14 @@
 // GEMM, stage, fold and norm (12 per VJP) spent most of their time in launches,
 // drains and partial sums through memory.
 //
-// A step attempt of k_chain_adj, and the training step it belongs to before and
-// now:
-//   64-256-256-64 FP32, 4096 rows   112 us   17.5 -> 6.2 ms
-//   the same, 333 rows              102 us   12.6 -> 4.3 ms
-//   2-50-2 FP32, one trajectory      27 us   14.6 -> 2.9 ms
+// A step attempt of k_chain_adj (median of the launches with work), and the
+// training step it belongs to before and now:
+//   32-256-256-32 FP32, 4096 rows   135 us   17.6 -> 6.2 ms
+//   the same, 333 rows              111 us   12.5 -> 4.3 ms
+//   2-50-2 FP32, one trajectory      31 us   13.6 -> 3.8 ms (host-bound: 2.5 to
+//                                            4 ms from machine to machine)
 //   17-512-512-16 flow, split BF16,
-//   8192 rows                       490 us   39.5 -> 14.3 ms
+//   8192 rows                       568 us   38.8 -> 13.7 ms
 // Bound by the matrix pipe and the phases around it: of a 16-row block's 43,000
 // cycles per stage (256-wide layers) 20,000 are MFMA, the rest layer
 // prologues, epilogues and barriers that two waves per SIMD only half hide; a
@@ -467,9 +468,9 @@ __device__ __forceinline__ bool wg_block(const ChainWgradArgs& a, int& tile, int
 // the operand of MFMA tile v, whose features are 4 (l % 16) + v.  32 B of
 // operands per lane feed 16 MFMAs (512 cycles), so neither LDS nor a second
 // read of the rows is needed; the four waves' sums meet in LDS at the end.
-// 64-256-256-64, 4096 rows: 60 us for the 5.6 GFLOP of a step's seven stages,
-// 94 TFLOP/s (a large FP32 product of the library: 129); one GEMM, one fold per
-// stage before.
+// 32-256-256-32, 4096 rows: 67 us for the 4.7 GFLOP of a step's seven stages,
+// 70 TFLOP/s, or 84 with the 64-wide tiles' padding of the outer layers (a large
+// FP32 product of the library: 129); one GEMM, one fold per stage before.
 constexpr int GT = 64;
 __global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
   const Ctl* ctl = a.ctl;
@@ -595,7 +596,7 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
 // FP32, ranges of 16 rows (small batches).  With one group of rows per range
 // the kernel above is a chain: a memory latency per stage and a sum over waves
 // in four LDS rounds (12.7 us for one trajectory's 2 tiles, 21 us for 333 rows
-// of 64-256-256-64; this one 6.4 and 13.9 us).
+// of 32-256-256-32; this one 6.5 and 13.9 us).
 // Here all stages' operands are requested at once, and a wave takes all 16 rows
 // of a quarter of the tile (inputs 4 i + wave), so nothing is summed across
 // waves.
@@ -700,8 +701,11 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32s(ChainWgradArgs a) {
 // long again as the products).  Loads are unconditional: rows
 // are padded to whole groups with zeros, columns past a layer's width repeat
 // the last ones and end in tile entries nobody reads.  17-512-512-16 flow, 8192
-// rows: 575 -> 360 us per step attempt, 39% of the matrix pipe (a large split
-// product of the library's rate would be 52%), HBM reads 2.4 -> 0.65 GB.
+// rows: 575 -> 384 us per step attempt, 39% of the matrix pipe (a large split
+// product of the library's rate would be 52%), HBM reads 2.4 -> 0.65 GB.  The
+// hidden layers' bias gradients are sums of the blocks' FP32 column sums, which
+// the row pass leaves: the planes hold ~16 bits of a term (7.6e-6 off where the
+// FP32 values are exact).
 constexpr int GS = 128, GS_PITCH = 160, GS_K = 32;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4;

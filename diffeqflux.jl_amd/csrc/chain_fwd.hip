@@ -7,11 +7,11 @@
 // chain of the wide layers (FP32) or by the weights' way from L2 (split BF16);
 // it replaces eight kernels per right-hand side whose launches and drains cost
 // more than their work at these sizes.  Six stages in one launch:
-//   64-256-256-64 FP32, 4096 rows 39 us, 333 or 1000 rows 31 us (16-row blocks
-//   36; a 1000-row solve 2.67 -> 0.95 ms in all)
-//   17-512-512-16 flow, split BF16, 8192 rows 185 us a step (31 us per
-//   right-hand side against 135 us; the density solve 12.2 -> 3.1 ms)
-//   2-50-2, one trajectory 11 us, of which half is instruction issue of the
+//   32-256-256-32 FP32, 4096 rows 65 us, 333 or 1000 rows 52 us (16-row blocks
+//   60; a 1000-row solve 2.69 -> 0.95 ms in all)
+//   17-512-512-16 flow, split BF16, 8192 rows 215 us a step (36 us per
+//   right-hand side against 135 us; the density solve 12.0 -> 3.0 ms)
+//   2-50-2, one trajectory 17 us, of which half is instruction issue of the
 //   stage inputs and epilogues: one wave per SIMD, nothing to overlap
 #include <algorithm>
 

@@ -708,11 +708,12 @@ bool chain_plan(node_handle* h, ChainModel& m) {
   for (int l = 0; l < h->L; ++l) mid = std::max(mid, std::min(h->layers[l].in, h->layers[l].out));
   // 64 x 4 tiles, blocks of 8 rows: less matrix time per block (a chain of one
   // MFMA per K step, ~17 cycles each, against two waves' shares of 32), worth it
-  // where a layer is wide both ways and the blocks fit the chip at once.  Fixed
-  // steps, forward / adjoint us at 300 rows, 16-row against 8-row blocks:
-  // 64-128-128-64 955 / 1921 and 1024 / 2067, 64-160-160-64 1257 / 2657 and
-  // 1132 / 2360, 64-256-256-64 1590 / 3366 and 1334 / 2919, 64-512-512-64
-  // 3678 / 7928 and 2422 / 5837; 8-1024-8 1028 / 2595 and 1106 / 2434.
+  // where a layer is wide both ways and the blocks fit the chip at once.  Times
+  // of 8-row against 16-row blocks, forward / adjoint of 16 fixed steps, 300 to
+  // 2048 rows: 64-128-128-64 1.07-1.10 / 1.07, 64-144-144-64 0.99-1.03 / 1.00,
+  // 64-160-160-64 0.90-0.94 / 0.90, 32-256-256-32 0.88 / 0.89-0.91, 64-512-512-64
+  // 0.66-0.72 / 0.73-0.79, 32-800-800-32 0.64-0.67 / 0.75-0.82.  At 2049 rows a
+  // CU gets a second block: 1.22-1.82 / 1.24-1.66 over the same models.
   const bool small = h->prec == NODE_PREC_FP32 && !h->cnf && mid > 128 && h->B <= 8 * 256;
   m.cw = small ? 4 : 16;
   m.tf = small ? 64 : 16;
@@ -730,9 +731,14 @@ bool chain_plan(node_handle* h, ChainModel& m) {
     if (l < h->L - 1) wide = std::max(wide, m.mtf[l] * m.tf);
   }
   if (wide > 1024 || (h->cnf && wide > 512)) return false;
-  // Past ~700k weights a block's way through them (2.2M: ~100 us per
-  // right-hand side, whatever the batch) costs what the GEMM path does at
-  // 4096 rows (split BF16) and twice that at 1000 (FP32: 116 against ~57).
+  // Up to 700k weights a solve and its adjoint take, against the GEMM path, at 1
+  // to 16,384 rows and both precisions (10 fixed steps): 64-512-512-64 (0.33M)
+  // 0.48-0.87 / 0.49-0.80, 64-500-500-500-64 (0.56M) 0.49-0.83 / 0.55-0.82,
+  // 32-800-800-32 (0.69M) 0.50-0.88 / 0.61-0.91, a 17-512-512-512-16 flow (0.54M)
+  // 0.29-0.71 / 0.41-0.78; at 32,768 and 65,536 rows (FP32) 0.93-1.01 / 0.83-1.00.
+  // Past it a block's way through the weights (2.2M: ~100 us per right-hand side,
+  // whatever the batch) costs what the GEMM path does at 4096 rows (split BF16)
+  // and twice that at 1000 (FP32: 116 against ~57).
   int64_t weights = 0;
   for (int l = 0; l < h->L; ++l) weights += (int64_t)h->layers[l].in * h->layers[l].out;
   if (weights > 700000) return false;

@@ -17,8 +17,8 @@ from oracle.mlp import MLP
 
 pytestmark = pytest.mark.gpu
 
-CLASSES = [  # (repeated 700 times; the last two so often that the stage data leaves
-             # LDS, and that slots take trajectories from the queue)
+CLASSES = [  # (repeated 700 times; the last two so often that slots take trajectories
+             # from the queue)
     ([3, 13, 3], ["tanh", "identity"]),
     ([2, 16, 16, 9, 2], ["tanh", "softplus", "sigmoid", "identity"]),
     ([9, 17, 31, 9], ["softplus", "tanh", "identity"]),
