@@ -402,6 +402,21 @@ __device__ __forceinline__ float chain_sum(const float* part, int mt, int kt, in
   return v;
 }
 
+// FP32: zeros where the four stored features at position f of tile t lie past the
+// layer's n.  Their weights are zero, but 0 x inf is not: a hidden value that
+// overflows would come back as NaN through the padding (the saturating layer
+// behind it is finite).  Split BF16 has no infinities to keep apart: their lo
+// plane is NaN.
+template <class PP> __device__ __forceinline__ f32x4v chain_keep(f32x4v v, int t, int f, int n) {
+  if constexpr (sizeof(typename PP::T) == 4) {
+    if (__builtin_amdgcn_readfirstlane(ChainK<PP>::TF * (t + 1)) > n) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = chain_feat(f + j) < n ? v[j] : 0.f;
+    }
+  }
+  return v;
+}
+
 // Runge-Kutta stage values u + dt sum_j A[s][j] k_j: the latest stage first,
 // the others in order, the first stage's product with dt * A (the GEMM path's
 // stage kernels' order; fused multiply-adds in words, since the compiler moves

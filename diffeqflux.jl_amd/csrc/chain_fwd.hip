@@ -148,16 +148,16 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
     for (int l = 0; l < L - 1; ++l) {
       const ChainBuf<PP> in{cur, m.pitch, plane}, o{other - cur, m.pitch, plane};
       const float* bias = lbias + l * m.wmax;
-      const int act = m.act[l];
+      const int act = m.act[l], nout = m.out[l];
       auto epi = [&](int t, int, f32x4v (&acc)[NT]) {
         const int f = TF * t + 4 * (lane / CW), r = lane & (CW - 1);
         const f32x4v bv = *(const f32x4v*)(bias + f);
 #pragma unroll
         for (int q = 0; q < (CNF ? NT / 2 : NT); ++q) {
           const f32x4v z = acc[q] + bv, y = act_f4(act, z);
-          chain_put4<PP>(o, CW * q + r, f, y);
+          chain_put4<PP>(o, CW * q + r, f, chain_keep<PP>(y, t, f, nout));
           if constexpr (CNF)
-            chain_put4<PP>(o, R + CW * q + r, f, acc[q + NT / 2] * act_d4(act, z, y));
+            chain_put4<PP>(o, R + CW * q + r, f, chain_keep<PP>(acc[q + NT / 2] * act_d4(act, z, y), t, f, nout));
         }
       };
       chain_layer<PP, NT, NW, INPLACE>(m.Wf[l], m.mtf[l], m.ktf[l], in, wave, lane, none,
