@@ -230,13 +230,13 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
           const int r = CW * q + (lane & (CW - 1));
-          const f32x4v z = acc[q] + bv, y = chain_keep<PP>(act_f4(act, z), t, f, nout);
+          const f32x4v z = chain_keep<PP>(acc[q] + bv, t, f, nout), y = act_f4(act, z);
           chain_put4<PP>(o, r, f, y);
           if constexpr (F32) *(f32x4v*)(hr + r * hw + f) = y;
           else sl[(t * NP + q) * 64] = act_d4(act, z, y);
           if constexpr (CNF) {
             const f32x4v d = act_d4(act, z, y);
-            const f32x4v tv = chain_keep<PP>(acc[q + NP] * d, t, f, nout);
+            const f32x4v tv = acc[q + NP] * d;
             chain_put4<PP>(o, R + r, f, tv);
             if constexpr (F32) *(f32x4v*)(hr + (R + r) * hw + f) = tv;
             // act'' adot in closed form (act' adot = t)
@@ -297,7 +297,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
     for (int l = ll; l >= 1; --l) {
       const ChainBuf<PP> in{cur, m.pitch, plane}, o{other - cur, m.pitch, plane};
       T* const dr = rows_at(ob, a.ops.d[l - 1], a.ops.w[l]);
-      const int dw = a.ops.w[l], act = m.act[l - 1], nin = m.in[l];
+      const int dw = a.ops.w[l], act = m.act[l - 1];
       float* const bsr = a.bsum + (((int64_t)slot * gridDim.x + blockIdx.x) * (L - 1) + l - 1) * a.bw;
       const T* const hr = rows_at(ob, a.ops.h[l], dw);
       const f32x4v* sl = (const f32x4v*)a.slope + (sbase + (int64_t)(l - 1) * a.stiles) * NP * 64 + lane;
@@ -329,11 +329,10 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_adj(ChainAdj
           f32x4v v = acc[q] * d;
           if constexpr (CNF) {
             v += acc[q + NP] * c2[i][q];
-            const f32x4v tv = chain_keep<PP>(acc[q + NP] * d, t, f, nin);
+            const f32x4v tv = acc[q + NP] * d;
             chain_put4<PP>(o, R + r, f, tv);
             if constexpr (F32) *(f32x4v*)(dr + (R + r) * dw + f) = tv;
           }
-          v = chain_keep<PP>(v, t, f, nin);
           chain_put4<PP>(o, r, f, v);
           if constexpr (F32) *(f32x4v*)(dr + r * dw + f) = v;
           else bs4 += v;

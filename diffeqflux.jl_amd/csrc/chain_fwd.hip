@@ -154,10 +154,10 @@ __global__ void __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) k_chain_fwd(ChainFwd
         const f32x4v bv = *(const f32x4v*)(bias + f);
 #pragma unroll
         for (int q = 0; q < (CNF ? NT / 2 : NT); ++q) {
-          const f32x4v z = acc[q] + bv, y = act_f4(act, z);
-          chain_put4<PP>(o, CW * q + r, f, chain_keep<PP>(y, t, f, nout));
+          const f32x4v z = chain_keep<PP>(acc[q] + bv, t, f, nout), y = act_f4(act, z);
+          chain_put4<PP>(o, CW * q + r, f, y);
           if constexpr (CNF)
-            chain_put4<PP>(o, R + CW * q + r, f, chain_keep<PP>(acc[q + NT / 2] * act_d4(act, z, y), t, f, nout));
+            chain_put4<PP>(o, R + CW * q + r, f, acc[q + NT / 2] * act_d4(act, z, y));
         }
       };
       chain_layer<PP, NT, NW, INPLACE>(m.Wf[l], m.mtf[l], m.ktf[l], in, wave, lane, none,
