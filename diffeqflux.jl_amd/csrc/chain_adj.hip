@@ -441,6 +441,10 @@ __device__ __forceinline__ int wg_slot(int mode, int s, int gsel) {
   return s == 0 ? gsel : s == 6 ? (gsel ^ 1) : s + 1;
 }
 
+// Whether stage s has a weight in the quadrature (the last one has none; it is
+// left out rather than multiplied by 0: its operands may have overflowed)
+__device__ __forceinline__ bool wg_quad(int mode, int s) { return mode != SM_STEP || s < 6; }
+
 // tile index -> layer, tile row (inputs) and column (outputs)
 __device__ __forceinline__ int wg_tile(const ChainWgradArgs& a, int tile, int& it, int& ot) {
   int l = 0;
@@ -539,12 +543,14 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32(ChainWgradArgs a) {
 #pragma unroll
     for (int x = 0; x < 4; ++x)
 #pragma unroll
-      for (int y = 0; y < 4; ++y) {
-        ab[x][y] += cb * g[x][y];
-        ae[x][y] += ce * g[x][y];
-      }
-    bb += cb * gb;
+      for (int y = 0; y < 4; ++y) ae[x][y] += ce * g[x][y];
     be += ce * gb;
+    if (!wg_quad(a.mode, s)) break;                // (the last stage)
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int y = 0; y < 4; ++y) ab[x][y] += cb * g[x][y];
+    bb += cb * gb;
   }
   // sum over the waves, two halves of the tile at a time; acc element (p, q, v)
   // of lane l is input 4 (4 (l / 16) + v) + p, output 4 (l % 16) + q
@@ -632,7 +638,7 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32s(ChainWgradArgs a) {
       dv[s][j] = *(const f32x4v*)(d + 4 * j * wo);
     }
   };
-  auto fold = [&](int s, float cb, float ce) {
+  auto fold = [&](int s, bool quad, float cb, float ce) {
     f32x4v gb = zero;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -642,10 +648,10 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32s(ChainWgradArgs a) {
       f32x4v g = zero;
 #pragma unroll
       for (int j = 0; j < 4; ++j) g = __builtin_amdgcn_mfma_f32_16x16x4f32(hv[s][j], dv[s][j][q], g, 0, 0, 0);
-      ab[q] += cb * g;
+      if (quad) ab[q] += cb * g;
       ae[q] += ce * g;
     }
-    bb += cb * gb;
+    if (quad) bb += cb * gb;
     be += ce * gb;
   };
   load(0);
@@ -653,9 +659,9 @@ __global__ void __launch_bounds__(256, 2) k_chain_wgrad32s(ChainWgradArgs a) {
 #pragma unroll
     for (int s = 1; s < 7; ++s) load(s);
 #pragma unroll
-    for (int s = 0; s < 7; ++s) fold(s, s < 6 ? chA[6][s] : 0.f, chBT[s]);
+    for (int s = 0; s < 7; ++s) fold(s, s < 6, chA[6][s < 6 ? s : 0], chBT[s]);
   } else {
-    fold(0, 1.f, 0.f);
+    fold(0, true, 1.f, 0.f);
   }
   // acc element (q, v) of lane l: input 4 (4 (l / 16) + v) + wave, output 4 (l % 16) + q
   const int64_t tsz = GT * (GT + 1);
@@ -768,7 +774,7 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
           const float ce = a.mode == SM_STEP ? chBT[s] : 0.f;
 #pragma unroll
           for (int v = 0; v < 8; ++v) {
-            bb[v] += cb * x[s][v >> 2][v & 3];
+            if (wg_quad(a.mode, s)) bb[v] += cb * x[s][v >> 2][v & 3];
             be[v] += ce * x[s][v >> 2][v & 3];
           }
         }
@@ -874,12 +880,16 @@ __global__ void __launch_bounds__(256, 1) k_chain_wgrad16(ChainWgradArgs a) {
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
-      for (int y = 0; y < 2; ++y) {
-        ab[x][y] += cb * g[x][y];
-        ae[x][y] += ce * g[x][y];
-      }
+      for (int y = 0; y < 2; ++y) ae[x][y] += ce * g[x][y];
 #pragma unroll
-    for (int v = 0; v < 8; ++v) { bb[v] += cb * gb[v]; be[v] += ce * gb[v]; }
+    for (int v = 0; v < 8; ++v) be[v] += ce * gb[v];
+    if (!wg_quad(a.mode, s)) break;                // (the last stage)
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int y = 0; y < 2; ++y) ab[x][y] += cb * g[x][y];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) bb[v] += cb * gb[v];
   }
   const int64_t tsz = GS * (GS + 1);
   float* out = a.part + ((int64_t)chunk * 2 * a.ntile + tile) * tsz;

@@ -44,3 +44,30 @@ def test_overflow_behind_a_saturating_layer(hidden, act):
     last = -(hidden[1] * 2 + 2)
     assert sb["retcode"] == 1 and rel(du0, gu) < 2e-5
     assert rel(dp[last:], gp[last:]) < 1e-4  # (the second layer's holds inf * 0)
+
+
+@pytest.mark.parametrize("prec,tol", [("fp32", 1e-4), ("bf16x3", 5e-4)])
+@pytest.mark.parametrize("B", [1, 600, 4097])
+@pytest.mark.parametrize("hidden", [[], [4]])
+def test_last_stage_outside_the_quadrature(hidden, B, prec, tol):
+    """lambda overflows in the last stage of a step, which has no weight in the
+    parameter gradient: lambda(t0) is inf, the gradient is the oracle's (bounds
+    of the fused step tests).  One step of z = w dt = 15: the stage values grow
+    by up to 900, the new state by 25442."""
+    from diffeqflux_hip import Handle
+    widths, acts = [1, *hidden, 1], ["identity"] * (len(hidden) + 1)
+    m = MLP(widths, acts)
+    p = np.float32([2.0**-7, 0] if not hidden else [2.0**-3] * 4 + [0] * 4 + [2.0**-6] * 4 + [0])
+    u0 = np.full((B, 1), 1e-6, np.float32)
+    kw, t1 = dict(adaptive=False, dt=1920.0), 1920.0
+    h = Handle(widths, acts, 0, prec, B)
+    h.set_params(p)
+    h.forward(u0, Handle.make_opts(0.0, t1, **kw))
+    ref = OA.forward(m, p.astype(np.float64), u0.astype(np.float64), 0.0, t1, saveat=[0.0, t1], **kw)
+    cot = np.zeros((2, B, 1), np.float32)
+    cot[1] = 5e34 / B
+    cot[1, 0] = 5e34
+    du0, dp, st = h.backward(cot)
+    gu, gp, _ = OA.backward(m, p.astype(np.float64), ref, list(cot.astype(np.float64)), **kw)
+    assert st["retcode"] == 1 and gu[0, 0] > 1e39 and np.isposinf(du0[0, 0])
+    assert np.linalg.norm(dp - gp) < tol * np.linalg.norm(gp)
