@@ -15,8 +15,8 @@
 // training step it belongs to before and now:
 //   32-256-256-32 FP32, 4096 rows   135 us   17.6 -> 6.2 ms
 //   the same, 333 rows              111 us   12.5 -> 4.3 ms
-//   2-50-2 FP32, one trajectory      31 us   13.6 -> 3.8 ms (host-bound: 2.5 to
-//                                            4 ms from machine to machine)
+//   2-50-2 FP32, one trajectory      31 us   13.6 -> 3.8 ms (29 to 66 steps by
+//                                            inputs: 2.5 to 5 ms)
 //   17-512-512-16 flow, split BF16,
 //   8192 rows                       568 us   38.8 -> 13.7 ms
 // Bound by the matrix pipe and the phases around it: of a 16-row block's 43,000
